@@ -162,6 +162,13 @@ AV1M_HD constexpr int dscan_off(int t) {
          : t == TX_8X16 ? 1424 : t == TX_16X8 ? 1552 : t == TX_16X32 ? 1680 : t == TX_32X16 ? 2192 : t == TX_4X16 ? 2704
          : t == TX_16X4 ? 2768 : t == TX_8X32 ? 2832 : 3088;
 }
+// the same for the sizes of at most 256 coefficients, whose scan indices fit a byte (the closed loop keeps these in LDS)
+constexpr int SCAN8_TOTAL = 1296;
+AV1M_HD constexpr bool scan8_has(int t) { return t != TX_32X32 && t != TX_64X64 && t != TX_16X32 && t != TX_32X16 && t != TX_32X64 && t != TX_64X32 && t != TX_16X64 && t != TX_64X16; }
+AV1M_HD constexpr int scan8_off(int t) {
+    return t == TX_4X4 ? 0 : t == TX_8X8 ? 16 : t == TX_16X16 ? 80 : t == TX_4X8 ? 336 : t == TX_8X4 ? 368 : t == TX_8X16 ? 400
+         : t == TX_16X8 ? 528 : t == TX_4X16 ? 656 : t == TX_16X4 ? 720 : t == TX_8X32 ? 784 : 1040;
+}
 // the coefficient context of tx size t (get_tx_size_context)
 AV1M_HD constexpr int txsz_ctx_of(int t) { return (av1t::Tx_Size_Sqr[t] + av1t::Tx_Size_Sqr_Up[t] + 1) >> 1; }
 
@@ -634,6 +641,7 @@ struct DevTables {
     float lamS[2][256];          // sqrt(lambda): the screening weight with satdLambda 1
     CostTab cost[4];
     uint16_t iscan[DSCAN_TOTAL]; // inverse default scans: iscan[dscan_off(t) + position] = scan index
+    uint8_t scan8[SCAN8_TOTAL], iscan8[SCAN8_TOTAL];   // default scans and their inverses at scan8_off(t), a byte per entry
 };
 
 // tunables of the search (the reference's GpParams, gp.h:29-68, for the knobs this core implements)

@@ -21,6 +21,9 @@ constexpr int tx_of(int W, int H) {
          : (W == 8 && H == 32) ? TX_8X32 : (W == 32 && H == 8) ? TX_32X8 : (W == 16 && H == 64) ? TX_16X64 : TX_64X16;
 }
 
+// global memory seen through its own address space: a generic pointer read back from LDS would go through flat
+// instructions, which wait on the LDS counter too
+template <typename T> using glb = __attribute__((address_space(1))) T;
 // LDS view of a type: accesses through it compile to ds_* instructions, also inside functions the compiler keeps out
 // of line (where a plain pointer would lose its address space and go through flat instructions)
 template <typename T> using lds = __attribute__((address_space(3))) T;
@@ -248,13 +251,12 @@ __device__ EvalOut grp_eval(RP res, FP tmp, QP q, const E &e, const TT &T) {
     {
         constexpr int OCF = W * TH / GW, OC = OCF < 1 ? 1 : OCF > 8 ? 8 : OCF, NI = W * (TH / OC);
         const auto *FcT = T.fwdT + T.fwdOff[ck][LH];
-        const auto *Fc = T.fwd + T.fwdOff[ck][LH];
         for (int it = lane; it < NI; it += GW) {
             const int j = it % W, i0 = (it / W) * OC, jj = flr ? W - 1 - j : j;
             float acc[OC];
             if (ck == K_IDT) {
 #pragma unroll
-                for (int o = 0; o < OC; o++) acc[o] = Fc[(i0 + o) * H + i0 + o] * (float)res[(fud ? H - 1 - (i0 + o) : i0 + o) * W + jj];
+                for (int o = 0; o < OC; o++) acc[o] = FcT[(i0 + o) * H + i0 + o] * (float)res[(fud ? H - 1 - (i0 + o) : i0 + o) * W + jj];
             } else {
 #pragma unroll
                 for (int o = 0; o < OC; o++) acc[o] = 0.f;
@@ -276,7 +278,6 @@ __device__ EvalOut grp_eval(RP res, FP tmp, QP q, const E &e, const TT &T) {
         constexpr int ORF = TW * TH / GW, OR = ORF < 1 ? 1 : ORF > TW ? TW : ORF, NR = TH * (TW / OR);
         static_assert(NR <= GW, "one row item per lane");
         const auto *FrT = T.fwdT + T.fwdOff[rk][LW];
-        const auto *Fr = T.fwd + T.fwdOff[rk][LW];
         const float scale = T.txScale[e.txSz];
         const int i = lane % TH, o0 = (lane / TH) * OR;
         auto *row = tmp + i * TS;
@@ -284,7 +285,7 @@ __device__ EvalOut grp_eval(RP res, FP tmp, QP q, const E &e, const TT &T) {
         if (lane < NR) {
             if (rk == K_IDT) {
 #pragma unroll
-                for (int o = 0; o < OR; o++) acc[o] = Fr[(o0 + o) * W + o0 + o] * row[o0 + o];
+                for (int o = 0; o < OR; o++) acc[o] = FrT[(o0 + o) * W + o0 + o] * row[o0 + o];
             } else {
 #pragma unroll
                 for (int o = 0; o < OR; o++) acc[o] = 0.f;
@@ -440,13 +441,12 @@ __device__ EvalOut half_eval(RP res, FP tmp, QP q, const E &e, const TT &T) {
     {
         constexpr int OCF = W * TH / 16, OC = OCF < 1 ? 1 : OCF > 8 ? 8 : OCF, NI = W * (TH / OC);
         const auto *FcT = T.fwdT + T.fwdOff[ck][LH];
-        const auto *Fc = T.fwd + T.fwdOff[ck][LH];
         for (int it = lane; it < NI; it += 16) {
             const int j = it % W, i0 = (it / W) * OC, jj = flr ? W - 1 - j : j;
             float acc[OC];
             if (ck == K_IDT) {
 #pragma unroll
-                for (int o = 0; o < OC; o++) acc[o] = Fc[(i0 + o) * H + i0 + o] * (float)res[(fud ? H - 1 - (i0 + o) : i0 + o) * W + jj];
+                for (int o = 0; o < OC; o++) acc[o] = FcT[(i0 + o) * H + i0 + o] * (float)res[(fud ? H - 1 - (i0 + o) : i0 + o) * W + jj];
             } else {
 #pragma unroll
                 for (int o = 0; o < OC; o++) acc[o] = 0.f;
@@ -467,7 +467,6 @@ __device__ EvalOut half_eval(RP res, FP tmp, QP q, const E &e, const TT &T) {
         constexpr int ORF = TW * TH / 16, OR = ORF < 1 ? 1 : ORF > TW ? TW : ORF, NR = TH * (TW / OR);
         static_assert(NR <= 16, "one row item per lane");
         const auto *FrT = T.fwdT + T.fwdOff[rk][LW];
-        const auto *Fr = T.fwd + T.fwdOff[rk][LW];
         const float scale = T.txScale[e.txSz];
         const int i = lane % TH, o0 = (lane / TH) * OR;
         auto *row = tmp + i * TS;
@@ -475,7 +474,7 @@ __device__ EvalOut half_eval(RP res, FP tmp, QP q, const E &e, const TT &T) {
         if (lane < NR) {
             if (rk == K_IDT) {
 #pragma unroll
-                for (int o = 0; o < OR; o++) acc[o] = Fr[(o0 + o) * W + o0 + o] * row[o0 + o];
+                for (int o = 0; o < OR; o++) acc[o] = FrT[(o0 + o) * W + o0 + o] * row[o0 + o];
             } else {
 #pragma unroll
                 for (int o = 0; o < OR; o++) acc[o] = 0.f;

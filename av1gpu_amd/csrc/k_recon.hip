@@ -38,29 +38,44 @@ struct RcSmall {
     int16_t lev[RC_LEV_TOTAL];
 };
 // scratch of one group evaluating a transform block with a side of 32 or 64 (DCT_DCT only)
+// The levels overlay the coefficients: the quantizer's round t writes levels 32 t .. 32 t + 31, the bytes of tmp's floats
+// 16 t .. 16 t + 15, and coefficient 32 t + k lies at float 32 t + k or later (row stride W + 1): read in this round
+// before its store (each lane's store depends on its own load) or in an earlier one.
 struct RcTeam {
-    float tmp[32 * 65];      // th x (W + 1): column-pass outputs, then the coefficients
-    int16_t q[1024];
+    float tmp[32 * 65];      // th x (W + 1): column-pass outputs, then the coefficients, then the levels
     uint16_t ea[EDGE_LEN], el[EDGE_LEN];
 };
-// the tables the small-block evaluations and the decisions read, staged once per workgroup
+template <typename X> __device__ __forceinline__ lds<int16_t> *team_lev(X &t) { return (lds<int16_t> *)(lds<char> *)t.tmp; }
+// The tables the evaluations and the decisions read, staged once per workgroup (the costs: per quantizer context of the
+// images it meets).  An evaluation reads them in chains (level -> context -> cost) that nothing else hides in one
+// workgroup's four waves.  From the device tables they were about 480 flat loads per wave and block; in LDS the closed loop
+// of a 512 x 512 image went 52.7 -> 48.7 ms, of 16 12 MP images 191 -> 175 ms (two workgroups per CU still fit: the
+// inverse's scratch and the levels share the evaluations' scratch).
 struct RcTabs {
     float fwdT[3 * 336];     // DCT, ADST, identity for n = 4, 8, 16, transposed (offsets fwdOff)
-    float fwd[3 * 336];      // the same, row-major (the identity kind reads its diagonal)
     int fwdOff[3][7];
     float txScale[19];
     float txg[19][16];
     uint8_t cbOff[19][25];         // Coeff_Base_Ctx_Offset
-    const uint16_t *iscan;         // the inverse default scans (device tables; read through the caches)
-    const CostTab *cost;           // the cost tables of the image's quantizer context (device tables)
+    uint8_t scan8[SCAN8_TOTAL], iscan8[SCAN8_TOTAL];   // default scans of up to 256 coefficients and their inverses
+    const uint16_t *iscan;         // the larger ones' inverses (device tables; read through the caches)
+    CostTab cost;                  // of the image's quantizer context
 };
-using RcEvalIn = EvalInT<const CostTab *>;
+using RcEvalIn = EvalInT<const lds<CostTab> *>;
 template <int TSZ>
-__device__ __forceinline__ const uint16_t *dscan_ptr(const lds<RcTabs> &) { return scan_of(TSZ, DCT_DCT); }
+__device__ __forceinline__ auto dscan_ptr(const lds<RcTabs> &T) {
+    constexpr int t = av1t::Adjusted_Tx_Size[TSZ];
+    if constexpr (scan8_has(t)) return (const lds<uint8_t> *)(T.scan8 + scan8_off(t));
+    else return scan_of(TSZ, DCT_DCT);
+}
 template <int TSZ>
 __device__ __forceinline__ const lds<uint8_t> *cboff_ptr(const lds<RcTabs> &T) { return T.cbOff[TSZ]; }
 template <int TSZ>
-__device__ __forceinline__ const uint16_t *iscan_ptr(const lds<RcTabs> &T) { return T.iscan + dscan_off(av1t::Adjusted_Tx_Size[TSZ]); }
+__device__ __forceinline__ auto iscan_ptr(const lds<RcTabs> &T) {
+    constexpr int t = av1t::Adjusted_Tx_Size[TSZ];
+    if constexpr (scan8_has(t)) return (const lds<uint8_t> *)(T.iscan8 + scan8_off(t));
+    else return T.iscan + dscan_off(t);
+}
 
 union RcScr {
     RcSmall s;
@@ -70,8 +85,8 @@ struct RcShared {
     RcScr u;
     RcTabs tab;
     uint16_t srcb[64 * 64];                  // source block of the current leaf: luma W x H, or U at 0 and V at 2048
-    int16_t inv[64 * 64];                    // inverse transform residual (the row pass clamps to 16 bits; the column
-                                             // outputs of a block passing the range checks are within 12)
+    Img img;                                 // descriptor of the superblock's image
+    int dcQ, acQ;                            // its quantizer steps
     uint16_t ea[3][EDGE_LEN], el[3][EDGE_LEN];   // unfiltered edges of the current tx block per plane
     int dcv[3], ft[3], hvL[3], hvA[3], px[3], py[3], mx[3], my[3];
     int skipCtx[3], dcCtx[3];
@@ -105,12 +120,23 @@ __device__ __forceinline__ const lds<RcTeam> &team_scr(const lds<RcShared> &S, i
     return g < RC_NTEAM ? S.u.t[g] : ((const lds<RcTeam> *)(const lds<char> *)(&S + 1))[g - RC_NTEAM];
 }
 
-template <typename Px> __device__ __forceinline__ Px *rec_plane(const Img &I, int p) { return (Px *)I.rec[p]; }
-template <typename Px> __device__ __forceinline__ const Px *src_plane(const Img &I, int p) { return (const Px *)I.src[p]; }
+template <typename Px> __device__ __forceinline__ glb<Px> *rec_plane(const lds<Img> &I, int p) { return (glb<Px> *)I.rec[p]; }
+template <typename Px> __device__ __forceinline__ const glb<Px> *src_plane(const lds<Img> &I, int p) { return (const glb<Px> *)I.src[p]; }
+__device__ __forceinline__ glb<uint8_t> *map8(uint8_t *p) { return (glb<uint8_t> *)p; }
+// Scratch of the exact inverse (the residual, W x H): the evaluations' scratch is free once the levels are decided.  The
+// levels and edges of team t and of t ^ 1 (the other plane of a chroma pair) must stay, so blocks with a side of 32 or 64
+// take the coefficients of team (t & 3) ^ 2, smaller ones group 0's.
+__device__ __forceinline__ lds<int16_t> *inv_scr(lds<RcShared> &S, int txSz, int team);
+
+__device__ __forceinline__ lds<int16_t> *inv_scr(lds<RcShared> &S, int txSz, int team) {
+    static_assert(sizeof(RcGroup::tmp) >= 16 * 16 * 2 && sizeof(RcTeam::tmp) >= 64 * 64 * 2 && RC_NTEAM == 4, "the inverse's scratch");
+    const bool big = tx_w(txSz) > 16 || tx_h(txSz) > 16;
+    return (lds<int16_t> *)(lds<char> *)(big ? S.u.t[(team & 3) ^ 2].tmp : S.u.s.g[0].tmp);
+}
 
 // get_filter_type (spec 7.11.2.8): 1 if the above or left block (chroma: the chroma-carrying one) uses a SMOOTH mode
-__device__ int filter_type(const Img &I, int plane, int mi_row, int mi_col, int availU, int availL) {
-    const uint8_t *m = plane ? I.mUV : I.mY;
+__device__ int filter_type(const lds<Img> &I, int plane, int mi_row, int mi_col, int availU, int availL) {
+    const glb<uint8_t> *m = map8(plane ? I.mUV : I.mY);
     auto smooth = [](int v) { return v == SMOOTH_PRED || v == SMOOTH_V_PRED || v == SMOOTH_H_PRED; };
     int a = 0, l = 0;
     if (availU) {
@@ -128,11 +154,11 @@ __device__ int filter_type(const Img &I, int plane, int mi_row, int mi_col, int 
 
 // coefficient contexts of a tx block from the context maps (spec get_tx_block ctx), by the 32 lanes of the group:
 // lane k reads the k-th 4x4 column above and row to the left
-__device__ void grp_txb_ctx(const Img &I, int plane, int txSz, int x4, int y4, int bsize, int tx0, int ty0, lds<int> *skipCtx,
+__device__ void grp_txb_ctx(const lds<Img> &I, int plane, int txSz, int x4, int y4, int bsize, int tx0, int ty0, lds<int> *skipCtx,
                             lds<int> *dcCtx) {
     const int lane = glane(), ss = plane ? I.ss : 0;
     const int stride = I.MiCols >> ss, maxX4 = I.MiCols >> ss, maxY4 = I.MiRows >> ss;
-    const uint8_t *L = I.cLvl[plane], *D = I.cDc[plane];
+    const glb<uint8_t> *L = map8(I.cLvl[plane]), *D = map8(I.cDc[plane]);
     const bool hasA = y4 > ((ty0 >> 2) >> ss), hasL = x4 > ((tx0 >> 2) >> ss);
     const int w = tx_w(txSz), h = tx_h(txSz), w4 = w >> 2, h4 = h >> 2;
     int top = 0, left = 0, topAny = 0, leftAny = 0, sgn = 0;
@@ -162,7 +188,7 @@ __device__ void grp_txb_ctx(const Img &I, int plane, int txSz, int x4, int y4, i
 template <typename Px>
 // fA / fL: the block's AvailU / AvailL for the edge filter type where they differ from the tx block's edges (a further
 // 4:4:4 chroma tx block inside its block); -1: the same
-__device__ void rc_edges(lds<RcShared> &S, const Img &I, int p, int px, int py, int lw, int lh, int haveL, int haveA, int haveAR, int haveBL,
+__device__ void rc_edges(lds<RcShared> &S, const lds<Img> &I, int p, int px, int py, int lw, int lh, int haveL, int haveA, int haveAR, int haveBL,
                          int mi_row, int mi_col, int fA = -1, int fL = -1) {
     const int ss = p ? I.ss : 0;
     const int maxX = ((I.MiCols * 4) >> ss) - 1, maxY = ((I.MiRows * 4) >> ss) - 1;
@@ -220,34 +246,34 @@ __device__ void grp_residual(lds<RcShared> &S, lds<uint16_t> *gea, lds<uint16_t>
 // one RD task (candidate c of plane p with tx type t) of a tx block up to 16x16 by the calling group: the residual
 // res is ready; the levels go to lev
 template <int W, int H>
-__device__ EvalOut grp_task(lds<RcShared> &S, lds<RcGroup> &X, const Img &I, int p, int c, int t, const lds<int16_t> *res,
+__device__ EvalOut grp_task(lds<RcShared> &S, lds<RcGroup> &X, const lds<Img> &I, int p, int c, int t, const lds<int16_t> *res,
                             lds<int16_t> *lev, const SearchParams &P) {
     RcEvalIn e;
     e.txSz = tx_of(W, H); e.txType = t; e.plane = p;
-    e.dcQ = dc_q(I.qindex, I.bd); e.acQ = ac_q(I.qindex, I.bd);
+    e.dcQ = S.dcQ; e.acQ = S.acQ;
     e.skipCtx = S.skipCtx[p]; e.dcCtx = S.dcCtx[p]; e.intraDir = p == 0 ? cand_mode(c) : 0; e.bd = I.bd;
     e.rnd = p ? P.rndC : P.rnd; e.zbin = p ? P.zbinC : P.zbin;
     e.resEnergy = 0.f;
-    e.C = S.tab.cost;
+    e.C = &S.tab.cost;
     return grp_eval<W, H>(res, X.tmp, lev, e, S.tab);
 }
 // the same task by half the group (blocks of up to 64 coefficients), with tmp its own part of the group's scratch
 template <int W, int H>
-__device__ EvalOut half_task(lds<RcShared> &S, lds<float> *tmp, const Img &I, int p, int c, int t, const lds<int16_t> *res,
+__device__ EvalOut half_task(lds<RcShared> &S, lds<float> *tmp, const lds<Img> &I, int p, int c, int t, const lds<int16_t> *res,
                              lds<int16_t> *lev, const SearchParams &P) {
     RcEvalIn e;
     e.txSz = tx_of(W, H); e.txType = t; e.plane = p;
-    e.dcQ = dc_q(I.qindex, I.bd); e.acQ = ac_q(I.qindex, I.bd);
+    e.dcQ = S.dcQ; e.acQ = S.acQ;
     e.skipCtx = S.skipCtx[p]; e.dcCtx = S.dcCtx[p]; e.intraDir = p == 0 ? cand_mode(c) : 0; e.bd = I.bd;
     e.rnd = p ? P.rndC : P.rnd; e.zbin = p ? P.zbinC : P.zbin;
     e.resEnergy = 0.f;
-    e.C = S.tab.cost;
+    e.C = &S.tab.cost;
     return half_eval<W, H>(res, tmp, lev, e, S.tab);
 }
 
 // one RD task (candidate c, 255 = CfL, of plane p; DCT_DCT) of a tx block with a side of 32 or 64 by the calling group
 template <int W, int H>
-__device__ EvalOut grp_task_big(lds<RcShared> &S, lds<RcTeam> &X, const Img &I, const DevTables &T, int p, int c,
+__device__ EvalOut grp_task_big(lds<RcShared> &S, lds<RcTeam> &X, const lds<Img> &I, const DevTables &T, int p, int c,
                                 const lds<uint16_t> *src, int sp, const SearchParams &P) {
     constexpr int LW = W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
     const int lane = glane(), bd = I.bd;
@@ -279,11 +305,11 @@ __device__ EvalOut grp_task_big(lds<RcShared> &S, lds<RcTeam> &X, const Img &I, 
     RcEvalIn e;
     e.resEnergy = grp_fwd_dct<W, H>(X.tmp, T, S.tab.txScale[txSz], res);
     e.txSz = txSz; e.txType = DCT_DCT; e.plane = p;
-    e.dcQ = dc_q(I.qindex, bd); e.acQ = ac_q(I.qindex, bd);
+    e.dcQ = S.dcQ; e.acQ = S.acQ;
     e.skipCtx = S.skipCtx[p]; e.dcCtx = S.dcCtx[p]; e.intraDir = p == 0 ? cand_mode(c) : 0; e.bd = bd;
     e.rnd = p ? P.rndC : P.rnd; e.zbin = p ? P.zbinC : P.zbin;
-    e.C = S.tab.cost;
-    return grp_qrate<W, H>(X.tmp, W + 1, X.q, e, S.tab);
+    e.C = &S.tab.cost;
+    return grp_qrate<W, H>(X.tmp, W + 1, team_lev(X), e, S.tab);
 }
 
 // ---- exact inverse transform + reconstruction by the workgroup (spec 7.13.3, 7.12.3 step 3) ----
@@ -320,7 +346,9 @@ __device__ __forceinline__ uint32_t inv_col(int j, int W, int ck, int bd, lds<in
 
 // dequantize + inverse + add the levels q (LDS, modified by the repair) onto dst; returns the number of repairs
 template <typename Px>
-__device__ __forceinline__ int wg_inverse_add(lds<RcShared> &S, lds<int16_t> *q, int txSz, int txType, int bd, int dcQ, int acQ, Px *dst, int pitch) {
+__device__ __forceinline__ int wg_inverse_add(lds<RcShared> &S, lds<int16_t> *q, lds<int16_t> *inv, int txSz, int txType, int bd, glb<Px> *dst,
+                                              int pitch) {
+    const int dcQ = S.dcQ, acQ = S.acQ;
     const int tid = threadIdx.x, lw = av1t::Tx_Width_Log2[txSz], lh = av1t::Tx_Height_Log2[txSz], W = 1 << lw, H = 1 << lh;
     const int tw = W > 32 ? 32 : W, th = H > 32 ? 32 : H, n = tw * th, den = dq_denom(txSz), dsh = den == 4 ? 2 : den == 2 ? 1 : 0;
     const bool rect = lw - lh == 1 || lh - lw == 1;
@@ -332,11 +360,11 @@ __device__ __forceinline__ int wg_inverse_add(lds<RcShared> &S, lds<int16_t> *q,
         uint32_t err = 0;
         if (tid < H) {
             switch (lw) {
-            case 2: err = inv_row<2>(tid, W, th, tw, q, dcQ, acQ, dsh, bd, rect, rk, rs, S.inv); break;
-            case 3: err = inv_row<3>(tid, W, th, tw, q, dcQ, acQ, dsh, bd, rect, rk, rs, S.inv); break;
-            case 4: err = inv_row<4>(tid, W, th, tw, q, dcQ, acQ, dsh, bd, rect, rk, rs, S.inv); break;
-            case 5: err = inv_row<5>(tid, W, th, tw, q, dcQ, acQ, dsh, bd, rect, rk, rs, S.inv); break;
-            default: err = inv_row<6>(tid, W, th, tw, q, dcQ, acQ, dsh, bd, rect, rk, rs, S.inv); break;
+            case 2: err = inv_row<2>(tid, W, th, tw, q, dcQ, acQ, dsh, bd, rect, rk, rs, inv); break;
+            case 3: err = inv_row<3>(tid, W, th, tw, q, dcQ, acQ, dsh, bd, rect, rk, rs, inv); break;
+            case 4: err = inv_row<4>(tid, W, th, tw, q, dcQ, acQ, dsh, bd, rect, rk, rs, inv); break;
+            case 5: err = inv_row<5>(tid, W, th, tw, q, dcQ, acQ, dsh, bd, rect, rk, rs, inv); break;
+            default: err = inv_row<6>(tid, W, th, tw, q, dcQ, acQ, dsh, bd, rect, rk, rs, inv); break;
             }
         }
         if (err) atomicOr(gen(&S.errFlag), (int)err);
@@ -344,11 +372,11 @@ __device__ __forceinline__ int wg_inverse_add(lds<RcShared> &S, lds<int16_t> *q,
         err = 0;
         if (tid < W) {
             switch (lh) {
-            case 2: err = inv_col<2>(tid, W, ck, bd, S.inv); break;
-            case 3: err = inv_col<3>(tid, W, ck, bd, S.inv); break;
-            case 4: err = inv_col<4>(tid, W, ck, bd, S.inv); break;
-            case 5: err = inv_col<5>(tid, W, ck, bd, S.inv); break;
-            default: err = inv_col<6>(tid, W, ck, bd, S.inv); break;
+            case 2: err = inv_col<2>(tid, W, ck, bd, inv); break;
+            case 3: err = inv_col<3>(tid, W, ck, bd, inv); break;
+            case 4: err = inv_col<4>(tid, W, ck, bd, inv); break;
+            case 5: err = inv_col<5>(tid, W, ck, bd, inv); break;
+            default: err = inv_col<6>(tid, W, ck, bd, inv); break;
             }
         }
         if (err) atomicOr(gen(&S.errFlag), (int)err);
@@ -365,8 +393,8 @@ __device__ __forceinline__ int wg_inverse_add(lds<RcShared> &S, lds<int16_t> *q,
     const int fud = flip_ud(txType), flr = flip_lr(txType), maxv = (1 << bd) - 1;
     for (int p = tid; p < W * H; p += RC_NT) {
         const int i = p >> lw, j = p & (W - 1);
-        Px *d = dst + (size_t)(fud ? H - 1 - i : i) * pitch + (flr ? W - 1 - j : j);
-        *d = (Px)clip3(0, maxv, (int)*d + S.inv[i * W + j]);
+        glb<Px> *d = dst + (size_t)(fud ? H - 1 - i : i) * pitch + (flr ? W - 1 - j : j);
+        *d = (Px)clip3(0, maxv, (int)*d + inv[i * W + j]);
     }
     __syncthreads();
     return fixes;
@@ -374,7 +402,7 @@ __device__ __forceinline__ int wg_inverse_add(lds<RcShared> &S, lds<int16_t> *q,
 
 // write the prediction of candidate c of plane p (edges prepared by group g, or the base edges) into dst (workgroup)
 template <typename Px>
-__device__ void wg_write_pred(const lds<RcShared> &S, const lds<uint16_t> *gea, const lds<uint16_t> *gel, int g, int p, int c, int lw, int lh, Px *dst,
+__device__ void wg_write_pred(const lds<RcShared> &S, const lds<uint16_t> *gea, const lds<uint16_t> *gel, int g, int p, int c, int lw, int lh, glb<Px> *dst,
                               int pitch, int bd) {
     const int W = 1 << lw, H = 1 << lh;
     const int m = c == 255 ? DC_PRED : cand_mode(c), pa = pangle(m, c == 255 ? 0 : cand_delta(c));
@@ -393,7 +421,7 @@ __device__ void wg_write_pred(const lds<RcShared> &S, const lds<uint16_t> *gea, 
 }
 
 // record the finished tx block with levels q: coefficients, txb entry, context maps, BlockDecoded (workgroup)
-__device__ int wg_record_txb(lds<RcShared> &S, const Batch &B, uint32_t sb, const Img &I, int p, int txSz, int txType, int x4, int y4,
+__device__ int wg_record_txb(lds<RcShared> &S, const Batch &B, uint32_t sb, const lds<Img> &I, int p, int txSz, int txType, int x4, int y4,
                              const lds<int16_t> *q) {
     const int tid = threadIdx.x, n = tx_ncoef(txSz);
     const uint32_t off = (uint32_t)S.nCoef;
@@ -401,12 +429,15 @@ __device__ int wg_record_txb(lds<RcShared> &S, const Batch &B, uint32_t sb, cons
         // eob: 1 + the largest scan index of a nonzero level (inverse default scan; rows for class VERT, columns for
         // HORIZ); cul: the sum of |level| before the eob, i.e. over every level (later ones are 0), capped at 63
         const int cls = tx_class(txType), tw = tx_w(txSz) > 32 ? 32 : tx_w(txSz), th = tx_h(txSz) > 32 ? 32 : tx_h(txSz);
-        const uint16_t *isc = S.tab.iscan + dscan_off(av1t::Adjusted_Tx_Size[txSz]);
+        const int adj = av1t::Adjusted_Tx_Size[txSz];
+        const bool s8 = scan8_has(adj);
+        const glb<uint16_t> *isc = (const glb<uint16_t> *)S.tab.iscan + dscan_off(adj);
+        const lds<uint8_t> *isc8 = S.tab.iscan8 + scan8_off(adj);
         int last = 0, cul = 0;
         for (int i = tid; i < n; i += 32) {
             const int v = q[i];
             if (v) {
-                const int c = cls == TX_CLASS_2D ? (int)isc[i] : cls == TX_CLASS_VERT ? i : (i % tw) * th + i / tw;
+                const int c = cls == TX_CLASS_2D ? (s8 ? (int)isc8[i] : (int)isc[i]) : cls == TX_CLASS_VERT ? i : (i % tw) * th + i / tw;
                 last = max(last, c + 1);
                 cul += abs(v);
             }
@@ -415,7 +446,7 @@ __device__ int wg_record_txb(lds<RcShared> &S, const Batch &B, uint32_t sb, cons
         cul = gsumi(cul);
         if (tid == 0) { S.eobOut = eob; S.culOut = min(cul, 63); }
     }
-    int16_t *oc = B.oCoeffs + (size_t)sb * B.coefCap + off;
+    glb<int16_t> *oc = (glb<int16_t> *)B.oCoeffs + (size_t)sb * B.coefCap + off;
     for (int i = tid; i < n; i += RC_NT) oc[i] = q[i];
     __syncthreads();
     const int eob = S.eobOut, cul = S.culOut, dcCat = q[0] < 0 ? 1 : q[0] > 0 ? 2 : 0;
@@ -425,8 +456,8 @@ __device__ int wg_record_txb(lds<RcShared> &S, const Batch &B, uint32_t sb, cons
     for (int k = tid; k < w4 * h4; k += RC_NT) {
         const int yy = k >> lw4, xx = k & (w4 - 1);
         if (y4 + yy < rows && x4 + xx < stride) {
-            I.cLvl[p][(size_t)(y4 + yy) * stride + x4 + xx] = (uint8_t)(eob ? cul : 0);
-            I.cDc[p][(size_t)(y4 + yy) * stride + x4 + xx] = (uint8_t)(eob ? dcCat : 0);
+            map8(I.cLvl[p])[(size_t)(y4 + yy) * stride + x4 + xx] = (uint8_t)(eob ? cul : 0);
+            map8(I.cDc[p])[(size_t)(y4 + yy) * stride + x4 + xx] = (uint8_t)(eob ? dcCat : 0);
         }
         S.bdm[p][r4 + yy + 1][c4 + xx + 1] = 1;
     }
@@ -453,7 +484,7 @@ __device__ __forceinline__ const lds<uint16_t> *stage_src(const lds<RcShared> &S
 // wg_luma_residuals; chroma tasks make their own in slot t; levels of task t go to S.u.s.lev[t].  Larger blocks:
 // team g (tasks g, g + nTeam, ..., run in descending order) keeps the levels and prepared edges of task g.
 template <int W, int H>
-__device__ __forceinline__ void wg_run_tasks(lds<RcShared> &S, const Img &I, const DevTables &T, const SearchParams &P, float lambda, bool lumaBits,
+__device__ __forceinline__ void wg_run_tasks(lds<RcShared> &S, const lds<Img> &I, const DevTables &T, const SearchParams &P, float lambda, bool lumaBits,
                              bool pickWinner) {
     constexpr bool big = W > 16 || H > 16;
     constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 4 ? 2 : H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
@@ -463,7 +494,7 @@ __device__ __forceinline__ void wg_run_tasks(lds<RcShared> &S, const Img &I, con
         static_assert((6 * nt > 14 ? 6 * nt : 14) * W * H <= RC_LEV_TOTAL, "the packed levels cannot hold every task");
     }
     const int g = gid(), lane = glane();
-    const CostTab &C = *S.tab.cost;
+    const lds<CostTab> &C = S.tab.cost;
     // blocks of up to 64 coefficients: 16 half groups, two tasks per group at once; luma residuals are ready, chroma
     // tasks first make theirs (one task per group, as below), then the halves evaluate
     bool done = false;
@@ -538,7 +569,7 @@ __device__ __forceinline__ void wg_run_tasks(lds<RcShared> &S, const Img &I, con
 
 // luma blocks up to 16x16: the residual of each candidate S.candC[k] into S.u.s.res[k] (group k)
 template <int W, int H>
-__device__ void wg_luma_residuals(lds<RcShared> &S, const Img &I) {
+__device__ void wg_luma_residuals(lds<RcShared> &S, const lds<Img> &I) {
     constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : 4, LH = H == 4 ? 2 : H == 8 ? 3 : 4;
     const int g = gid();
     if (g < S.nCand)
@@ -549,7 +580,7 @@ __device__ void wg_luma_residuals(lds<RcShared> &S, const Img &I) {
 // the levels of the winning task t, and (larger blocks) the team holding them with its prepared edges: the team's
 // kept task is t (t < nTeam), or it evaluates t again
 template <int W, int H>
-__device__ __forceinline__ lds<int16_t> *wg_final_levels(lds<RcShared> &S, const Img &I, const DevTables &T, const SearchParams &P, int t, int &team) {
+__device__ __forceinline__ lds<int16_t> *wg_final_levels(lds<RcShared> &S, const lds<Img> &I, const DevTables &T, const SearchParams &P, int t, int &team) {
     team = (W > 16 || H > 16) ? t % S.nTeam : t % RC_NG;
     if constexpr (W > 16 || H > 16) {
         if (t >= S.nTeam) {   // overwritten by a task of the same team that ran after it
@@ -557,7 +588,7 @@ __device__ __forceinline__ lds<int16_t> *wg_final_levels(lds<RcShared> &S, const
             if (gid() == team) grp_task_big<W, H>(S, team_scr(S, team), I, T, p, S.taskC[t], stage_src(S, p), W, P);
             __syncthreads();
         }
-        return team_scr(S, team).q;
+        return team_lev(team_scr(S, team));
     } else {
         return S.u.s.lev + t * (W * H);
     }
@@ -566,7 +597,7 @@ __device__ __forceinline__ lds<int16_t> *wg_final_levels(lds<RcShared> &S, const
 // write the prediction of task t of plane p (into dst): larger blocks predict again from team g's prepared edges;
 // blocks up to 16x16 take source minus the kept residual (slot k)
 template <int W, int H, typename Px>
-__device__ void wg_final_pred(const lds<RcShared> &S, const Img &I, int p, int t, int k, int team, Px *dst, int pitch) {
+__device__ void wg_final_pred(const lds<RcShared> &S, const lds<Img> &I, int p, int t, int k, int team, glb<Px> *dst, int pitch) {
     constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 4 ? 2 : H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
     if constexpr (W > 16 || H > 16) {
         wg_write_pred<Px>(S, I.edgeFilter ? team_scr(S, team).ea : nullptr, team_scr(S, team).el, team, p, S.taskC[t], LW, LH, dst, pitch, I.bd);
@@ -579,14 +610,14 @@ __device__ void wg_final_pred(const lds<RcShared> &S, const Img &I, int p, int t
 }
 
 template <int W, int H, typename Px>
-__device__ void rc_luma(lds<RcShared> &S, const Batch &B, const SearchParams &P, uint32_t sb, const Img &I, int bsize, int x, int y, int availU,
+__device__ void rc_luma(lds<RcShared> &S, const Batch &B, const SearchParams &P, uint32_t sb, const lds<Img> &I, int bsize, int x, int y, int availU,
                         int availL, int tx0, int ty0, float lambda) {
     constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 4 ? 2 : H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
     const DevTables &T = *B.T;
     const int tid = threadIdx.x, txSz = tx_of(W, H);
     const int sbr4 = (y >> 2) & 15, sbc4 = (x >> 2) & 15, mi_row = y >> 2, mi_col = x >> 2;
     {
-        const Px *src = src_plane<Px>(I, 0) + (size_t)y * I.spitch[0] + x;
+        const glb<Px> *src = src_plane<Px>(I, 0) + (size_t)y * I.spitch[0] + x;
         for (int q = tid; q < W * H; q += RC_NT) S.srcb[q] = src[(size_t)(q >> LW) * I.spitch[0] + (q & (W - 1))];
     }
     if (gid() == 0)
@@ -600,8 +631,8 @@ __device__ void rc_luma(lds<RcShared> &S, const Batch &B, const SearchParams &P,
         const int set = tx_set_intra(txSz);
         if (w < nc) S.candC[w] = br.cand[w];
         if (w == 0) {
-            S.am = av1t::Intra_Mode_Context[availU ? I.mY[(size_t)(mi_row - 1) * I.MiCols + mi_col] : DC_PRED];
-            S.lm = av1t::Intra_Mode_Context[availL ? I.mY[(size_t)mi_row * I.MiCols + mi_col - 1] : DC_PRED];
+            S.am = av1t::Intra_Mode_Context[availU ? map8(I.mY)[(size_t)(mi_row - 1) * I.MiCols + mi_col] : DC_PRED];
+            S.lm = av1t::Intra_Mode_Context[availL ? map8(I.mY)[(size_t)mi_row * I.MiCols + mi_col - 1] : DC_PRED];
             S.nCand = nc;
             S.bsize = bsize;
         }
@@ -646,10 +677,10 @@ __device__ void rc_luma(lds<RcShared> &S, const Batch &B, const SearchParams &P,
     const int win = S.win;
     int team;
     lds<int16_t> *q = wg_final_levels<W, H>(S, I, T, P, win, team);
-    Px *dst = rec_plane<Px>(I, 0) + (size_t)y * I.pitch[0] + x;
+    glb<Px> *dst = rec_plane<Px>(I, 0) + (size_t)y * I.pitch[0] + x;
     wg_final_pred<W, H, Px>(S, I, 0, win, S.taskK[win], team, dst, I.pitch[0]);
     if (S.taskE[win] > 0) {
-        const int fixes = wg_inverse_add<Px>(S, q, txSz, S.taskT[win], I.bd, dc_q(I.qindex, I.bd), ac_q(I.qindex, I.bd), dst, I.pitch[0]);
+        const int fixes = wg_inverse_add<Px>(S, q, inv_scr(S, txSz, team), txSz, S.taskT[win], I.bd, dst, I.pitch[0]);
         if (fixes && tid == 0) atomicAdd(&B.stats[3], 1u);
     }
     const int eob = wg_record_txb(S, B, sb, I, 0, txSz, S.taskT[win], x >> 2, y >> 2, q);
@@ -658,11 +689,11 @@ __device__ void rc_luma(lds<RcShared> &S, const Batch &B, const SearchParams &P,
 }
 
 template <int W, int H, typename Px>
-__device__ void rc_chroma(lds<RcShared> &S, const Batch &B, const SearchParams &P, uint32_t sb, const Img &I, int bsize, int mi_row, int mi_col,
+__device__ void rc_chroma(lds<RcShared> &S, const Batch &B, const SearchParams &P, uint32_t sb, const lds<Img> &I, int bsize, int mi_row, int mi_col,
                           int availUC, int availLC, int tx0, int ty0, float lambda) {
     constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 4 ? 2 : H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
     const DevTables &T = *B.T;
-    const CostTab &C = *S.tab.cost;
+    const lds<CostTab> &C = S.tab.cost;
     const int tid = threadIdx.x, ss = I.ss, bd = I.bd, txSz = tx_of(W, H);
     const int cx = (mi_col >> ss) * 4, cy = (mi_row >> ss) * 4, x4 = cx >> 2, y4 = cy >> 2;
     const int sbr4 = (mi_row & 15) >> ss, sbc4 = (mi_col & 15) >> ss;
@@ -674,7 +705,7 @@ __device__ void rc_chroma(lds<RcShared> &S, const Batch &B, const SearchParams &
     if (gid() == 2) grp_txb_ctx(I, 1, txSz, x4, y4, bsize, tx0, ty0, &S.skipCtx[1], &S.dcCtx[1]);
     if (gid() == 3) grp_txb_ctx(I, 2, txSz, x4, y4, bsize, tx0, ty0, &S.skipCtx[2], &S.dcCtx[2]);
     {
-        const Px *gU = src_plane<Px>(I, 1) + (size_t)cy * I.spitch[1] + cx, *gV = src_plane<Px>(I, 2) + (size_t)cy * I.spitch[2] + cx;
+        const glb<Px> *gU = src_plane<Px>(I, 1) + (size_t)cy * I.spitch[1] + cx, *gV = src_plane<Px>(I, 2) + (size_t)cy * I.spitch[2] + cx;
         for (int q = tid; q < W * H; q += RC_NT) {
             S.srcb[q] = gU[(size_t)(q >> LW) * I.spitch[1] + (q & (W - 1))];
             S.srcb[2048 + q] = gV[(size_t)(q >> LW) * I.spitch[2] + (q & (W - 1))];
@@ -705,7 +736,7 @@ __device__ void rc_chroma(lds<RcShared> &S, const Batch &B, const SearchParams &
             for (int ly = mi_row * 4; ly < mi_row * 4 + 4 * bh4(bsize); ly += th)
                 for (int lx = mi_col * 4; lx < mi_col * 4 + 4 * bw4(bsize); lx += tw)
                     if (lx < I.MiCols * 4 && ly < I.MiRows * 4) { maxLumaW = lx + tw; maxLumaH = ly + th; }
-            const Px *luma = rec_plane<Px>(I, 0);
+            const glb<Px> *luma = rec_plane<Px>(I, 0);
             const int lp = I.pitch[0], i = tid >> LW, j = tid & (W - 1);
             const bool in = tid < W * H;
             int v = 0;
@@ -773,7 +804,7 @@ __device__ void rc_chroma(lds<RcShared> &S, const Batch &B, const SearchParams &
         for (int ly = mi_row * 4; ly < mi_row * 4 + 4 * bh4(bsize); ly += th)
             for (int lx = mi_col * 4; lx < mi_col * 4 + 4 * bw4(bsize); lx += tw)
                 if (lx < I.MiCols * 4 && ly < I.MiRows * 4) { maxLumaW = lx + tw; maxLumaH = ly + th; }
-        const Px *luma = rec_plane<Px>(I, 0);
+        const glb<Px> *luma = rec_plane<Px>(I, 0);
         const int lp = I.pitch[0];
         int sum = 0;
         for (int q = tid; q < W * H; q += RC_NT) {
@@ -1015,10 +1046,10 @@ __device__ void rc_chroma(lds<RcShared> &S, const Batch &B, const SearchParams &
         const int t = win + p - 1;
         int team;
         lds<int16_t> *q = wg_final_levels<W, H>(S, I, T, P, t, team);
-        Px *dst = rec_plane<Px>(I, p) + (size_t)cy * I.pitch[p] + cx;
+        glb<Px> *dst = rec_plane<Px>(I, p) + (size_t)cy * I.pitch[p] + cx;
         wg_final_pred<W, H, Px>(S, I, p, t, t, team, dst, I.pitch[p]);
         if (S.taskE[t] > 0) {
-            const int fixes = wg_inverse_add<Px>(S, q, txSz, uvTxType, bd, dc_q(I.qindex, bd), ac_q(I.qindex, bd), dst, I.pitch[p]);
+            const int fixes = wg_inverse_add<Px>(S, q, inv_scr(S, txSz, team), txSz, uvTxType, bd, dst, I.pitch[p]);
             if (fixes && tid == 0) atomicAdd(&B.stats[3], 1u);
         }
         int eob = wg_record_txb(S, B, sb, I, p, txSz, uvTxType, x4, y4, q);
@@ -1033,7 +1064,7 @@ __device__ void rc_chroma(lds<RcShared> &S, const Batch &B, const SearchParams &
             if (gid() == 1) grp_txb_ctx(I, p, txSz, x4 + (ox >> 2), y4 + (oy >> 2), bsize, tx0, ty0, &S.skipCtx[p], &S.dcCtx[p]);
             {
                 lds<uint16_t> *sd = S.srcb + (p == 2 ? 2048 : 0);
-                const Px *g = src_plane<Px>(I, p) + (size_t)(cy + oy) * I.spitch[p] + cx + ox;
+                const glb<Px> *g = src_plane<Px>(I, p) + (size_t)(cy + oy) * I.spitch[p] + cx + ox;
                 for (int i = tid; i < W * H; i += RC_NT) sd[i] = g[(size_t)(i >> LW) * I.spitch[p] + (i & (W - 1))];
             }
             if (tid == 0) { S.taskC[0] = winC; S.taskT[0] = uvTxType; S.taskP[0] = p; S.nTask = 1; }
@@ -1041,10 +1072,10 @@ __device__ void rc_chroma(lds<RcShared> &S, const Batch &B, const SearchParams &
             wg_run_tasks<W, H>(S, I, T, P, lambda, false, false);
             int tm;
             lds<int16_t> *qk = wg_final_levels<W, H>(S, I, T, P, 0, tm);
-            Px *dk = rec_plane<Px>(I, p) + (size_t)(cy + oy) * I.pitch[p] + cx + ox;
+            glb<Px> *dk = rec_plane<Px>(I, p) + (size_t)(cy + oy) * I.pitch[p] + cx + ox;
             wg_final_pred<W, H, Px>(S, I, p, 0, 0, tm, dk, I.pitch[p]);
             if (S.taskE[0] > 0) {
-                const int fixes = wg_inverse_add<Px>(S, qk, txSz, uvTxType, bd, dc_q(I.qindex, bd), ac_q(I.qindex, bd), dk, I.pitch[p]);
+                const int fixes = wg_inverse_add<Px>(S, qk, inv_scr(S, txSz, tm), txSz, uvTxType, bd, dk, I.pitch[p]);
                 if (fixes && tid == 0) atomicAdd(&B.stats[3], 1u);
             }
             eob |= wg_record_txb(S, B, sb, I, p, txSz, uvTxType, x4 + (ox >> 2), y4 + (oy >> 2), qk);
@@ -1058,31 +1089,44 @@ __device__ void rc_chroma(lds<RcShared> &S, const Batch &B, const SearchParams &
     }
 }
 
-// stage the cost tables of quantizer context qctx (and, when first, the small forward matrices) in LDS
-__device__ void stage_tables(lds<RcShared> &S, const DevTables &T, int qctx, bool matrices) {
+// stage the cost tables of quantizer context qctx (and, when first, the tables of every image) in LDS
+__device__ void stage_tables(lds<RcShared> &S, const DevTables &T, int qctx, bool first) {
     const int tid = threadIdx.x;
-    if (tid == 0) { S.tab.cost = &T.cost[qctx]; S.tab.iscan = T.iscan; }
-    if (matrices) {
+    static_assert(sizeof(CostTab) % 4 == 0, "the cost tables are floats");
+    {
+        const float *c = (const float *)&T.cost[qctx];
+        lds<float> *d = (lds<float> *)(lds<char> *)&S.tab.cost;
+        for (int k = tid; k < (int)(sizeof(CostTab) / 4); k += RC_NT) d[k] = c[k];
+    }
+    if (first) {
+        if (tid == 0) S.tab.iscan = T.iscan;
         for (int k = tid; k < 3 * 336; k += RC_NT) {
             const int kind = k / 336, r = k % 336, ln = r < 16 ? 2 : r < 80 ? 3 : 4, e = r - (ln == 2 ? 0 : ln == 3 ? 16 : 80);
             S.tab.fwdT[k] = T.fwdT[T.fwdOff[kind][ln] + e];
-            S.tab.fwd[k] = T.fwd[T.fwdOff[kind][ln] + e];
         }
         if (tid < 21) S.tab.fwdOff[tid / 7][tid % 7] = (tid / 7) * 336 + ((tid % 7) == 3 ? 16 : (tid % 7) == 4 ? 80 : 0);
         if (tid < 19) S.tab.txScale[tid] = T.txScale[tid];
         for (int k = tid; k < 19 * 16; k += RC_NT) S.tab.txg[k / 16][k % 16] = T.txg[k / 16][k % 16];
         for (int k = tid; k < 19 * 25; k += RC_NT) S.tab.cbOff[k / 25][k % 25] = (&av1t::Coeff_Base_Ctx_Offset[0][0][0])[k];
+        for (int k = tid; k < SCAN8_TOTAL; k += RC_NT) { S.tab.scan8[k] = T.scan8[k]; S.tab.iscan8[k] = T.iscan8[k]; }
     }
 }
 
 // the closed loop of superblock sb (the workgroup; the tables staged for its image's quantizer context)
 template <typename Px>
 __device__ void recon_sb(lds<RcShared> &S, const Batch &B, const SearchParams &P, uint32_t sb) {
-    const Img &I = B.img[B.sbImg[sb]];
+    const int tid = threadIdx.x;
+    {   // the image's descriptor, read in place in LDS from here on
+        static_assert(sizeof(Img) % 4 == 0, "the descriptor is copied by words");
+        const uint32_t *g = (const uint32_t *)&B.img[B.sbImg[sb]];
+        lds<uint32_t> *d = (lds<uint32_t> *)(lds<char> *)&S.img;
+        for (int k = tid; k < (int)(sizeof(Img) / 4); k += RC_NT) d[k] = g[k];
+    }
+    __syncthreads();
+    const lds<Img> &I = S.img;
     const DevTables &T = *B.T;
     const uint32_t local = sb - I.sbBase;
     const int sbc = (int)(local % I.sbCols), sbr = (int)(local / I.sbCols), sbx = sbc * 64, sby = sbr * 64;
-    const int tid = threadIdx.x;
     int tc = 0, tr = 0;
     while (tc + 1 < I.tileCols && sbx >= I.tileColStart[tc + 1] * 4) tc++;
     while (tr + 1 < I.tileRows && sby >= I.tileRowStart[tr + 1] * 4) tr++;
@@ -1097,7 +1141,7 @@ __device__ void recon_sb(lds<RcShared> &S, const Batch &B, const SearchParams &P
         if (yy == (16 >> ss) && xx == -1) v = 0;
         S.bdm[p][yy + 1][xx + 1] = v;
     }
-    if (tid == 0) { S.nTxb = 0; S.nCoef = 0; S.flopsOn = B.flops != nullptr; S.flops = 0; }
+    if (tid == 0) { S.nTxb = 0; S.nCoef = 0; S.flopsOn = B.flops != nullptr; S.flops = 0; S.dcQ = dc_q(I.qindex, I.bd); S.acQ = ac_q(I.qindex, I.bd); }
     __syncthreads();
     const float lambda = T.lambda[I.bd == 10][I.qindex] * P.lambdaMul;
     const int nLeaves = B.leafCount[sb];
@@ -1135,11 +1179,11 @@ __device__ void recon_sb(lds<RcShared> &S, const Batch &B, const SearchParams &P
             const int r = mi_row + k / bw, c = mi_col + k % bw;
             if (r < I.MiRows && c < I.MiCols) {
                 const size_t o = (size_t)r * I.MiCols + c;
-                I.mY[o] = (uint8_t)yMode;
-                if (hasC) I.mUV[o] = (uint8_t)uv;
-                I.mSkip[o] = (uint8_t)skip;
-                I.mMiSize[o] = (uint8_t)bsize;
-                I.mTx[o] = (uint8_t)txSz;
+                map8(I.mY)[o] = (uint8_t)yMode;
+                if (hasC) map8(I.mUV)[o] = (uint8_t)uv;
+                map8(I.mSkip)[o] = (uint8_t)skip;
+                map8(I.mMiSize)[o] = (uint8_t)bsize;
+                map8(I.mTx)[o] = (uint8_t)txSz;
             }
         }
         if (tid == 0) {

@@ -168,6 +168,11 @@ void build_tables(DevTables &T) {
         const uint16_t *s = scan_of(t, DCT_DCT);
         const int n = av1t::Tx_Width[t] * av1t::Tx_Height[t];
         for (int k = 0; k < n; k++) T.iscan[dscan_off(t) + s[k]] = (uint16_t)k;
+        if (scan8_has(t))
+            for (int k = 0; k < n; k++) {
+                T.scan8[scan8_off(t) + k] = (uint8_t)s[k];
+                T.iscan8[scan8_off(t) + s[k]] = (uint8_t)k;
+            }
     }
 }
 
