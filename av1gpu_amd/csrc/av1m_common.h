@@ -723,12 +723,15 @@ struct AnHooks {
     const uint32_t *base;
 };
 
-// the device work queue of the persistent closed-loop schedule
+// the device work queue of the persistent closed-loop schedule: an item is a superblock's luma or its chroma
+constexpr uint32_t RC_CHROMA = 0x80000000u;   // item flag: the superblock's chroma
 struct RcQueue {
-    const uint32_t *order;       // [n] superblocks in anti-diagonal wavefront order (step, image)
-    uint32_t n;
+    const uint32_t *order;       // [n] items, every one behind those it depends on
+    uint32_t n, nSb;
     uint32_t *head;              // next item to take
-    uint32_t *done;              // [nSb] set when a superblock is complete
+    uint32_t *prog;              // [2][nSb] progress of each superblock's luma and chroma: bits 0-7 rows (of 4 luma samples)
+                                 // of its right edge, 8-15 columns of its bottom edge, 16-31 blocks that are complete
+    int fine;                    // published after every block, else when the superblock is complete
     uint32_t *abort;             // raised by a wait that ran out of time
     uint64_t spinTicks;          // wait limit in wall-clock ticks
 };

@@ -696,9 +696,9 @@ static int encode_impl(av1mi_encoder *enc, const av1mi_frame_in *in, int n, av1m
         A.add(mapMem[i], 5 * mi + 2 * (mi + 2 * c1));
         mapTotal += 5 * mi + 2 * (mi + 2 * c1);
     }
-    uint32_t *dStats, *dDone, *dQctl;
+    uint32_t *dStats, *dProg, *dQctl;
     unsigned long long *dFlops = nullptr;
-    A.add(dStats, 8); A.add(dDone, nSb); A.add(dQctl, 2);
+    A.add(dStats, 8); A.add(dProg, 2 * (size_t)nSb); A.add(dQctl, 2);
     if (enc->countWork) A.add(dFlops, 64);
     // the CDEF output planes (the reconstruction's geometry), zeroed like it
     std::vector<uint8_t *> cdefMem(n, nullptr);
@@ -739,9 +739,12 @@ static int encode_impl(av1mi_encoder *enc, const av1mi_frame_in *in, int n, av1m
     for (auto &v : steps) { stepOff.push_back((uint32_t)stepFlat.size()); stepFlat.insert(stepFlat.end(), v.begin(), v.end()); }
     stepOff.push_back((uint32_t)stepFlat.size());
     if (stepFlat.size() != nSb) { snprintf(err, errlen, "internal: wavefront order covers %zu of %u superblocks", stepFlat.size(), nSb); return -1; }
-    uint32_t *dSteps, *dLnMask = nullptr;
+    // the persistent schedule's items: each superblock's luma, and its chroma (none of monochrome frames)
+    uint32_t nItems = nSb;
+    for (int i = 0; i < n; i++) if (!imgs[i].mono) nItems += (uint32_t)(imgs[i].sbCols * imgs[i].sbRows);
+    uint32_t *dSteps, *dOrder, *dLnMask = nullptr;
     PackOff *dPO;
-    A.add(dSteps, stepFlat.size()); A.add(dPO, nSb);
+    A.add(dSteps, stepFlat.size()); A.add(dOrder, nItems); A.add(dPO, nSb);
     // deblocking work units per image (pass 0: each plane's rows x 4-sample columns; pass 1: 4-sample rows x columns)
     uint64_t *dDbStart = nullptr;
     std::vector<uint64_t> dbStart(2 * ((size_t)n + 1), 0);
@@ -786,6 +789,29 @@ static int encode_impl(av1mi_encoder *enc, const av1mi_frame_in *in, int n, av1m
     const int wpe = occ ? occ : (uint64_t)nSb >= (uint64_t)std::max(1, enc->cus) * std::max<size_t>(1, steps.size()) ? 2 : 1;
     const int slots = enc->slots[bd == 10][wpe - 1] > 0 ? enc->slots[bd == 10][wpe - 1] : 1;
     const uint32_t qBlocks = enc->cfg.queueBlocks > 0 ? (uint32_t)enc->cfg.queueBlocks : (uint32_t)std::max(1, enc->cus * slots);
+    // Progress per block when the workgroups outnumber what the wavefront keeps ready: a superblock then starts beside
+    // its unfinished neighbours and its chroma runs one block behind its luma.  Else per superblock, the chroma of a step
+    // behind the luma of the next one, so that no workgroup is held by a wait.
+    // One 512 x 512 image (128 items, 22 steps): 20.2 ms per block on MI355X, 48.7 ms with the whole superblock as one item.
+    const bool fine = (uint64_t)nItems <= (uint64_t)qBlocks * std::max<size_t>(1, steps.size());
+    std::vector<uint32_t> order;
+    order.reserve(nItems);
+    {
+        auto luma = [&](size_t k) { for (uint32_t sb : steps[k]) order.push_back(sb); };
+        auto chroma = [&](size_t k) { for (uint32_t sb : steps[k]) if (!imgs[sbImg[sb]].mono) order.push_back(sb | RC_CHROMA); };
+        for (size_t k = 0; k < steps.size(); k++) {
+            if (fine) {
+                for (uint32_t sb : steps[k]) {
+                    order.push_back(sb);
+                    if (!imgs[sbImg[sb]].mono) order.push_back(sb | RC_CHROMA);
+                }
+            } else {
+                luma(k);
+                if (k) chroma(k - 1);
+                if (k + 1 == steps.size()) chroma(k);
+            }
+        }
+    }
     // ---- device memory: stream-ordered per call, or the captured plan's (graph mode) ----
     bool capture = false;
     const bool graph = enc->cfg.graph && !na;
@@ -798,7 +824,7 @@ static int encode_impl(av1mi_encoder *enc, const av1mi_frame_in *in, int n, av1m
         A.bind(na->mem);
     } else if (graph) {
         std::vector<uint64_t> key = sig;
-        key.insert(key.end(), {(uint64_t)anS, (uint64_t)sched, (uint64_t)qBlocks, (uint64_t)A.total, (uint64_t)wpe});
+        key.insert(key.end(), {(uint64_t)anS, (uint64_t)sched, (uint64_t)qBlocks, (uint64_t)A.total, (uint64_t)wpe, (uint64_t)fine});
         if (enc->plan.key != key) {
             drop_plan(enc);
             HCK(hipMalloc(&enc->plan.mem, A.total));
@@ -867,9 +893,9 @@ static int encode_impl(av1mi_encoder *enc, const av1mi_frame_in *in, int n, av1m
             for (size_t k = 0; k + 1 < stepOff.size(); k++) launch_recon(B, P, dSteps + stepOff[k], stepOff[k + 1] - stepOff[k], bd, s);
         } else {
             RcQueue Q;
-            Q.order = dSteps; Q.n = nSb; Q.head = dQctl; Q.abort = dQctl + 1; Q.done = dDone;
+            Q.order = dOrder; Q.n = nItems; Q.nSb = nSb; Q.head = dQctl; Q.abort = dQctl + 1; Q.prog = dProg; Q.fine = fine;
             Q.spinTicks = enc->clockHz * 30;   // no legitimate wait comes near 30 s
-            launch_recon_queue(B, P, Q, std::min<uint32_t>(qBlocks, nSb), bd, wpe, s);
+            launch_recon_queue(B, P, Q, std::min<uint32_t>(qBlocks, nItems), bd, wpe, s);
         }
         return hipGetLastError() == hipSuccess ? 0 : -1;
     };
@@ -878,6 +904,7 @@ static int encode_impl(av1mi_encoder *enc, const av1mi_frame_in *in, int n, av1m
             HCK(hipMemcpy(dShStart, shStart.data(), shStart.size() * 4, hipMemcpyHostToDevice));
             HCK(hipMemcpy(dSbImg, sbImg.data(), (size_t)nSb * 4, hipMemcpyHostToDevice));
             HCK(hipMemcpy(dSteps, stepFlat.data(), stepFlat.size() * 4, hipMemcpyHostToDevice));
+            HCK(hipMemcpy(dOrder, order.data(), order.size() * 4, hipMemcpyHostToDevice));
             HCK(hipStreamBeginCapture(enc->cap, hipStreamCaptureModeThreadLocal));
             const int r = device_part(enc->cap, false);
             hipGraph_t g = nullptr;
@@ -901,11 +928,12 @@ static int encode_impl(av1mi_encoder *enc, const av1mi_frame_in *in, int n, av1m
         HCK(hipMemcpyAsync(dImg, imgs.data(), n * sizeof(Img), hipMemcpyHostToDevice, st));
         HCK(hipMemcpyAsync(dShStart, shStart.data(), shStart.size() * 4, hipMemcpyHostToDevice, st));
         HCK(hipMemcpyAsync(dSbImg, sbImg.data(), (size_t)nSb * 4, hipMemcpyHostToDevice, st));
-        HCK(hipMemcpyAsync(dSteps, stepFlat.data(), stepFlat.size() * 4, hipMemcpyHostToDevice, st));
+        if (sched == 1) HCK(hipMemcpyAsync(dSteps, stepFlat.data(), stepFlat.size() * 4, hipMemcpyHostToDevice, st));
+        else HCK(hipMemcpyAsync(dOrder, order.data(), order.size() * 4, hipMemcpyHostToDevice, st));
         if (device_part(st, true)) { snprintf(err, errlen, "HIP: launch failed (%s)", hipGetErrorString(hipGetLastError())); A.release(st); return -1; }
     }
     tm.schedule = (uint32_t)sched;
-    tm.queueBlocks = sched == 1 ? 0 : std::min<uint32_t>(qBlocks, nSb);
+    tm.queueBlocks = sched == 1 ? 0 : std::min<uint32_t>(qBlocks, nItems);
     tm.anStreams = (uint32_t)anS;
     tm.graph = (uint32_t)graph;
     tm.tuned = tu && cand < 0 ? 1u : 0u;

@@ -1,8 +1,15 @@
-// Closed-loop decisions and reconstruction: one 256-thread workgroup (8 groups of 32 lanes) per 64x64 superblock,
-// launched per wavefront step (SBs whose left, above and above-right neighbours are complete).  Inside the SB the
+// Closed-loop decisions and reconstruction: one 256-thread workgroup (8 groups of 32 lanes) per 64x64 superblock and plane
+// kind (luma, or both chroma planes), from a persistent queue or one launch per wavefront step.  Inside the superblock the
 // leaves run in decode order exactly as the decoder sees them: BlockDecoded state, real reconstructed edges, exact
 // coefficient contexts from the 4x4 maps.  Reference: encoder/src/k_recon.cuh:1692-1808 (kernel), 822-1213 (luma),
 // 1220-1686 (chroma), 139-197 (inverse + add), 203-238 (contexts), 685-730 (records).
+//
+// What bounds it: the latency of the chain of blocks.  A block's steps depend on each other and on the blocks before it,
+// so a superblock keeps one workgroup's four waves mostly waiting, and an image keeps about one superblock per wavefront
+// column ready.  Two splits shorten the chain: luma needs nothing of chroma, so the two run as separate items beside each
+// other; and progress published per block lets a superblock start beside its unfinished neighbours (recon_part).
+// Closed loop of one 512 x 512 image 48.7 -> 20.2 ms, 24 MP learned 115 -> 54 ms; 16 images of 12 MP 175 -> 119 ms (per
+// superblock there; the smaller items also spill less).
 //
 // Per block:
 //   luma    every re-checked analysis candidate x every intra tx type of the set (tx blocks up to 16x16; DCT_DCT only
@@ -109,7 +116,10 @@ struct RcShared {
     int flopsOn;                             // count the forward-transform work (Batch::flops set)
     unsigned long long flops;                // of the superblock so far
     int am, lm, mode, delta, uvMode, uvDelta, nuv, bsize;
-    uint32_t qItem;                          // persistent schedule: the superblock taken
+    uint32_t qItem;                          // persistent schedule: the item taken
+    uint16_t leaf[MAX_LEAVES];               // the superblock's blocks: size | x4 << 5 | y4 << 9
+    uint32_t known[4];                       // last seen progress of the left, above and above-right superblock and of the
+                                             // superblock's own luma; [0] bit 31: a wait failed
 };
 
 // scratch of transform team g: the first RC_NTEAM share the union with the small-block scratch, the others follow RcShared
@@ -610,7 +620,7 @@ __device__ void wg_final_pred(const lds<RcShared> &S, const lds<Img> &I, int p, 
 }
 
 template <int W, int H, typename Px>
-__device__ void rc_luma(lds<RcShared> &S, const Batch &B, const SearchParams &P, uint32_t sb, const lds<Img> &I, int bsize, int x, int y, int availU,
+__device__ __noinline__ void rc_luma(lds<RcShared> &S, const Batch &B, const SearchParams &P, uint32_t sb, const lds<Img> &I, int bsize, int x, int y, int availU,
                         int availL, int tx0, int ty0, float lambda) {
     constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 4 ? 2 : H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
     const DevTables &T = *B.T;
@@ -689,7 +699,7 @@ __device__ void rc_luma(lds<RcShared> &S, const Batch &B, const SearchParams &P,
 }
 
 template <int W, int H, typename Px>
-__device__ void rc_chroma(lds<RcShared> &S, const Batch &B, const SearchParams &P, uint32_t sb, const lds<Img> &I, int bsize, int mi_row, int mi_col,
+__device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const SearchParams &P, uint32_t sb, const lds<Img> &I, int bsize, int mi_row, int mi_col,
                           int availUC, int availLC, int tx0, int ty0, float lambda) {
     constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 4 ? 2 : H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
     const DevTables &T = *B.T;
@@ -1112,15 +1122,58 @@ __device__ void stage_tables(lds<RcShared> &S, const DevTables &T, int qctx, boo
     }
 }
 
-// the closed loop of superblock sb (the workgroup; the tables staged for its image's quantizer context)
-template <typename Px>
-__device__ void recon_sb(lds<RcShared> &S, const Batch &B, const SearchParams &P, uint32_t sb) {
+// number and coefficients of the chroma tx blocks of a block that carries chroma (4:4:4 blocks with a 64-sample side hold
+// several per plane, coded where they start inside the coded area; the first always)
+__device__ __forceinline__ void chroma_size(const lds<Img> &I, int bsize, int mi_row, int mi_col, int &nTxb, int &nCoef) {
+    const int t = uv_tx_size(bsize, I.ss), w4 = tx_w(t) >> 2, h4 = tx_h(t) >> 2;
+    int n = 1;
+    if (!I.ss && (bw4(bsize) > w4 || bh4(bsize) > h4)) {
+        n = 0;
+        for (int y = 0; y < bh4(bsize); y += h4)
+            for (int x = 0; x < bw4(bsize); x += w4) n += (x == 0 && y == 0) || (mi_col + x < I.MiCols && mi_row + y < I.MiRows);
+    }
+    nTxb = 2 * n;
+    nCoef = 2 * n * tx_ncoef(t);
+}
+
+// wait (one thread) until the byte of progress word f at bit `shift` (16: the 16-bit block count) is at least need; the
+// word last seen in seen; false when the wait ran out of time or another workgroup aborted
+__device__ bool wait_progress(const uint32_t *f, int shift, uint32_t need, const RcQueue &Q, uint32_t &seen) {
+    const uint32_t mask = shift == 16 ? 0x7FFFu : 0xFFu;
+    const uint64_t t0 = wall_clock64();
+    for (;;) {
+        seen = __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (((seen >> shift) & mask) >= need) break;
+        if (__hip_atomic_load(Q.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return false;
+        if (wall_clock64() - t0 > Q.spinTicks) {
+            __hip_atomic_store(Q.abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return false;
+        }
+        __builtin_amdgcn_s_sleep(2);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    return true;
+}
+
+// The closed loop of the luma (PL 0) or the chroma (PL 1) of superblock sb, by the workgroup (the tables staged for its
+// image's quantizer context).  Luma reads nothing of chroma; chroma reads its own block's luma reconstruction, mode and
+// end of block and, like luma, its own plane kind's neighbours, so the two are separate items whose chains run beside
+// each other.  Q null: one launch per wavefront step (every neighbour complete, luma before chroma in one workgroup).
+// Q->fine: before each block on the superblock's left or upper edge the workgroup waits for the neighbours' samples that
+// block can read (twice its size along the edge), and after every block it publishes its own progress; blocks along the
+// right (bottom) edge of a superblock come in ascending row (column) order whatever the partition, so two counts tell
+// how far an edge is.  False: a wait failed (the schedule is being aborted).
+template <typename Px, int PL>
+__device__ bool recon_part(lds<RcShared> &S, const Batch &B, const SearchParams &P, uint32_t sb, const RcQueue *Q) {
     const int tid = threadIdx.x;
-    {   // the image's descriptor, read in place in LDS from here on
+    {   // the image's descriptor, read in place in LDS from here on, and the blocks
         static_assert(sizeof(Img) % 4 == 0, "the descriptor is copied by words");
         const uint32_t *g = (const uint32_t *)&B.img[B.sbImg[sb]];
         lds<uint32_t> *d = (lds<uint32_t> *)(lds<char> *)&S.img;
         for (int k = tid; k < (int)(sizeof(Img) / 4); k += RC_NT) d[k] = g[k];
+        const Leaf lf = B.leaves[(size_t)sb * MAX_LEAVES + tid];
+        static_assert(RC_NT == MAX_LEAVES && BLOCK_INVALID <= 32, "a thread per block, 5 + 4 + 4 bits");
+        S.leaf[tid] = (uint16_t)(lf.bsize | lf.x4 << 5 | lf.y4 << 9);
     }
     __syncthreads();
     const lds<Img> &I = S.img;
@@ -1141,24 +1194,95 @@ __device__ void recon_sb(lds<RcShared> &S, const Batch &B, const SearchParams &P
         if (yy == (16 >> ss) && xx == -1) v = 0;
         S.bdm[p][yy + 1][xx + 1] = v;
     }
-    if (tid == 0) { S.nTxb = 0; S.nCoef = 0; S.flopsOn = B.flops != nullptr; S.flops = 0; S.dcQ = dc_q(I.qindex, I.bd); S.acQ = ac_q(I.qindex, I.bd); }
+    if (tid == 0) {
+        S.flopsOn = B.flops != nullptr; S.flops = 0; S.dcQ = dc_q(I.qindex, I.bd); S.acQ = ac_q(I.qindex, I.bd);
+        for (int k = 0; k < 4; k++) S.known[k] = 0;
+    }
     __syncthreads();
     const float lambda = T.lambda[I.bd == 10][I.qindex] * P.lambdaMul;
     const int nLeaves = B.leafCount[sb];
+    // the neighbours inside the tile and how much of them the coded area holds (units of 4 luma samples)
+    const bool fine = Q && Q->fine;
+    const uint32_t *prog = fine ? Q->prog + (size_t)PL * Q->nSb + sb : nullptr;
+    const bool hasLeft = sbx > tx0, hasUp = sby > ty0, hasUpR = hasUp && (sbc + 1) * 16 < miColEnd;
+    const int inRows = min(16, I.MiRows - sbr * 16), inCols = min(16, I.MiCols - sbc * 16), inColsR = min(16, I.MiCols - sbc * 16 - 16);
+    uint32_t knL = 0, knU = 0, knR = 0, knY = 0;
+    uint32_t ownR = 0, ownB = 0;   // this superblock's edges so far
+    int nTxb = 0, nCoef = 0;       // of the superblock before the block
     for (int li = 0; li < nLeaves; li++) {
-        const Leaf lf = B.leaves[(size_t)sb * MAX_LEAVES + li];
-        const int bsize = lf.bsize, x = sbx + lf.x4 * 4, y = sby + lf.y4 * 4, mi_row = y >> 2, mi_col = x >> 2;
+        const int lf = __builtin_amdgcn_readfirstlane((int)S.leaf[li]);
+        const int bsize = lf & 31, lx4 = (lf >> 5) & 15, ly4 = lf >> 9, x = sbx + lx4 * 4, y = sby + ly4 * 4, mi_row = y >> 2, mi_col = x >> 2;
+        const int bw = bw4(bsize), bh = bh4(bsize);
         auto inside = [&](int r, int c) { return c >= (tx0 >> 2) && c < miColEnd && r >= (ty0 >> 2) && r < miRowEnd; };
-        const int availU = inside(mi_row - 1, mi_col), availL = inside(mi_row, mi_col - 1);
         const int hasC = has_chroma(bsize, mi_row, mi_col, I.mono, I.ss);
-        const int availUC = hasC ? ((I.ss && bh4(bsize) == 1) ? inside(mi_row - 2, mi_col) : availU) : 0;
-        const int availLC = hasC ? ((I.ss && bw4(bsize) == 1) ? inside(mi_row, mi_col - 2) : availL) : 0;
-        const uint32_t firstTxb = (uint32_t)S.nTxb;
         const int txSz = av1t::Max_Tx_Size_Rect[bsize];
+        int cTxb = 0, cCoef = 0;
+        if (hasC) chroma_size(I, bsize, mi_row, mi_col, cTxb, cCoef);
+        const int firstTxb = nTxb, firstCoef = nCoef;
+        nTxb += 1 + cTxb;
+        nCoef += tx_ncoef(txSz) + cCoef;
+        if (PL && !hasC) continue;
+        // the block's luma area in the superblock; chroma of a 4-sample side covers the block before it too
+        const int ax = PL && I.ss && bw == 1 ? lx4 - 1 : lx4, ay = PL && I.ss && bh == 1 ? ly4 - 1 : ly4;
+        const int aw = lx4 + bw - ax, ah = ly4 + bh - ay;
+        if (fine) {
+            const uint32_t needL = hasLeft && ax == 0 ? min(ay + 2 * ah, inRows) : 0;
+            const uint32_t needU = hasUp && ay == 0 ? min(ax + 2 * aw, inCols) : 0;
+            const uint32_t needR = hasUpR && ay == 0 && ax + 2 * aw > 16 ? min(ax + 2 * aw - 16, inColsR) : 0;
+            if ((knL & 0xFF) < needL || ((knU >> 8) & 0xFF) < needU || ((knR >> 8) & 0xFF) < needR || (PL && (int)(knY >> 16) < li + 1)) {
+                if (tid == 0) {
+                    uint32_t l = knL, u = knU, r = knR, yp = knY;
+                    bool ok = true;
+                    if (needL) ok = wait_progress(prog - 1, 0, needL, *Q, l);
+                    if (ok && needU) ok = wait_progress(prog - I.sbCols, 8, needU, *Q, u);
+                    if (ok && needR) ok = wait_progress(prog - I.sbCols + 1, 8, needR, *Q, r);
+                    if (ok && PL) ok = wait_progress(Q->prog + sb, 16, li + 1, *Q, yp);
+                    S.known[0] = ok ? l & 0x7FFFFFFFu : 0x80000000u; S.known[1] = u; S.known[2] = r; S.known[3] = yp;
+                }
+                __syncthreads();
+                knL = S.known[0]; knU = S.known[1]; knR = S.known[2]; knY = S.known[3];
+                if (knL & 0x80000000u) return false;
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            }
+        }
+        if (tid == 0) { S.nTxb = firstTxb + PL; S.nCoef = firstCoef + (PL ? tx_ncoef(txSz) : 0); }
+        RecBlock *const rb = B.oBlocks + (size_t)sb * MAX_LEAVES + li;
+        int skip = 0;
+        if constexpr (PL == 0) {
+            const int availU = inside(mi_row - 1, mi_col), availL = inside(mi_row, mi_col - 1);
 #define RC_LUMA(w, h) rc_luma<w, h, Px>(S, B, P, sb, I, bsize, x, y, availU, availL, tx0, ty0, lambda)
-        AV1M_TX_SWITCH(txSz, RC_LUMA)
+            AV1M_TX_SWITCH(txSz, RC_LUMA)
 #undef RC_LUMA
-        if (hasC) {
+            __syncthreads();
+            skip = S.winEob[0] == 0;   // of the luma; the chroma item completes the record of a block that carries chroma
+            const int yMode = S.mode;
+            for (int k = tid; k < bw * bh; k += RC_NT) {
+                const int r = mi_row + k / bw, c = mi_col + k % bw;
+                if (r < I.MiRows && c < I.MiCols) {
+                    const size_t o = (size_t)r * I.MiCols + c;
+                    map8(I.mY)[o] = (uint8_t)yMode;
+                    if (!hasC) map8(I.mSkip)[o] = (uint8_t)skip;
+                    map8(I.mMiSize)[o] = (uint8_t)bsize;
+                    map8(I.mTx)[o] = (uint8_t)txSz;
+                }
+            }
+            if (tid == 0) {
+                RecBlock b;
+                b.mi_row = (uint16_t)mi_row; b.mi_col = (uint16_t)mi_col; b.bsize = (uint8_t)bsize; b.skip = (uint8_t)skip; b.tx_depth = 0;
+                b.y_mode = (uint8_t)yMode;
+                b.angle_delta_y = (int8_t)(bsize >= BLOCK_8X8 && is_dir(yMode) ? S.delta : 0);
+                b.uv_mode = 0; b.angle_delta_uv = 0; b.cfl_alpha_u = 0; b.cfl_alpha_v = 0;
+                b.filter_intra = 0; b.cdef_idx = 0; b.sb_qindex = 0;
+                *rb = b;
+                B.oBlockTxb[(size_t)sb * MAX_LEAVES + li] = (uint16_t)firstTxb;
+                atomicAdd(&B.stats[0], 1u);
+                if (skip && !hasC) atomicAdd(&B.stats[1], 1u);
+            }
+        } else {
+            const int availUC = (I.ss && bh == 1) ? inside(mi_row - 2, mi_col) : inside(mi_row - 1, mi_col);
+            const int availLC = (I.ss && bw == 1) ? inside(mi_row, mi_col - 2) : inside(mi_row, mi_col - 1);
+            if (tid == 0) { S.mode = rb->y_mode; S.winEob[0] = !rb->skip; }
+            __syncthreads();
             const int uvTx = uv_tx_size(bsize, I.ss);
 #define RC_CHROMA(w, h) rc_chroma<w, h, Px>(S, B, P, sb, I, bsize, mi_row, mi_col, availUC, availLC, tx0, ty0, lambda * P.lambdaCMul)
             switch (uvTx) {
@@ -1169,47 +1293,46 @@ __device__ void recon_sb(lds<RcShared> &S, const Batch &B, const SearchParams &P
             case TX_8X32: RC_CHROMA(8, 32); break; default: RC_CHROMA(32, 8); break;
             }
 #undef RC_CHROMA
-        } else if (tid == 0) {
-            S.winEob[1] = S.winEob[2] = 0; S.uvMode = 0; S.uvDelta = 0; S.cflAlpha[0] = S.cflAlpha[1] = 0;
-        }
-        __syncthreads();
-        const int skip = S.winEob[0] == 0 && S.winEob[1] == 0 && S.winEob[2] == 0;
-        const int yMode = S.mode, uv = S.uvMode, bw = bw4(bsize), bh = bh4(bsize);
-        for (int k = tid; k < bw * bh; k += RC_NT) {
-            const int r = mi_row + k / bw, c = mi_col + k % bw;
-            if (r < I.MiRows && c < I.MiCols) {
-                const size_t o = (size_t)r * I.MiCols + c;
-                map8(I.mY)[o] = (uint8_t)yMode;
-                if (hasC) map8(I.mUV)[o] = (uint8_t)uv;
-                map8(I.mSkip)[o] = (uint8_t)skip;
-                map8(I.mMiSize)[o] = (uint8_t)bsize;
-                map8(I.mTx)[o] = (uint8_t)txSz;
+            __syncthreads();
+            skip = S.winEob[0] == 0 && S.winEob[1] == 0 && S.winEob[2] == 0;
+            const int uv = S.uvMode;
+            for (int k = tid; k < bw * bh; k += RC_NT) {
+                const int r = mi_row + k / bw, c = mi_col + k % bw;
+                if (r < I.MiRows && c < I.MiCols) {
+                    const size_t o = (size_t)r * I.MiCols + c;
+                    map8(I.mUV)[o] = (uint8_t)uv;
+                    map8(I.mSkip)[o] = (uint8_t)skip;
+                }
+            }
+            if (tid == 0) {
+                const bool cfl = uv == UV_CFL_PRED;
+                rb->skip = (uint8_t)skip;
+                rb->uv_mode = (uint8_t)uv;
+                rb->angle_delta_uv = (int8_t)(bsize >= BLOCK_8X8 && is_dir(uv) ? S.uvDelta : 0);
+                rb->cfl_alpha_u = (int8_t)(cfl ? S.cflAlpha[0] : 0);
+                rb->cfl_alpha_v = (int8_t)(cfl ? S.cflAlpha[1] : 0);
+                if (skip) atomicAdd(&B.stats[1], 1u);
+                if (cfl) atomicAdd(&B.stats[2], 1u);
             }
         }
-        if (tid == 0) {
-            RecBlock b;
-            b.mi_row = (uint16_t)mi_row; b.mi_col = (uint16_t)mi_col; b.bsize = (uint8_t)bsize; b.skip = (uint8_t)skip; b.tx_depth = 0;
-            b.y_mode = (uint8_t)yMode;
-            b.angle_delta_y = (int8_t)(bsize >= BLOCK_8X8 && is_dir(yMode) ? S.delta : 0);
-            b.uv_mode = (uint8_t)(hasC ? uv : 0);
-            b.angle_delta_uv = (int8_t)(hasC && bsize >= BLOCK_8X8 && is_dir(uv) ? S.uvDelta : 0);
-            const bool cfl = hasC && uv == UV_CFL_PRED;
-            b.cfl_alpha_u = (int8_t)(cfl ? S.cflAlpha[0] : 0); b.cfl_alpha_v = (int8_t)(cfl ? S.cflAlpha[1] : 0);
-            b.filter_intra = 0; b.cdef_idx = 0; b.sb_qindex = 0;
-            B.oBlocks[(size_t)sb * MAX_LEAVES + li] = b;
-            B.oBlockTxb[(size_t)sb * MAX_LEAVES + li] = (uint16_t)firstTxb;
-            atomicAdd(&B.stats[0], 1u);
-            if (skip) atomicAdd(&B.stats[1], 1u);
-            if (cfl) atomicAdd(&B.stats[2], 1u);
-        }
+        if (ax + aw == 16) ownR = ay + ah;
+        if (ay + ah == 16) ownB = ax + aw;
         __syncthreads();
+        if (fine && tid == RC_NT - 64) {   // wave 3, the one with the least to do while the next block is set up
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            __hip_atomic_store(Q->prog + (size_t)PL * Q->nSb + sb, ownR | ownB << 8 | (uint32_t)(li + 1) << 16, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
     if (tid == 0) {
-        SbOut o;
-        o.nBlocks = (uint32_t)nLeaves; o.nTxb = (uint32_t)S.nTxb; o.nCoeffs = (uint32_t)S.nCoef; o.pad = 0;
-        B.sbOut[sb] = o;
+        if constexpr (PL == 0) {
+            SbOut o;
+            o.nBlocks = (uint32_t)nLeaves; o.nTxb = (uint32_t)nTxb; o.nCoeffs = (uint32_t)nCoef; o.pad = 0;
+            B.sbOut[sb] = o;
+        }
         if (S.flopsOn && S.flops) atomicAdd(&B.flops[32 + (sb & 31)], S.flops);
     }
+    return true;
 }
 
 // RcShared allows two workgroups per compute unit.  WPE 2 holds the registers to 256 so both fit (more superblocks in
@@ -1245,29 +1368,17 @@ AV1M_RC_KERNEL(2) k_recon(RcStepArgs) {
     if (threadIdx.x == 0) S.nTeam = RC_NTEAM;
     stage_tables(S, *B.T, B.img[B.sbImg[sb]].qctx, true);
     __syncthreads();
-    recon_sb<Px>(S, B, P, sb);
+    recon_part<Px, 0>(S, B, P, sb, nullptr);
+    __syncthreads();
+    if (!S.img.mono) recon_part<Px, 1>(S, B, P, sb, nullptr);
 }
 
-// wait (thread 0) until superblock flag f is set; false when the wait ran out of time or another workgroup aborted
-__device__ bool wait_done(const uint32_t *f, const RcQueue &Q) {
-    const uint64_t t0 = wall_clock64();
-    while (__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) {
-        if (__hip_atomic_load(Q.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return false;
-        if (wall_clock64() - t0 > Q.spinTicks) {
-            __hip_atomic_store(Q.abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return false;
-        }
-        __builtin_amdgcn_s_sleep(2);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    return true;
-}
-
-// Persistent schedule: every workgroup pulls superblocks from the queue (the anti-diagonal wavefront order of all
-// images of the batch) and starts each as soon as its left and above-right (above, at a tile's right edge)
-// neighbours inside its tile are done.  Items are taken in an order where every dependency was taken earlier by a
-// running workgroup, so the waits always end; a wait that exceeds the time limit raises the abort flag, which makes
-// every workgroup stop taking items and return.
+// Persistent schedule: every workgroup pulls items (a superblock's luma or chroma) from the queue, the anti-diagonal
+// wavefront order of all images of the batch, and starts each as soon as what it depends on is done: its left and
+// above-right (above, at a tile's right edge) neighbours of the same plane kind inside its tile and, for chroma, its own
+// luma -- all of them before the item starts, or block by block (Q.fine, recon_part).  An item's dependencies stand
+// before it in the queue, so they were taken earlier by a running workgroup and the waits always end; a wait that
+// exceeds the time limit raises the abort flag, which makes every workgroup stop taking items and return.
 template <typename Px, int WPE>
 AV1M_RC_KERNEL(WPE) k_recon_queue(RcQueueArgs) {
     extern __shared__ __align__(16) char smraw[];
@@ -1284,38 +1395,46 @@ AV1M_RC_KERNEL(WPE) k_recon_queue(RcQueueArgs) {
             uint32_t it = Q.n;
             if (!__hip_atomic_load(Q.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
                 it = __hip_atomic_fetch_add(Q.head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            uint32_t sb = 0xFFFFFFFFu;
+            uint32_t item = 0xFFFFFFFFu;
             if (it < Q.n) {
-                sb = Q.order[it];
-                const Img &I = B.img[B.sbImg[sb]];
-                const uint32_t local = sb - I.sbBase;
-                const int c = (int)(local % I.sbCols), r = (int)(local / I.sbCols);
-                int tc = 0, tr = 0;
-                while (tc + 1 < I.tileCols && c * 16 >= I.tileColStart[tc + 1]) tc++;
-                while (tr + 1 < I.tileRows && r * 16 >= I.tileRowStart[tr + 1]) tr++;
-                const int c0 = I.tileColStart[tc] >> 4, c1 = (I.tileColStart[tc + 1] + 15) >> 4, r0 = I.tileRowStart[tr] >> 4;
-                bool ok = true;
-                if (c > c0) ok = wait_done(Q.done + sb - 1, Q);
-                if (ok && r > r0) ok = wait_done(Q.done + sb - I.sbCols + (c + 1 < c1 ? 1 : 0), Q);
-                if (!ok) sb = 0xFFFFFFFFu;
+                item = Q.order[it];
+                if (!Q.fine) {
+                    const uint32_t sb = item & ~RC_CHROMA, *prog = Q.prog + ((item & RC_CHROMA) ? Q.nSb : 0) + sb;
+                    const Img &I = B.img[B.sbImg[sb]];
+                    const uint32_t local = sb - I.sbBase;
+                    const int c = (int)(local % I.sbCols), r = (int)(local / I.sbCols);
+                    int tc = 0, tr = 0;
+                    while (tc + 1 < I.tileCols && c * 16 >= I.tileColStart[tc + 1]) tc++;
+                    while (tr + 1 < I.tileRows && r * 16 >= I.tileRowStart[tr + 1]) tr++;
+                    const int c0 = I.tileColStart[tc] >> 4, c1 = (I.tileColStart[tc + 1] + 15) >> 4, r0 = I.tileRowStart[tr] >> 4;
+                    bool ok = true;
+                    uint32_t seen;
+                    if (item & RC_CHROMA) ok = wait_progress(Q.prog + sb, 0, 16, Q, seen);
+                    if (ok && c > c0) ok = wait_progress(prog - 1, 0, 16, Q, seen);
+                    if (ok && r > r0) ok = wait_progress(prog - I.sbCols + (c + 1 < c1 ? 1 : 0), 0, 16, Q, seen);
+                    if (!ok) item = 0xFFFFFFFFu;
+                }
             }
-            S.qItem = sb;
+            S.qItem = item;
         }
         __syncthreads();
-        const uint32_t sb = S.qItem;
-        if (sb == 0xFFFFFFFFu) break;
+        const uint32_t item = S.qItem;
+        if (item == 0xFFFFFFFFu) break;
         // the neighbours' reconstruction, maps and contexts were published with release at agent scope
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        const uint32_t sb = item & ~RC_CHROMA;
         const int qctx = B.img[B.sbImg[sb]].qctx;
         if (qctx != staged) {
             stage_tables(S, *B.T, qctx, staged < 0);
             staged = qctx;
         }
         __syncthreads();
-        recon_sb<Px>(S, B, P, sb);
+        const bool ok = (item & RC_CHROMA) ? recon_part<Px, 1>(S, B, P, sb, &Q) : recon_part<Px, 0>(S, B, P, sb, &Q);
+        if (!ok) break;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
         __syncthreads();
-        if (tid == 0) __hip_atomic_store(Q.done + sb, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (tid == 0)   // complete: both edges and every block
+            __hip_atomic_store(Q.prog + ((item & RC_CHROMA) ? Q.nSb : 0) + sb, 0x7FFF1010u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 

@@ -8,7 +8,8 @@
 
 namespace av1m {
 
-constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)AV1MI_NOALLOC_SCRATCH_MIB << 20;
+// (the last 64 KiB hold the closed loop's item order and progress words: 16 bytes for each of the at most 3.9 k superblocks)
+constexpr size_t NOALLOC_SCRATCH_BYTES = ((size_t)AV1MI_NOALLOC_SCRATCH_MIB << 20) + (64 << 10);
 
 static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
 
