@@ -2,6 +2,7 @@
 // dequantizer and inverse transforms, intra prediction primitives, and the structures the kernels exchange.
 // Compiled by hipcc for gfx950 device code and for the host side of the library.
 #pragma once
+#include <math.h>
 #include <stdint.h>
 #include "av1_spec_tables.h"
 
@@ -126,6 +127,16 @@ AV1M_HD int dq_denom(int t) {
 }
 AV1M_HD int dc_q(int q, int bd) { return av1t::Dc_Qlookup[(bd - 8) >> 1][clip3(0, 255, q)]; }
 AV1M_HD int ac_q(int q, int bd) { return av1t::Ac_Qlookup[(bd - 8) >> 1][clip3(0, 255, q)]; }
+// n / d rounded to nearest for d an integer step (4 .. 2^15) and y = 1 / d rounded to nearest: Markstein's correction
+// (P. W. Markstein, "Computation of elementary functions on the IBM RISC System/6000 processor", 1990).  n - q d is exact
+// in one fma while q is near n / d, so the first correction brings q (two roundings off) within one unit in the last
+// place, and from there q + r y rounds to n / d.  Quotients too small for that (n - q d below the smallest normal number)
+// lie under every dead zone.  Five operations where a division that has no reciprocal at hand takes about eleven.
+AV1M_HD float quot_step(float n, float d, float y) {
+    float q = n * y;
+    q = fmaf(fmaf(-q, d, n), y, q);
+    return fmaf(fmaf(-q, d, n), y, q);
+}
 // spec 7.12.3 step 1 without quantizer matrices: |level * q| & 0xFFFFFF, / dqDenom (a shift: 1, 2, 4), clamp 2^(7+bd)
 AV1M_HD int dequant(int level, int q, int denShift, int bd) {
     const int dq = level * q;

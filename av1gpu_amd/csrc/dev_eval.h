@@ -98,6 +98,7 @@ __device__ __forceinline__ int gargmin(float v, int i) {
 template <typename CP>
 struct EvalInT {
     int txSz, txType, plane, dcQ, acQ, skipCtx, dcCtx, intraDir, bd;
+    float dcRcp, acRcp;   // 1 / dcQ, 1 / acQ rounded to nearest
     float rnd, zbin, resEnergy;
     CP C;
 };
@@ -144,58 +145,57 @@ __device__ float base_bits(const E &e, int eob) {
     return b;
 }
 
-// scan position of index c in a tx block of the adjusted size TW x TH: class VERT scans rows (raster order), HORIZ
-// columns (Mrow / Mcol scans), 2D the default zig-zag scan dscan
-template <int TW, int TH, int CLS, typename SP>
-__device__ __forceinline__ int scan_pos(int c, SP dscan) {
-    if constexpr (CLS == TX_CLASS_VERT) return c;
-    else if constexpr (CLS == TX_CLASS_HORIZ) return (c % TH) * TW + c / TH;
-    else return dscan[c];
-}
-
-// bits of the coefficient at scan position c (< eob) of a tx block of size TSZ and class CLS given the levels q
-// (natural order, stride = adjusted width); cbOff: Coeff_Base_Ctx_Offset[TSZ] (5 x 5)
-template <int TSZ, int CLS, typename QP, typename SP, typename OP, typename CT>
-__device__ float coeff_bits(int c, int eob, QP q, SP dscan, OP cbOff, int pt, int dcCtx, const CT &C) {
+// Bits of the coefficient at scan position c (< eob) of a tx block of size TSZ given the levels q (natural order, stride =
+// adjusted width); sk: the scan and context class (0: 2D, default zig-zag scan dscan; 1: HORIZ, columns; 2: VERT, rows),
+// always 0 for sizes with a side over 16; cbOff: Coeff_Base_Ctx_Offset[TSZ] (5 x 5).
+// One path for the three classes, whose neighbour positions differ in data only, so the lanes of a wave that evaluate
+// different tx types do not run the classes one after the other; the five neighbours are read once for both contexts.
+template <int TSZ, typename QP, typename SP, typename OP, typename CT>
+__device__ __forceinline__ float coeff_bits(int c, int eob, int sk, QP q, SP dscan, OP cbOff, int pt, int dcCtx, const CT &C) {
     constexpr int ctx = txsz_ctx_of(TSZ), adj = av1t::Adjusted_Tx_Size[TSZ];
-    constexpr int bwl = av1t::Tx_Width_Log2[adj], width = 1 << bwl, height = av1t::Tx_Height[adj];
-    const int pos = scan_pos<width, height, CLS>(c, dscan), qv = q[pos], v = qv < 0 ? -qv : qv, level = v < 15 ? v : 15;
-    const int row = pos >> bwl, col = pos - (row << bwl);
-    float b;
-    if (c == eob - 1) {
-        const int bctx = c == 0 ? 0 : c <= (height << bwl) / 8 ? 1 : c <= (height << bwl) / 4 ? 2 : 3;
-        b = C.coeff_base_eob[ctx][pt][bctx][min(level, 3) - 1];
-    } else {
-        int mag = 0;
-#pragma unroll
-        for (int k = 0; k < 5; k++) {
-            const int rr = row + av1t::Sig_Ref_Diff_Offset[CLS][k][0], cc = col + av1t::Sig_Ref_Diff_Offset[CLS][k][1];
-            if (rr < height && cc < width) { const int a = q[(rr << bwl) + cc]; mag += min(a < 0 ? -a : a, 3); }
-        }
-        int bctx = min((mag + 1) >> 1, 4);
-        if constexpr (CLS == TX_CLASS_2D) bctx = (row == 0 && col == 0) ? 0 : bctx + cbOff[min(row, 4) * 5 + min(col, 4)];
-        else bctx += min(CLS == TX_CLASS_VERT ? row : col, 2) == 0 ? av1t::Coeff_Base_Pos_Ctx_Offset[0]
-                   : min(CLS == TX_CLASS_VERT ? row : col, 2) == 1 ? av1t::Coeff_Base_Pos_Ctx_Offset[1] : av1t::Coeff_Base_Pos_Ctx_Offset[2];
-        b = C.coeff_base[ctx][pt][bctx][min(level, 3)];
+    constexpr int bwl = av1t::Tx_Width_Log2[adj], width = 1 << bwl, lbh = av1t::Tx_Height_Log2[adj], height = 1 << lbh;
+    constexpr bool only2d = width > 16 || height > 16;
+    int pos = dscan[c];
+    if constexpr (!only2d) pos = sk == 0 ? pos : sk == 1 ? ((c & (height - 1)) << bwl) + (c >> lbh) : c;
+    const int row = pos >> bwl, col = pos & (width - 1);
+    auto at = [&](int dr, int dc) -> int {   // |level| of the neighbour at (row + dr, col + dc), 0 outside
+        const bool in = row + dr < height && col + dc < width;
+        const int a = q[in ? pos + (dr << bwl) + dc : pos];
+        return in ? (a < 0 ? -a : a) : 0;
+    };
+    static_assert(av1t::Sig_Ref_Diff_Offset[0][2][0] == 1 && av1t::Sig_Ref_Diff_Offset[1][2][1] == 2 && av1t::Sig_Ref_Diff_Offset[2][4][0] == 4,
+                  "neighbour order: right, below, then the class's own three");
+    int a2, a3, a4;
+    const int qv = q[pos], a0 = at(0, 1), a1 = at(1, 0);
+    if constexpr (only2d) {
+        a2 = at(1, 1); a3 = at(0, 2); a4 = at(2, 0);
+    } else {   // the class's own three: (1,1) (0,2) (2,0) / (0,2) (0,3) (0,4) / (2,0) (3,0) (4,0)
+        a2 = at(sk == 2 ? 2 : 1 - sk, sk == 2 ? 0 : 1 + sk);
+        a3 = at(sk == 2 ? 3 : 0, sk == 2 ? 0 : 2 + sk);
+        a4 = at(sk == 2 ? 4 : sk == 1 ? 0 : 2, sk == 1 ? 4 : 0);
     }
+    const int v = qv < 0 ? -qv : qv, level = v < 15 ? v : 15;
+    const int m5 = min(a0, 3) + min(a1, 3) + min(a2, 3) + min(a3, 3) + min(a4, 3);
+    const int m = min((m5 + 1) >> 1, 4);
+    int bctx = pos == 0 ? 0 : m + (int)cbOff[min(row, 4) * 5 + min(col, 4)];
+    if constexpr (!only2d) {
+        static_assert(av1t::Coeff_Base_Pos_Ctx_Offset[0] == 26 && av1t::Coeff_Base_Pos_Ctx_Offset[1] == 31 && av1t::Coeff_Base_Pos_Ctx_Offset[2] == 36,
+                      "26 + 5 min(position, 2)");
+        bctx = sk == 0 ? bctx : m + 26 + 5 * min(sk == 1 ? col : row, 2);
+    }
+    const int ectx = c == 0 ? 0 : c <= (height << bwl) / 8 ? 1 : c <= (height << bwl) / 4 ? 2 : 3;
+    const auto *pb = c == eob - 1 ? &C.coeff_base_eob[ctx][pt][ectx][min(max(level, 1), 3) - 1] : &C.coeff_base[ctx][pt][bctx][min(level, 3)];
+    float b = *pb;
     if (level > 2) {
-        int mag = 0;
+        const int mb = min((min(a0, 15) + min(a1, 15) + min(a2, 15) + 1) >> 1, 6);
+        bool near0 = row < 2 && col < 2;
+        if constexpr (!only2d) near0 = sk == 0 ? near0 : sk == 1 ? col == 0 : row == 0;
+        const auto *br = C.coeff_br[min(ctx, (int)TX_32X32)][pt][pos == 0 ? mb : near0 ? mb + 7 : mb + 14];
+        // up to four symbols of at most 3: n3 full ones, then the rest
+        const int rem = level - 3, n3 = (rem * 11) >> 5;   // rem / 3 for 0 .. 12
+        const float full = br[3], rest = br[rem - 3 * n3];
 #pragma unroll
-        for (int k = 0; k < 3; k++) {
-            const int rr = row + av1t::Mag_Ref_Offset_With_Tx_Class[CLS][k][0], cc = col + av1t::Mag_Ref_Offset_With_Tx_Class[CLS][k][1];
-            if (rr < height && cc < width) { const int a = q[rr * width + cc]; mag += min(a < 0 ? -a : a, 15); }
-        }
-        mag = min((mag + 1) >> 1, 6);
-        const int brctx = pos == 0 ? mag : CLS == TX_CLASS_2D ? ((row < 2 && col < 2) ? mag + 7 : mag + 14)
-                        : CLS == TX_CLASS_HORIZ ? (col == 0 ? mag + 7 : mag + 14) : (row == 0 ? mag + 7 : mag + 14);
-        const auto *br = C.coeff_br[min(ctx, (int)TX_32X32)][pt][brctx];
-        int rem = level - 3;
-        for (int i = 0; i < 4; i++) {
-            const int k = min(rem, 3);
-            b += br[k];
-            rem -= k;
-            if (k < 3) break;
-        }
+        for (int i = 0; i < 4; i++) b = i < n3 ? b + full : i == n3 ? b + rest : b;
     }
     if (v) {
         b += c == 0 ? C.dc_sign[pt][dcCtx][qv < 0] : 1.0f;
@@ -204,14 +204,14 @@ __device__ float coeff_bits(int c, int eob, QP q, SP dscan, OP cbOff, int pt, in
     return b;
 }
 
-// eob and rate of the levels q of a tx block of size TSZ, class CLS, by the group (all lanes return both); last: the
+// eob and rate of the levels q of a tx block of size TSZ, class sk, by the group (all lanes return both); last: the
 // lane's share of the eob (1 + the largest scan index of a nonzero level among the positions the lane quantized)
-template <int TSZ, int CLS, typename QP, typename SP, typename OP, typename E>
-__device__ void grp_rate(QP q, SP dscan, OP cbOff, const E &e, int last, int &eobOut, float &bitsOut) {
+template <int TSZ, typename QP, typename SP, typename OP, typename E>
+__device__ __forceinline__ void grp_rate(QP q, SP dscan, OP cbOff, const E &e, int sk, int last, int &eobOut, float &bitsOut) {
     const int lane = glane();
     const int eob = gmaxi(last);
     float bits = lane == 0 ? base_bits<TSZ>(e, eob) : 0.f;
-    for (int c = lane; c < eob; c += GW) bits += coeff_bits<TSZ, CLS>(c, eob, q, dscan, cbOff, e.plane > 0, e.dcCtx, *e.C);
+    for (int c = lane; c < eob; c += GW) bits += coeff_bits<TSZ>(c, eob, sk, q, dscan, cbOff, e.plane > 0, e.dcCtx, *e.C);
     eobOut = eob;
     bitsOut = gsum(bits);
 }
@@ -328,7 +328,7 @@ __device__ __forceinline__ EvalOut grp_qrate(FP tmp, int ts, QP q, const E &e, c
     for (int idx = lane; idx < N; idx += GW) {
         const float v = tmp[(idx >> LTW) * ts + (idx & (TW - 1))];
         const int step = idx == 0 ? e.dcQ : e.acQ;
-        const float a = fabsf(v) * (float)den / (float)step;
+        const float a = quot_step(fabsf(v) * (float)den, (float)step, idx == 0 ? e.dcRcp : e.acRcp);
         int l = a < e.zbin ? 0 : (int)(a + e.rnd);
         l = min(l, 16383);
         const int qv = v < 0 ? -l : l;
@@ -349,9 +349,7 @@ __device__ __forceinline__ EvalOut grp_qrate(FP tmp, int ts, QP q, const E &e, c
     const auto cbOff = cboff_ptr<TSZ>(T);
     int eob;
     EvalOut o;
-    if (sk == 0) grp_rate<TSZ, TX_CLASS_2D>(q, dscan, cbOff, e, last, eob, o.R);
-    else if (sk == 1) grp_rate<TSZ, TX_CLASS_HORIZ>(q, dscan, cbOff, e, last, eob, o.R);
-    else grp_rate<TSZ, TX_CLASS_VERT>(q, dscan, cbOff, e, last, eob, o.R);
+    grp_rate<TSZ>(q, dscan, cbOff, e, sk, last, eob, o.R);
     const float g = T.txg[e.txSz][e.txType];
     o.D = g * distS;
     if (W == 64 || H == 64) {
@@ -393,7 +391,7 @@ __device__ EvalOut half_qrate(FP tmp, int ts, QP q, const E &e, const TT &T) {
         for (int idx = lane + 16 * h; idx < N; idx += GW) {
             const float v = tmp[(idx >> LTW) * ts + (idx & (TW - 1))];
             const int step = idx == 0 ? e.dcQ : e.acQ;
-            const float a = fabsf(v) * (float)den / (float)step;
+            const float a = quot_step(fabsf(v) * (float)den, (float)step, idx == 0 ? e.dcRcp : e.acRcp);
             int l = a < e.zbin ? 0 : (int)(a + e.rnd);
             l = min(l, 16383);
             const int qv = v < 0 ? -l : l;
@@ -413,15 +411,13 @@ __device__ EvalOut half_qrate(FP tmp, int ts, QP q, const E &e, const TT &T) {
     const auto cbOff = cboff_ptr<TSZ>(T);
     const int eob = hmaxi(last);
     float b0 = lane == 0 ? base_bits<TSZ>(e, eob) : 0.f, b1 = 0.f;
-    if (sk == 0) {
-        for (int c = lane; c < eob; c += GW) b0 += coeff_bits<TSZ, TX_CLASS_2D>(c, eob, q, dscan, cbOff, e.plane > 0, e.dcCtx, *e.C);
-        for (int c = lane + 16; c < eob; c += GW) b1 += coeff_bits<TSZ, TX_CLASS_2D>(c, eob, q, dscan, cbOff, e.plane > 0, e.dcCtx, *e.C);
-    } else if (sk == 1) {
-        for (int c = lane; c < eob; c += GW) b0 += coeff_bits<TSZ, TX_CLASS_HORIZ>(c, eob, q, dscan, cbOff, e.plane > 0, e.dcCtx, *e.C);
-        for (int c = lane + 16; c < eob; c += GW) b1 += coeff_bits<TSZ, TX_CLASS_HORIZ>(c, eob, q, dscan, cbOff, e.plane > 0, e.dcCtx, *e.C);
-    } else {
-        for (int c = lane; c < eob; c += GW) b0 += coeff_bits<TSZ, TX_CLASS_VERT>(c, eob, q, dscan, cbOff, e.plane > 0, e.dcCtx, *e.C);
-        for (int c = lane + 16; c < eob; c += GW) b1 += coeff_bits<TSZ, TX_CLASS_VERT>(c, eob, q, dscan, cbOff, e.plane > 0, e.dcCtx, *e.C);
+    // the lane's two virtual lanes side by side: their chains of reads overlap
+    for (int c = lane; c < eob; c += GW) {
+        const int d = c + 16 < N ? c + 16 : c;
+        const float v0 = coeff_bits<TSZ>(c, eob, sk, q, dscan, cbOff, e.plane > 0, e.dcCtx, *e.C);
+        const float v1 = coeff_bits<TSZ>(d, eob, sk, q, dscan, cbOff, e.plane > 0, e.dcCtx, *e.C);
+        b0 += v0;
+        if (c + 16 < eob) b1 += v1;
     }
     EvalOut o;
     o.R = hsum2(b0, b1);

@@ -359,7 +359,8 @@ __global__ void __launch_bounds__(an_groups(W, H) * 32) __attribute__((amdgpu_wa
         const int hasC = has_chroma(BS, y >> 2, x >> 2, I.mono, I.ss);
         const float overhead = (hasC ? P.uvOverheadBits : 0.f) + T.avgSkip0;
         EvalIn e;
-        e.txSz = TXS; e.plane = 0; e.dcQ = dc_q(I.qindex, bd); e.acQ = ac_q(I.qindex, bd); e.skipCtx = 0; e.dcCtx = 0;
+        e.txSz = TXS; e.plane = 0; e.dcQ = dc_q(I.qindex, bd); e.acQ = ac_q(I.qindex, bd);
+        e.dcRcp = 1.f / (float)e.dcQ; e.acRcp = 1.f / (float)e.acQ; e.skipCtx = 0; e.dcCtx = 0;
         e.bd = bd; e.rnd = P.rnd; e.zbin = P.zbin; e.resEnergy = 0.f; e.C = &C; e.intraDir = 0; e.txType = 0;
         float bestJ = INF;
         int bestK = 0, bestTx = DCT_DCT, resK = -1;

@@ -94,6 +94,7 @@ struct RcShared {
     uint16_t srcb[64 * 64];                  // source block of the current leaf: luma W x H, or U at 0 and V at 2048
     Img img;                                 // descriptor of the superblock's image
     int dcQ, acQ;                            // its quantizer steps
+    float dcRcp, acRcp;                      // 1 / dcQ, 1 / acQ
     uint16_t ea[3][EDGE_LEN], el[3][EDGE_LEN];   // unfiltered edges of the current tx block per plane
     int dcv[3], ft[3], hvL[3], hvA[3], px[3], py[3], mx[3], my[3];
     int skipCtx[3], dcCtx[3];
@@ -260,7 +261,7 @@ __device__ EvalOut grp_task(lds<RcShared> &S, lds<RcGroup> &X, const lds<Img> &I
                             lds<int16_t> *lev, const SearchParams &P) {
     RcEvalIn e;
     e.txSz = tx_of(W, H); e.txType = t; e.plane = p;
-    e.dcQ = S.dcQ; e.acQ = S.acQ;
+    e.dcQ = S.dcQ; e.acQ = S.acQ; e.dcRcp = S.dcRcp; e.acRcp = S.acRcp;
     e.skipCtx = S.skipCtx[p]; e.dcCtx = S.dcCtx[p]; e.intraDir = p == 0 ? cand_mode(c) : 0; e.bd = I.bd;
     e.rnd = p ? P.rndC : P.rnd; e.zbin = p ? P.zbinC : P.zbin;
     e.resEnergy = 0.f;
@@ -273,7 +274,7 @@ __device__ EvalOut half_task(lds<RcShared> &S, lds<float> *tmp, const lds<Img> &
                              lds<int16_t> *lev, const SearchParams &P) {
     RcEvalIn e;
     e.txSz = tx_of(W, H); e.txType = t; e.plane = p;
-    e.dcQ = S.dcQ; e.acQ = S.acQ;
+    e.dcQ = S.dcQ; e.acQ = S.acQ; e.dcRcp = S.dcRcp; e.acRcp = S.acRcp;
     e.skipCtx = S.skipCtx[p]; e.dcCtx = S.dcCtx[p]; e.intraDir = p == 0 ? cand_mode(c) : 0; e.bd = I.bd;
     e.rnd = p ? P.rndC : P.rnd; e.zbin = p ? P.zbinC : P.zbin;
     e.resEnergy = 0.f;
@@ -315,7 +316,7 @@ __device__ EvalOut grp_task_big(lds<RcShared> &S, lds<RcTeam> &X, const lds<Img>
     RcEvalIn e;
     e.resEnergy = grp_fwd_dct<W, H>(X.tmp, T, S.tab.txScale[txSz], res);
     e.txSz = txSz; e.txType = DCT_DCT; e.plane = p;
-    e.dcQ = S.dcQ; e.acQ = S.acQ;
+    e.dcQ = S.dcQ; e.acQ = S.acQ; e.dcRcp = S.dcRcp; e.acRcp = S.acRcp;
     e.skipCtx = S.skipCtx[p]; e.dcCtx = S.dcCtx[p]; e.intraDir = p == 0 ? cand_mode(c) : 0; e.bd = bd;
     e.rnd = p ? P.rndC : P.rnd; e.zbin = p ? P.zbinC : P.zbin;
     e.C = &S.tab.cost;
@@ -516,8 +517,11 @@ __device__ __forceinline__ void wg_run_tasks(lds<RcShared> &S, const lds<Img> &I
                              S.u.s.res[t], I.bd);
             __syncthreads();
         }
-        const int h = lane >> 4;
-        for (int t = 2 * g + h; t < S.nTask; t += 2 * RC_NG) {
+        // slot -> task with the candidates of one tx type side by side (the luma tasks are candidate-major), so the four
+        // halves of a wave mostly run the same kinds of pass
+        const int h = lane >> 4, nc = lumaBits && S.nTask % S.nCand == 0 ? S.nCand : 1, nt = S.nTask / nc;
+        for (int s = 2 * g + h; s < S.nTask; s += 2 * RC_NG) {
+            const int t = (s % nc) * nt + s / nc;
             const int c = S.taskC[t], tt = S.taskT[t], p = S.taskP[t];
             const EvalOut o = half_task<W, H>(S, S.u.s.g[g].tmp + h * 136, I, p, c, tt, S.u.s.res[lumaBits ? S.taskK[t] : t], S.u.s.lev + t * (W * H), P);
             float J;
@@ -1196,6 +1200,7 @@ __device__ bool recon_part(lds<RcShared> &S, const Batch &B, const SearchParams 
     }
     if (tid == 0) {
         S.flopsOn = B.flops != nullptr; S.flops = 0; S.dcQ = dc_q(I.qindex, I.bd); S.acQ = ac_q(I.qindex, I.bd);
+        S.dcRcp = 1.f / (float)S.dcQ; S.acRcp = 1.f / (float)S.acQ;
         for (int k = 0; k < 4; k++) S.known[k] = 0;
     }
     __syncthreads();
