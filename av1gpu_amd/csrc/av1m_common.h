@@ -742,7 +742,6 @@ struct RcQueue {
     uint32_t *head;              // next item to take
     uint32_t *prog;              // [2][nSb] progress of each superblock's luma and chroma: bits 0-7 rows (of 4 luma samples)
                                  // of its right edge, 8-15 columns of its bottom edge, 16-31 blocks that are complete
-    int fine;                    // published after every block, else when the superblock is complete
     uint32_t *abort;             // raised by a wait that ran out of time
     uint64_t spinTicks;          // wait limit in wall-clock ticks
 };

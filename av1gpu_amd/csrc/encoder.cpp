@@ -789,28 +789,17 @@ static int encode_impl(av1mi_encoder *enc, const av1mi_frame_in *in, int n, av1m
     const int wpe = occ ? occ : (uint64_t)nSb >= (uint64_t)std::max(1, enc->cus) * std::max<size_t>(1, steps.size()) ? 2 : 1;
     const int slots = enc->slots[bd == 10][wpe - 1] > 0 ? enc->slots[bd == 10][wpe - 1] : 1;
     const uint32_t qBlocks = enc->cfg.queueBlocks > 0 ? (uint32_t)enc->cfg.queueBlocks : (uint32_t)std::max(1, enc->cus * slots);
-    // Progress per block when the workgroups outnumber what the wavefront keeps ready: a superblock then starts beside
-    // its unfinished neighbours and its chroma runs one block behind its luma.  Else per superblock, the chroma of a step
-    // behind the luma of the next one, so that no workgroup is held by a wait.
-    // One 512 x 512 image (128 items, 22 steps): 20.2 ms per block on MI355X, 48.7 ms with the whole superblock as one item.
-    const bool fine = (uint64_t)nItems <= (uint64_t)qBlocks * std::max<size_t>(1, steps.size());
+    // The persistent schedule's items, the chroma of a step behind the luma of the next one: progress is published per
+    // block, so an item runs beside its unfinished neighbours, and the lag keeps workgroups from being held by chroma
+    // that waits for its luma (16 images of 12 MP, closed loop on MI355X: 94 ms; 105 ms with each superblock's chroma
+    // right behind its luma, 116 ms with neighbours complete before an item starts).
     std::vector<uint32_t> order;
     order.reserve(nItems);
-    {
-        auto luma = [&](size_t k) { for (uint32_t sb : steps[k]) order.push_back(sb); };
-        auto chroma = [&](size_t k) { for (uint32_t sb : steps[k]) if (!imgs[sbImg[sb]].mono) order.push_back(sb | RC_CHROMA); };
-        for (size_t k = 0; k < steps.size(); k++) {
-            if (fine) {
-                for (uint32_t sb : steps[k]) {
-                    order.push_back(sb);
-                    if (!imgs[sbImg[sb]].mono) order.push_back(sb | RC_CHROMA);
-                }
-            } else {
-                luma(k);
-                if (k) chroma(k - 1);
-                if (k + 1 == steps.size()) chroma(k);
-            }
-        }
+    for (size_t k = 0; k <= steps.size(); k++) {
+        if (k < steps.size()) order.insert(order.end(), steps[k].begin(), steps[k].end());
+        if (k)
+            for (uint32_t sb : steps[k - 1])
+                if (!imgs[sbImg[sb]].mono) order.push_back(sb | RC_CHROMA);
     }
     // ---- device memory: stream-ordered per call, or the captured plan's (graph mode) ----
     bool capture = false;
@@ -824,7 +813,7 @@ static int encode_impl(av1mi_encoder *enc, const av1mi_frame_in *in, int n, av1m
         A.bind(na->mem);
     } else if (graph) {
         std::vector<uint64_t> key = sig;
-        key.insert(key.end(), {(uint64_t)anS, (uint64_t)sched, (uint64_t)qBlocks, (uint64_t)A.total, (uint64_t)wpe, (uint64_t)fine});
+        key.insert(key.end(), {(uint64_t)anS, (uint64_t)sched, (uint64_t)qBlocks, (uint64_t)A.total, (uint64_t)wpe});
         if (enc->plan.key != key) {
             drop_plan(enc);
             HCK(hipMalloc(&enc->plan.mem, A.total));
@@ -893,7 +882,7 @@ static int encode_impl(av1mi_encoder *enc, const av1mi_frame_in *in, int n, av1m
             for (size_t k = 0; k + 1 < stepOff.size(); k++) launch_recon(B, P, dSteps + stepOff[k], stepOff[k + 1] - stepOff[k], bd, s);
         } else {
             RcQueue Q;
-            Q.order = dOrder; Q.n = nItems; Q.nSb = nSb; Q.head = dQctl; Q.abort = dQctl + 1; Q.prog = dProg; Q.fine = fine;
+            Q.order = dOrder; Q.n = nItems; Q.nSb = nSb; Q.head = dQctl; Q.abort = dQctl + 1; Q.prog = dProg;
             Q.spinTicks = enc->clockHz * 30;   // no legitimate wait comes near 30 s
             launch_recon_queue(B, P, Q, std::min<uint32_t>(qBlocks, nItems), bd, wpe, s);
         }

@@ -1163,10 +1163,10 @@ __device__ bool wait_progress(const uint32_t *f, int shift, uint32_t need, const
 // image's quantizer context).  Luma reads nothing of chroma; chroma reads its own block's luma reconstruction, mode and
 // end of block and, like luma, its own plane kind's neighbours, so the two are separate items whose chains run beside
 // each other.  Q null: one launch per wavefront step (every neighbour complete, luma before chroma in one workgroup).
-// Q->fine: before each block on the superblock's left or upper edge the workgroup waits for the neighbours' samples that
-// block can read (twice its size along the edge), and after every block it publishes its own progress; blocks along the
-// right (bottom) edge of a superblock come in ascending row (column) order whatever the partition, so two counts tell
-// how far an edge is.  False: a wait failed (the schedule is being aborted).
+// Else, before each block on the superblock's left or upper edge the workgroup waits for the neighbours' samples that
+// block can read (twice its size along the edge) and for chroma for its luma, and after every block it publishes its own
+// progress; blocks along the right (bottom) edge of a superblock come in ascending row (column) order whatever the
+// partition, so two counts tell how far an edge is.  False: a wait failed (the schedule is being aborted).
 template <typename Px, int PL>
 __device__ bool recon_part(lds<RcShared> &S, const Batch &B, const SearchParams &P, uint32_t sb, const RcQueue *Q) {
     const int tid = threadIdx.x;
@@ -1207,8 +1207,7 @@ __device__ bool recon_part(lds<RcShared> &S, const Batch &B, const SearchParams 
     const float lambda = T.lambda[I.bd == 10][I.qindex] * P.lambdaMul;
     const int nLeaves = B.leafCount[sb];
     // the neighbours inside the tile and how much of them the coded area holds (units of 4 luma samples)
-    const bool fine = Q && Q->fine;
-    const uint32_t *prog = fine ? Q->prog + (size_t)PL * Q->nSb + sb : nullptr;
+    uint32_t *const prog = Q ? Q->prog + (size_t)PL * Q->nSb + sb : nullptr;
     const bool hasLeft = sbx > tx0, hasUp = sby > ty0, hasUpR = hasUp && (sbc + 1) * 16 < miColEnd;
     const int inRows = min(16, I.MiRows - sbr * 16), inCols = min(16, I.MiCols - sbc * 16), inColsR = min(16, I.MiCols - sbc * 16 - 16);
     uint32_t knL = 0, knU = 0, knR = 0, knY = 0;
@@ -1230,7 +1229,7 @@ __device__ bool recon_part(lds<RcShared> &S, const Batch &B, const SearchParams 
         // the block's luma area in the superblock; chroma of a 4-sample side covers the block before it too
         const int ax = PL && I.ss && bw == 1 ? lx4 - 1 : lx4, ay = PL && I.ss && bh == 1 ? ly4 - 1 : ly4;
         const int aw = lx4 + bw - ax, ah = ly4 + bh - ay;
-        if (fine) {
+        if (Q) {
             const uint32_t needL = hasLeft && ax == 0 ? min(ay + 2 * ah, inRows) : 0;
             const uint32_t needU = hasUp && ay == 0 ? min(ax + 2 * aw, inCols) : 0;
             const uint32_t needR = hasUpR && ay == 0 && ax + 2 * aw > 16 ? min(ax + 2 * aw - 16, inColsR) : 0;
@@ -1323,10 +1322,9 @@ __device__ bool recon_part(lds<RcShared> &S, const Batch &B, const SearchParams 
         if (ax + aw == 16) ownR = ay + ah;
         if (ay + ah == 16) ownB = ax + aw;
         __syncthreads();
-        if (fine && tid == RC_NT - 64) {   // wave 3, the one with the least to do while the next block is set up
+        if (Q && tid == RC_NT - 64) {   // wave 3, the one with the least to do while the next block is set up
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-            __hip_atomic_store(Q->prog + (size_t)PL * Q->nSb + sb, ownR | ownB << 8 | (uint32_t)(li + 1) << 16, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(prog, ownR | ownB << 8 | (uint32_t)(li + 1) << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
     if (tid == 0) {
@@ -1379,10 +1377,10 @@ AV1M_RC_KERNEL(2) k_recon(RcStepArgs) {
 }
 
 // Persistent schedule: every workgroup pulls items (a superblock's luma or chroma) from the queue, the anti-diagonal
-// wavefront order of all images of the batch, and starts each as soon as what it depends on is done: its left and
-// above-right (above, at a tile's right edge) neighbours of the same plane kind inside its tile and, for chroma, its own
-// luma -- all of them before the item starts, or block by block (Q.fine, recon_part).  An item's dependencies stand
-// before it in the queue, so they were taken earlier by a running workgroup and the waits always end; a wait that
+// wavefront order of all images of the batch, and runs it beside what it depends on: its left, above and above-right
+// neighbours of the same plane kind inside its tile and, for chroma, its own luma (recon_part waits block by block).  An
+// item's dependencies stand before it in the queue, so they were taken earlier by a running workgroup and the waits
+// always end; a wait that
 // exceeds the time limit raises the abort flag, which makes every workgroup stop taking items and return.
 template <typename Px, int WPE>
 AV1M_RC_KERNEL(WPE) k_recon_queue(RcQueueArgs) {
@@ -1400,33 +1398,11 @@ AV1M_RC_KERNEL(WPE) k_recon_queue(RcQueueArgs) {
             uint32_t it = Q.n;
             if (!__hip_atomic_load(Q.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
                 it = __hip_atomic_fetch_add(Q.head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            uint32_t item = 0xFFFFFFFFu;
-            if (it < Q.n) {
-                item = Q.order[it];
-                if (!Q.fine) {
-                    const uint32_t sb = item & ~RC_CHROMA, *prog = Q.prog + ((item & RC_CHROMA) ? Q.nSb : 0) + sb;
-                    const Img &I = B.img[B.sbImg[sb]];
-                    const uint32_t local = sb - I.sbBase;
-                    const int c = (int)(local % I.sbCols), r = (int)(local / I.sbCols);
-                    int tc = 0, tr = 0;
-                    while (tc + 1 < I.tileCols && c * 16 >= I.tileColStart[tc + 1]) tc++;
-                    while (tr + 1 < I.tileRows && r * 16 >= I.tileRowStart[tr + 1]) tr++;
-                    const int c0 = I.tileColStart[tc] >> 4, c1 = (I.tileColStart[tc + 1] + 15) >> 4, r0 = I.tileRowStart[tr] >> 4;
-                    bool ok = true;
-                    uint32_t seen;
-                    if (item & RC_CHROMA) ok = wait_progress(Q.prog + sb, 0, 16, Q, seen);
-                    if (ok && c > c0) ok = wait_progress(prog - 1, 0, 16, Q, seen);
-                    if (ok && r > r0) ok = wait_progress(prog - I.sbCols + (c + 1 < c1 ? 1 : 0), 0, 16, Q, seen);
-                    if (!ok) item = 0xFFFFFFFFu;
-                }
-            }
-            S.qItem = item;
+            S.qItem = it < Q.n ? Q.order[it] : 0xFFFFFFFFu;
         }
         __syncthreads();
         const uint32_t item = S.qItem;
         if (item == 0xFFFFFFFFu) break;
-        // the neighbours' reconstruction, maps and contexts were published with release at agent scope
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         const uint32_t sb = item & ~RC_CHROMA;
         const int qctx = B.img[B.sbImg[sb]].qctx;
         if (qctx != staged) {
