@@ -91,18 +91,35 @@ AV1M_HD int chroma_tx_type(int uvTx, int uvMode) {
     const int t = av1t::Mode_To_Txfm[uvMode];
     return tx_in_set(tx_set_intra(uvTx), t) ? t : DCT_DCT;
 }
-AV1M_HD constexpr int tx_class(int t) {
+// Properties of a tx type, two bits each packed by type: a shift where comparisons would become branches
+// scan and context class
+AV1M_HD constexpr int tx_class_of(int t) {
     return (t == V_DCT || t == V_ADST || t == V_FLIPADST) ? TX_CLASS_VERT : (t == H_DCT || t == H_ADST || t == H_FLIPADST) ? TX_CLASS_HORIZ : TX_CLASS_2D;
 }
-// 1-D kinds of the row (horizontal) and column (vertical) passes; flips
-AV1M_HD constexpr int row_kind(int t) {
+// 1-D kinds of the row (horizontal) and column (vertical) passes
+AV1M_HD constexpr int row_kind_of(int t) {
     return (t == DCT_DCT || t == ADST_DCT || t == FLIPADST_DCT || t == H_DCT) ? K_DCT
          : (t == IDTX || t == V_DCT || t == V_ADST || t == V_FLIPADST) ? K_IDT : K_ADST;
 }
-AV1M_HD constexpr int col_kind(int t) {
+AV1M_HD constexpr int col_kind_of(int t) {
     return (t == DCT_DCT || t == DCT_ADST || t == DCT_FLIPADST || t == V_DCT) ? K_DCT
          : (t == IDTX || t == H_DCT || t == H_ADST || t == H_FLIPADST) ? K_IDT : K_ADST;
 }
+// flips: bit 0 rows upside down, bit 1 columns left to right
+AV1M_HD constexpr int flips_of(int t) {
+    return ((t == FLIPADST_DCT || t == FLIPADST_ADST || t == V_FLIPADST || t == FLIPADST_FLIPADST) ? 1 : 0) |
+           ((t == DCT_FLIPADST || t == ADST_FLIPADST || t == H_FLIPADST || t == FLIPADST_FLIPADST) ? 2 : 0);
+}
+template <typename F> constexpr uint32_t pack_types(F f) {
+    uint32_t v = 0;
+    for (int t = 0; t < 16; t++) v |= (uint32_t)f(t) << (2 * t);
+    return v;
+}
+AV1M_HD constexpr int tx_class(int t) { constexpr uint32_t p = pack_types(tx_class_of); return (p >> (2 * t)) & 3; }
+AV1M_HD constexpr int row_kind(int t) { constexpr uint32_t p = pack_types(row_kind_of); return (p >> (2 * t)) & 3; }
+AV1M_HD constexpr int col_kind(int t) { constexpr uint32_t p = pack_types(col_kind_of); return (p >> (2 * t)) & 3; }
+AV1M_HD constexpr int flip_ud(int t) { constexpr uint32_t p = pack_types(flips_of); return (p >> (2 * t)) & 1; }
+AV1M_HD constexpr int flip_lr(int t) { constexpr uint32_t p = pack_types(flips_of); return (p >> (2 * t + 1)) & 1; }
 // Algorithmic forward-transform FLOPs of one evaluation of a W x H transform block of type t (work accounting): 2 per
 // fmaf of the column pass (W columns x min(H, 32) kept outputs x H taps) and of the row pass (min(H, 32) rows x
 // min(W, 32) kept outputs x W taps), 1 per multiply of an identity kind's pass and of the row output scale.
@@ -119,8 +136,6 @@ AV1M_HD constexpr uint32_t set_flops(int W, int H, int set) {
         if (av1t::Tx_Type_In_Set_Intra[set][t]) f += fwd_flops(W, H, t);
     return f;
 }
-AV1M_HD int flip_ud(int t) { return t == FLIPADST_DCT || t == FLIPADST_ADST || t == V_FLIPADST || t == FLIPADST_FLIPADST; }
-AV1M_HD int flip_lr(int t) { return t == DCT_FLIPADST || t == ADST_FLIPADST || t == H_FLIPADST || t == FLIPADST_FLIPADST; }
 AV1M_HD int dq_denom(int t) {
     return (t == TX_64X64 || t == TX_32X64 || t == TX_64X32) ? 4
          : (t == TX_32X32 || t == TX_16X32 || t == TX_32X16 || t == TX_16X64 || t == TX_64X16) ? 2 : 1;

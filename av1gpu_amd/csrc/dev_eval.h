@@ -39,16 +39,25 @@ template <typename T> __device__ __forceinline__ cst<T> *uni(const T *p) {
     return (cst<T> *)(((uint64_t)hi << 32) | lo);
 }
 
+// levels laid over the coefficients they come from: stores through this type may alias the float loads
+typedef int16_t __attribute__((may_alias)) lev16;
+
 __device__ __forceinline__ int glane() { return threadIdx.x & 31; }
 __device__ __forceinline__ int gid() { return threadIdx.x >> 5; }
-// the value of lane (this lane xor M) within the 32-lane group, every lane active: M = 1, 2 by DPP quad permutes
-// ([1,0,3,2], [2,3,0,1]), M = 4, 8, 16 by ds_swizzle in bit-mask mode (and 0x1f, or 0, xor M)
+// the value of lane (this lane xor M) within the 32-lane group, every lane active, in vector registers only: M = 1, 2 by
+// DPP quad permutes ([1,0,3,2], [2,3,0,1]), 4 as a mirror of 8 lanes (xor 7) and of 4 (xor 3), 8 as a rotation of the 16-lane
+// row, 16 by swapping rows (v_permlane16_swap).  ds_swizzle, which reaches the same lanes, waits on the LDS unit each time.
 template <int M>
 __device__ __forceinline__ int lane_xor(int v) {
     static_assert(M == 1 || M == 2 || M == 4 || M == 8 || M == 16, "lane_xor: one lane bit of the 32-lane group");
     if constexpr (M == 1) return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);
     else if constexpr (M == 2) return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false);
-    else return __builtin_amdgcn_ds_swizzle(v, 0x1F | (M << 10));
+    else if constexpr (M == 4) return __builtin_amdgcn_update_dpp(0, __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, false), 0x1B, 0xF, 0xF, false);
+    else if constexpr (M == 8) return __builtin_amdgcn_update_dpp(0, v, 0x128, 0xF, 0xF, false);
+    else {   // the pair after the swap: (even row's value, odd row's value) in every lane
+        const auto p = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+        return (int)((threadIdx.x & 16) ? p[0] : p[1]);
+    }
 }
 template <int M>
 __device__ __forceinline__ float lane_xorf(float v) { return __int_as_float(lane_xor<M>(__float_as_int(v))); }
@@ -107,42 +116,42 @@ struct EvalOut { float D, R; int eob; };
 
 __device__ __forceinline__ int txsz_ctx(int t) { return (av1t::Tx_Size_Sqr[t] + av1t::Tx_Size_Sqr_Up[t] + 1) >> 1; }
 
-// txb_skip, luma tx type and eob position bits of a tx block of size TSZ
+// txb_skip, luma tx type and eob position bits of a tx block of size TSZ (no branch per lane: the terms that do not apply
+// are read at clamped positions and dropped)
 template <int TSZ, typename E>
-__device__ float base_bits(const E &e, int eob) {
+__device__ __forceinline__ float base_bits(const E &e, int eob) {
     const auto &C = *e.C;
     constexpr int t = TSZ, ctx = txsz_ctx_of(t);
-    if (eob == 0) return C.txb_skip[ctx][e.skipCtx][1];
-    float b = C.txb_skip[ctx][e.skipCtx][0];
     const int pt = e.plane > 0;
-    if (e.plane == 0) {
-        constexpr int set = tx_set_intra(t), sqr = av1t::Tx_Size_Sqr[t];
-        if constexpr (set == TX_SET_INTRA_1) {
-            int idx = 0;
+    const float skip = C.txb_skip[ctx][e.skipCtx][eob == 0 ? 1 : 0];
+    float b = skip;
+    constexpr int set = tx_set_intra(t), sqr = av1t::Tx_Size_Sqr[t];
+    if constexpr (set == TX_SET_INTRA_1) {
+        int idx = 0;
 #pragma unroll
-            for (int i = 0; i < 7; i++) idx = av1t::Tx_Type_Intra_Inv_Set1[i] == e.txType ? i : idx;
-            b += C.tx_set1[sqr][e.intraDir][idx];
-        } else if constexpr (set == TX_SET_INTRA_2) {
-            int idx = 0;
+        for (int i = 0; i < 7; i++) idx = av1t::Tx_Type_Intra_Inv_Set1[i] == e.txType ? i : idx;
+        const float x = C.tx_set1[sqr][e.intraDir][idx];
+        b += pt ? 0.f : x;
+    } else if constexpr (set == TX_SET_INTRA_2) {
+        int idx = 0;
 #pragma unroll
-            for (int i = 0; i < 5; i++) idx = av1t::Tx_Type_Intra_Inv_Set2[i] == e.txType ? i : idx;
-            b += C.tx_set2[sqr][e.intraDir][idx];
-        }
+        for (int i = 0; i < 5; i++) idx = av1t::Tx_Type_Intra_Inv_Set2[i] == e.txType ? i : idx;
+        const float x = C.tx_set2[sqr][e.intraDir][idx];
+        b += pt ? 0.f : x;
     }
     constexpr int lw = av1t::Tx_Width_Log2[t], lh = av1t::Tx_Height_Log2[t];
     constexpr int ms = (lw < 5 ? lw : 5) + (lh < 5 ? lh : 5) - 4;
-    const int eobPt = eob <= 2 ? eob : 2 + (31 - __clz(eob - 1));
+    const int eobPt = eob <= 2 ? max(eob, 1) : 2 + (31 - __clz(eob - 1));
     const int ec = tx_class(e.txType) == TX_CLASS_2D ? 0 : 1;
     const float p = ms == 0 ? C.eob_pt16[pt][ec][eobPt - 1] : ms == 1 ? C.eob_pt32[pt][ec][eobPt - 1]
                   : ms == 2 ? C.eob_pt64[pt][ec][eobPt - 1] : ms == 3 ? C.eob_pt128[pt][ec][eobPt - 1]
                   : ms == 4 ? C.eob_pt256[pt][ec][eobPt - 1] : ms == 5 ? C.eob_pt512[pt][eobPt - 1] : C.eob_pt1024[pt][eobPt - 1];
     b += p;
-    if (eobPt >= 3) {
-        const int rem = eob - ((1 << (eobPt - 2)) + 1);
-        b += C.eob_extra[ctx][pt][eobPt - 3][(rem >> (eobPt - 3)) & 1];
-        b += (float)(eobPt - 3);
-    }
-    return b;
+    const int x = max(eobPt - 3, 0), rem = eob - ((1 << (x + 1)) + 1);
+    const float ex = C.eob_extra[ctx][pt][x][(rem >> x) & 1];
+    b += eobPt >= 3 ? ex : 0.f;
+    b += (float)x;
+    return eob == 0 ? skip : b;
 }
 
 // Bits of the coefficient at scan position c (< eob) of a tx block of size TSZ given the levels q (natural order, stride =
@@ -158,10 +167,10 @@ __device__ __forceinline__ float coeff_bits(int c, int eob, int sk, QP q, SP dsc
     int pos = dscan[c];
     if constexpr (!only2d) pos = sk == 0 ? pos : sk == 1 ? ((c & (height - 1)) << bwl) + (c >> lbh) : c;
     const int row = pos >> bwl, col = pos & (width - 1);
-    auto at = [&](int dr, int dc) -> int {   // |level| of the neighbour at (row + dr, col + dc), 0 outside
-        const bool in = row + dr < height && col + dc < width;
-        const int a = q[in ? pos + (dr << bwl) + dc : pos];
-        return in ? (a < 0 ? -a : a) : 0;
+    auto at = [&](int dr, int dc) -> int {   // |level| of the neighbour at (row + dr, col + dc), 0 outside (masked, no branch)
+        const int in = ((row + dr - height) & (col + dc - width)) >> 31;
+        const int a = q[pos + (((dr << bwl) + dc) & in)];
+        return max(a, -a) & in;
     };
     static_assert(av1t::Sig_Ref_Diff_Offset[0][2][0] == 1 && av1t::Sig_Ref_Diff_Offset[1][2][1] == 2 && av1t::Sig_Ref_Diff_Offset[2][4][0] == 4,
                   "neighbour order: right, below, then the class's own three");
@@ -174,7 +183,8 @@ __device__ __forceinline__ float coeff_bits(int c, int eob, int sk, QP q, SP dsc
         a3 = at(sk == 2 ? 3 : 0, sk == 2 ? 0 : 2 + sk);
         a4 = at(sk == 2 ? 4 : sk == 1 ? 0 : 2, sk == 1 ? 4 : 0);
     }
-    const int v = qv < 0 ? -qv : qv, level = v < 15 ? v : 15;
+    const int v = max(qv, -qv), level = min(v, 15);
+    const float sgn = (&C.dc_sign[pt][dcCtx][0])[qv < 0];
     const int m5 = min(a0, 3) + min(a1, 3) + min(a2, 3) + min(a3, 3) + min(a4, 3);
     const int m = min((m5 + 1) >> 1, 4);
     int bctx = pos == 0 ? 0 : m + (int)cbOff[min(row, 4) * 5 + min(col, 4)];
@@ -185,7 +195,7 @@ __device__ __forceinline__ float coeff_bits(int c, int eob, int sk, QP q, SP dsc
     }
     const int ectx = c == 0 ? 0 : c <= (height << bwl) / 8 ? 1 : c <= (height << bwl) / 4 ? 2 : 3;
     const auto *pb = c == eob - 1 ? &C.coeff_base_eob[ctx][pt][ectx][min(max(level, 1), 3) - 1] : &C.coeff_base[ctx][pt][bctx][min(level, 3)];
-    float b = *pb;
+    float b = *pb, golomb = 0.f;
     if (level > 2) {
         const int mb = min((min(a0, 15) + min(a1, 15) + min(a2, 15) + 1) >> 1, 6);
         bool near0 = row < 2 && col < 2;
@@ -195,13 +205,11 @@ __device__ __forceinline__ float coeff_bits(int c, int eob, int sk, QP q, SP dsc
         const int rem = level - 3, n3 = (rem * 11) >> 5;   // rem / 3 for 0 .. 12
         const float full = br[3], rest = br[rem - 3 * n3];
 #pragma unroll
-        for (int i = 0; i < 4; i++) b = i < n3 ? b + full : i == n3 ? b + rest : b;
+        for (int i = 0; i < 4; i++) b += i < n3 ? full : i == n3 ? rest : 0.f;
+        golomb = v > 14 ? (float)(2 * (31 - __clz(max(v - 14, 1))) + 1) : 0.f;
     }
-    if (v) {
-        b += c == 0 ? C.dc_sign[pt][dcCtx][qv < 0] : 1.0f;
-        if (v > 14) b += (float)(2 * (31 - __clz(v - 14)) + 1);
-    }
-    return b;
+    b += v ? (c == 0 ? sgn : 1.0f) : 0.f;   // the sign, then the Golomb part (sums with 0 are exact)
+    return b + golomb;
 }
 
 // eob and rate of the levels q of a tx block of size TSZ, class sk, by the group (all lanes return both); last: the
@@ -210,7 +218,8 @@ template <int TSZ, typename QP, typename SP, typename OP, typename E>
 __device__ __forceinline__ void grp_rate(QP q, SP dscan, OP cbOff, const E &e, int sk, int last, int &eobOut, float &bitsOut) {
     const int lane = glane();
     const int eob = gmaxi(last);
-    float bits = lane == 0 ? base_bits<TSZ>(e, eob) : 0.f;
+    const float base = base_bits<TSZ>(e, eob);
+    float bits = lane == 0 ? base : 0.f;
     for (int c = lane; c < eob; c += GW) bits += coeff_bits<TSZ>(c, eob, sk, q, dscan, cbOff, e.plane > 0, e.dcCtx, *e.C);
     eobOut = eob;
     bitsOut = gsum(bits);
@@ -325,19 +334,21 @@ __device__ __forceinline__ EvalOut grp_qrate(FP tmp, int ts, QP q, const E &e, c
     const int den = dq_denom(e.txSz), dsh = den == 4 ? 2 : den == 2 ? 1 : 0;
     float dist = 0.f, kept = 0.f;
     int last = 0;
-    for (int idx = lane; idx < N; idx += GW) {
-        const float v = tmp[(idx >> LTW) * ts + (idx & (TW - 1))];
+    constexpr int NE = (N + GW - 1) / GW;   // per lane; a 4x4 leaves the upper half of the lanes a zero
+#pragma unroll 4
+    for (int t = 0; t < NE; t++) {
+        const int idx = N < GW ? lane & (N - 1) : lane + GW * t;
+        float v = tmp[(idx >> LTW) * ts + (idx & (TW - 1))];
+        if constexpr (N < GW) v = lane < N ? v : 0.f;
         const int step = idx == 0 ? e.dcQ : e.acQ;
         const float a = quot_step(fabsf(v) * (float)den, (float)step, idx == 0 ? e.dcRcp : e.acRcp);
         int l = a < e.zbin ? 0 : (int)(a + e.rnd);
         l = min(l, 16383);
         const int qv = v < 0 ? -l : l;
-        q[idx] = (int16_t)qv;
-        if (l) {
-            const int c = sk == 0 ? (int)iscan[idx] : sk == 1 ? (idx & (TW - 1)) * TH + (idx >> LTW) : idx;
-            last = max(last, c + 1);
-        }
-        const float dq = l ? (float)dequant(qv, step, dsh, e.bd) : 0.f;
+        if (N >= GW || lane < N) q[idx] = (int16_t)qv;
+        const int c0 = (int)iscan[idx], c = sk == 0 ? c0 : sk == 1 ? (idx & (TW - 1)) * TH + (idx >> LTW) : idx;
+        last = max(last, l ? c + 1 : 0);
+        const float dq = (float)dequant(qv, step, dsh, e.bd);   // 0 for level 0
         const float d = v - dq;
         const float sq = d * d;
         dist = dist + sq;
@@ -387,30 +398,29 @@ __device__ EvalOut half_qrate(FP tmp, int ts, QP q, const E &e, const TT &T) {
     float dist[2] = {0.f, 0.f};
     int last = 0;
 #pragma unroll
-    for (int h = 0; h < 2; h++)
-        for (int idx = lane + 16 * h; idx < N; idx += GW) {
-            const float v = tmp[(idx >> LTW) * ts + (idx & (TW - 1))];
-            const int step = idx == 0 ? e.dcQ : e.acQ;
-            const float a = quot_step(fabsf(v) * (float)den, (float)step, idx == 0 ? e.dcRcp : e.acRcp);
-            int l = a < e.zbin ? 0 : (int)(a + e.rnd);
-            l = min(l, 16383);
-            const int qv = v < 0 ? -l : l;
-            q[idx] = (int16_t)qv;
-            if (l) {
-                const int c = sk == 0 ? (int)iscan[idx] : sk == 1 ? (idx & (TW - 1)) * TH + (idx >> LTW) : idx;
-                last = max(last, c + 1);
-            }
-            const float dq = l ? (float)dequant(qv, step, dsh, e.bd) : 0.f;
-            const float d = v - dq;
-            const float sq = d * d;
-            dist[h] = dist[h] + sq;
-        }
+    for (int t = 0; t < N / 16; t++) {   // virtual lane lane + 16 (t & 1)
+        const int idx = lane + 16 * t;
+        const float v = tmp[(idx >> LTW) * ts + (idx & (TW - 1))];
+        const int step = idx == 0 ? e.dcQ : e.acQ;
+        const float a = quot_step(fabsf(v) * (float)den, (float)step, idx == 0 ? e.dcRcp : e.acRcp);
+        int l = a < e.zbin ? 0 : (int)(a + e.rnd);
+        l = min(l, 16383);
+        const int qv = v < 0 ? -l : l;
+        q[idx] = (int16_t)qv;
+        const int c0 = (int)iscan[idx], c = sk == 0 ? c0 : sk == 1 ? (idx & (TW - 1)) * TH + (idx >> LTW) : idx;
+        last = max(last, l ? c + 1 : 0);
+        const float dq = (float)dequant(qv, step, dsh, e.bd);
+        const float d = v - dq;
+        const float sq = d * d;
+        dist[t & 1] = dist[t & 1] + sq;
+    }
     const float distS = hsum2(dist[0], dist[1]);
     gsync();
     const auto dscan = dscan_ptr<TSZ>(T);
     const auto cbOff = cboff_ptr<TSZ>(T);
     const int eob = hmaxi(last);
-    float b0 = lane == 0 ? base_bits<TSZ>(e, eob) : 0.f, b1 = 0.f;
+    const float base = base_bits<TSZ>(e, eob);
+    float b0 = lane == 0 ? base : 0.f, b1 = 0.f;
     // the lane's two virtual lanes side by side: their chains of reads overlap
     for (int c = lane; c < eob; c += GW) {
         const int d = c + 16 < N ? c + 16 : c;

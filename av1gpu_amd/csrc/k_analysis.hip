@@ -29,7 +29,7 @@ struct EvalScrDirect {
     static constexpr int TS = W + 1, TH = H > 32 ? 32 : H;
     float tmp[TH * TS];
     static_assert((W > 32 ? 32 : W) * TH * 2 <= TH * TS * 4, "the levels fit in the coefficients' space");
-    __device__ int16_t *lev() { return reinterpret_cast<int16_t *>(tmp); }
+    __device__ lev16 *lev() { return reinterpret_cast<lev16 *>(tmp); }
 };
 template <int W, int H>
 struct AnScr {

@@ -320,7 +320,7 @@ __device__ EvalOut grp_task_big(lds<RcShared> &S, lds<RcTeam> &X, const lds<Img>
     e.skipCtx = S.skipCtx[p]; e.dcCtx = S.dcCtx[p]; e.intraDir = p == 0 ? cand_mode(c) : 0; e.bd = bd;
     e.rnd = p ? P.rndC : P.rnd; e.zbin = p ? P.zbinC : P.zbin;
     e.C = &S.tab.cost;
-    return grp_qrate<W, H>(X.tmp, W + 1, team_lev(X), e, S.tab);
+    return grp_qrate<W, H>(X.tmp, W + 1, (lds<lev16> *)team_lev(X), e, S.tab);
 }
 
 // ---- exact inverse transform + reconstruction by the workgroup (spec 7.13.3, 7.12.3 step 3) ----
