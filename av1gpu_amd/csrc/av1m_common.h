@@ -611,6 +611,70 @@ AV1M_HD void pred_col(int mode, int pa, int dcv, int i0, int di, int j, int lw, 
         }
     }
 }
+// The 4x4 samples at rows i0.., columns j0.. of a predicted block from unfiltered edges (no upsampling), raster order: the mode
+// and the direction's steps are settled once for the sixteen.  Along a row of zones 1 and 2 the position in AboveRow moves
+// by one sample and its fraction stays, so a row takes five samples for its four; along a column the same holds for
+// LeftCol.  Equal to pred_px at every sample.
+template <typename P>
+AV1M_HD void pred_4x4(int mode, int pa, int dcv, int i0, int j0, int lw, int lh, const P *A, const P *L, int (&o)[16]) {
+    const int w = 1 << lw, h = 1 << lh;
+    if (mode == DC_PRED) {
+        for (int k = 0; k < 16; k++) o[k] = dcv;
+    } else if (is_dir(mode)) {
+        if (pa <= 90) {   // 90: the sample above
+            const int dx = pa == 90 ? 0 : av1t::Dr_Intra_Derivative[pa], mb = w + h - 1;
+            for (int i = 0; i < 4; i++) {
+                const int idx = (i0 + i + 1) * dx, base = (idx >> 6) + j0, sh = (idx >> 1) & 0x1F;
+                int a[5];
+                for (int j = 0; j < 5; j++) a[j] = A[base + j < mb ? base + j : mb];
+                for (int j = 0; j < 4; j++) o[4 * i + j] = (a[j] * (32 - sh) + a[j + 1] * sh + 16) >> 5;
+            }
+        } else if (pa < 180) {
+            const int dx = av1t::Dr_Intra_Derivative[180 - pa], dy = av1t::Dr_Intra_Derivative[pa - 90];
+            for (int i = 0; i < 4; i++) {
+                const int ia = -(i0 + i + 1) * dx, ba = (ia >> 6) + j0, sa = (ia >> 1) & 0x1F;
+                for (int j = 0; j < 4; j++) {
+                    const int il = -(j0 + j + 1) * dy, bl = (il >> 6) + i0 + i, sl = (il >> 1) & 0x1F;
+                    const bool above = ba + j >= -1;
+                    const P *s = above ? A + ba + j : L + bl;
+                    const int sh = above ? sa : sl;
+                    o[4 * i + j] = (s[0] * (32 - sh) + s[1] * sh + 16) >> 5;
+                }
+            }
+        } else {   // 180: the sample to the left
+            const int dy = pa == 180 ? 0 : av1t::Dr_Intra_Derivative[270 - pa];
+            for (int j = 0; j < 4; j++) {
+                const int idx = (j0 + j + 1) * dy, base = (idx >> 6) + i0, sh = (idx >> 1) & 0x1F;
+                int a[5];
+                for (int i = 0; i < 5; i++) a[i] = L[base + i];
+                for (int i = 0; i < 4; i++) o[4 * i + j] = (a[i] * (32 - sh) + a[i + 1] * sh + 16) >> 5;
+            }
+        }
+    } else {
+        int a[4], l[4];
+        for (int k = 0; k < 4; k++) { a[k] = A[j0 + k]; l[k] = L[i0 + k]; }
+        if (mode == PAETH_PRED) {
+            const int tl = A[-1];
+            for (int i = 0; i < 4; i++)
+                for (int j = 0; j < 4; j++) {
+                    const int dl = a[j] - tl, dt = l[i] - tl, dtl = dl + dt;   // base - left, base - above, base - top left
+                    const int pL = dl < 0 ? -dl : dl, pT = dt < 0 ? -dt : dt, pTL = dtl < 0 ? -dtl : dtl;
+                    o[4 * i + j] = (pL <= pT && pL <= pTL) ? l[i] : pT <= pTL ? a[j] : tl;
+                }
+        } else {
+            // the SMOOTH modes as in pred_col: SMOOTH_V / SMOOTH_H take a second copy of their own direction's pair
+            const uint8_t *wx = sm_weights(lw), *wy = sm_weights(lh);
+            const int lb = L[h - 1], ar = A[w - 1];
+            for (int i = 0; i < 4; i++) {
+                const int wi = wy[i0 + i];
+                for (int j = 0; j < 4; j++) {
+                    const int wj = wx[j0 + j], vv = wi * a[j] + (256 - wi) * lb, hh = wj * l[i] + (256 - wj) * ar;
+                    o[4 * i + j] = ((mode == SMOOTH_PRED ? vv + hh : mode == SMOOTH_V_PRED ? 2 * vv : 2 * hh) + 256) >> 9;
+                }
+            }
+        }
+    }
+}
 AV1M_HD int edge_strength(int w, int h, int ft, int delta) {
     const int d = delta < 0 ? -delta : delta, s = w + h;
     if (ft == 0) {

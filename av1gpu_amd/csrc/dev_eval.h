@@ -233,13 +233,12 @@ __device__ __forceinline__ const uint8_t *cboff_ptr(const DevTables &) { return 
 template <int TSZ>
 __device__ __forceinline__ const uint16_t *iscan_ptr(const DevTables &T) { return T.iscan + dscan_off(av1t::Adjusted_Tx_Size[TSZ]); }
 
-// Evaluation scratch of one group in LDS, for tx blocks up to W x H
+// Evaluation scratch of one group in LDS, for tx blocks of W x H up to 16 x 16
 template <int W, int H>
 struct EvalScr {
-    static constexpr int TS = W + 1, TH = H > 32 ? 32 : H;
     int16_t res[W * H];
-    float tmp[TH * TS];
-    int16_t q[(W > 32 ? 32 : W) * TH];
+    float tmp[H * (W + 1)];
+    int16_t q[W * H];
 };
 
 template <int W, int H, typename FP, typename QP, typename E, typename TT>
@@ -250,8 +249,8 @@ __device__ __forceinline__ EvalOut grp_qrate(FP tmp, int ts, QP q, const E &e, c
 // return the same values.
 template <int W, int H, typename RP, typename FP, typename QP, typename E, typename TT>
 __device__ EvalOut grp_eval(RP res, FP tmp, QP q, const E &e, const TT &T) {
-    constexpr int TW = W > 32 ? 32 : W, TH = H > 32 ? 32 : H, TS = W + 1;
-    constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 4 ? 2 : H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
+    constexpr int TW = W, TH = H, TS = W + 1;
+    constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : 4, LH = H == 4 ? 2 : H == 8 ? 3 : 4;
     const int lane = glane();
     const int rk = row_kind(e.txType), ck = col_kind(e.txType), fud = flip_ud(e.txType), flr = flip_lr(e.txType);
     // Outputs per item chosen so that a pass fills the group's 32 lanes where the block allows (at most 8 per item):
@@ -321,18 +320,19 @@ __device__ EvalOut grp_eval(RP res, FP tmp, QP q, const E &e, const TT &T) {
 // region at tmp + i * ts), levels into q (natural order, tw x th).  All lanes of the group return the same values.
 template <int W, int H, typename FP, typename QP, typename E, typename TT>
 __device__ __forceinline__ EvalOut grp_qrate(FP tmp, int ts, QP q, const E &e, const TT &T) {
-    constexpr int TW = W > 32 ? 32 : W, TH = H > 32 ? 32 : H;
-    constexpr int LTW = TW == 4 ? 2 : TW == 8 ? 3 : TW == 16 ? 4 : 5;
+    static_assert(W <= 16 && H <= 16, "larger tx blocks: wave_qrate");
+    constexpr int TW = W, TH = H;
+    constexpr int LTW = TW == 4 ? 2 : TW == 8 ? 3 : 4;
     constexpr int N = TW * TH;
     const int lane = glane();
     constexpr int TSZ = tx_of(W, H);
     const int cls = tx_class(e.txType);
     // the scan of the rate: the default (2D) scan, rows (class VERT: raster order) or columns (class HORIZ)
-    const int sk = (W > 16 || H > 16 || cls == TX_CLASS_2D) ? 0 : cls == TX_CLASS_HORIZ ? 1 : 2;
+    const int sk = cls == TX_CLASS_2D ? 0 : cls == TX_CLASS_HORIZ ? 1 : 2;
     const auto iscan = iscan_ptr<TSZ>(T);
     // ---- quantization + distortion (virtual lane = physical lane), and the eob ----
     const int den = dq_denom(e.txSz), dsh = den == 4 ? 2 : den == 2 ? 1 : 0;
-    float dist = 0.f, kept = 0.f;
+    float dist = 0.f;
     int last = 0;
     constexpr int NE = (N + GW - 1) / GW;   // per lane; a 4x4 leaves the upper half of the lanes a zero
 #pragma unroll 4
@@ -352,7 +352,6 @@ __device__ __forceinline__ EvalOut grp_qrate(FP tmp, int ts, QP q, const E &e, c
         const float d = v - dq;
         const float sq = d * d;
         dist = dist + sq;
-        kept = fmaf(v, v, kept);
     }
     const float distS = gsum(dist);
     gsync();
@@ -363,10 +362,6 @@ __device__ __forceinline__ EvalOut grp_qrate(FP tmp, int ts, QP q, const E &e, c
     grp_rate<TSZ>(q, dscan, cbOff, e, sk, last, eob, o.R);
     const float g = T.txg[e.txSz][e.txType];
     o.D = g * distS;
-    if (W == 64 || H == 64) {
-        const float keptS = gsum(kept);
-        o.D = o.D + fmaxf(0.f, fmaf(-g, keptS, e.resEnergy));
-    }
     o.eob = eob;
     return o;
 }
@@ -503,88 +498,228 @@ __device__ EvalOut half_eval(RP res, FP tmp, QP q, const E &e, const TT &T) {
     return half_qrate<W, H>(tmp, TS, q, e, T);
 }
 
-// 2-D forward DCT_DCT of a W x H residual with a side of 32 or 64 by the 32 lanes of the group, the residual produced
-// on the fly: res(k0, j, r) fills r[0 .. CH) with rows k0 .. k0 + CH - 1 of column j.  Column pass: lane = column (two columns, j and j + 32, for W = 64), one fmaf chain per kept
-// output over k ascending with the matrix coefficient a wave-uniform scalar operand; row pass: lane = row.  The
-// coefficients (scaled) land in tmp (row i at tmp + i * (W + 1), tw x th kept).  Returns the residual energy sum over the
-// raster order (W or H = 64: the energy the dropped coefficients carry), else 0.
+// ---- tx blocks with a side of 32 or 64 (DCT_DCT only), by a whole wave ----
+// Each forward-transform output is one fmaf chain over ascending k, and so is each element of an FP32 MFMA: the 16x16x4
+// instruction adds its four products in ascending k with a rounding per product (checked on MI355X against fmaf chains,
+// 1.4 M elements over three value ranges, none different).  So both passes run on the matrix cores under the same
+// arithmetic contract, at twice the FMA rate of the vector unit and without an operand load per product.
+__device__ __forceinline__ int wlane() { return threadIdx.x & 63; }
+// (the value of this 32-lane half's partner lane in the lower half, in the upper half), in every lane
+struct Halves { float lo, hi; };
+__device__ __forceinline__ Halves halves(float v) {
+    const auto p = __builtin_amdgcn_permlane32_swap((unsigned)__float_as_int(v), (unsigned)__float_as_int(v), false, false);
+    return Halves{__int_as_float((int)p[0]), __int_as_float((int)p[1])};
+}
+__device__ __forceinline__ int other_half(int v) {
+    const auto p = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+    return (int)((threadIdx.x & 32) ? p[0] : p[1]);
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// the residual energy as 32 sequential float sums over the raster order (virtual lane v: elements v, v + 32, ...), for
+// sums past 2^24, whose order of additions matters; res(i0, di, j, r) fills r with rows i0, i0 + di, ... of column j
 template <int W, int H, typename Res>
-__device__ __forceinline__ float grp_fwd_dct(lds<float> *tmp, const DevTables &T, float scale, Res res) {
-    constexpr int TW = W > 32 ? 32 : W, TH = H > 32 ? 32 : H, TS = W + 1;
+__device__ __forceinline__ float wave_energy_seq(Res res) {
+    const int v = threadIdx.x & 31;
+    float e = 0.f;
+    for (int k = 0; k < H; k++) {
+        int r[1];
+        if constexpr (W == 64) {
+            res(k, 1, v, r);
+            e = e + (float)(r[0] * r[0]);
+            res(k, 1, v + 32, r);
+            e = e + (float)(r[0] * r[0]);
+        } else if constexpr (W == 32) {
+            res(k, 1, v, r);
+            e = e + (float)(r[0] * r[0]);
+        } else {   // W = 16: element v + 32 t is column v & 15 of row 2 t + (v >> 4)
+            if ((k & 1) == (v >> 4)) {
+                res(k, 1, v & 15, r);
+                e = e + (float)(r[0] * r[0]);
+            }
+        }
+    }
+    return e;
+}
+
+// Forward DCT of a W x H residual made on the fly by res (above), by the 64 lanes of the wave.  Column pass as Y^T = X^T
+// Fc^T: lane l supplies rows k = 4 s + g (g = l / 16) of its column, so the prediction of a sample is made once, in the lane
+// that feeds it to the matrix core; the columns of a 16-column tile go to the lanes in the order 4 (m % 4) + m / 4, which
+// makes accumulator register r of lane group g column 4 r + g -- the operand the row pass (Y Fr^T) wants of that lane, so
+// nothing moves between the passes.  The kept th x tw coefficients (scaled) land in tmp (row stride TS).  Returns the
+// energy sum over the raster order where a side is 64, else 0.
+template <int W, int H, int TS, typename FP, typename Res>
+__device__ __forceinline__ float wave_fwd_dct(FP tmp, const DevTables &T, float scale, Res res) {
+    constexpr int TW = W > 32 ? 32 : W, TH = H > 32 ? 32 : H;
     constexpr int LW = W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
+    constexpr int NJ = W < 16 ? 1 : W / 16, NI = TH < 16 ? 1 : TH / 16, NO = TW < 16 ? 1 : TW / 16, KS = H / 4, RS = W / 4, CH = KS < 8 ? KS : 8;
     constexpr bool E64 = W == 64 || H == 64;
-    constexpr int NC = W == 64 ? 2 : 1;
-    constexpr int CH = H < 8 ? H : 8;   // residual rows made per call of res (its mode tests once per run)
-    const int lane = glane();
-    cst<DevTables> *TU = uni(&T);
-    cst<float> *FcT = TU->fwdT + TU->fwdOff[K_DCT][LH];
-    cst<float> *FrT = TU->fwdT + TU->fwdOff[K_DCT][LW];
-    float en = 0.f, eo = 0.f;
-    if (lane < W) {
-        float acc[NC][TH];
+    const int l = wlane(), n = l & 15, g = l >> 4, jm = 4 * (n & 3) + (n >> 2);
+    const DevTables *TU = (const DevTables *)uni(&T);
+    const glb<float> *const FcT0 = (const glb<float> *)TU->fwdT + TU->fwdOff[K_DCT][LH];
+    const glb<float> *const FrT0 = (const glb<float> *)TU->fwdT + TU->fwdOff[K_DCT][LW];
+    uint32_t en0 = 0, en1 = 0;   // squares of the even and the odd column tiles
+    f32x4 z[NI][NO];
 #pragma unroll
-        for (int i = 0; i < TH; i++) { acc[0][i] = 0.f; if constexpr (NC == 2) acc[NC - 1][i] = 0.f; }
-        for (int k0 = 0; k0 < H; k0 += CH) {
-            int ra[CH], rb[CH];
-            res(k0, lane, ra);
-            if constexpr (NC == 2) res(k0, lane + 32, rb);
+    for (int it = 0; it < NI; it++)
 #pragma unroll
-            for (int kk = 0; kk < CH; kk++) {
-                const int k = k0 + kk, r0 = ra[kk], r1 = NC == 2 ? rb[kk] : 0;
-                if constexpr (E64) {
-                    // raster-order virtual lane l holds elements l, l + 32, ...: W = 64 alternates columns l and l + 32
-                    // per row; W = 32 is column l; W = 16 (16x64) splits column l & 15 into even (lane l) and odd rows
-                    // (l + 16)
-                    if constexpr (W == 64) { en = en + (float)(r0 * r0); en = en + (float)(r1 * r1); }
-                    else if constexpr (W == 32) en = en + (float)(r0 * r0);
-                    else { if (k & 1) eo = eo + (float)(r0 * r0); else en = en + (float)(r0 * r0); }
-                }
-                const float x0 = (float)r0, x1 = (float)r1;
-                cst<float> *f = FcT + k * H;
+        for (int ot = 0; ot < NO; ot++) z[it][ot] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // a column tile at a time through both passes (the row pass's k are the columns in ascending order); rolled, since the
+    // prediction's modes make it the larger part of the code
+#pragma unroll 1
+    for (int jt = 0; jt < NJ; jt++) {
+        const int j = 16 * jt + jm;
+        f32x4 y[NI];
 #pragma unroll
-                for (int i = 0; i < TH; i++) {
-                    const float fi = f[i];
-                    acc[0][i] = fmaf(fi, x0, acc[0][i]);
-                    if constexpr (NC == 2) acc[NC - 1][i] = fmaf(fi, x1, acc[NC - 1][i]);
+        for (int it = 0; it < NI; it++) y[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // the matrix operands are read again for each run of rows (and candidate): hoisted out of the loops they would hold
+        // 30-60 registers through the whole search and spill as many others
+        const glb<float> *FrT = FrT0;
+#pragma unroll 1
+        for (int s0 = 0; s0 < KS; s0 += CH) {
+            const glb<float> *FcT = FcT0;
+            asm volatile("" : "+s"(FcT), "+s"(FrT));
+            int r[CH];
+            res(4 * s0 + g, 4, W < 16 ? j & (W - 1) : j, r);
+            if constexpr (E64) {
+                uint32_t q = 0;
+#pragma unroll
+                for (int s = 0; s < CH; s++) q += (uint32_t)(r[s] * r[s]);
+                en0 += (jt & 1) ? 0u : q;
+                en1 += (jt & 1) ? q : 0u;
+            }
+#pragma unroll
+            for (int s = 0; s < CH; s++) {
+                const float x = W < 16 && j >= W ? 0.f : (float)r[s];
+#pragma unroll
+                for (int it = 0; it < NI; it++) {
+                    const int i = 16 * it + n;
+                    float f = FcT[(4 * (s0 + s) + g) * H + (TH < 16 ? i & (TH - 1) : i)];
+                    if constexpr (TH < 16) f = i < TH ? f : 0.f;
+                    y[it] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, f, y[it], 0, 0, 0);
                 }
             }
         }
 #pragma unroll
-        for (int i = 0; i < TH; i++) {
-            tmp[i * TS + lane] = acc[0][i];
-            if constexpr (NC == 2) tmp[i * TS + lane + 32] = acc[NC - 1][i];
+        for (int s = 0; s < (RS < 4 ? RS : 4); s++) {
+#pragma unroll
+            for (int ot = 0; ot < NO; ot++) {
+                const int o = 16 * ot + n;
+                float f = FrT[(16 * jt + 4 * s + g) * W + (TW < 16 ? o & (TW - 1) : o)];
+                if constexpr (TW < 16) f = o < TW ? f : 0.f;
+#pragma unroll
+                for (int it = 0; it < NI; it++) z[it][ot] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[it][s], f, z[it][ot], 0, 0, 0);
+            }
         }
     }
-    if constexpr (E64 && W == 16) {
-        const float o = __shfl_xor(eo, 16, 32);
-        if (lane >= 16) en = o;
-    }
+#pragma unroll
+    for (int it = 0; it < NI; it++)
+#pragma unroll
+        for (int ot = 0; ot < NO; ot++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int i = 16 * it + 4 * g + r, o = 16 * ot + n;
+                if ((TH >= 16 || i < TH) && (TW >= 16 || o < TW)) tmp[i * TS + o] = z[it][ot][r] * scale;
+            }
     gsync();
-    if (lane < TH) {
-        float acc[TW];
-#pragma unroll
-        for (int o = 0; o < TW; o++) acc[o] = 0.f;
-        lds<float> *row = tmp + lane * TS;
-#pragma unroll 2
-        for (int k = 0; k < W; k++) {
-            const float x = row[k];
-            cst<float> *f = FrT + k * W;
-#pragma unroll
-            for (int o = 0; o < TW; o++) acc[o] = fmaf(f[o], x, acc[o]);
+    if constexpr (E64) {
+        // the virtual lanes' sums as integers: v = 16 (column tile parity) + column in the tile (W = 16: + 16 (row parity),
+        // which is g & 1), each over the lanes of the other rows; a sum below 2^24 is what any order of float additions gives
+        uint32_t a = en0, b = en1;
+        float f;
+        bool exact;
+        if constexpr (W == 16) {
+            a += (uint32_t)other_half((int)a);
+            exact = a < (1u << 24);
+            f = (float)a;
+            f += lane_xorf<16>(f);
+        } else {
+            a += (uint32_t)lane_xor<16>((int)a); a += (uint32_t)other_half((int)a);
+            b += (uint32_t)lane_xor<16>((int)b); b += (uint32_t)other_half((int)b);
+            exact = a < (1u << 24) && b < (1u << 24);
+            f = (float)a + (float)b;
         }
-#pragma unroll
-        for (int o = 0; o < TW; o++) row[o] = acc[o] * scale;
+        if (__any(!exact)) return gsum(wave_energy_seq<W, H>(res));
+        // the butterfly over the column bits: columns 4 (n % 4) + n / 4, so steps 8, 4, 2, 1 are lanes xor 2, 1, 8, 4
+        f += lane_xorf<2>(f); f += lane_xorf<1>(f); f += lane_xorf<8>(f); f += lane_xorf<4>(f);
+        return f;
     }
-    gsync();
-    return E64 ? gsum(en) : 0.f;
+    return 0.f;
 }
 
-// sum of r^2 over a W x H residual in raster order (32 virtual lanes)
-template <int W, int H, typename RP>
-__device__ float grp_res_energy(RP res) {
-    float e = 0.f;
-    for (int p = glane(); p < W * H; p += GW) e += (float)(res[p] * res[p]);
-    return gsum(e);
+// Quantization, distortion and rate of those coefficients (row stride ts), levels into q (natural order; may overlay tmp: every
+// coefficient is read before the first level is written).  Each virtual lane v of the 32-lane form is two lanes here: the
+// lower half's takes the first half of its elements, the upper half's the rest, and the sequential sums are handed over
+// once; the rate's scan positions alternate between the two.  All lanes return the same values.
+template <int W, int H, typename FP, typename QP, typename E, typename TT>
+__device__ __forceinline__ EvalOut wave_qrate(FP tmp, int ts, QP q, const E &e, const TT &T) {
+    constexpr int TW = W > 32 ? 32 : W, TH = H > 32 ? 32 : H;
+    constexpr int LTW = TW == 8 ? 3 : TW == 16 ? 4 : 5;
+    constexpr int N = TW * TH, NE = N / 64, TSZ = tx_of(W, H);
+    constexpr bool E64 = W == 64 || H == 64;
+    const int v = threadIdx.x & 31, h = (threadIdx.x >> 5) & 1;
+    const auto iscan = iscan_ptr<TSZ>(T);
+    const int den = dq_denom(e.txSz), dsh = den == 4 ? 2 : den == 2 ? 1 : 0;
+    float x[NE], sq[NE];
+#pragma unroll
+    for (int u = 0; u < NE; u++) {
+        const int idx = v + 32 * (NE * h + u);
+        x[u] = tmp[(idx >> LTW) * ts + (idx & (TW - 1))];
+    }
+    gsync();
+    int last = 0;
+#pragma unroll
+    for (int u = 0; u < NE; u++) {
+        const int idx = v + 32 * (NE * h + u);
+        const int step = idx == 0 ? e.dcQ : e.acQ;
+        const float a = quot_step(fabsf(x[u]) * (float)den, (float)step, idx == 0 ? e.dcRcp : e.acRcp);
+        int l = a < e.zbin ? 0 : (int)(a + e.rnd);
+        l = min(l, 16383);
+        const int qv = x[u] < 0 ? -l : l;
+        q[idx] = (int16_t)qv;
+        last = max(last, l ? (int)iscan[idx] + 1 : 0);
+        const float d = x[u] - (float)dequant(qv, step, dsh, e.bd);
+        sq[u] = d * d;
+    }
+    float dist = 0.f, kept = 0.f;
+#pragma unroll
+    for (int u = 0; u < NE; u++) {
+        dist = dist + sq[u];
+        if constexpr (E64) kept = fmaf(x[u], x[u], kept);
+    }
+    dist = halves(dist).lo;
+    if constexpr (E64) kept = halves(kept).lo;
+#pragma unroll
+    for (int u = 0; u < NE; u++) {
+        dist = dist + sq[u];
+        if constexpr (E64) kept = fmaf(x[u], x[u], kept);
+    }
+    const float distS = gsum(halves(dist).hi);
+    gsync();
+    const auto dscan = dscan_ptr<TSZ>(T);
+    const auto cbOff = cboff_ptr<TSZ>(T);
+    last = max(last, other_half(last));
+    const int eob = __builtin_amdgcn_readfirstlane(gmaxi(last));
+    const float base = base_bits<TSZ>(e, eob);
+    float bits = v == 0 ? base : 0.f;
+    for (int c0 = 0; c0 < eob; c0 += 64) {
+        const int c = c0 + 32 * h + v;
+        const float b = coeff_bits<TSZ>(min(c, N - 1), eob, 0, q, dscan, cbOff, e.plane > 0, e.dcCtx, *e.C);
+        const Halves p = halves(c < eob ? b : 0.f);
+        bits += p.lo;
+        bits += p.hi;
+    }
+    EvalOut o;
+    o.R = gsum(bits);
+    const float g = T.txg[e.txSz][e.txType];
+    o.D = g * distS;
+    if constexpr (E64) {
+        const float keptS = gsum(halves(kept).hi);
+        o.D = o.D + fmaxf(0.f, fmaf(-g, keptS, e.resEnergy));
+    }
+    o.eob = eob;
+    return o;
 }
 
 // ---- intra edge preparation by a group: av1g_edge_prepare's integer arithmetic (spec 7.11.2.4 step 4, 7.11.2.9-12)

@@ -15,32 +15,32 @@
 
 namespace av1m {
 
-// Shapes at least 32 wide try DCT_DCT only: their evaluation takes the forward DCT with the residual made on the fly
-// from the prediction (grp_fwd_dct: wave-uniform matrix operands), so no residual array sits in LDS.  The levels
-// overlay the coefficients (lev): the quantizer's round t writes levels 32 t .. 32 t + 31, i.e. the bytes of
-// coefficients 16 t .. 16 t + 15 of the row-major tmp, whose raster index is at most 16 t + 15 -- read in an earlier
-// round, or in this one before its store (each lane's store depends on its own load); nothing reads the coefficients
-// after the quantizer.  64 x 64 and 64 x 32: 19.7 KB per two-group workgroup, 8 per CU (2 waves per SIMD, the VGPR
-// limit) instead of 6.
+// Shapes with a side of 32 or 64 try DCT_DCT only and take a whole wave per block: both passes of the forward DCT on the
+// matrix cores, with the residual made on the fly from the prediction, so no residual array sits in LDS, and the
+// screening's 4x4s over 64 lanes.  The levels overlay the coefficients (wave_qrate reads every coefficient first).
+// Against a 32-lane group per block with FMA chains, together with the screening's prediction by whole 4x4s: 64x64 8.7 ->
+// 5.3 ms, 64x32 9.5 -> 5.8, 32x32 4.8 -> 4.1 on 16 images of 12 MP, and a single block's latency, which is what a small
+// image waits for, 1054 -> 371 us (64x64), 617 -> 236 us (64x32).
 template <int W, int H>
-constexpr bool an_direct() { return W >= 32; }
+constexpr bool an_wave() { return W >= 32 || H >= 32; }
 template <int W, int H>
-struct EvalScrDirect {
-    static constexpr int TS = W + 1, TH = H > 32 ? 32 : H;
+struct EvalScrWave {
+    static constexpr int TW = W > 32 ? 32 : W, TH = H > 32 ? 32 : H, TS = TW + 1;
     float tmp[TH * TS];
-    static_assert((W > 32 ? 32 : W) * TH * 2 <= TH * TS * 4, "the levels fit in the coefficients' space");
     __device__ lev16 *lev() { return reinterpret_cast<lev16 *>(tmp); }
 };
 template <int W, int H>
 struct AnScr {
-    std::conditional_t<an_direct<W, H>(), EvalScrDirect<W, H>, EvalScr<W, H>> ev;
+    std::conditional_t<an_wave<W, H>(), EvalScrWave<W, H>, EvalScr<W, H>> ev;
     uint16_t ea[EDGE_LEN], el[EDGE_LEN];   // source edges
     uint16_t pa[EDGE_LEN], pl[EDGE_LEN];   // edge-filtered copies of the candidate under evaluation
     int satdI[32];
     int cand[32];
 };
 
-constexpr int an_groups(int W, int H) { return W * H <= 256 ? 8 : W * H <= 1024 ? 4 : 2; }
+// threads of a workgroup and blocks it takes at a time: 8 groups of 32 lanes, or 4 waves for the shapes of a wave per block
+constexpr int AN_NT = 256;
+constexpr int an_groups(int W, int H) { return W >= 32 || H >= 32 ? AN_NT / 64 : AN_NT / 32; }
 
 struct TileBox { int x0, y0, x1, y1; };
 __device__ __forceinline__ TileBox tile_box(const Img &I, int x, int y) {
@@ -67,37 +67,33 @@ __device__ __forceinline__ int ol_decoded(int px, int py, int x, int y, const Ti
 }
 
 // Occupancy target per shape, in waves per SIMD.  At 4 the compiler keeps a kernel under 128 VGPRs and the extra waves
-// hide the LDS and table latency, which outweighs the spills that costs most small shapes; the shapes listed at 3
-// spill 150-340 bytes per lane at 4 or 5 and run faster with 168 VGPRs (measured on MI355X, kernel trace of the
-// 256-image batch with every shape at each of the targets 2 .. 6, the fastest kept per shape: analysis 642 -> 626 ms;
-// 8x16 63 -> 56 ms).  The 64-wide shapes take 2: 256 VGPRs and no AGPRs (the two share one 512-entry file per lane,
-// so any AGPR beyond 256 VGPRs leaves one wave per SIMD); with the levels over the coefficients that gave 64x64
-// 94 -> 49 ms and 64x32 71 -> 56 ms on the same batch.  Where LDS allows fewer waves than the target the compiler
-// notes that it cannot reach it; the build silences that.
+// hide the LDS and table latency, which outweighs the spills that costs most small shapes; 8x16, 16x8 and 16x16 spill
+// 150-340 bytes per lane at 4 and run faster with 168 VGPRs, as do the shapes of a wave per block (MI355X, 16 images of 12
+// MP, learned: 64x64 9.7 / 7.3 / 6.9 ms, 64x32 9.3 / 7.9 / 8.4, 32x64 9.7 / 7.6 / 7.6, 32x16 6.4 / 5.1 / 6.0, 16x32 5.6 / 5.0
+// / 6.3 at 2 / 3 / 4; all ten 50.9 / 41.0 / 43.8).  Where LDS allows fewer waves than the target the compiler notes that
+// it cannot reach it; the build silences that.
 constexpr int an_wpe(int W, int H) {
-    return W == 64 ? 2
-         : (W == 8 && H == 16) || (W == 16 && H == 8) || (W == 16 && H == 16) || (W == 16 && H == 32) || (W == 32 && H == 32) ||
-                   (W == 32 && H == 64)
-             ? 3
-             : 4;
+    return W >= 32 || H >= 32 || (W == 8 && H == 16) || (W == 16 && H == 8) || (W == 16 && H == 16) ? 3 : 4;
 }
 // HOOKS: the instance that reads an external screener's candidates and / or a block list (AnHook); the default instance
 // has neither, so their registers do not weigh on it.
 template <int W, int H, int BS, typename Px, bool HOOKS>
-__global__ void __launch_bounds__(an_groups(W, H) * 32) __attribute__((amdgpu_waves_per_eu(an_wpe(W, H)))) k_analysis(Batch B, SearchParams P,
+__global__ void __launch_bounds__(AN_NT) __attribute__((amdgpu_waves_per_eu(an_wpe(W, H)))) k_analysis(Batch B, SearchParams P,
                                                                                                       uint32_t nTotal, AnHook hk) {
     constexpr int NG = an_groups(W, H), TXS = tx_of(W, H);
     constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 4 ? 2 : H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
     constexpr int NSUB = (W / 4) * (H / 4), NSX = W / 4;
     __shared__ AnScr<W, H> sm[NG];
-    AnScr<W, H> &S = sm[gid()];
+    constexpr bool WAVE = an_wave<W, H>();
+    const int blk = WAVE ? threadIdx.x >> 6 : gid();   // the two halves of a wave do the same in what is not spread over 64
+    AnScr<W, H> &S = sm[blk];
     const DevTables &T = *B.T;
     const int lane = glane();
     const uint32_t *starts = B.shStart + (size_t)BS * (B.nimg + 1);
     const int set = tx_set_intra(TXS);
     // a block list (k_an_blank has set every record of the shape to "not analysed"): the groups take its entries
     const uint32_t nItems = (HOOKS && hk.list) ? min(*hk.count, nTotal) : nTotal;
-    for (uint32_t item = blockIdx.x * NG + gid(); item < nItems; item += gridDim.x * NG) {
+    for (uint32_t item = blockIdx.x * NG + blk; item < nItems; item += gridDim.x * NG) {
         const uint32_t gb = (HOOKS && hk.list) ? hk.list[item] : item;
         if (HOOKS && gb >= nTotal) continue;   // an entry outside the shape
         int lo = 0, hi = B.nimg - 1;
@@ -222,7 +218,7 @@ __global__ void __launch_bounds__(an_groups(W, H) * 32) __attribute__((amdgpu_wa
                 gsync();
                 return;
             }
-            if constexpr (NSUB <= 8) {
+            if constexpr (NSUB < 4 || (NSUB <= 8 && NSY < 2)) {
                 constexpr int PIX = NSUB * 16, SEG = PIX < GW ? PIX : GW, NPL = PIX > GW ? PIX / GW : 1;
                 // the pixel of item base + lane is (lane % SEG) + 32 k, k = (base / 32) % NPL, for every candidate: the
                 // lane's NPL source samples are loaded once
@@ -253,35 +249,43 @@ __global__ void __launch_bounds__(an_groups(W, H) * 32) __attribute__((amdgpu_wa
                 gsync();
                 return;
             }
-            if constexpr (NSUB >= GW) {
-                // every candidate gives lane l the same 4x4s (l, l + 32, ...): each is loaded once and screened for all
-                // the candidates in turn, the group summing each candidate's costs (integers: any order)
-                for (int sb = lane; sb < NSUB; sb += GW) {
+            if constexpr (WAVE) {
+                // lane l of the wave keeps 4x4 l % NSUB (l, l + 64, ... where there are more), loaded once for all the
+                // candidates; 64 / NSUB candidates at a time where there are fewer, the lanes of each summing its costs
+                constexpr int LPC = NSUB < 64 ? NSUB : 64, CPR = 64 / LPC;
+                static_assert(NSUB >= 16 && (NSUB <= 64 || NSUB % 64 == 0), "whole segments of 4x4s");
+                const int wl = wlane();
+                for (int sb = wl % LPC; sb < NSUB; sb += LPC) {
                     const int sx = (sb % NSX) * 4, sy = (sb / NSX) * 4;
                     int sv[16];
 #pragma unroll
                     for (int i = 0; i < 4; i++)
 #pragma unroll
                         for (int j = 0; j < 4; j++) sv[i * 4 + j] = src[(sy + i) * sp + sx + j];
-                    for (int ci = c0; ci < c1; ci++) {
-                        const int c = S.cand[ci], m = cand_mode(c), pa = pangle(m, cand_delta(c));
+                    for (int cq = c0; cq < c1; cq += CPR) {
+                        const int ci = cq + wl / LPC;
                         int d[16];
 #pragma unroll
-                        for (int j = 0; j < 4; j++) {   // one run of pred_col per column of the 4x4
-                            int r[4];
-                            pred_col(m, pa, dcv, sy, 1, sx + j, LW, LH, A, L, 0, 0, r);
+                        for (int q = 0; q < 16; q++) d[q] = 0;
+                        if (ci < c1) {
+                            int c = S.cand[ci];
+                            if constexpr (CPR == 1) c = __builtin_amdgcn_readfirstlane(c);   // one candidate: scalar branches
+                            const int m = cand_mode(c), pa = pangle(m, cand_delta(c));
+                            int r[16];
+                            pred_4x4(m, pa, dcv, sy, sx, LW, LH, A, L, r);
 #pragma unroll
-                            for (int i = 0; i < 4; i++) d[i * 4 + j] = sv[i * 4 + j] - r[i];
+                            for (int q = 0; q < 16; q++) d[q] = sv[q] - r[q];
                         }
-                        const int v = seg_sumi<GW>(hadamard4(d));
-                        if (lane == 0) S.satdI[ci] += v;
+                        int v = seg_sumi<LPC < GW ? LPC : GW>(hadamard4(d));
+                        if constexpr (LPC == 64) v += other_half(v);
+                        if (wl % LPC == 0 && ci < c1) S.satdI[ci] += v;
                     }
                 }
                 gsync();
                 return;
             }
             if constexpr (NSUB == 16) {
-                // the same with 16 4x4s: lane l keeps 4x4 l % 16, two candidates a round (one per half)
+                // every candidate gives lane l the same 4x4 (l % 16): loaded once, two candidates a round (one per half)
                 const int sb = lane & 15, sx = (sb % NSX) * 4, sy = (sb / NSX) * 4;
                 int sv[16];
 #pragma unroll
@@ -295,13 +299,10 @@ __global__ void __launch_bounds__(an_groups(W, H) * 32) __attribute__((amdgpu_wa
                     for (int q = 0; q < 16; q++) d[q] = 0;
                     if (ci < c1) {
                         const int c = S.cand[ci], m = cand_mode(c), pa = pangle(m, cand_delta(c));
+                        int r[16];
+                        pred_4x4(m, pa, dcv, sy, sx, LW, LH, A, L, r);
 #pragma unroll
-                        for (int j = 0; j < 4; j++) {
-                            int r[4];
-                            pred_col(m, pa, dcv, sy, 1, sx + j, LW, LH, A, L, 0, 0, r);
-#pragma unroll
-                            for (int i = 0; i < 4; i++) d[i * 4 + j] = sv[i * 4 + j] - r[i];
-                        }
+                        for (int q = 0; q < 16; q++) d[q] = sv[q] - r[q];
                     }
                     const int v = seg_sumi<16>(hadamard4(d));
                     if ((lane & 15) == 0 && ci < c1) S.satdI[ci] += v;
@@ -309,29 +310,6 @@ __global__ void __launch_bounds__(an_groups(W, H) * 32) __attribute__((amdgpu_wa
                 gsync();
                 return;
             }
-            constexpr int SEG = NSUB < GW ? NSUB : GW;
-            const int items = (c1 - c0) * NSUB;
-            for (int base = 0; base < items; base += GW) {
-                const int it = base + lane;
-                int v = 0, ci = c0;
-                if (it < items) {
-                    ci = c0 + it / NSUB;
-                    const int sb = it % NSUB, sx = (sb % NSX) * 4, sy = (sb / NSX) * 4;
-                    const int c = S.cand[ci], m = cand_mode(c), pa = pangle(m, cand_delta(c));
-                    int d[16];
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {   // one run of pred_col per column of the 4x4
-                        int r[4];
-                        pred_col(m, pa, dcv, sy, 1, sx + j, LW, LH, A, L, 0, 0, r);
-#pragma unroll
-                        for (int i = 0; i < 4; i++) d[i * 4 + j] = (int)src[(sy + i) * sp + sx + j] - r[i];
-                    }
-                    v = hadamard4(d);
-                }
-                v = seg_sumi<SEG>(v);
-                if (it < items && (it & (SEG - 1)) == 0) atomicAdd(&S.satdI[ci], v);
-            }
-            gsync();
         };
         screen(0, n13);
         float js = lane < n13 ? fmaf(lamS, mbits(S.cand[lane]), (float)S.satdI[lane] * 0.25f) : INF;
@@ -368,8 +346,10 @@ __global__ void __launch_bounds__(an_groups(W, H) * 32) __attribute__((amdgpu_wa
         for (int st = 0; st < nSteps; st++) {
             const int k = st < nK ? st : bestK, t = st < nK ? DCT_DCT : st - nK + 1;
             if (t != DCT_DCT && !tx_in_set(set, t)) continue;
-            const int c = S.cand[top[k]], m = cand_mode(c), pa = pangle(m, cand_delta(c));
-            if constexpr (an_direct<W, H>()) {   // DCT_DCT only (st < nK): prediction and forward DCT in one pass
+            int c = S.cand[top[k]];
+            if constexpr (WAVE) c = __builtin_amdgcn_readfirstlane(c);
+            const int m = cand_mode(c), pa = pangle(m, cand_delta(c));
+            if constexpr (WAVE) {   // DCT_DCT only (st < nK): prediction and forward DCT in one pass
                 const uint16_t *EA = A, *EL = L;
                 int upA = 0, upL = 0;
                 if (I.edgeFilter && is_dir(m)) {
@@ -379,17 +359,16 @@ __global__ void __launch_bounds__(an_groups(W, H) * 32) __attribute__((amdgpu_wa
                     EA = S.pa + EDGE_OFF;
                     EL = S.pl + EDGE_OFF;
                 }
-                auto res = [&](int i0, int j, auto &r) {
-                    pred_col(m, pa, dcv, i0, 1, j, LW, LH, EA, EL, upA, upL, r);
+                auto res = [&](int i0, int di, int j, auto &r) {
+                    pred_col(m, pa, dcv, i0, di, j, LW, LH, EA, EL, upA, upL, r);
                     constexpr int CH = sizeof(r) / sizeof(r[0]);
 #pragma unroll
-                    for (int c = 0; c < CH; c++) r[c] = (int)src[(i0 + c) * sp + j] - r[c];
+                    for (int c = 0; c < CH; c++) r[c] = (int)src[(i0 + c * di) * sp + j] - r[c];
                 };
-                lds<float> *tl = (lds<float> *)(lds<char> *)(char *)S.ev.tmp;
-                e.resEnergy = grp_fwd_dct<W, H>(tl, T, T.txScale[TXS], res);
+                e.resEnergy = wave_fwd_dct<W, H, decltype(S.ev)::TS>(S.ev.tmp, T, T.txScale[TXS], res);
                 e.txType = DCT_DCT;
                 e.intraDir = m;
-                const EvalOut o = grp_qrate<W, H>(S.ev.tmp, W + 1, S.ev.lev(), e, T);
+                const EvalOut o = wave_qrate<W, H>(S.ev.tmp, decltype(S.ev)::TS, S.ev.lev(), e, T);
                 const float J = fmaf(lambda, (o.R + mbits(c)) + overhead, o.D);
                 if (J < bestJ) { bestJ = J; bestK = k; }
                 gsync();
@@ -411,7 +390,6 @@ __global__ void __launch_bounds__(an_groups(W, H) * 32) __attribute__((amdgpu_wa
                     S.ev.res[p] = (int16_t)((int)src[i * sp + j] - pr);
                 }
                 gsync();
-                e.resEnergy = (W == 64 || H == 64) ? grp_res_energy<W, H>(S.ev.res) : 0.f;
                 resK = k;
             }
             e.txType = t;
@@ -425,7 +403,7 @@ __global__ void __launch_bounds__(an_groups(W, H) * 32) __attribute__((amdgpu_wa
             gsync();
             }
         }
-        if (lane == 0) {
+        if (WAVE ? wlane() == 0 : lane == 0) {
             out.J = nK ? bestJ : INF;
             out.tx = (uint8_t)bestTx;
             int n = 0;
@@ -484,18 +462,18 @@ static void launch_an(const Batch &B, const SearchParams &P, uint32_t n, int bd,
     // share nothing here)
     const bool hooked = hk.ext || hk.list;
     constexpr int M = an_slot_mult(W, H);
-    const uint32_t c = bd == 10 ? (hooked ? an_grid_cap(k_analysis<W, H, BS, uint16_t, true>, NG * 32, M)
-                                          : an_grid_cap(k_analysis<W, H, BS, uint16_t, false>, NG * 32, M))
-                                : (hooked ? an_grid_cap(k_analysis<W, H, BS, uint8_t, true>, NG * 32, M)
-                                          : an_grid_cap(k_analysis<W, H, BS, uint8_t, false>, NG * 32, M));
+    const uint32_t c = bd == 10 ? (hooked ? an_grid_cap(k_analysis<W, H, BS, uint16_t, true>, AN_NT, M)
+                                          : an_grid_cap(k_analysis<W, H, BS, uint16_t, false>, AN_NT, M))
+                                : (hooked ? an_grid_cap(k_analysis<W, H, BS, uint8_t, true>, AN_NT, M)
+                                          : an_grid_cap(k_analysis<W, H, BS, uint8_t, false>, AN_NT, M));
     uint32_t grid = (n + NG - 1) / NG;
     if (grid > c) grid = c;
     if (bd == 10) {
-        if (hooked) hipLaunchKernelGGL((k_analysis<W, H, BS, uint16_t, true>), dim3(grid), dim3(NG * 32), 0, st, B, P, n, hk);
-        else hipLaunchKernelGGL((k_analysis<W, H, BS, uint16_t, false>), dim3(grid), dim3(NG * 32), 0, st, B, P, n, hk);
+        if (hooked) hipLaunchKernelGGL((k_analysis<W, H, BS, uint16_t, true>), dim3(grid), dim3(AN_NT), 0, st, B, P, n, hk);
+        else hipLaunchKernelGGL((k_analysis<W, H, BS, uint16_t, false>), dim3(grid), dim3(AN_NT), 0, st, B, P, n, hk);
     } else {
-        if (hooked) hipLaunchKernelGGL((k_analysis<W, H, BS, uint8_t, true>), dim3(grid), dim3(NG * 32), 0, st, B, P, n, hk);
-        else hipLaunchKernelGGL((k_analysis<W, H, BS, uint8_t, false>), dim3(grid), dim3(NG * 32), 0, st, B, P, n, hk);
+        if (hooked) hipLaunchKernelGGL((k_analysis<W, H, BS, uint8_t, true>), dim3(grid), dim3(AN_NT), 0, st, B, P, n, hk);
+        else hipLaunchKernelGGL((k_analysis<W, H, BS, uint8_t, false>), dim3(grid), dim3(AN_NT), 0, st, B, P, n, hk);
     }
 }
 

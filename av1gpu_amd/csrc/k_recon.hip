@@ -23,10 +23,8 @@
 namespace av1m {
 
 constexpr int RC_NT = 256, RC_NG = 8;
-// transform teams for tx blocks with a side of 32 or 64 (groups 0 .. nTeam - 1): RC_NTEAM of them inside RcShared keep
-// the workgroup's LDS under half a compute unit's, so two workgroups share a CU; the one-workgroup-per-CU instance adds
-// RC_NTEAM more after RcShared (every group a team)
-constexpr int RC_NTEAM = 4;
+// transform teams for tx blocks with a side of 32 or 64: the waves
+constexpr int RC_NTEAM = RC_NT / 64;
 
 constexpr int RC_SMALL_RES = 16;
 // levels of every task of a tx block up to 16x16, packed by the block's size (task t at t * W * H): at most 6 candidates
@@ -44,12 +42,10 @@ struct RcSmall {
     int16_t res[RC_SMALL_RES][256];
     int16_t lev[RC_LEV_TOTAL];
 };
-// scratch of one group evaluating a transform block with a side of 32 or 64 (DCT_DCT only)
-// The levels overlay the coefficients: the quantizer's round t writes levels 32 t .. 32 t + 31, the bytes of tmp's floats
-// 16 t .. 16 t + 15, and coefficient 32 t + k lies at float 32 t + k or later (row stride W + 1): read in this round
-// before its store (each lane's store depends on its own load) or in an earlier one.
+// scratch of one wave evaluating a transform block with a side of 32 or 64 (DCT_DCT only): the kept coefficients, which the
+// levels overlay, and the prepared edges
 struct RcTeam {
-    float tmp[32 * 65];      // th x (W + 1): column-pass outputs, then the coefficients, then the levels
+    float tmp[32 * 33];
     uint16_t ea[EDGE_LEN], el[EDGE_LEN];
 };
 template <typename X> __device__ __forceinline__ lds<int16_t> *team_lev(X &t) { return (lds<int16_t> *)(lds<char> *)t.tmp; }
@@ -84,9 +80,14 @@ __device__ __forceinline__ auto iscan_ptr(const lds<RcTabs> &T) {
     else return T.iscan + dscan_off(t);
 }
 
+struct RcBig {
+    RcTeam t[RC_NTEAM];
+    int16_t inv[64 * 64];    // inverse transform residual (the row pass clamps to 16 bits; the column outputs of a block
+                             // passing the range checks are within 12)
+};
 union RcScr {
     RcSmall s;
-    RcTeam t[RC_NTEAM];
+    RcBig b;
 };
 struct RcShared {
     RcScr u;
@@ -98,7 +99,7 @@ struct RcShared {
     uint16_t ea[3][EDGE_LEN], el[3][EDGE_LEN];   // unfiltered edges of the current tx block per plane
     int dcv[3], ft[3], hvL[3], hvA[3], px[3], py[3], mx[3], my[3];
     int skipCtx[3], dcCtx[3];
-    int gup[RC_NG][2];                       // upsampling flags of each group's prepared edges
+    int gup[RC_NG][2];                       // upsampling flags of each group's (team's) prepared edges
     uint8_t bdm[3][18][18];                  // BlockDecoded[plane][y + 1][x + 1]
     int taskC[64], taskT[64], taskP[64], taskE[64], taskK[64];   // candidate, tx type, plane, eob, residual slot
     int candC[8], nCand;                     // luma: the re-checked candidates
@@ -113,7 +114,6 @@ struct RcShared {
     int satdI[32], uvc[32];
     float uvJ[32];                           // screening costs of the UV candidates
     int nTxb, nCoef, errFlag, nzFlag, eobOut, culOut;
-    int nTeam;                               // transform teams: RC_NTEAM, or 2 * RC_NTEAM with the extra ones after RcShared
     int flopsOn;                             // count the forward-transform work (Batch::flops set)
     unsigned long long flops;                // of the superblock so far
     int am, lm, mode, delta, uvMode, uvDelta, nuv, bsize;
@@ -123,26 +123,13 @@ struct RcShared {
                                              // superblock's own luma; [0] bit 31: a wait failed
 };
 
-// scratch of transform team g: the first RC_NTEAM share the union with the small-block scratch, the others follow RcShared
-__device__ __forceinline__ lds<RcTeam> &team_scr(lds<RcShared> &S, int g) {
-    return g < RC_NTEAM ? S.u.t[g] : ((lds<RcTeam> *)(lds<char> *)(&S + 1))[g - RC_NTEAM];
-}
-__device__ __forceinline__ const lds<RcTeam> &team_scr(const lds<RcShared> &S, int g) {
-    return g < RC_NTEAM ? S.u.t[g] : ((const lds<RcTeam> *)(const lds<char> *)(&S + 1))[g - RC_NTEAM];
-}
-
 template <typename Px> __device__ __forceinline__ glb<Px> *rec_plane(const lds<Img> &I, int p) { return (glb<Px> *)I.rec[p]; }
 template <typename Px> __device__ __forceinline__ const glb<Px> *src_plane(const lds<Img> &I, int p) { return (const glb<Px> *)I.src[p]; }
 __device__ __forceinline__ glb<uint8_t> *map8(uint8_t *p) { return (glb<uint8_t> *)p; }
-// Scratch of the exact inverse (the residual, W x H): the evaluations' scratch is free once the levels are decided.  The
-// levels and edges of team t and of t ^ 1 (the other plane of a chroma pair) must stay, so blocks with a side of 32 or 64
-// take the coefficients of team (t & 3) ^ 2, smaller ones group 0's.
-__device__ __forceinline__ lds<int16_t> *inv_scr(lds<RcShared> &S, int txSz, int team);
-
-__device__ __forceinline__ lds<int16_t> *inv_scr(lds<RcShared> &S, int txSz, int team) {
-    static_assert(sizeof(RcGroup::tmp) >= 16 * 16 * 2 && sizeof(RcTeam::tmp) >= 64 * 64 * 2 && RC_NTEAM == 4, "the inverse's scratch");
-    const bool big = tx_w(txSz) > 16 || tx_h(txSz) > 16;
-    return (lds<int16_t> *)(lds<char> *)(big ? S.u.t[(team & 3) ^ 2].tmp : S.u.s.g[0].tmp);
+// scratch of the exact inverse (the residual, W x H): the small blocks' evaluations are done with theirs by then
+__device__ __forceinline__ lds<int16_t> *inv_scr(lds<RcShared> &S, int txSz) {
+    static_assert(sizeof(RcGroup::tmp) >= 16 * 16 * 2, "the inverse's scratch");
+    return tx_w(txSz) > 16 || tx_h(txSz) > 16 ? S.u.b.inv : (lds<int16_t> *)(lds<char> *)S.u.s.g[0].tmp;
 }
 
 // get_filter_type (spec 7.11.2.8): 1 if the above or left block (chroma: the chroma-carrying one) uses a SMOOTH mode
@@ -282,11 +269,13 @@ __device__ EvalOut half_task(lds<RcShared> &S, lds<float> *tmp, const lds<Img> &
     return half_eval<W, H>(res, tmp, lev, e, S.tab);
 }
 
-// one RD task (candidate c, 255 = CfL, of plane p; DCT_DCT) of a tx block with a side of 32 or 64 by the calling group
+// one RD task (candidate c, 255 = CfL, of plane p; DCT_DCT) of a tx block with a side of 32 or 64 by the calling wave (its
+// two groups prepare the same edges)
 template <int W, int H>
-__device__ EvalOut grp_task_big(lds<RcShared> &S, lds<RcTeam> &X, const lds<Img> &I, const DevTables &T, int p, int c,
-                                const lds<uint16_t> *src, int sp, const SearchParams &P) {
+__device__ EvalOut wave_task(lds<RcShared> &S, lds<RcTeam> &X, int team, const lds<Img> &I, const DevTables &T, int p, int c,
+                             const lds<uint16_t> *src, int sp, const SearchParams &P) {
     constexpr int LW = W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
+    constexpr int TS = (W > 32 ? 32 : W) + 1;
     const int lane = glane(), bd = I.bd;
     const int m = c == 255 ? DC_PRED : cand_mode(c), pa = pangle(m, c == 255 ? 0 : cand_delta(c));
     const lds<uint16_t> *EA = S.ea[p] + EDGE_OFF, *EL = S.el[p] + EDGE_OFF;
@@ -299,28 +288,28 @@ __device__ EvalOut grp_task_big(lds<RcShared> &S, lds<RcTeam> &X, const lds<Img>
         EA = X.ea + EDGE_OFF;
         EL = X.el + EDGE_OFF;
     }
-    if (lane == 0) { S.gup[gid()][0] = upA; S.gup[gid()][1] = upL; }
+    if (wlane() == 0) { S.gup[team][0] = upA; S.gup[team][1] = upL; }
     const int dcv = S.dcv[p], alpha = c == 255 ? S.cflAlpha[p - 1] : 0, cavg = S.cflAvg;
-    auto res = [&](int i0, int j, auto &r) {
+    auto res = [&](int i0, int di, int j, auto &r) {
         constexpr int CH = sizeof(r) / sizeof(r[0]);
         if (c == 255) {
 #pragma unroll
-            for (int k = 0; k < CH; k++) r[k] = clip3(0, (1 << bd) - 1, dcv + round2signed(alpha * (S.cflL[(i0 + k) * W + j] - cavg), 6));
+            for (int k = 0; k < CH; k++) r[k] = clip3(0, (1 << bd) - 1, dcv + round2signed(alpha * (S.cflL[(i0 + k * di) * W + j] - cavg), 6));
         } else {
-            pred_col(m, pa, dcv, i0, 1, j, LW, LH, EA, EL, upA, upL, r);
+            pred_col(m, pa, dcv, i0, di, j, LW, LH, EA, EL, upA, upL, r);
         }
 #pragma unroll
-        for (int k = 0; k < CH; k++) r[k] = (int)src[(i0 + k) * sp + j] - r[k];
+        for (int k = 0; k < CH; k++) r[k] = (int)src[(i0 + k * di) * sp + j] - r[k];
     };
     const int txSz = tx_of(W, H);
     RcEvalIn e;
-    e.resEnergy = grp_fwd_dct<W, H>(X.tmp, T, S.tab.txScale[txSz], res);
+    e.resEnergy = wave_fwd_dct<W, H, TS>(X.tmp, T, S.tab.txScale[txSz], res);
     e.txSz = txSz; e.txType = DCT_DCT; e.plane = p;
     e.dcQ = S.dcQ; e.acQ = S.acQ; e.dcRcp = S.dcRcp; e.acRcp = S.acRcp;
     e.skipCtx = S.skipCtx[p]; e.dcCtx = S.dcCtx[p]; e.intraDir = p == 0 ? cand_mode(c) : 0; e.bd = bd;
     e.rnd = p ? P.rndC : P.rnd; e.zbin = p ? P.zbinC : P.zbin;
     e.C = &S.tab.cost;
-    return grp_qrate<W, H>(X.tmp, W + 1, (lds<lev16> *)team_lev(X), e, S.tab);
+    return wave_qrate<W, H>(X.tmp, TS, (lds<lev16> *)team_lev(X), e, S.tab);
 }
 
 // ---- exact inverse transform + reconstruction by the workgroup (spec 7.13.3, 7.12.3 step 3) ----
@@ -493,7 +482,7 @@ __device__ __forceinline__ const lds<uint16_t> *stage_src(const lds<RcShared> &S
 // J = fmaf(lambda, R + extra, D) with extra = luma mode bits (plane 0) or 0; S.taskJ / taskE.  Then S.win = the first
 // minimum over the tasks.  Blocks up to 16x16: luma tasks read the residual of their candidate (S.taskK), made by
 // wg_luma_residuals; chroma tasks make their own in slot t; levels of task t go to S.u.s.lev[t].  Larger blocks:
-// team g (tasks g, g + nTeam, ..., run in descending order) keeps the levels and prepared edges of task g.
+// team g (tasks g, g + RC_NTEAM, ..., run in descending order) keeps the levels and prepared edges of task g.
 template <int W, int H>
 __device__ __forceinline__ void wg_run_tasks(lds<RcShared> &S, const lds<Img> &I, const DevTables &T, const SearchParams &P, float lambda, bool lumaBits,
                              bool pickWinner) {
@@ -537,15 +526,18 @@ __device__ __forceinline__ void wg_run_tasks(lds<RcShared> &S, const lds<Img> &I
             gsync();
         }
     }
-    const int NGT = big ? S.nTeam : RC_NG;   // big tasks: the teams (groups 0 .. nTeam - 1)
-    // a team keeps the levels and prepared edges of its last task only: it runs its tasks in descending order, so the
-    // first tasks -- the analysis's best candidates, the likeliest winners -- are the ones kept
-    const int tFirst = big ? (g < S.nTask ? g + ((S.nTask - 1 - g) / NGT) * NGT : -1) : g, tStep = big ? -NGT : NGT;
-    if (!done && g < NGT) for (int t = tFirst; t >= 0 && t < S.nTask; t += tStep) {
-        const int c = S.taskC[t], tt = S.taskT[t], p = S.taskP[t];
+    // big tasks: one per team at a time.  A team keeps the levels and prepared edges of its last task only: it runs its
+    // tasks in descending order, so the first tasks -- the analysis's best candidates, the likeliest winners -- are kept
+    constexpr int NGT = big ? RC_NTEAM : RC_NG;
+    const int me = big ? (int)(threadIdx.x >> 6) : g;
+    const int tFirst = big ? (me < S.nTask ? me + ((S.nTask - 1 - me) / NGT) * NGT : -1) : me, tStep = big ? -NGT : NGT;
+    if (!done) for (int t = tFirst; t >= 0 && t < S.nTask; t += tStep) {
+        int c = S.taskC[t], p = S.taskP[t];
+        const int tt = S.taskT[t];
+        if constexpr (big) { c = __builtin_amdgcn_readfirstlane(c); p = __builtin_amdgcn_readfirstlane(p); }   // the wave's task
         EvalOut o;
         if constexpr (big) {
-            o = grp_task_big<W, H>(S, team_scr(S, g), I, T, p, c, stage_src(S, p), W, P);
+            o = wave_task<W, H>(S, S.u.b.t[me], me, I, T, p, c, stage_src(S, p), W, P);
         } else {
             if (!lumaBits)   // chroma: this task's own residual
                 grp_residual<W, H>(S, I.edgeFilter ? S.u.s.g[g].ea : nullptr, S.u.s.g[g].el, p, c, stage_src(S, p), W, S.u.s.res[t], I.bd);
@@ -592,17 +584,17 @@ __device__ void wg_luma_residuals(lds<RcShared> &S, const lds<Img> &I) {
 }
 
 // the levels of the winning task t, and (larger blocks) the team holding them with its prepared edges: the team's
-// kept task is t (t < nTeam), or it evaluates t again
+// kept task is t (t < RC_NTEAM), or it evaluates t again
 template <int W, int H>
 __device__ __forceinline__ lds<int16_t> *wg_final_levels(lds<RcShared> &S, const lds<Img> &I, const DevTables &T, const SearchParams &P, int t, int &team) {
-    team = (W > 16 || H > 16) ? t % S.nTeam : t % RC_NG;
+    team = (W > 16 || H > 16) ? t % RC_NTEAM : t % RC_NG;
     if constexpr (W > 16 || H > 16) {
-        if (t >= S.nTeam) {   // overwritten by a task of the same team that ran after it
+        if (t >= RC_NTEAM) {   // overwritten by a task of the same team that ran after it
             const int p = S.taskP[t];
-            if (gid() == team) grp_task_big<W, H>(S, team_scr(S, team), I, T, p, S.taskC[t], stage_src(S, p), W, P);
+            if ((int)(threadIdx.x >> 6) == team) wave_task<W, H>(S, S.u.b.t[team], team, I, T, p, S.taskC[t], stage_src(S, p), W, P);
             __syncthreads();
         }
-        return team_lev(team_scr(S, team));
+        return team_lev(S.u.b.t[team]);
     } else {
         return S.u.s.lev + t * (W * H);
     }
@@ -614,7 +606,7 @@ template <int W, int H, typename Px>
 __device__ void wg_final_pred(const lds<RcShared> &S, const lds<Img> &I, int p, int t, int k, int team, glb<Px> *dst, int pitch) {
     constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 4 ? 2 : H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
     if constexpr (W > 16 || H > 16) {
-        wg_write_pred<Px>(S, I.edgeFilter ? team_scr(S, team).ea : nullptr, team_scr(S, team).el, team, p, S.taskC[t], LW, LH, dst, pitch, I.bd);
+        wg_write_pred<Px>(S, I.edgeFilter ? S.u.b.t[team].ea : nullptr, S.u.b.t[team].el, team, p, S.taskC[t], LW, LH, dst, pitch, I.bd);
     } else {
         const lds<uint16_t> *src = stage_src(S, p);
         const lds<int16_t> *res = S.u.s.res[k];
@@ -694,7 +686,7 @@ __device__ __noinline__ void rc_luma(lds<RcShared> &S, const Batch &B, const Sea
     glb<Px> *dst = rec_plane<Px>(I, 0) + (size_t)y * I.pitch[0] + x;
     wg_final_pred<W, H, Px>(S, I, 0, win, S.taskK[win], team, dst, I.pitch[0]);
     if (S.taskE[win] > 0) {
-        const int fixes = wg_inverse_add<Px>(S, q, inv_scr(S, txSz, team), txSz, S.taskT[win], I.bd, dst, I.pitch[0]);
+        const int fixes = wg_inverse_add<Px>(S, q, inv_scr(S, txSz), txSz, S.taskT[win], I.bd, dst, I.pitch[0]);
         if (fixes && tid == 0) atomicAdd(&B.stats[3], 1u);
     }
     const int eob = wg_record_txb(S, B, sb, I, 0, txSz, S.taskT[win], x >> 2, y >> 2, q);
@@ -970,14 +962,12 @@ __device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const S
                 const int sx = (sbk % NSX) * 4, sy = (sbk / NSX) * 4, c = S.uvc[ci], m = cand_mode(c), pa = pangle(m, cand_delta(c));
                 const lds<uint16_t> *s = p == 1 ? srcU : srcV;
                 const lds<uint16_t> *A = S.ea[p] + EDGE_OFF, *L = S.el[p] + EDGE_OFF;
-                int d[16];
+                int d[16], r[16];
+                pred_4x4(m, pa, S.dcv[p], sy, sx, LW, LH, A, L, r);
 #pragma unroll
-                for (int j = 0; j < 4; j++) {   // one run of pred_col per column of the 4x4
-                    int r[4];
-                    pred_col(m, pa, S.dcv[p], sy, 1, sx + j, LW, LH, A, L, 0, 0, r);
+                for (int i = 0; i < 4; i++)
 #pragma unroll
-                    for (int i = 0; i < 4; i++) d[i * 4 + j] = (int)s[(sy + i) * sp + sx + j] - r[i];
-                }
+                    for (int j = 0; j < 4; j++) d[i * 4 + j] = (int)s[(sy + i) * sp + sx + j] - r[i * 4 + j];
                 v = hadamard4(d);
             }
             v = seg_sumi<SEG>(v);
@@ -1063,7 +1053,7 @@ __device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const S
         glb<Px> *dst = rec_plane<Px>(I, p) + (size_t)cy * I.pitch[p] + cx;
         wg_final_pred<W, H, Px>(S, I, p, t, t, team, dst, I.pitch[p]);
         if (S.taskE[t] > 0) {
-            const int fixes = wg_inverse_add<Px>(S, q, inv_scr(S, txSz, team), txSz, uvTxType, bd, dst, I.pitch[p]);
+            const int fixes = wg_inverse_add<Px>(S, q, inv_scr(S, txSz), txSz, uvTxType, bd, dst, I.pitch[p]);
             if (fixes && tid == 0) atomicAdd(&B.stats[3], 1u);
         }
         int eob = wg_record_txb(S, B, sb, I, p, txSz, uvTxType, x4, y4, q);
@@ -1089,7 +1079,7 @@ __device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const S
             glb<Px> *dk = rec_plane<Px>(I, p) + (size_t)(cy + oy) * I.pitch[p] + cx + ox;
             wg_final_pred<W, H, Px>(S, I, p, 0, 0, tm, dk, I.pitch[p]);
             if (S.taskE[0] > 0) {
-                const int fixes = wg_inverse_add<Px>(S, qk, inv_scr(S, txSz, tm), txSz, uvTxType, bd, dk, I.pitch[p]);
+                const int fixes = wg_inverse_add<Px>(S, qk, inv_scr(S, txSz), txSz, uvTxType, bd, dk, I.pitch[p]);
                 if (fixes && tid == 0) atomicAdd(&B.stats[3], 1u);
             }
             eob |= wg_record_txb(S, B, sb, I, p, txSz, uvTxType, x4 + (ox >> 2), y4 + (oy >> 2), qk);
@@ -1339,9 +1329,8 @@ __device__ bool recon_part(lds<RcShared> &S, const Batch &B, const SearchParams 
 }
 
 // RcShared allows two workgroups per compute unit.  WPE 2 holds the registers to 256 so both fit (more superblocks in
-// flight: batches); WPE 1 is one workgroup per CU, which spends the registers and the rest of the LDS on the latency of
-// one superblock (fewer spills, eight transform teams: a single image, whose closed loop is bound by its chain of
-// superblocks).  The same results either way.
+// flight: batches); WPE 1 is one workgroup per CU, which spends the registers on the latency of one superblock (fewer
+// spills: a single image, whose closed loop is bound by its chain of superblocks).  The same results either way.
 #define AV1M_RC_KERNEL(WPE) __global__ void __launch_bounds__(RC_NT) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 
 // The kernels' one parameter, read in place in the kernarg segment (it is the segment's first argument): handing a
@@ -1368,7 +1357,6 @@ AV1M_RC_KERNEL(2) k_recon(RcStepArgs) {
     const Batch &B = A.B;
     const SearchParams &P = A.P;
     const uint32_t sb = A.sbList[blockIdx.x];
-    if (threadIdx.x == 0) S.nTeam = RC_NTEAM;
     stage_tables(S, *B.T, B.img[B.sbImg[sb]].qctx, true);
     __syncthreads();
     recon_part<Px, 0>(S, B, P, sb, nullptr);
@@ -1392,7 +1380,6 @@ AV1M_RC_KERNEL(WPE) k_recon_queue(RcQueueArgs) {
     const RcQueue &Q = A.Q;
     const int tid = threadIdx.x;
     int staged = -1;
-    if (tid == 0) S.nTeam = WPE == 1 ? 2 * RC_NTEAM : RC_NTEAM;
     for (;;) {
         if (tid == 0) {
             uint32_t it = Q.n;
@@ -1420,29 +1407,24 @@ AV1M_RC_KERNEL(WPE) k_recon_queue(RcQueueArgs) {
 }
 
 static_assert(sizeof(RcShared) <= 80 * 1024, "the closed loop's LDS exceeds half a compute unit's 160 KiB");
-static_assert(alignof(RcShared) >= alignof(RcTeam) && sizeof(RcShared) + RC_NTEAM * sizeof(RcTeam) <= 160 * 1024,
-              "the eight-team instance's LDS exceeds a compute unit's");
-// dynamic LDS of the instance at WPE workgroups per CU
-constexpr size_t rc_smem(int wpe) { return sizeof(RcShared) + (wpe == 1 ? RC_NTEAM * sizeof(RcTeam) : 0); }
-size_t recon_smem_bytes() { return rc_smem(1); }
+// dynamic LDS of every instance
+constexpr size_t rc_smem() { return sizeof(RcShared); }
+size_t recon_smem_bytes() { return rc_smem(); }
 
 int recon_prepare(int bd) {
-    const int s2 = (int)rc_smem(2), s1 = (int)rc_smem(1);
-    const hipError_t e = bd == 10 ? hipFuncSetAttribute((const void *)k_recon<uint16_t>, hipFuncAttributeMaxDynamicSharedMemorySize, s2)
-                                  : hipFuncSetAttribute((const void *)k_recon<uint8_t>, hipFuncAttributeMaxDynamicSharedMemorySize, s2);
-    hipError_t f = bd == 10 ? hipFuncSetAttribute((const void *)k_recon_queue<uint16_t, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, s1)
-                            : hipFuncSetAttribute((const void *)k_recon_queue<uint8_t, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, s1);
-    if (f == hipSuccess)
-        f = bd == 10 ? hipFuncSetAttribute((const void *)k_recon_queue<uint16_t, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, s2)
-                     : hipFuncSetAttribute((const void *)k_recon_queue<uint8_t, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, s2);
-    return e == hipSuccess && f == hipSuccess ? 0 : -1;
+    const void *k[3] = {bd == 10 ? (const void *)k_recon<uint16_t> : (const void *)k_recon<uint8_t>,
+                        bd == 10 ? (const void *)k_recon_queue<uint16_t, 1> : (const void *)k_recon_queue<uint8_t, 1>,
+                        bd == 10 ? (const void *)k_recon_queue<uint16_t, 2> : (const void *)k_recon_queue<uint8_t, 2>};
+    for (const void *f : k)
+        if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)rc_smem()) != hipSuccess) return -1;
+    return 0;
 }
 
 void launch_recon(const Batch &B, const SearchParams &P, const uint32_t *dSbList, uint32_t n, int bd, hipStream_t st) {
     if (!n) return;
     const RcStepArgs a{B, P, dSbList};
-    if (bd == 10) hipLaunchKernelGGL(k_recon<uint16_t>, dim3(n), dim3(RC_NT), rc_smem(2), st, a);
-    else hipLaunchKernelGGL(k_recon<uint8_t>, dim3(n), dim3(RC_NT), rc_smem(2), st, a);
+    if (bd == 10) hipLaunchKernelGGL(k_recon<uint16_t>, dim3(n), dim3(RC_NT), rc_smem(), st, a);
+    else hipLaunchKernelGGL(k_recon<uint8_t>, dim3(n), dim3(RC_NT), rc_smem(), st, a);
 }
 
 // resident workgroups of the persistent kernel per compute unit
@@ -1450,11 +1432,11 @@ int recon_queue_slots(int bd, int wpe) {
     int n = 0;
     hipError_t e;
     if (wpe == 2)
-        e = bd == 10 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_recon_queue<uint16_t, 2>, RC_NT, rc_smem(2))
-                     : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_recon_queue<uint8_t, 2>, RC_NT, rc_smem(2));
+        e = bd == 10 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_recon_queue<uint16_t, 2>, RC_NT, rc_smem())
+                     : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_recon_queue<uint8_t, 2>, RC_NT, rc_smem());
     else
-        e = bd == 10 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_recon_queue<uint16_t, 1>, RC_NT, rc_smem(1))
-                     : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_recon_queue<uint8_t, 1>, RC_NT, rc_smem(1));
+        e = bd == 10 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_recon_queue<uint16_t, 1>, RC_NT, rc_smem())
+                     : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_recon_queue<uint8_t, 1>, RC_NT, rc_smem());
     return e == hipSuccess ? n : 0;
 }
 
@@ -1462,11 +1444,11 @@ void launch_recon_queue(const Batch &B, const SearchParams &P, const RcQueue &Q,
     if (!Q.n || !blocks) return;
     const RcQueueArgs a{B, P, Q};
     if (wpe == 2) {
-        if (bd == 10) hipLaunchKernelGGL((k_recon_queue<uint16_t, 2>), dim3(blocks), dim3(RC_NT), rc_smem(2), st, a);
-        else hipLaunchKernelGGL((k_recon_queue<uint8_t, 2>), dim3(blocks), dim3(RC_NT), rc_smem(2), st, a);
+        if (bd == 10) hipLaunchKernelGGL((k_recon_queue<uint16_t, 2>), dim3(blocks), dim3(RC_NT), rc_smem(), st, a);
+        else hipLaunchKernelGGL((k_recon_queue<uint8_t, 2>), dim3(blocks), dim3(RC_NT), rc_smem(), st, a);
     } else {
-        if (bd == 10) hipLaunchKernelGGL((k_recon_queue<uint16_t, 1>), dim3(blocks), dim3(RC_NT), rc_smem(1), st, a);
-        else hipLaunchKernelGGL((k_recon_queue<uint8_t, 1>), dim3(blocks), dim3(RC_NT), rc_smem(1), st, a);
+        if (bd == 10) hipLaunchKernelGGL((k_recon_queue<uint16_t, 1>), dim3(blocks), dim3(RC_NT), rc_smem(), st, a);
+        else hipLaunchKernelGGL((k_recon_queue<uint8_t, 1>), dim3(blocks), dim3(RC_NT), rc_smem(), st, a);
     }
 }
 
