@@ -79,7 +79,16 @@ AV1M_HD int is_dir(int m) { return m >= V_PRED && m <= D67_PRED; }
 AV1M_HD int cand_mode(int c) { return c >> 3; }
 AV1M_HD int cand_delta(int c) { return (c & 7) - 3; }
 AV1M_HD int cand_pack(int m, int d) { return (m << 3) | (d + 3); }
-AV1M_HD int pangle(int mode, int delta) { return is_dir(mode) ? av1t::Mode_To_Angle[mode] + 3 * delta : 0; }
+// Mode_To_Angle of the directional modes V_PRED .. D67_PRED, a byte each (a shift instead of a table read)
+constexpr uint64_t pack_angles() {
+    uint64_t v = 0;
+    for (int m = V_PRED; m <= D67_PRED; m++) v |= (uint64_t)av1t::Mode_To_Angle[m] << (8 * (m - V_PRED));
+    return v;
+}
+AV1M_HD int pangle(int mode, int delta) {
+    constexpr uint64_t a = pack_angles();
+    return is_dir(mode) ? (int)((a >> (8 * (mode - V_PRED))) & 0xFF) + 3 * delta : 0;
+}
 
 AV1M_HD constexpr int tx_set_intra(int t) {
     if (av1t::Tx_Size_Sqr_Up[t] >= TX_32X32) return TX_SET_DCTONLY;

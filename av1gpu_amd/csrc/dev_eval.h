@@ -728,7 +728,9 @@ template <typename P>
 __device__ void grp_edge_filter(P *buf, int sz, int strength) {
     if (!strength) return;
     const int lane = glane();
-    const uint8_t *K = av1t::Intra_Edge_Kernel[strength - 1];
+    // Intra_Edge_Kernel[strength - 1]: 0 4 8 4 0 / 0 5 6 5 0 / 2 4 4 4 2
+    static_assert(av1t::Intra_Edge_Kernel[0][2] == 8 && av1t::Intra_Edge_Kernel[1][1] == 5 && av1t::Intra_Edge_Kernel[2][0] == 2, "edge kernel");
+    const int k0 = strength == 3 ? 2 : 0, k1 = strength == 2 ? 5 : 4, k2 = 10 - 2 * strength;
     int v[5];
 #pragma unroll
     for (int k = 0; k < 5; k++) {
@@ -736,7 +738,7 @@ __device__ void grp_edge_filter(P *buf, int sz, int strength) {
         int s = 0;
         if (i < sz) {
 #pragma unroll
-            for (int j = 0; j < 5; j++) s += K[j] * buf[clip3(0, sz - 1, i - 2 + j) - 1];
+            for (int j = 0; j < 5; j++) s += (j == 2 ? k2 : j == 1 || j == 3 ? k1 : k0) * buf[clip3(0, sz - 1, i - 2 + j) - 1];
         }
         v[k] = (s + 8) >> 4;
     }

@@ -353,7 +353,7 @@ __global__ void __launch_bounds__(AN_NT) __attribute__((amdgpu_waves_per_eu(an_w
                 const uint16_t *EA = A, *EL = L;
                 int upA = 0, upL = 0;
                 if (I.edgeFilter && is_dir(m)) {
-                    for (int i = lane; i < EDGE_LEN; i += GW) { S.pa[i] = S.ea[i]; S.pl[i] = S.el[i]; }
+                    for (int i = lane + EDGE_OFF - 2; i < EDGE_OFF + W + H + 2; i += GW) { S.pa[i] = S.ea[i]; S.pl[i] = S.el[i]; }
                     gsync();
                     grp_edge_prepare(pa, LW, LH, 0, haveL, haveA, x, y, maxX, maxY, S.pa + EDGE_OFF, S.pl + EDGE_OFF, bd, upA, upL);
                     EA = S.pa + EDGE_OFF;
@@ -378,7 +378,7 @@ __global__ void __launch_bounds__(AN_NT) __attribute__((amdgpu_waves_per_eu(an_w
                 const uint16_t *EA = A, *EL = L;
                 int upA = 0, upL = 0;
                 if (I.edgeFilter && is_dir(m)) {
-                    for (int i = lane; i < EDGE_LEN; i += GW) { S.pa[i] = S.ea[i]; S.pl[i] = S.el[i]; }
+                    for (int i = lane + EDGE_OFF - 2; i < EDGE_OFF + W + H + 2; i += GW) { S.pa[i] = S.ea[i]; S.pl[i] = S.el[i]; }
                     gsync();
                     grp_edge_prepare(pa, LW, LH, 0, haveL, haveA, x, y, maxX, maxY, S.pa + EDGE_OFF, S.pl + EDGE_OFF, bd, upA, upL);
                     EA = S.pa + EDGE_OFF;

@@ -113,7 +113,7 @@ struct RcShared {
     unsigned long long acc64[8];
     int satdI[32], uvc[32];
     float uvJ[32];                           // screening costs of the UV candidates
-    int nTxb, nCoef, errFlag, nzFlag, eobOut, culOut;
+    int errFlag[2], nzFlag[2];               // range violations, nonzero levels left (luma or U, V)
     int flopsOn;                             // count the forward-transform work (Batch::flops set)
     unsigned long long flops;                // of the superblock so far
     int am, lm, mode, delta, uvMode, uvDelta, nuv, bsize;
@@ -126,12 +126,6 @@ struct RcShared {
 template <typename Px> __device__ __forceinline__ glb<Px> *rec_plane(const lds<Img> &I, int p) { return (glb<Px> *)I.rec[p]; }
 template <typename Px> __device__ __forceinline__ const glb<Px> *src_plane(const lds<Img> &I, int p) { return (const glb<Px> *)I.src[p]; }
 __device__ __forceinline__ glb<uint8_t> *map8(uint8_t *p) { return (glb<uint8_t> *)p; }
-// scratch of the exact inverse (the residual, W x H): the small blocks' evaluations are done with theirs by then
-__device__ __forceinline__ lds<int16_t> *inv_scr(lds<RcShared> &S, int txSz) {
-    static_assert(sizeof(RcGroup::tmp) >= 16 * 16 * 2, "the inverse's scratch");
-    return tx_w(txSz) > 16 || tx_h(txSz) > 16 ? S.u.b.inv : (lds<int16_t> *)(lds<char> *)S.u.s.g[0].tmp;
-}
-
 // get_filter_type (spec 7.11.2.8): 1 if the above or left block (chroma: the chroma-carrying one) uses a SMOOTH mode
 __device__ int filter_type(const lds<Img> &I, int plane, int mi_row, int mi_col, int availU, int availL) {
     const glb<uint8_t> *m = map8(plane ? I.mUV : I.mY);
@@ -213,7 +207,7 @@ __device__ void grp_residual(lds<RcShared> &S, lds<uint16_t> *gea, lds<uint16_t>
     int upA = 0, upL = 0;
     const bool filt = c != 255 && is_dir(m) && gea != nullptr;
     if (filt) {
-        for (int i = lane; i < EDGE_LEN; i += GW) { gea[i] = S.ea[p][i]; gel[i] = S.el[p][i]; }
+        for (int i = lane + EDGE_OFF - 2; i < EDGE_OFF + W + H + 2; i += GW) { gea[i] = S.ea[p][i]; gel[i] = S.el[p][i]; }   // the filled part
         gsync();
         grp_edge_prepare(pa, lw, lh, S.ft[p], S.hvL[p], S.hvA[p], S.px[p], S.py[p], S.mx[p], S.my[p], gea + EDGE_OFF, gel + EDGE_OFF, bd, upA,
                          upL);
@@ -281,7 +275,7 @@ __device__ EvalOut wave_task(lds<RcShared> &S, lds<RcTeam> &X, int team, const l
     const lds<uint16_t> *EA = S.ea[p] + EDGE_OFF, *EL = S.el[p] + EDGE_OFF;
     int upA = 0, upL = 0;
     if (c != 255 && is_dir(m) && I.edgeFilter) {
-        for (int i = lane; i < EDGE_LEN; i += GW) { X.ea[i] = S.ea[p][i]; X.el[i] = S.el[p][i]; }
+        for (int i = lane + EDGE_OFF - 2; i < EDGE_OFF + W + H + 2; i += GW) { X.ea[i] = S.ea[p][i]; X.el[i] = S.el[p][i]; }
         gsync();
         grp_edge_prepare(pa, LW, LH, S.ft[p], S.hvL[p], S.hvA[p], S.px[p], S.py[p], S.mx[p], S.my[p], X.ea + EDGE_OFF, X.el + EDGE_OFF, bd,
                          upA, upL);
@@ -342,135 +336,6 @@ __device__ __forceinline__ uint32_t inv_col(int j, int W, int ck, int bd, lds<in
 #pragma unroll
     for (int i = 0; i < N; i++) res[i * W + j] = (int16_t)round2l(Tv[i], 4);
     return err;
-}
-
-// dequantize + inverse + add the levels q (LDS, modified by the repair) onto dst; returns the number of repairs
-template <typename Px>
-__device__ __forceinline__ int wg_inverse_add(lds<RcShared> &S, lds<int16_t> *q, lds<int16_t> *inv, int txSz, int txType, int bd, glb<Px> *dst,
-                                              int pitch) {
-    const int dcQ = S.dcQ, acQ = S.acQ;
-    const int tid = threadIdx.x, lw = av1t::Tx_Width_Log2[txSz], lh = av1t::Tx_Height_Log2[txSz], W = 1 << lw, H = 1 << lh;
-    const int tw = W > 32 ? 32 : W, th = H > 32 ? 32 : H, n = tw * th, den = dq_denom(txSz), dsh = den == 4 ? 2 : den == 2 ? 1 : 0;
-    const bool rect = lw - lh == 1 || lh - lw == 1;
-    const int rk = row_kind(txType), ck = col_kind(txType), rs = av1t::Transform_Row_Shift[txSz];
-    int fixes = 0;
-    for (;;) {
-        if (tid == 0) { S.errFlag = 0; S.nzFlag = 0; }
-        __syncthreads();
-        uint32_t err = 0;
-        if (tid < H) {
-            switch (lw) {
-            case 2: err = inv_row<2>(tid, W, th, tw, q, dcQ, acQ, dsh, bd, rect, rk, rs, inv); break;
-            case 3: err = inv_row<3>(tid, W, th, tw, q, dcQ, acQ, dsh, bd, rect, rk, rs, inv); break;
-            case 4: err = inv_row<4>(tid, W, th, tw, q, dcQ, acQ, dsh, bd, rect, rk, rs, inv); break;
-            case 5: err = inv_row<5>(tid, W, th, tw, q, dcQ, acQ, dsh, bd, rect, rk, rs, inv); break;
-            default: err = inv_row<6>(tid, W, th, tw, q, dcQ, acQ, dsh, bd, rect, rk, rs, inv); break;
-            }
-        }
-        if (err) atomicOr(gen(&S.errFlag), (int)err);
-        __syncthreads();
-        err = 0;
-        if (tid < W) {
-            switch (lh) {
-            case 2: err = inv_col<2>(tid, W, ck, bd, inv); break;
-            case 3: err = inv_col<3>(tid, W, ck, bd, inv); break;
-            case 4: err = inv_col<4>(tid, W, ck, bd, inv); break;
-            case 5: err = inv_col<5>(tid, W, ck, bd, inv); break;
-            default: err = inv_col<6>(tid, W, ck, bd, inv); break;
-            }
-        }
-        if (err) atomicOr(gen(&S.errFlag), (int)err);
-        __syncthreads();
-        if (!S.errFlag) break;
-        fixes++;
-        for (int i = tid; i < n; i += RC_NT) {
-            q[i] = (int16_t)(q[i] / 2);
-            if (q[i]) S.nzFlag = 1;
-        }
-        __syncthreads();
-        if (!S.nzFlag) return fixes;
-    }
-    const int fud = flip_ud(txType), flr = flip_lr(txType), maxv = (1 << bd) - 1;
-    for (int p = tid; p < W * H; p += RC_NT) {
-        const int i = p >> lw, j = p & (W - 1);
-        glb<Px> *d = dst + (size_t)(fud ? H - 1 - i : i) * pitch + (flr ? W - 1 - j : j);
-        *d = (Px)clip3(0, maxv, (int)*d + inv[i * W + j]);
-    }
-    __syncthreads();
-    return fixes;
-}
-
-// write the prediction of candidate c of plane p (edges prepared by group g, or the base edges) into dst (workgroup)
-template <typename Px>
-__device__ void wg_write_pred(const lds<RcShared> &S, const lds<uint16_t> *gea, const lds<uint16_t> *gel, int g, int p, int c, int lw, int lh, glb<Px> *dst,
-                              int pitch, int bd) {
-    const int W = 1 << lw, H = 1 << lh;
-    const int m = c == 255 ? DC_PRED : cand_mode(c), pa = pangle(m, c == 255 ? 0 : cand_delta(c));
-    const bool filt = c != 255 && is_dir(m) && gea != nullptr;
-    const lds<uint16_t> *EA = filt ? gea + EDGE_OFF : S.ea[p] + EDGE_OFF, *EL = filt ? gel + EDGE_OFF : S.el[p] + EDGE_OFF;
-    const int upA = filt ? S.gup[g][0] : 0, upL = filt ? S.gup[g][1] : 0, dcv = S.dcv[p];
-    for (int q = threadIdx.x; q < W * H; q += RC_NT) {
-        const int i = q >> lw, j = q & (W - 1);
-        int pr;
-        if (c == 255) pr = clip3(0, (1 << bd) - 1, dcv + round2signed(S.cflAlpha[p - 1] * (S.cflL[i * W + j] - S.cflAvg), 6));
-        else if (m == DC_PRED) pr = dcv;
-        else pr = pred_px(m, pa, i, j, lw, lh, EA, EL, upA, upL);
-        dst[(size_t)i * pitch + j] = (Px)pr;
-    }
-    __syncthreads();
-}
-
-// record the finished tx block with levels q: coefficients, txb entry, context maps, BlockDecoded (workgroup)
-__device__ int wg_record_txb(lds<RcShared> &S, const Batch &B, uint32_t sb, const lds<Img> &I, int p, int txSz, int txType, int x4, int y4,
-                             const lds<int16_t> *q) {
-    const int tid = threadIdx.x, n = tx_ncoef(txSz);
-    const uint32_t off = (uint32_t)S.nCoef;
-    if (tid < 32) {
-        // eob: 1 + the largest scan index of a nonzero level (inverse default scan; rows for class VERT, columns for
-        // HORIZ); cul: the sum of |level| before the eob, i.e. over every level (later ones are 0), capped at 63
-        const int cls = tx_class(txType), tw = tx_w(txSz) > 32 ? 32 : tx_w(txSz), th = tx_h(txSz) > 32 ? 32 : tx_h(txSz);
-        const int adj = av1t::Adjusted_Tx_Size[txSz];
-        const bool s8 = scan8_has(adj);
-        const glb<uint16_t> *isc = (const glb<uint16_t> *)S.tab.iscan + dscan_off(adj);
-        const lds<uint8_t> *isc8 = S.tab.iscan8 + scan8_off(adj);
-        int last = 0, cul = 0;
-        for (int i = tid; i < n; i += 32) {
-            const int v = q[i];
-            if (v) {
-                const int c = cls == TX_CLASS_2D ? (s8 ? (int)isc8[i] : (int)isc[i]) : cls == TX_CLASS_VERT ? i : (i % tw) * th + i / tw;
-                last = max(last, c + 1);
-                cul += abs(v);
-            }
-        }
-        const int eob = gmaxi(last);
-        cul = gsumi(cul);
-        if (tid == 0) { S.eobOut = eob; S.culOut = min(cul, 63); }
-    }
-    glb<int16_t> *oc = (glb<int16_t> *)B.oCoeffs + (size_t)sb * B.coefCap + off;
-    for (int i = tid; i < n; i += RC_NT) oc[i] = q[i];
-    __syncthreads();
-    const int eob = S.eobOut, cul = S.culOut, dcCat = q[0] < 0 ? 1 : q[0] > 0 ? 2 : 0;
-    const int ss = p ? I.ss : 0, stride = I.MiCols >> ss, rows = I.MiRows >> ss;
-    const int w4 = tx_w(txSz) >> 2, h4 = tx_h(txSz) >> 2, lw4 = av1t::Tx_Width_Log2[txSz] - 2;
-    const int r4 = y4 & ((16 >> ss) - 1), c4 = x4 & ((16 >> ss) - 1);
-    for (int k = tid; k < w4 * h4; k += RC_NT) {
-        const int yy = k >> lw4, xx = k & (w4 - 1);
-        if (y4 + yy < rows && x4 + xx < stride) {
-            map8(I.cLvl[p])[(size_t)(y4 + yy) * stride + x4 + xx] = (uint8_t)(eob ? cul : 0);
-            map8(I.cDc[p])[(size_t)(y4 + yy) * stride + x4 + xx] = (uint8_t)(eob ? dcCat : 0);
-        }
-        S.bdm[p][r4 + yy + 1][c4 + xx + 1] = 1;
-    }
-    if (tid == 0) {
-        RecTxb t;
-        t.coeff_off = off; t.x4 = (uint16_t)x4; t.y4 = (uint16_t)y4; t.plane = (uint8_t)p; t.tx_size = (uint8_t)txSz;
-        t.tx_type = (uint8_t)(p == 0 && eob == 0 ? DCT_DCT : txType); t.flags = 0; t.eob = (uint16_t)eob; t.reserved = 0;
-        B.oTxb[(size_t)sb * B.txbCap + S.nTxb] = t;
-    }
-    __syncthreads();
-    if (tid == 0) { S.nTxb++; S.nCoef += n; }
-    __syncthreads();
-    return eob;
 }
 
 // source of plane p in the staging buffer
@@ -583,41 +448,143 @@ __device__ void wg_luma_residuals(lds<RcShared> &S, const lds<Img> &I) {
     __syncthreads();
 }
 
-// the levels of the winning task t, and (larger blocks) the team holding them with its prepared edges: the team's
-// kept task is t (t < RC_NTEAM), or it evaluates t again
-template <int W, int H>
-__device__ __forceinline__ lds<int16_t> *wg_final_levels(lds<RcShared> &S, const lds<Img> &I, const DevTables &T, const SearchParams &P, int t, int &team) {
-    team = (W > 16 || H > 16) ? t % RC_NTEAM : t % RC_NG;
-    if constexpr (W > 16 || H > 16) {
-        if (t >= RC_NTEAM) {   // overwritten by a task of the same team that ran after it
-            const int p = S.taskP[t];
-            if ((int)(threadIdx.x >> 6) == team) wave_task<W, H>(S, S.u.b.t[team], team, I, T, p, S.taskC[t], stage_src(S, p), W, P);
+// The end of a tx block (luma: NP 1, plane p0 = 0; chroma: NP 2, U and V side by side in the halves of the workgroup, V's
+// task t0 + 1 behind U's t0): the winner's levels and prepared edges (a larger block evaluates the task again if its team
+// ran another after it), exact dequantization and inverse transform with the conformance repair (spec 7.13.3, 7.12.3
+// step 3: halve the levels until no range is violated), prediction + residual written once, then the record: levels, txb
+// entry (index txb, + txbStep for V), context maps, BlockDecoded.  One wave of each half keeps the record, so the only
+// barriers are those of the inverse and one at the end.  (px, py): the tx block's first sample in its planes.
+template <int W, int H, int NP, typename Px>
+__device__ __forceinline__ void wg_finish(lds<RcShared> &S, const Batch &B, const SearchParams &P, const DevTables &T, uint32_t sb, const lds<Img> &I,
+                                          int t0, int slot0, int txType, int px, int py, uint32_t txb, uint32_t txbStep, uint32_t coef) {
+    constexpr bool big = W > 16 || H > 16;
+    constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 4 ? 2 : H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
+    constexpr int TW = W > 32 ? 32 : W, TH = H > 32 ? 32 : H, N = TW * TH, txSz = tx_of(W, H), NT = RC_NT / NP;
+    static_assert(NP == 1 || (H <= NT && W <= NT && W * H <= 32 * 32), "U and V share the workgroup and the inverse's scratch");
+    const int half = NP == 2 ? (int)(threadIdx.x >> 7) : 0, tl = (int)threadIdx.x & (NT - 1);
+    const int p = NP == 2 ? 1 + half : 0, t = t0 + half, slot = slot0 + half, bd = I.bd;
+    const int team = t % (big ? RC_NTEAM : RC_NG);
+    if constexpr (big) {
+        if (t0 >= RC_NTEAM) {
+            const int wv = (int)(threadIdx.x >> 6);
+            const int tw = wv == t0 % RC_NTEAM ? t0 : NP == 2 && wv == (t0 + 1) % RC_NTEAM ? t0 + 1 : -1;
+            if (tw >= 0) {
+                const int tp = __builtin_amdgcn_readfirstlane(S.taskP[tw]), tc = __builtin_amdgcn_readfirstlane(S.taskC[tw]);
+                wave_task<W, H>(S, S.u.b.t[wv], wv, I, T, tp, tc, stage_src(S, tp), W, P);
+            }
             __syncthreads();
         }
-        return team_lev(S.u.b.t[team]);
-    } else {
-        return S.u.s.lev + t * (W * H);
     }
-}
-
-// write the prediction of task t of plane p (into dst): larger blocks predict again from team g's prepared edges;
-// blocks up to 16x16 take source minus the kept residual (slot k)
-template <int W, int H, typename Px>
-__device__ void wg_final_pred(const lds<RcShared> &S, const lds<Img> &I, int p, int t, int k, int team, glb<Px> *dst, int pitch) {
-    constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 4 ? 2 : H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
-    if constexpr (W > 16 || H > 16) {
-        wg_write_pred<Px>(S, I.edgeFilter ? S.u.b.t[team].ea : nullptr, S.u.b.t[team].el, team, p, S.taskC[t], LW, LH, dst, pitch, I.bd);
-    } else {
-        const lds<uint16_t> *src = stage_src(S, p);
-        const lds<int16_t> *res = S.u.s.res[k];
-        for (int q = threadIdx.x; q < W * H; q += RC_NT) dst[(size_t)(q >> LW) * pitch + (q & (W - 1))] = (Px)((int)src[q] - res[q]);
-        __syncthreads();
+    lds<int16_t> *q = big ? team_lev(S.u.b.t[team]) : S.u.s.lev + t * (W * H);
+    static_assert(sizeof(RcGroup::tmp) >= 16 * 16 * 2, "the inverse's scratch of a small block: a group's");
+    lds<int16_t> *inv = big ? S.u.b.inv + half * (32 * 32) : (lds<int16_t> *)(lds<char> *)S.u.s.g[half].tmp;
+    int eob = S.taskE[t], fixes = 0;
+    bool add = eob > 0;
+    if (NP == 2 ? (S.taskE[t0] > 0 || S.taskE[t0 + 1] > 0) : add) {
+        constexpr int den = (W == 64 && H >= 32) || (H == 64 && W >= 32) ? 4 : W * H > 256 ? 2 : 1;
+        const int dsh = den == 4 ? 2 : den == 2 ? 1 : 0, rk = row_kind(txType), ck = col_kind(txType);
+        constexpr bool rect = W == 2 * H || H == 2 * W;
+        for (;;) {
+            uint32_t err = 0;
+            if (add && tl < H) err = inv_row<LW>(tl, W, TH, TW, q, S.dcQ, S.acQ, dsh, bd, rect, rk, av1t::Transform_Row_Shift[txSz], inv);
+            if (err) atomicOr(gen(&S.errFlag[half]), (int)err);
+            __syncthreads();
+            err = 0;
+            if (add && tl < W) err = inv_col<LH>(tl, W, ck, bd, inv);
+            if (err) atomicOr(gen(&S.errFlag[half]), (int)err);
+            __syncthreads();
+            const int bad = S.errFlag[half];
+            if (!(S.errFlag[0] | S.errFlag[1])) break;
+            __syncthreads();
+            if (tl == 0) { S.errFlag[half] = 0; S.nzFlag[half] = 0; }
+            __syncthreads();
+            if (bad) {
+                fixes++;
+                for (int i = tl; i < N; i += NT) {
+                    q[i] = (int16_t)(q[i] / 2);
+                    if (q[i]) S.nzFlag[half] = 1;
+                }
+            }
+            __syncthreads();
+            if (bad && !S.nzFlag[half]) add = false;
+        }
+        if (fixes && tl == 0) atomicAdd(&B.stats[3], 1u);
     }
+    // prediction + residual
+    {
+        const int maxv = (1 << bd) - 1, fud = flip_ud(txType), flr = flip_lr(txType), pitch = I.pitch[p];
+        glb<Px> *dst = rec_plane<Px>(I, p) + (size_t)py * pitch + px;
+        if constexpr (big) {
+            const int c = S.taskC[t], m = c == 255 ? DC_PRED : cand_mode(c), pa = pangle(m, c == 255 ? 0 : cand_delta(c));
+            const bool filt = c != 255 && is_dir(m) && I.edgeFilter;
+            const lds<uint16_t> *EA = (filt ? S.u.b.t[team].ea : S.ea[p]) + EDGE_OFF, *EL = (filt ? S.u.b.t[team].el : S.el[p]) + EDGE_OFF;
+            const int upA = filt ? S.gup[team][0] : 0, upL = filt ? S.gup[team][1] : 0, dcv = S.dcv[p];
+            for (int k = tl; k < W * H; k += NT) {
+                const int i = k >> LW, j = k & (W - 1);
+                int v;
+                if (c == 255) v = clip3(0, maxv, dcv + round2signed(S.cflAlpha[p == 2] * (S.cflL[k] - S.cflAvg), 6));
+                else if (m == DC_PRED) v = dcv;
+                else v = pred_px(m, pa, i, j, LW, LH, EA, EL, upA, upL);
+                if (add) v = clip3(0, maxv, v + inv[k]);   // DCT_DCT: no flips
+                dst[(size_t)i * pitch + j] = (Px)v;
+            }
+        } else {
+            const lds<uint16_t> *src = stage_src(S, p);
+            const lds<int16_t> *res = S.u.s.res[slot];
+            for (int k = tl; k < W * H; k += NT) {
+                const int i = k >> LW, j = k & (W - 1);
+                int v = (int)src[k] - res[k];
+                if (add) v = clip3(0, maxv, v + inv[((fud ? H - 1 - i : i) << LW) + (flr ? W - 1 - j : j)]);
+                dst[(size_t)i * pitch + j] = (Px)v;
+            }
+        }
+    }
+    // record
+    coef += half * (txbStep * N);
+    {
+        glb<uint32_t> *oc = (glb<uint32_t> *)((glb<int16_t> *)B.oCoeffs + (size_t)sb * B.coefCap + coef);   // coef: a multiple of 16
+        const lds<uint32_t> *qw = (const lds<uint32_t> *)(const lds<char> *)q;
+        for (int i = tl; i < N / 2; i += NT) oc[i] = qw[i];
+    }
+    if (tl < 64) {   // a wave
+        int cul = 0, last = 0;   // the sum of |level| (before the eob, i.e. over every level: later ones are 0)
+        for (int i = tl; i < N; i += 64) { const int v = q[i]; cul += max(v, -v); }
+        cul = gsumi(cul);
+        cul = min(cul + other_half(cul), 63);
+        if (fixes) {   // the eob of the halved levels: 1 + the largest scan index of a nonzero one
+            const auto isc = iscan_ptr<txSz>(S.tab);
+            const int cls = tx_class(txType);
+            for (int i = tl; i < N; i += 64)
+                if (q[i]) last = max(last, 1 + (cls == TX_CLASS_2D ? (int)isc[i] : cls == TX_CLASS_VERT ? i : (i % TW) * TH + i / TW));
+            last = gmaxi(last);
+            eob = max(last, other_half(last));
+        }
+        const int dcCat = q[0] < 0 ? 1 : q[0] > 0 ? 2 : 0;
+        const int ss = p ? I.ss : 0, stride = I.MiCols >> ss, rows = I.MiRows >> ss, x4 = px >> 2, y4 = py >> 2;
+        const int r4 = y4 & ((16 >> ss) - 1), c4 = x4 & ((16 >> ss) - 1);
+        constexpr int W4 = W / 4, H4 = H / 4, LW4 = LW - 2;
+        for (int k = tl; k < W4 * H4; k += 64) {
+            const int yy = k >> LW4, xx = k & (W4 - 1);
+            if (y4 + yy < rows && x4 + xx < stride) {
+                map8(I.cLvl[p])[(size_t)(y4 + yy) * stride + x4 + xx] = (uint8_t)(eob ? cul : 0);
+                map8(I.cDc[p])[(size_t)(y4 + yy) * stride + x4 + xx] = (uint8_t)(eob ? dcCat : 0);
+            }
+            S.bdm[p][r4 + yy + 1][c4 + xx + 1] = 1;
+        }
+        if (tl == 0) {
+            RecTxb r;
+            r.coeff_off = coef; r.x4 = (uint16_t)x4; r.y4 = (uint16_t)y4; r.plane = (uint8_t)p; r.tx_size = (uint8_t)txSz;
+            r.tx_type = (uint8_t)(p == 0 && eob == 0 ? DCT_DCT : txType); r.flags = 0; r.eob = (uint16_t)eob; r.reserved = 0;
+            B.oTxb[(size_t)sb * B.txbCap + txb + half * txbStep] = r;
+            S.winEob[p] = eob;
+        }
+    }
+    __syncthreads();
 }
 
 template <int W, int H, typename Px>
 __device__ __noinline__ void rc_luma(lds<RcShared> &S, const Batch &B, const SearchParams &P, uint32_t sb, const lds<Img> &I, int bsize, int x, int y, int availU,
-                        int availL, int tx0, int ty0, float lambda) {
+                        int availL, int tx0, int ty0, float lambda, uint32_t txb, uint32_t coef) {
     constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 4 ? 2 : H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
     const DevTables &T = *B.T;
     const int tid = threadIdx.x, txSz = tx_of(W, H);
@@ -681,22 +648,13 @@ __device__ __noinline__ void rc_luma(lds<RcShared> &S, const Batch &B, const Sea
         wg_run_tasks<W, H>(S, I, T, P, lambda, true, true);
     }
     const int win = S.win;
-    int team;
-    lds<int16_t> *q = wg_final_levels<W, H>(S, I, T, P, win, team);
-    glb<Px> *dst = rec_plane<Px>(I, 0) + (size_t)y * I.pitch[0] + x;
-    wg_final_pred<W, H, Px>(S, I, 0, win, S.taskK[win], team, dst, I.pitch[0]);
-    if (S.taskE[win] > 0) {
-        const int fixes = wg_inverse_add<Px>(S, q, inv_scr(S, txSz), txSz, S.taskT[win], I.bd, dst, I.pitch[0]);
-        if (fixes && tid == 0) atomicAdd(&B.stats[3], 1u);
-    }
-    const int eob = wg_record_txb(S, B, sb, I, 0, txSz, S.taskT[win], x >> 2, y >> 2, q);
-    if (tid == 0) { S.mode = cand_mode(S.taskC[win]); S.delta = cand_delta(S.taskC[win]); S.winEob[0] = eob; }
-    __syncthreads();
+    if (tid == 0) { S.mode = cand_mode(S.taskC[win]); S.delta = cand_delta(S.taskC[win]); }
+    wg_finish<W, H, 1, Px>(S, B, P, T, sb, I, win, S.taskK[win], S.taskT[win], x, y, txb, 0, coef);
 }
 
 template <int W, int H, typename Px>
 __device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const SearchParams &P, uint32_t sb, const lds<Img> &I, int bsize, int mi_row, int mi_col,
-                          int availUC, int availLC, int tx0, int ty0, float lambda) {
+                          int availUC, int availLC, int tx0, int ty0, float lambda, uint32_t txb, uint32_t coef, int nTxb) {
     constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 4 ? 2 : H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
     const DevTables &T = *B.T;
     const lds<CostTab> &C = S.tab.cost;
@@ -995,7 +953,8 @@ __device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const S
         S.uvJ[l] = js;
         gsync();
         int rank = 0, fin = 0;
-        for (int j = 0; j < nuv; j++) {
+#pragma unroll
+        for (int j = 0; j < 19; j++) {   // candidates past nuv are INF
             const float o = S.uvJ[j];
             rank += (o < js || (o == js && j < l)) ? 1 : 0;
             fin += o < INF ? 1 : 0;
@@ -1040,55 +999,45 @@ __device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const S
         }
     }
     __syncthreads();
-    const int win = S.win, uvTxType = S.taskT[win], winC = S.taskC[win], nTask0 = S.nTask;
-    // 4:4:4 blocks with a 64-sample side hold several chroma tx blocks (nTx > 1): the decision above is the first
-    // one's; each further one (raster order, U's then V's) gets its edges from the reconstruction, its own contexts
-    // and a closed-loop final quantization with the chosen mode (a one-task run in slot 0 / team 0: the winning pair is
-    // (even, odd), so V's kept task survives U's further blocks), and is not coded outside the coded area
-    const int nTxX = ss ? 1 : (4 * bw4(bsize)) / W, nTxY = ss ? 1 : (4 * bh4(bsize)) / H;
-    for (int p = 1; p <= 2; p++) {
-        const int t = win + p - 1;
-        int team;
-        lds<int16_t> *q = wg_final_levels<W, H>(S, I, T, P, t, team);
-        glb<Px> *dst = rec_plane<Px>(I, p) + (size_t)cy * I.pitch[p] + cx;
-        wg_final_pred<W, H, Px>(S, I, p, t, t, team, dst, I.pitch[p]);
-        if (S.taskE[t] > 0) {
-            const int fixes = wg_inverse_add<Px>(S, q, inv_scr(S, txSz), txSz, uvTxType, bd, dst, I.pitch[p]);
-            if (fixes && tid == 0) atomicAdd(&B.stats[3], 1u);
-        }
-        int eob = wg_record_txb(S, B, sb, I, p, txSz, uvTxType, x4, y4, q);
-        // only a chroma tx block with a 32-sample side belongs to a 64-sided 4:4:4 block
-        if constexpr (W == 32 || H == 32) for (int k = 1; k < nTxX * nTxY; k++) {
+    // 4:4:4 blocks with a 64-sample side hold several chroma tx blocks per plane (raster order, U's then V's in the record):
+    // the decision above is the first one's; each further one gets its edges from the reconstruction, its own contexts and
+    // a closed-loop final quantization with the chosen mode, and is not coded outside the coded area
+    const int win = S.win, uvTxType = S.taskT[win], winC = S.taskC[win];
+    const uint32_t perPlane = (uint32_t)nTxb / 2;
+    wg_finish<W, H, 2, Px>(S, B, P, T, sb, I, win, win, uvTxType, cx, cy, txb, perPlane, coef);
+    // only a chroma tx block with a 32-sample side belongs to a 64-sided 4:4:4 block
+    if constexpr (W == 32 || H == 32) if (perPlane > 1) {
+        const int nTxX = (4 * bw4(bsize)) / W, nTxY = (4 * bh4(bsize)) / H;
+        int eobU = S.winEob[1], eobV = S.winEob[2];
+        uint32_t n = 0;
+        for (int k = 1; k < nTxX * nTxY; k++) {
             const int ox = (k % nTxX) * W, oy = (k / nTxX) * H;
             if (x4 + (ox >> 2) >= I.MiCols || y4 + (oy >> 2) >= I.MiRows) continue;
+            n++;
             const int r4 = sbr4 + (oy >> 2), c4 = sbc4 + (ox >> 2);
-            if (gid() == 0)
+            if (gid() < 2) {
+                const int p = 1 + gid();
                 rc_edges<Px>(S, I, p, cx + ox, cy + oy, LW, LH, availLC || ox > 0, availUC || oy > 0, S.bdm[p][r4][c4 + (W >> 2) + 1],
                              S.bdm[p][r4 + (H >> 2) + 1][c4], mi_row, mi_col, availUC, availLC);
-            if (gid() == 1) grp_txb_ctx(I, p, txSz, x4 + (ox >> 2), y4 + (oy >> 2), bsize, tx0, ty0, &S.skipCtx[p], &S.dcCtx[p]);
-            {
+            }
+            if (gid() == 2 || gid() == 3) {
+                const int p = gid() - 1;
+                grp_txb_ctx(I, p, txSz, x4 + (ox >> 2), y4 + (oy >> 2), bsize, tx0, ty0, &S.skipCtx[p], &S.dcCtx[p]);
+            }
+            for (int p = 1; p <= 2; p++) {
                 lds<uint16_t> *sd = S.srcb + (p == 2 ? 2048 : 0);
                 const glb<Px> *g = src_plane<Px>(I, p) + (size_t)(cy + oy) * I.spitch[p] + cx + ox;
                 for (int i = tid; i < W * H; i += RC_NT) sd[i] = g[(size_t)(i >> LW) * I.spitch[p] + (i & (W - 1))];
             }
-            if (tid == 0) { S.taskC[0] = winC; S.taskT[0] = uvTxType; S.taskP[0] = p; S.nTask = 1; }
+            if (tid < 2) { S.taskC[tid] = winC; S.taskT[tid] = uvTxType; S.taskP[tid] = 1 + tid; }
+            if (tid == 0) S.nTask = 2;
             __syncthreads();
             wg_run_tasks<W, H>(S, I, T, P, lambda, false, false);
-            int tm;
-            lds<int16_t> *qk = wg_final_levels<W, H>(S, I, T, P, 0, tm);
-            glb<Px> *dk = rec_plane<Px>(I, p) + (size_t)(cy + oy) * I.pitch[p] + cx + ox;
-            wg_final_pred<W, H, Px>(S, I, p, 0, 0, tm, dk, I.pitch[p]);
-            if (S.taskE[0] > 0) {
-                const int fixes = wg_inverse_add<Px>(S, qk, inv_scr(S, txSz), txSz, uvTxType, bd, dk, I.pitch[p]);
-                if (fixes && tid == 0) atomicAdd(&B.stats[3], 1u);
-            }
-            eob |= wg_record_txb(S, B, sb, I, p, txSz, uvTxType, x4 + (ox >> 2), y4 + (oy >> 2), qk);
+            wg_finish<W, H, 2, Px>(S, B, P, T, sb, I, 0, 0, uvTxType, cx + ox, cy + oy, txb + n, perPlane, coef + n * tx_ncoef(txSz));
+            eobU |= S.winEob[1]; eobV |= S.winEob[2];
         }
-        if (nTxX * nTxY > 1) {   // V's first tx block reads the decision's tasks again
-            if (tid == 0) S.nTask = nTask0;
-            __syncthreads();
-        }
-        if (tid == 0) S.winEob[p] = eob;
+        __syncthreads();
+        if (tid == 0) { S.winEob[1] = eobU; S.winEob[2] = eobV; }
         __syncthreads();
     }
 }
@@ -1192,6 +1141,7 @@ __device__ bool recon_part(lds<RcShared> &S, const Batch &B, const SearchParams 
         S.flopsOn = B.flops != nullptr; S.flops = 0; S.dcQ = dc_q(I.qindex, I.bd); S.acQ = ac_q(I.qindex, I.bd);
         S.dcRcp = 1.f / (float)S.dcQ; S.acRcp = 1.f / (float)S.acQ;
         for (int k = 0; k < 4; k++) S.known[k] = 0;
+        S.errFlag[0] = S.errFlag[1] = 0;
     }
     __syncthreads();
     const float lambda = T.lambda[I.bd == 10][I.qindex] * P.lambdaMul;
@@ -1206,7 +1156,7 @@ __device__ bool recon_part(lds<RcShared> &S, const Batch &B, const SearchParams 
     for (int li = 0; li < nLeaves; li++) {
         const int lf = __builtin_amdgcn_readfirstlane((int)S.leaf[li]);
         const int bsize = lf & 31, lx4 = (lf >> 5) & 15, ly4 = lf >> 9, x = sbx + lx4 * 4, y = sby + ly4 * 4, mi_row = y >> 2, mi_col = x >> 2;
-        const int bw = bw4(bsize), bh = bh4(bsize);
+        const int bw = bw4(bsize), bh = bh4(bsize), lbw = 31 - __clz(bw);
         auto inside = [&](int r, int c) { return c >= (tx0 >> 2) && c < miColEnd && r >= (ty0 >> 2) && r < miRowEnd; };
         const int hasC = has_chroma(bsize, mi_row, mi_col, I.mono, I.ss);
         const int txSz = av1t::Max_Tx_Size_Rect[bsize];
@@ -1239,19 +1189,18 @@ __device__ bool recon_part(lds<RcShared> &S, const Batch &B, const SearchParams 
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             }
         }
-        if (tid == 0) { S.nTxb = firstTxb + PL; S.nCoef = firstCoef + (PL ? tx_ncoef(txSz) : 0); }
         RecBlock *const rb = B.oBlocks + (size_t)sb * MAX_LEAVES + li;
         int skip = 0;
         if constexpr (PL == 0) {
             const int availU = inside(mi_row - 1, mi_col), availL = inside(mi_row, mi_col - 1);
-#define RC_LUMA(w, h) rc_luma<w, h, Px>(S, B, P, sb, I, bsize, x, y, availU, availL, tx0, ty0, lambda)
+#define RC_LUMA(w, h) rc_luma<w, h, Px>(S, B, P, sb, I, bsize, x, y, availU, availL, tx0, ty0, lambda, firstTxb, firstCoef)
             AV1M_TX_SWITCH(txSz, RC_LUMA)
 #undef RC_LUMA
             __syncthreads();
             skip = S.winEob[0] == 0;   // of the luma; the chroma item completes the record of a block that carries chroma
             const int yMode = S.mode;
             for (int k = tid; k < bw * bh; k += RC_NT) {
-                const int r = mi_row + k / bw, c = mi_col + k % bw;
+                const int r = mi_row + (k >> lbw), c = mi_col + (k & (bw - 1));
                 if (r < I.MiRows && c < I.MiCols) {
                     const size_t o = (size_t)r * I.MiCols + c;
                     map8(I.mY)[o] = (uint8_t)yMode;
@@ -1278,7 +1227,8 @@ __device__ bool recon_part(lds<RcShared> &S, const Batch &B, const SearchParams 
             if (tid == 0) { S.mode = rb->y_mode; S.winEob[0] = !rb->skip; }
             __syncthreads();
             const int uvTx = uv_tx_size(bsize, I.ss);
-#define RC_CHROMA(w, h) rc_chroma<w, h, Px>(S, B, P, sb, I, bsize, mi_row, mi_col, availUC, availLC, tx0, ty0, lambda * P.lambdaCMul)
+#define RC_CHROMA(w, h) rc_chroma<w, h, Px>(S, B, P, sb, I, bsize, mi_row, mi_col, availUC, availLC, tx0, ty0, lambda * P.lambdaCMul, \
+                                                   firstTxb + 1, firstCoef + tx_ncoef(txSz), cTxb)
             switch (uvTx) {
             case TX_4X4: RC_CHROMA(4, 4); break; case TX_8X8: RC_CHROMA(8, 8); break; case TX_16X16: RC_CHROMA(16, 16); break;
             case TX_32X32: RC_CHROMA(32, 32); break; case TX_4X8: RC_CHROMA(4, 8); break; case TX_8X4: RC_CHROMA(8, 4); break;
@@ -1291,7 +1241,7 @@ __device__ bool recon_part(lds<RcShared> &S, const Batch &B, const SearchParams 
             skip = S.winEob[0] == 0 && S.winEob[1] == 0 && S.winEob[2] == 0;
             const int uv = S.uvMode;
             for (int k = tid; k < bw * bh; k += RC_NT) {
-                const int r = mi_row + k / bw, c = mi_col + k % bw;
+                const int r = mi_row + (k >> lbw), c = mi_col + (k & (bw - 1));
                 if (r < I.MiRows && c < I.MiCols) {
                     const size_t o = (size_t)r * I.MiCols + c;
                     map8(I.mUV)[o] = (uint8_t)uv;
