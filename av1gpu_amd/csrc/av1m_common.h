@@ -513,45 +513,51 @@ AV1M_HD const uint8_t *sm_weights(int l) {
     return l == 2 ? av1t::Sm_Weights_Tx_4x4 : l == 3 ? av1t::Sm_Weights_Tx_8x8 : l == 4 ? av1t::Sm_Weights_Tx_16x16
          : l == 5 ? av1t::Sm_Weights_Tx_32x32 : av1t::Sm_Weights_Tx_64x64;
 }
+// Where the predictors read the spec's direction steps and smooth weights: the constant tables, or a copy (the closed loop
+// keeps one in LDS)
+struct PredTables {
+    AV1M_HD int step(int pa) const { return av1t::Dr_Intra_Derivative[pa]; }
+    AV1M_HD const uint8_t *weights(int l) const { return sm_weights(l); }
+};
 // one predicted sample (row i, column j) of a non-DC mode from AboveRow / LeftCol (index 0 = first sample, -1 the
 // corner; after upsampling index -2 exists)
-template <typename P>
-AV1M_HD int pred_px(int mode, int pa, int i, int j, int lw, int lh, const P *A, const P *L, int upA, int upL) {
+template <typename P, typename TB = PredTables>
+AV1M_HD int pred_px(int mode, int pa, int i, int j, int lw, int lh, const P *A, const P *L, int upA, int upL, const TB &tb = TB()) {
     const int w = 1 << lw, h = 1 << lh;
     if (is_dir(mode)) {
         if (pa == 90) return A[j];
         if (pa == 180) return L[i];
         if (pa < 90) {
-            const int dx = av1t::Dr_Intra_Derivative[pa], idx = (i + 1) * dx;
+            const int dx = tb.step(pa), idx = (i + 1) * dx;
             const int base = (idx >> (6 - upA)) + (j << upA), sh = ((idx << upA) >> 1) & 0x1F, mb = (w + h - 1) << upA;
             return base < mb ? (A[base] * (32 - sh) + A[base + 1] * sh + 16) >> 5 : A[mb];
         }
         if (pa < 180) {
-            const int dx = av1t::Dr_Intra_Derivative[180 - pa];
+            const int dx = tb.step(180 - pa);
             int idx = (j << 6) - (i + 1) * dx;
             if ((idx >> (6 - upA)) >= -(1 << upA)) {
                 const int base = idx >> (6 - upA), sh = ((idx * (1 << upA)) >> 1) & 0x1F;
                 return (A[base] * (32 - sh) + A[base + 1] * sh + 16) >> 5;
             }
-            const int dy = av1t::Dr_Intra_Derivative[pa - 90];
+            const int dy = tb.step(pa - 90);
             idx = (i << 6) - (j + 1) * dy;
             const int base = idx >> (6 - upL), sh = ((idx * (1 << upL)) >> 1) & 0x1F;
             return (L[base] * (32 - sh) + L[base + 1] * sh + 16) >> 5;
         }
-        const int dy = av1t::Dr_Intra_Derivative[270 - pa], idx = (j + 1) * dy;
+        const int dy = tb.step(270 - pa), idx = (j + 1) * dy;
         const int base = (idx >> (6 - upL)) + (i << upL), sh = ((idx << upL) >> 1) & 0x1F;
         return (L[base] * (32 - sh) + L[base + 1] * sh + 16) >> 5;
     }
     if (mode == SMOOTH_PRED) {
-        const uint8_t *wx = sm_weights(lw), *wy = sm_weights(lh);
+        const auto wx = tb.weights(lw), wy = tb.weights(lh);
         return (wy[i] * A[j] + (256 - wy[i]) * L[h - 1] + wx[j] * L[i] + (256 - wx[j]) * A[w - 1] + 256) >> 9;
     }
     if (mode == SMOOTH_V_PRED) {
-        const uint8_t *wy = sm_weights(lh);
+        const auto wy = tb.weights(lh);
         return (wy[i] * A[j] + (256 - wy[i]) * L[h - 1] + 128) >> 8;
     }
     if (mode == SMOOTH_H_PRED) {
-        const uint8_t *wx = sm_weights(lw);
+        const auto wx = tb.weights(lw);
         return (wx[j] * L[i] + (256 - wx[j]) * A[w - 1] + 128) >> 8;
     }
     const int a = A[j], l = L[i], tl = A[-1], base = a + l - tl;   // PAETH
@@ -561,9 +567,9 @@ AV1M_HD int pred_px(int mode, int pa, int i, int j, int lw, int lh, const P *A, 
 // CH predicted samples of column j, rows i0, i0 + di, ..., i0 + (CH - 1) di, of any mode (DC_PRED: dcv): pred_px's
 // cases with the mode and zone tests made once for the CH samples, so a group whose lanes share the mode branches once
 // per run of samples instead of once per sample
-template <int CH, typename P>
+template <int CH, typename P, typename TB = PredTables>
 AV1M_HD void pred_col(int mode, int pa, int dcv, int i0, int di, int j, int lw, int lh, const P *A, const P *L, int upA, int upL,
-                      int (&o)[CH]) {
+                      int (&o)[CH], const TB &tb = TB()) {
     const int w = 1 << lw, h = 1 << lh;
     if (mode == DC_PRED) {
         for (int c = 0; c < CH; c++) o[c] = dcv;
@@ -574,14 +580,14 @@ AV1M_HD void pred_col(int mode, int pa, int dcv, int i0, int di, int j, int lw, 
         } else if (pa == 180) {
             for (int c = 0; c < CH; c++) o[c] = L[i0 + c * di];
         } else if (pa < 90) {
-            const int dx = av1t::Dr_Intra_Derivative[pa], mb = (w + h - 1) << upA, am = A[mb];
+            const int dx = tb.step(pa), mb = (w + h - 1) << upA, am = A[mb];
             for (int c = 0; c < CH; c++) {
                 const int idx = (i0 + c * di + 1) * dx;
                 const int base = (idx >> (6 - upA)) + (j << upA), sh = ((idx << upA) >> 1) & 0x1F;
                 o[c] = base < mb ? (A[base] * (32 - sh) + A[base + 1] * sh + 16) >> 5 : am;
             }
         } else if (pa < 180) {
-            const int dx = av1t::Dr_Intra_Derivative[180 - pa], dy = av1t::Dr_Intra_Derivative[pa - 90];
+            const int dx = tb.step(180 - pa), dy = tb.step(pa - 90);
             for (int c = 0; c < CH; c++) {
                 const int i = i0 + c * di;
                 const int ia = (j << 6) - (i + 1) * dx;
@@ -595,7 +601,7 @@ AV1M_HD void pred_col(int mode, int pa, int dcv, int i0, int di, int j, int lw, 
                 }
             }
         } else {
-            const int dy = av1t::Dr_Intra_Derivative[270 - pa], idx = (j + 1) * dy, sh = ((idx << upL) >> 1) & 0x1F;
+            const int dy = tb.step(270 - pa), idx = (j + 1) * dy, sh = ((idx << upL) >> 1) & 0x1F;
             for (int c = 0; c < CH; c++) {
                 const int base = (idx >> (6 - upL)) + ((i0 + c * di) << upL);
                 o[c] = (L[base] * (32 - sh) + L[base + 1] * sh + 16) >> 5;
@@ -611,7 +617,7 @@ AV1M_HD void pred_col(int mode, int pa, int dcv, int i0, int di, int j, int lw, 
     } else {
         // the SMOOTH modes: (x + 128) >> 8 = (2x + 256) >> 9, so SMOOTH_V / SMOOTH_H are SMOOTH with the other
         // direction's pair replaced by a second copy of their own
-        const uint8_t *wx = sm_weights(lw), *wy = sm_weights(lh);
+        const auto wx = tb.weights(lw), wy = tb.weights(lh);
         const int a = A[j], lb = L[h - 1], ar = A[w - 1], wj = wx[j];
         for (int c = 0; c < CH; c++) {
             const int i = i0 + c * di, wi = wy[i], l = L[i];
@@ -624,14 +630,14 @@ AV1M_HD void pred_col(int mode, int pa, int dcv, int i0, int di, int j, int lw, 
 // and the direction's steps are settled once for the sixteen.  Along a row of zones 1 and 2 the position in AboveRow moves
 // by one sample and its fraction stays, so a row takes five samples for its four; along a column the same holds for
 // LeftCol.  Equal to pred_px at every sample.
-template <typename P>
-AV1M_HD void pred_4x4(int mode, int pa, int dcv, int i0, int j0, int lw, int lh, const P *A, const P *L, int (&o)[16]) {
+template <typename P, typename TB = PredTables>
+AV1M_HD void pred_4x4(int mode, int pa, int dcv, int i0, int j0, int lw, int lh, const P *A, const P *L, int (&o)[16], const TB &tb = TB()) {
     const int w = 1 << lw, h = 1 << lh;
     if (mode == DC_PRED) {
         for (int k = 0; k < 16; k++) o[k] = dcv;
     } else if (is_dir(mode)) {
         if (pa <= 90) {   // 90: the sample above
-            const int dx = pa == 90 ? 0 : av1t::Dr_Intra_Derivative[pa], mb = w + h - 1;
+            const int dx = pa == 90 ? 0 : tb.step(pa), mb = w + h - 1;
             for (int i = 0; i < 4; i++) {
                 const int idx = (i0 + i + 1) * dx, base = (idx >> 6) + j0, sh = (idx >> 1) & 0x1F;
                 int a[5];
@@ -639,7 +645,7 @@ AV1M_HD void pred_4x4(int mode, int pa, int dcv, int i0, int j0, int lw, int lh,
                 for (int j = 0; j < 4; j++) o[4 * i + j] = (a[j] * (32 - sh) + a[j + 1] * sh + 16) >> 5;
             }
         } else if (pa < 180) {
-            const int dx = av1t::Dr_Intra_Derivative[180 - pa], dy = av1t::Dr_Intra_Derivative[pa - 90];
+            const int dx = tb.step(180 - pa), dy = tb.step(pa - 90);
             for (int i = 0; i < 4; i++) {
                 const int ia = -(i0 + i + 1) * dx, ba = (ia >> 6) + j0, sa = (ia >> 1) & 0x1F;
                 for (int j = 0; j < 4; j++) {
@@ -651,7 +657,7 @@ AV1M_HD void pred_4x4(int mode, int pa, int dcv, int i0, int j0, int lw, int lh,
                 }
             }
         } else {   // 180: the sample to the left
-            const int dy = pa == 180 ? 0 : av1t::Dr_Intra_Derivative[270 - pa];
+            const int dy = pa == 180 ? 0 : tb.step(270 - pa);
             for (int j = 0; j < 4; j++) {
                 const int idx = (j0 + j + 1) * dy, base = (idx >> 6) + i0, sh = (idx >> 1) & 0x1F;
                 int a[5];
@@ -672,7 +678,7 @@ AV1M_HD void pred_4x4(int mode, int pa, int dcv, int i0, int j0, int lw, int lh,
                 }
         } else {
             // the SMOOTH modes as in pred_col: SMOOTH_V / SMOOTH_H take a second copy of their own direction's pair
-            const uint8_t *wx = sm_weights(lw), *wy = sm_weights(lh);
+            const auto wx = tb.weights(lw), wy = tb.weights(lh);
             const int lb = L[h - 1], ar = A[w - 1];
             for (int i = 0; i < 4; i++) {
                 const int wi = wy[i0 + i];

@@ -26,7 +26,7 @@ constexpr int RC_NT = 256, RC_NG = 8;
 // transform teams for tx blocks with a side of 32 or 64: the waves
 constexpr int RC_NTEAM = RC_NT / 64;
 
-constexpr int RC_SMALL_RES = 16;
+constexpr int RC_SMALL_RES = 14;   // 6 luma candidates, or 2 planes x 7 chroma candidates
 // levels of every task of a tx block up to 16x16, packed by the block's size (task t at t * W * H): at most 6 candidates
 // x 7 tx types of 128 coefficients, 6 x 5 of 256 (16x16: intra set 2), or 2 planes x 7 chroma candidates of 256
 constexpr int RC_LEV_TOTAL = 7680;
@@ -61,8 +61,15 @@ struct RcTabs {
     float txg[19][16];
     uint8_t cbOff[19][25];         // Coeff_Base_Ctx_Offset
     uint8_t scan8[SCAN8_TOTAL], iscan8[SCAN8_TOTAL];   // default scans of up to 256 coefficients and their inverses
+    uint16_t step[90];             // Dr_Intra_Derivative
+    uint8_t smooth[124];           // the smooth weights, n = 4, 8, .. 64 at n - 4
     const uint16_t *iscan;         // the larger ones' inverses (device tables; read through the caches)
     CostTab cost;                  // of the image's quantizer context
+};
+struct RcPredTables {
+    const lds<RcTabs> &T;
+    __device__ __forceinline__ int step(int pa) const { return T.step[pa]; }
+    __device__ __forceinline__ const lds<uint8_t> *weights(int l) const { return T.smooth + (1 << l) - 4; }
 };
 using RcEvalIn = EvalInT<const lds<CostTab> *>;
 template <int TSZ>
@@ -89,11 +96,15 @@ union RcScr {
     RcSmall s;
     RcBig b;
 };
+struct BlockCand { uint8_t cand[MAXK], ncand, tx; };   // the tail of BlockRes
 struct RcShared {
     RcScr u;
     RcTabs tab;
-    uint16_t srcb[64 * 64];                  // source block of the current leaf: luma W x H, or U at 0 and V at 2048
+    uint16_t srcb[64 * 64];                  // source: the superblock's luma, or its chroma, U at 0 and V at 2048 (4:4:4: of
+                                             // the current tx block only)
+    int srcAt, srcSp;                        // the current block in it, and its row stride
     Img img;                                 // descriptor of the superblock's image
+    SearchParams prm;                        // the launch's search parameters
     int dcQ, acQ;                            // its quantizer steps
     float dcRcp, acRcp;                      // 1 / dcQ, 1 / acQ
     uint16_t ea[3][EDGE_LEN], el[3][EDGE_LEN];   // unfiltered edges of the current tx block per plane
@@ -101,7 +112,8 @@ struct RcShared {
     int skipCtx[3], dcCtx[3];
     int gup[RC_NG][2];                       // upsampling flags of each group's (team's) prepared edges
     uint8_t bdm[3][18][18];                  // BlockDecoded[plane][y + 1][x + 1]
-    int taskC[64], taskT[64], taskP[64], taskE[64], taskK[64];   // candidate, tx type, plane, eob, residual slot
+    uint8_t taskC[64], taskT[64], taskP[64], taskK[64];   // candidate, tx type, plane, residual slot
+    uint16_t taskE[64];                      // eob
     int candC[8], nCand;                     // luma: the re-checked candidates
     float taskJ[64];
     int nTask;
@@ -119,6 +131,7 @@ struct RcShared {
     int am, lm, mode, delta, uvMode, uvDelta, nuv, bsize;
     uint32_t qItem;                          // persistent schedule: the item taken
     uint16_t leaf[MAX_LEAVES];               // the superblock's blocks: size | x4 << 5 | y4 << 9
+    uint32_t cand[MAX_LEAVES][2];            // luma: their analysis candidates (6 bytes), count and tx type (BlockRes)
     uint32_t known[4];                       // last seen progress of the left, above and above-right superblock and of the
                                              // superblock's own luma; [0] bit 31: a wait failed
 };
@@ -223,7 +236,7 @@ __device__ void grp_residual(lds<RcShared> &S, lds<uint16_t> *gea, lds<uint16_t>
 #pragma unroll
             for (int k = 0; k < CH; k++) r[k] = clip3(0, (1 << bd) - 1, dcv + round2signed(alpha * (S.cflL[(i0 + k * DI) * W + j] - avg), 6));
         } else {
-            pred_col(m, pa, dcv, i0, DI, j, lw, lh, EA, EL, upA, upL, r);
+            pred_col(m, pa, dcv, i0, DI, j, lw, lh, EA, EL, upA, upL, r, RcPredTables{S.tab});
         }
 #pragma unroll
         for (int k = 0; k < CH; k++) {
@@ -239,7 +252,7 @@ __device__ void grp_residual(lds<RcShared> &S, lds<uint16_t> *gea, lds<uint16_t>
 // res is ready; the levels go to lev
 template <int W, int H>
 __device__ EvalOut grp_task(lds<RcShared> &S, lds<RcGroup> &X, const lds<Img> &I, int p, int c, int t, const lds<int16_t> *res,
-                            lds<int16_t> *lev, const SearchParams &P) {
+                            lds<int16_t> *lev, const lds<SearchParams> &P) {
     RcEvalIn e;
     e.txSz = tx_of(W, H); e.txType = t; e.plane = p;
     e.dcQ = S.dcQ; e.acQ = S.acQ; e.dcRcp = S.dcRcp; e.acRcp = S.acRcp;
@@ -252,7 +265,7 @@ __device__ EvalOut grp_task(lds<RcShared> &S, lds<RcGroup> &X, const lds<Img> &I
 // the same task by half the group (blocks of up to 64 coefficients), with tmp its own part of the group's scratch
 template <int W, int H>
 __device__ EvalOut half_task(lds<RcShared> &S, lds<float> *tmp, const lds<Img> &I, int p, int c, int t, const lds<int16_t> *res,
-                             lds<int16_t> *lev, const SearchParams &P) {
+                             lds<int16_t> *lev, const lds<SearchParams> &P) {
     RcEvalIn e;
     e.txSz = tx_of(W, H); e.txType = t; e.plane = p;
     e.dcQ = S.dcQ; e.acQ = S.acQ; e.dcRcp = S.dcRcp; e.acRcp = S.acRcp;
@@ -267,7 +280,7 @@ __device__ EvalOut half_task(lds<RcShared> &S, lds<float> *tmp, const lds<Img> &
 // two groups prepare the same edges)
 template <int W, int H>
 __device__ EvalOut wave_task(lds<RcShared> &S, lds<RcTeam> &X, int team, const lds<Img> &I, const DevTables &T, int p, int c,
-                             const lds<uint16_t> *src, int sp, const SearchParams &P) {
+                             const lds<uint16_t> *src, int sp, const lds<SearchParams> &P) {
     constexpr int LW = W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
     constexpr int TS = (W > 32 ? 32 : W) + 1;
     const int lane = glane(), bd = I.bd;
@@ -290,7 +303,7 @@ __device__ EvalOut wave_task(lds<RcShared> &S, lds<RcTeam> &X, int team, const l
 #pragma unroll
             for (int k = 0; k < CH; k++) r[k] = clip3(0, (1 << bd) - 1, dcv + round2signed(alpha * (S.cflL[(i0 + k * di) * W + j] - cavg), 6));
         } else {
-            pred_col(m, pa, dcv, i0, di, j, LW, LH, EA, EL, upA, upL, r);
+            pred_col(m, pa, dcv, i0, di, j, LW, LH, EA, EL, upA, upL, r, RcPredTables{S.tab});
         }
 #pragma unroll
         for (int k = 0; k < CH; k++) r[k] = (int)src[(i0 + k * di) * sp + j] - r[k];
@@ -339,7 +352,7 @@ __device__ __forceinline__ uint32_t inv_col(int j, int W, int ck, int bd, lds<in
 }
 
 // source of plane p in the staging buffer
-__device__ __forceinline__ const lds<uint16_t> *stage_src(const lds<RcShared> &S, int p) { return S.srcb + (p == 2 ? 2048 : 0); }
+__device__ __forceinline__ const lds<uint16_t> *stage_src(const lds<RcShared> &S, int p) { return S.srcb + S.srcAt + (p == 2 ? 2048 : 0); }
 
 // Inlined into each per-shape leaf function (rc_luma / rc_chroma): as a call of its own it would run on the ~140
 // registers outside the callee-saved ones and spill; inlined, the leaf function's one frame covers it.
@@ -349,7 +362,7 @@ __device__ __forceinline__ const lds<uint16_t> *stage_src(const lds<RcShared> &S
 // wg_luma_residuals; chroma tasks make their own in slot t; levels of task t go to S.u.s.lev[t].  Larger blocks:
 // team g (tasks g, g + RC_NTEAM, ..., run in descending order) keeps the levels and prepared edges of task g.
 template <int W, int H>
-__device__ __forceinline__ void wg_run_tasks(lds<RcShared> &S, const lds<Img> &I, const DevTables &T, const SearchParams &P, float lambda, bool lumaBits,
+__device__ __forceinline__ void wg_run_tasks(lds<RcShared> &S, const lds<Img> &I, const DevTables &T, const lds<SearchParams> &P, float lambda, bool lumaBits,
                              bool pickWinner) {
     constexpr bool big = W > 16 || H > 16;
     constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 4 ? 2 : H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
@@ -367,7 +380,7 @@ __device__ __forceinline__ void wg_run_tasks(lds<RcShared> &S, const lds<Img> &I
         done = true;
         if (!lumaBits) {
             for (int t = g; t < S.nTask; t += RC_NG)
-                grp_residual<W, H>(S, I.edgeFilter ? S.u.s.g[g].ea : nullptr, S.u.s.g[g].el, S.taskP[t], S.taskC[t], stage_src(S, S.taskP[t]), W,
+                grp_residual<W, H>(S, I.edgeFilter ? S.u.s.g[g].ea : nullptr, S.u.s.g[g].el, S.taskP[t], S.taskC[t], stage_src(S, S.taskP[t]), S.srcSp,
                              S.u.s.res[t], I.bd);
             __syncthreads();
         }
@@ -402,10 +415,10 @@ __device__ __forceinline__ void wg_run_tasks(lds<RcShared> &S, const lds<Img> &I
         if constexpr (big) { c = __builtin_amdgcn_readfirstlane(c); p = __builtin_amdgcn_readfirstlane(p); }   // the wave's task
         EvalOut o;
         if constexpr (big) {
-            o = wave_task<W, H>(S, S.u.b.t[me], me, I, T, p, c, stage_src(S, p), W, P);
+            o = wave_task<W, H>(S, S.u.b.t[me], me, I, T, p, c, stage_src(S, p), S.srcSp, P);
         } else {
             if (!lumaBits)   // chroma: this task's own residual
-                grp_residual<W, H>(S, I.edgeFilter ? S.u.s.g[g].ea : nullptr, S.u.s.g[g].el, p, c, stage_src(S, p), W, S.u.s.res[t], I.bd);
+                grp_residual<W, H>(S, I.edgeFilter ? S.u.s.g[g].ea : nullptr, S.u.s.g[g].el, p, c, stage_src(S, p), S.srcSp, S.u.s.res[t], I.bd);
             o = grp_task<W, H>(S, S.u.s.g[g], I, p, c, tt, S.u.s.res[lumaBits ? S.taskK[t] : t], S.u.s.lev + t * (W * H), P);
         }
         float J;
@@ -444,7 +457,7 @@ __device__ void wg_luma_residuals(lds<RcShared> &S, const lds<Img> &I) {
     constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : 4, LH = H == 4 ? 2 : H == 8 ? 3 : 4;
     const int g = gid();
     if (g < S.nCand)
-        grp_residual<W, H>(S, I.edgeFilter ? S.u.s.g[g].ea : nullptr, S.u.s.g[g].el, 0, S.candC[g], stage_src(S, 0), W, S.u.s.res[g], I.bd);
+        grp_residual<W, H>(S, I.edgeFilter ? S.u.s.g[g].ea : nullptr, S.u.s.g[g].el, 0, S.candC[g], stage_src(S, 0), S.srcSp, S.u.s.res[g], I.bd);
     __syncthreads();
 }
 
@@ -455,7 +468,7 @@ __device__ void wg_luma_residuals(lds<RcShared> &S, const lds<Img> &I) {
 // entry (index txb, + txbStep for V), context maps, BlockDecoded.  One wave of each half keeps the record, so the only
 // barriers are those of the inverse and one at the end.  (px, py): the tx block's first sample in its planes.
 template <int W, int H, int NP, typename Px>
-__device__ __forceinline__ void wg_finish(lds<RcShared> &S, const Batch &B, const SearchParams &P, const DevTables &T, uint32_t sb, const lds<Img> &I,
+__device__ __forceinline__ void wg_finish(lds<RcShared> &S, const Batch &B, const lds<SearchParams> &P, const DevTables &T, uint32_t sb, const lds<Img> &I,
                                           int t0, int slot0, int txType, int px, int py, uint32_t txb, uint32_t txbStep, uint32_t coef) {
     constexpr bool big = W > 16 || H > 16;
     constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 4 ? 2 : H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
@@ -470,7 +483,7 @@ __device__ __forceinline__ void wg_finish(lds<RcShared> &S, const Batch &B, cons
             const int tw = wv == t0 % RC_NTEAM ? t0 : NP == 2 && wv == (t0 + 1) % RC_NTEAM ? t0 + 1 : -1;
             if (tw >= 0) {
                 const int tp = __builtin_amdgcn_readfirstlane(S.taskP[tw]), tc = __builtin_amdgcn_readfirstlane(S.taskC[tw]);
-                wave_task<W, H>(S, S.u.b.t[wv], wv, I, T, tp, tc, stage_src(S, tp), W, P);
+                wave_task<W, H>(S, S.u.b.t[wv], wv, I, T, tp, tc, stage_src(S, tp), S.srcSp, P);
             }
             __syncthreads();
         }
@@ -524,7 +537,7 @@ __device__ __forceinline__ void wg_finish(lds<RcShared> &S, const Batch &B, cons
                 int v;
                 if (c == 255) v = clip3(0, maxv, dcv + round2signed(S.cflAlpha[p == 2] * (S.cflL[k] - S.cflAvg), 6));
                 else if (m == DC_PRED) v = dcv;
-                else v = pred_px(m, pa, i, j, LW, LH, EA, EL, upA, upL);
+                else v = pred_px(m, pa, i, j, LW, LH, EA, EL, upA, upL, RcPredTables{S.tab});
                 if (add) v = clip3(0, maxv, v + inv[k]);   // DCT_DCT: no flips
                 dst[(size_t)i * pitch + j] = (Px)v;
             }
@@ -533,7 +546,7 @@ __device__ __forceinline__ void wg_finish(lds<RcShared> &S, const Batch &B, cons
             const lds<int16_t> *res = S.u.s.res[slot];
             for (int k = tl; k < W * H; k += NT) {
                 const int i = k >> LW, j = k & (W - 1);
-                int v = (int)src[k] - res[k];
+                int v = (int)src[i * S.srcSp + j] - res[k];
                 if (add) v = clip3(0, maxv, v + inv[((fud ? H - 1 - i : i) << LW) + (flr ? W - 1 - j : j)]);
                 dst[(size_t)i * pitch + j] = (Px)v;
             }
@@ -583,23 +596,19 @@ __device__ __forceinline__ void wg_finish(lds<RcShared> &S, const Batch &B, cons
 }
 
 template <int W, int H, typename Px>
-__device__ __noinline__ void rc_luma(lds<RcShared> &S, const Batch &B, const SearchParams &P, uint32_t sb, const lds<Img> &I, int bsize, int x, int y, int availU,
-                        int availL, int tx0, int ty0, float lambda, uint32_t txb, uint32_t coef) {
+__device__ __noinline__ void rc_luma(lds<RcShared> &S, const Batch &B, const lds<SearchParams> &P, uint32_t sb, const lds<Img> &I, int bsize, int x, int y, int availU,
+                        int availL, int tx0, int ty0, float lambda, int li, uint32_t txb, uint32_t coef) {
     constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 4 ? 2 : H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
     const DevTables &T = *B.T;
     const int tid = threadIdx.x, txSz = tx_of(W, H);
     const int sbr4 = (y >> 2) & 15, sbc4 = (x >> 2) & 15, mi_row = y >> 2, mi_col = x >> 2;
-    {
-        const glb<Px> *src = src_plane<Px>(I, 0) + (size_t)y * I.spitch[0] + x;
-        for (int q = tid; q < W * H; q += RC_NT) S.srcb[q] = src[(size_t)(q >> LW) * I.spitch[0] + (q & (W - 1))];
-    }
     if (gid() == 0)
         rc_edges<Px>(S, I, 0, x, y, LW, LH, availL, availU, S.bdm[0][sbr4][sbc4 + (W >> 2) + 1], S.bdm[0][sbr4 + (H >> 2) + 1][sbc4],
                      mi_row, mi_col);
     if (gid() == 2) grp_txb_ctx(I, 0, txSz, mi_col, mi_row, bsize, tx0, ty0, &S.skipCtx[0], &S.dcCtx[0]);
     if (tid >= 128 && tid < 192) {   // wave 2: the tasks (candidate k, tx type t), k-major, types ascending
         const int w = tid - 128;
-        const BlockRes &br = B.blk[I.shOff[bsize] + (uint32_t)(y / (4 * bh4(bsize))) * I.shNbx[bsize] + x / (4 * bw4(bsize))];
+        const lds<BlockCand> &br = *(const lds<BlockCand> *)(const lds<char> *)S.cand[li];
         const int nc = max(1, min((int)br.ncand, P.Krecheck));
         const int set = tx_set_intra(txSz);
         if (w < nc) S.candC[w] = br.cand[w];
@@ -636,7 +645,7 @@ __device__ __noinline__ void rc_luma(lds<RcShared> &S, const Batch &B, const Sea
         // tx-type pass for the pass-1 winner (txAllCL off): the other types of the set
         if (tid == 0) {
             const int c0 = S.taskC[S.win], k0 = S.taskK[S.win], n0 = S.nTask;
-            const BlockRes &br = B.blk[I.shOff[bsize] + (uint32_t)(y / (4 * bh4(bsize))) * I.shNbx[bsize] + x / (4 * bw4(bsize))];
+            const lds<BlockCand> &br = *(const lds<BlockCand> *)(const lds<char> *)S.cand[li];
             int n = n0;
             for (int t = 1; t < 16; t++)
                 if (tx_in_set(tx_set_intra(txSz), t) && !(c0 == br.cand[0] && t == br.tx)) {
@@ -653,7 +662,7 @@ __device__ __noinline__ void rc_luma(lds<RcShared> &S, const Batch &B, const Sea
 }
 
 template <int W, int H, typename Px>
-__device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const SearchParams &P, uint32_t sb, const lds<Img> &I, int bsize, int mi_row, int mi_col,
+__device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const lds<SearchParams> &P, uint32_t sb, const lds<Img> &I, int bsize, int mi_row, int mi_col,
                           int availUC, int availLC, int tx0, int ty0, float lambda, uint32_t txb, uint32_t coef, int nTxb) {
     constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 4 ? 2 : H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
     const DevTables &T = *B.T;
@@ -668,7 +677,7 @@ __device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const S
     }
     if (gid() == 2) grp_txb_ctx(I, 1, txSz, x4, y4, bsize, tx0, ty0, &S.skipCtx[1], &S.dcCtx[1]);
     if (gid() == 3) grp_txb_ctx(I, 2, txSz, x4, y4, bsize, tx0, ty0, &S.skipCtx[2], &S.dcCtx[2]);
-    {
+    if (!ss) {   // (4:2:0: the superblock's chroma is there)
         const glb<Px> *gU = src_plane<Px>(I, 1) + (size_t)cy * I.spitch[1] + cx, *gV = src_plane<Px>(I, 2) + (size_t)cy * I.spitch[2] + cx;
         for (int q = tid; q < W * H; q += RC_NT) {
             S.srcb[q] = gU[(size_t)(q >> LW) * I.spitch[1] + (q & (W - 1))];
@@ -678,8 +687,8 @@ __device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const S
     if (tid < 32) S.satdI[tid] = 0;
     if (tid < 8) S.acc64[tid] = 0;
     __syncthreads();
-    constexpr int sp = W;
-    const lds<uint16_t> *srcU = S.srcb, *srcV = S.srcb + 2048;
+    const int sp = S.srcSp;
+    const lds<uint16_t> *srcU = stage_src(S, 1), *srcV = stage_src(S, 2);
     const bool cflOk = P.cfl && cfl_allowed(bsize);
     const float lamS = P.satdLambda * T.lamS[bd == 10][I.qindex];   // the luma lambda's screening weight
     const int yMode = S.mode;
@@ -874,7 +883,7 @@ __device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const S
                     const lds<uint16_t> *s = p == 1 ? srcU : srcV;
                     const lds<uint16_t> *A = S.ea[p] + EDGE_OFF, *L = S.el[p] + EDGE_OFF;
                     int pr[NSY];
-                    pred_col(m, pa, S.dcv[p], sy0, 4, sx, LW, LH, A, L, 0, 0, pr);
+                    pred_col(m, pa, S.dcv[p], sy0, 4, sx, LW, LH, A, L, 0, 0, pr, RcPredTables{S.tab});
 #pragma unroll
                     for (int k = 0; k < NSY; k++) d[k] = (int)s[(sy0 + 4 * k) * sp + sx] - pr[k];
                 }
@@ -900,7 +909,7 @@ __device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const S
                     const int c = S.uvc[ci], m = cand_mode(c), pa = pangle(m, cand_delta(c));
                     const lds<uint16_t> *s = p == 1 ? srcU : srcV;
                     const lds<uint16_t> *A = S.ea[p] + EDGE_OFF, *L = S.el[p] + EDGE_OFF;
-                    const int pr = m == DC_PRED ? S.dcv[p] : pred_px(m, pa, sy, sx, LW, LH, A, L, 0, 0);
+                    const int pr = m == DC_PRED ? S.dcv[p] : pred_px(m, pa, sy, sx, LW, LH, A, L, 0, 0, RcPredTables{S.tab});
                     v = (int)s[sy * sp + sx] - pr;
                 }
                 v = seg_sumi<GW>(hadamard4_lanes(v));
@@ -921,7 +930,7 @@ __device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const S
                 const lds<uint16_t> *s = p == 1 ? srcU : srcV;
                 const lds<uint16_t> *A = S.ea[p] + EDGE_OFF, *L = S.el[p] + EDGE_OFF;
                 int d[16], r[16];
-                pred_4x4(m, pa, S.dcv[p], sy, sx, LW, LH, A, L, r);
+                pred_4x4(m, pa, S.dcv[p], sy, sx, LW, LH, A, L, r, RcPredTables{S.tab});
 #pragma unroll
                 for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -1043,7 +1052,7 @@ __device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const S
 }
 
 // stage the cost tables of quantizer context qctx (and, when first, the tables of every image) in LDS
-__device__ void stage_tables(lds<RcShared> &S, const DevTables &T, int qctx, bool first) {
+__device__ void stage_tables(lds<RcShared> &S, const DevTables &T, const SearchParams &P, int qctx, bool first) {
     const int tid = threadIdx.x;
     static_assert(sizeof(CostTab) % 4 == 0, "the cost tables are floats");
     {
@@ -1053,6 +1062,7 @@ __device__ void stage_tables(lds<RcShared> &S, const DevTables &T, int qctx, boo
     }
     if (first) {
         if (tid == 0) S.tab.iscan = T.iscan;
+        if (tid < (int)(sizeof(SearchParams) / 4)) ((lds<uint32_t> *)(lds<char> *)&S.prm)[tid] = ((const uint32_t *)&P)[tid];
         for (int k = tid; k < 3 * 336; k += RC_NT) {
             const int kind = k / 336, r = k % 336, ln = r < 16 ? 2 : r < 80 ? 3 : 4, e = r - (ln == 2 ? 0 : ln == 3 ? 16 : 80);
             S.tab.fwdT[k] = T.fwdT[T.fwdOff[kind][ln] + e];
@@ -1061,6 +1071,8 @@ __device__ void stage_tables(lds<RcShared> &S, const DevTables &T, int qctx, boo
         if (tid < 19) S.tab.txScale[tid] = T.txScale[tid];
         for (int k = tid; k < 19 * 16; k += RC_NT) S.tab.txg[k / 16][k % 16] = T.txg[k / 16][k % 16];
         for (int k = tid; k < 19 * 25; k += RC_NT) S.tab.cbOff[k / 25][k % 25] = (&av1t::Coeff_Base_Ctx_Offset[0][0][0])[k];
+        if (tid < 90) S.tab.step[tid] = av1t::Dr_Intra_Derivative[tid];
+        if (tid >= 4 && tid < 128) S.tab.smooth[tid - 4] = sm_weights(31 - __clz(tid))[tid - (1 << (31 - __clz(tid)))];
         for (int k = tid; k < SCAN8_TOTAL; k += RC_NT) { S.tab.scan8[k] = T.scan8[k]; S.tab.iscan8[k] = T.iscan8[k]; }
     }
 }
@@ -1107,8 +1119,9 @@ __device__ bool wait_progress(const uint32_t *f, int shift, uint32_t need, const
 // progress; blocks along the right (bottom) edge of a superblock come in ascending row (column) order whatever the
 // partition, so two counts tell how far an edge is.  False: a wait failed (the schedule is being aborted).
 template <typename Px, int PL>
-__device__ bool recon_part(lds<RcShared> &S, const Batch &B, const SearchParams &P, uint32_t sb, const RcQueue *Q) {
+__device__ bool recon_part(lds<RcShared> &S, const Batch &B, uint32_t sb, const RcQueue *Q) {
     const int tid = threadIdx.x;
+    const lds<SearchParams> &P = S.prm;
     {   // the image's descriptor, read in place in LDS from here on, and the blocks
         static_assert(sizeof(Img) % 4 == 0, "the descriptor is copied by words");
         const uint32_t *g = (const uint32_t *)&B.img[B.sbImg[sb]];
@@ -1123,6 +1136,25 @@ __device__ bool recon_part(lds<RcShared> &S, const Batch &B, const SearchParams 
     const DevTables &T = *B.T;
     const uint32_t local = sb - I.sbBase;
     const int sbc = (int)(local % I.sbCols), sbr = (int)(local / I.sbCols), sbx = sbc * 64, sby = sbr * 64;
+    const int nLeaves = B.leafCount[sb];
+    // what the blocks will want of global memory whatever they decide: the source, and for luma the candidates
+    if constexpr (PL == 0) {
+        const glb<Px> *src = src_plane<Px>(I, 0) + (size_t)sby * I.spitch[0] + sbx;
+        for (int k = tid; k < 64 * 64; k += RC_NT) S.srcb[k] = src[(size_t)(k >> 6) * I.spitch[0] + (k & 63)];
+        if (tid < nLeaves) {
+            const int lf = S.leaf[tid], bs = lf & 31, x4 = (lf >> 5) & 15, y4 = lf >> 9;
+            static_assert(offsetof(BlockRes, cand) == 4 && sizeof(BlockRes) == 12, "candidates, count and type: the last two words");
+            const glb<uint32_t> *r = (const glb<uint32_t> *)(B.blk + I.shOff[bs] + (uint32_t)((sby + 4 * y4) / (4 * bh4(bs))) * I.shNbx[bs] +
+                                                             (sbx + 4 * x4) / (4 * bw4(bs)));
+            S.cand[tid][0] = r[1];
+            S.cand[tid][1] = r[2];
+        }
+    } else if (I.ss) {
+        for (int k = tid; k < 2 * 32 * 32; k += RC_NT) {
+            const int p = 1 + (k >> 10), y = (k >> 5) & 31, x = k & 31;
+            S.srcb[(p - 1) * 2048 + (k & 1023)] = (src_plane<Px>(I, p) + (size_t)(sby / 2 + y) * I.spitch[p] + sbx / 2)[x];
+        }
+    }
     int tc = 0, tr = 0;
     while (tc + 1 < I.tileCols && sbx >= I.tileColStart[tc + 1] * 4) tc++;
     while (tr + 1 < I.tileRows && sby >= I.tileRowStart[tr + 1] * 4) tr++;
@@ -1145,7 +1177,6 @@ __device__ bool recon_part(lds<RcShared> &S, const Batch &B, const SearchParams 
     }
     __syncthreads();
     const float lambda = T.lambda[I.bd == 10][I.qindex] * P.lambdaMul;
-    const int nLeaves = B.leafCount[sb];
     // the neighbours inside the tile and how much of them the coded area holds (units of 4 luma samples)
     uint32_t *const prog = Q ? Q->prog + (size_t)PL * Q->nSb + sb : nullptr;
     const bool hasLeft = sbx > tx0, hasUp = sby > ty0, hasUpR = hasUp && (sbc + 1) * 16 < miColEnd;
@@ -1189,11 +1220,15 @@ __device__ bool recon_part(lds<RcShared> &S, const Batch &B, const SearchParams 
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             }
         }
+        if (tid == 0) {
+            S.srcAt = PL == 0 ? ly4 * 256 + lx4 * 4 : I.ss ? (ay >> 1) * 128 + (ax >> 1) * 4 : 0;
+            S.srcSp = PL == 0 ? 64 : I.ss ? 32 : tx_w(uv_tx_size(bsize, 0));
+        }
         RecBlock *const rb = B.oBlocks + (size_t)sb * MAX_LEAVES + li;
         int skip = 0;
         if constexpr (PL == 0) {
             const int availU = inside(mi_row - 1, mi_col), availL = inside(mi_row, mi_col - 1);
-#define RC_LUMA(w, h) rc_luma<w, h, Px>(S, B, P, sb, I, bsize, x, y, availU, availL, tx0, ty0, lambda, firstTxb, firstCoef)
+#define RC_LUMA(w, h) rc_luma<w, h, Px>(S, B, P, sb, I, bsize, x, y, availU, availL, tx0, ty0, lambda, li, firstTxb, firstCoef)
             AV1M_TX_SWITCH(txSz, RC_LUMA)
 #undef RC_LUMA
             __syncthreads();
@@ -1305,13 +1340,12 @@ AV1M_RC_KERNEL(2) k_recon(RcStepArgs) {
     lds<RcShared> &S = *(lds<RcShared> *)(lds<char> *)smraw;
     const RcStepArgs &A = kernel_args<RcStepArgs>();
     const Batch &B = A.B;
-    const SearchParams &P = A.P;
     const uint32_t sb = A.sbList[blockIdx.x];
-    stage_tables(S, *B.T, B.img[B.sbImg[sb]].qctx, true);
+    stage_tables(S, *B.T, A.P, B.img[B.sbImg[sb]].qctx, true);
     __syncthreads();
-    recon_part<Px, 0>(S, B, P, sb, nullptr);
+    recon_part<Px, 0>(S, B, sb, nullptr);
     __syncthreads();
-    if (!S.img.mono) recon_part<Px, 1>(S, B, P, sb, nullptr);
+    if (!S.img.mono) recon_part<Px, 1>(S, B, sb, nullptr);
 }
 
 // Persistent schedule: every workgroup pulls items (a superblock's luma or chroma) from the queue, the anti-diagonal
@@ -1326,7 +1360,6 @@ AV1M_RC_KERNEL(WPE) k_recon_queue(RcQueueArgs) {
     lds<RcShared> &S = *(lds<RcShared> *)(lds<char> *)smraw;
     const RcQueueArgs &A = kernel_args<RcQueueArgs>();
     const Batch &B = A.B;
-    const SearchParams &P = A.P;
     const RcQueue &Q = A.Q;
     const int tid = threadIdx.x;
     int staged = -1;
@@ -1343,11 +1376,11 @@ AV1M_RC_KERNEL(WPE) k_recon_queue(RcQueueArgs) {
         const uint32_t sb = item & ~RC_CHROMA;
         const int qctx = B.img[B.sbImg[sb]].qctx;
         if (qctx != staged) {
-            stage_tables(S, *B.T, qctx, staged < 0);
+            stage_tables(S, *B.T, A.P, qctx, staged < 0);
             staged = qctx;
         }
         __syncthreads();
-        const bool ok = (item & RC_CHROMA) ? recon_part<Px, 1>(S, B, P, sb, &Q) : recon_part<Px, 0>(S, B, P, sb, &Q);
+        const bool ok = (item & RC_CHROMA) ? recon_part<Px, 1>(S, B, sb, &Q) : recon_part<Px, 0>(S, B, sb, &Q);
         if (!ok) break;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
         __syncthreads();
