@@ -7,6 +7,8 @@
 // by the xor butterfly 16, 8, 4, 2, 1; J = fmaf(lambda, bits, D).  Which physical lane computes a chain does not
 // change a value, so the passes spread their chains over the group freely.
 #pragma once
+#include <type_traits>
+#include <cstddef>
 #include "av1m_common.h"
 
 namespace av1m {
@@ -154,37 +156,66 @@ __device__ __forceinline__ float base_bits(const E &e, int eob) {
     return eob == 0 ? skip : b;
 }
 
-// Bits of the coefficient at scan position c (< eob) of a tx block of size TSZ given the levels q (natural order, stride =
-// adjusted width); sk: the scan and context class (0: 2D, default zig-zag scan dscan; 1: HORIZ, columns; 2: VERT, rows),
-// always 0 for sizes with a side over 16; cbOff: Coeff_Base_Ctx_Offset[TSZ] (5 x 5).
-// One path for the three classes, whose neighbour positions differ in data only, so the lanes of a wave that evaluate
-// different tx types do not run the classes one after the other; the five neighbours are read once for both contexts.
-template <int TSZ, typename QP, typename SP, typename OP, typename CT>
-__device__ __forceinline__ float coeff_bits(int c, int eob, int sk, QP q, SP dscan, OP cbOff, int pt, int dcCtx, const CT &C) {
+// The levels' magnitudes for the contexts: bytes min(|level|, 15) with four columns to the right and four rows below the
+// block that stay 0, so a neighbour is one read at a fixed distance with neither bounds nor absolute value (against reading
+// the levels: 45 of the 120 vector instructions per coefficient).  They are laid over the coefficients, which are all in
+// registers by then.
+template <int TW>
+constexpr int lv_stride() { return TW + 4; }
+__device__ __forceinline__ uint8_t *lv_of(float *p) { return (uint8_t *)p; }
+__device__ __forceinline__ lds<uint8_t> *lv_of(lds<float> *p) { return (lds<uint8_t> *)p; }
+typedef uint32_t __attribute__((may_alias)) word_a;
+__device__ __forceinline__ void lv_zero(uint8_t *p) { *(word_a *)p = 0; }
+__device__ __forceinline__ void lv_zero(lds<uint8_t> *p) { *(lds<word_a> *)p = 0; }
+// the margins of a TW x TH block by NL lanes
+template <int TW, int TH, int NL, typename LV>
+__device__ __forceinline__ void lv_margins(LV lv, int lane) {
+    constexpr int S = lv_stride<TW>(), NW = TH + S;   // words: one right of each row, S below
+    static_assert(TW % 4 == 0, "the margins are whole words");
+#pragma unroll
+    for (int k = 0; k < NW; k += NL) {
+        const int w = k + lane;
+        if (w < NW) lv_zero(lv + (w < TH ? w * S + TW : TH * S + 4 * (w - TH)));
+    }
+}
+
+// What the coefficients of one tx block share: the distances of the class's own three neighbours, (1,1) (0,2) (2,0) / (0,2) (0,3)
+// (0,4) / (2,0) (3,0) (4,0) for sk 0 (2D) / 1 (HORIZ) / 2 (VERT), and the cost of the DC's sign
+struct CoefIn {
+    int sk, d2, d3, d4;
+    float dcSign;
+};
+template <int TSZ, typename QP, typename E>
+__device__ __forceinline__ CoefIn coef_in(QP q, const E &e, int sk) {
+    constexpr int S = lv_stride<av1t::Tx_Width[av1t::Adjusted_Tx_Size[TSZ]]>();
+    static_assert(av1t::Sig_Ref_Diff_Offset[0][2][0] == 1 && av1t::Sig_Ref_Diff_Offset[1][2][1] == 2 && av1t::Sig_Ref_Diff_Offset[2][4][0] == 4,
+                  "neighbour order: right, below, then the class's own three");
+    return CoefIn{sk, sk == 0 ? S + 1 : sk == 1 ? 2 : 2 * S, sk == 0 ? 2 : sk == 1 ? 3 : 3 * S, sk == 1 ? 4 : sk == 0 ? 2 * S : 4 * S,
+                  (&(*e.C).dc_sign[e.plane > 0][e.dcCtx][0])[q[0] < 0]};
+}
+
+// Bits of the coefficient at scan position c (< eob) of a tx block of size TSZ given its magnitudes lv and levels q (natural
+// order, stride = adjusted width); in.sk: the scan and context class (0: 2D, default zig-zag scan dscan; 1: HORIZ, columns;
+// 2: VERT, rows), always 0 for sizes with a side over 16; cbOff: Coeff_Base_Ctx_Offset[TSZ] (5 x 5).  One path for the three
+// classes, whose neighbour positions differ in data only, so the lanes of a wave that evaluate different tx types do not
+// run the classes one after the other; the five neighbours are read once for both contexts.
+template <int TSZ, typename LV, typename QP, typename SP, typename OP, typename CT>
+__device__ __forceinline__ float coeff_bits(int c, int eob, const CoefIn &in, LV lv, QP q, SP dscan, OP cbOff, int pt, const CT &C) {
     constexpr int ctx = txsz_ctx_of(TSZ), adj = av1t::Adjusted_Tx_Size[TSZ];
-    constexpr int bwl = av1t::Tx_Width_Log2[adj], width = 1 << bwl, lbh = av1t::Tx_Height_Log2[adj], height = 1 << lbh;
+    constexpr int bwl = av1t::Tx_Width_Log2[adj], width = 1 << bwl, lbh = av1t::Tx_Height_Log2[adj], height = 1 << lbh, S = lv_stride<width>();
     constexpr bool only2d = width > 16 || height > 16;
+    const int sk = in.sk;
     int pos = dscan[c];
     if constexpr (!only2d) pos = sk == 0 ? pos : sk == 1 ? ((c & (height - 1)) << bwl) + (c >> lbh) : c;
     const int row = pos >> bwl, col = pos & (width - 1);
-    auto at = [&](int dr, int dc) -> int {   // |level| of the neighbour at (row + dr, col + dc), 0 outside (masked, no branch)
-        const int in = ((row + dr - height) & (col + dc - width)) >> 31;
-        const int a = q[pos + (((dr << bwl) + dc) & in)];
-        return max(a, -a) & in;
-    };
-    static_assert(av1t::Sig_Ref_Diff_Offset[0][2][0] == 1 && av1t::Sig_Ref_Diff_Offset[1][2][1] == 2 && av1t::Sig_Ref_Diff_Offset[2][4][0] == 4,
-                  "neighbour order: right, below, then the class's own three");
+    const auto at = lv + row * S + col;
+    const int level = at[0], a0 = at[1], a1 = at[S];
     int a2, a3, a4;
-    const int qv = q[pos], a0 = at(0, 1), a1 = at(1, 0);
     if constexpr (only2d) {
-        a2 = at(1, 1); a3 = at(0, 2); a4 = at(2, 0);
-    } else {   // the class's own three: (1,1) (0,2) (2,0) / (0,2) (0,3) (0,4) / (2,0) (3,0) (4,0)
-        a2 = at(sk == 2 ? 2 : 1 - sk, sk == 2 ? 0 : 1 + sk);
-        a3 = at(sk == 2 ? 3 : 0, sk == 2 ? 0 : 2 + sk);
-        a4 = at(sk == 2 ? 4 : sk == 1 ? 0 : 2, sk == 1 ? 4 : 0);
+        a2 = at[S + 1]; a3 = at[2]; a4 = at[2 * S];
+    } else {
+        a2 = at[in.d2]; a3 = at[in.d3]; a4 = at[in.d4];
     }
-    const int v = max(qv, -qv), level = min(v, 15);
-    const float sgn = (&C.dc_sign[pt][dcCtx][0])[qv < 0];
     const int m5 = min(a0, 3) + min(a1, 3) + min(a2, 3) + min(a3, 3) + min(a4, 3);
     const int m = min((m5 + 1) >> 1, 4);
     int bctx = pos == 0 ? 0 : m + (int)cbOff[min(row, 4) * 5 + min(col, 4)];
@@ -197,30 +228,32 @@ __device__ __forceinline__ float coeff_bits(int c, int eob, int sk, QP q, SP dsc
     const auto *pb = c == eob - 1 ? &C.coeff_base_eob[ctx][pt][ectx][min(max(level, 1), 3) - 1] : &C.coeff_base[ctx][pt][bctx][min(level, 3)];
     float b = *pb, golomb = 0.f;
     if (level > 2) {
-        const int mb = min((min(a0, 15) + min(a1, 15) + min(a2, 15) + 1) >> 1, 6);
+        const int mb = min((a0 + a1 + a2 + 1) >> 1, 6);
         bool near0 = row < 2 && col < 2;
         if constexpr (!only2d) near0 = sk == 0 ? near0 : sk == 1 ? col == 0 : row == 0;
         const auto *br = C.coeff_br[min(ctx, (int)TX_32X32)][pt][pos == 0 ? mb : near0 ? mb + 7 : mb + 14];
         // up to four symbols of at most 3: n3 full ones, then the rest
         const int rem = level - 3, n3 = (rem * 11) >> 5;   // rem / 3 for 0 .. 12
         const float full = br[3], rest = br[rem - 3 * n3];
+        const int qv = q[pos], v = max(qv, -qv);
 #pragma unroll
         for (int i = 0; i < 4; i++) b += i < n3 ? full : i == n3 ? rest : 0.f;
         golomb = v > 14 ? (float)(2 * (31 - __clz(max(v - 14, 1))) + 1) : 0.f;
     }
-    b += v ? (c == 0 ? sgn : 1.0f) : 0.f;   // the sign, then the Golomb part (sums with 0 are exact)
+    b += level ? (c == 0 ? in.dcSign : 1.0f) : 0.f;   // the sign, then the Golomb part (sums with 0 are exact)
     return b + golomb;
 }
 
-// eob and rate of the levels q of a tx block of size TSZ, class sk, by the group (all lanes return both); last: the
+// eob and rate of the levels of a tx block of size TSZ, class sk, by the group (all lanes return both); last: the
 // lane's share of the eob (1 + the largest scan index of a nonzero level among the positions the lane quantized)
-template <int TSZ, typename QP, typename SP, typename OP, typename E>
-__device__ __forceinline__ void grp_rate(QP q, SP dscan, OP cbOff, const E &e, int sk, int last, int &eobOut, float &bitsOut) {
+template <int TSZ, typename LV, typename QP, typename SP, typename OP, typename E>
+__device__ __forceinline__ void grp_rate(LV lv, QP q, SP dscan, OP cbOff, const E &e, int sk, int last, int &eobOut, float &bitsOut) {
     const int lane = glane();
     const int eob = gmaxi(last);
     const float base = base_bits<TSZ>(e, eob);
+    const CoefIn in = coef_in<TSZ>(q, e, sk);
     float bits = lane == 0 ? base : 0.f;
-    for (int c = lane; c < eob; c += GW) bits += coeff_bits<TSZ>(c, eob, sk, q, dscan, cbOff, e.plane > 0, e.dcCtx, *e.C);
+    for (int c = lane; c < eob; c += GW) bits += coeff_bits<TSZ>(c, eob, in, lv, q, dscan, cbOff, e.plane > 0, *e.C);
     eobOut = eob;
     bitsOut = gsum(bits);
 }
@@ -239,16 +272,17 @@ struct EvalScr {
     int16_t res[W * H];
     float tmp[H * (W + 1)];
     int16_t q[W * H];
+    __device__ std::nullptr_t lv() { return nullptr; }
 };
 
-template <int W, int H, typename FP, typename QP, typename E, typename TT>
-__device__ __forceinline__ EvalOut grp_qrate(FP tmp, int ts, QP q, const E &e, const TT &T);
+template <int W, int H, typename FP, typename QP, typename E, typename TT, typename LV>
+__device__ __forceinline__ EvalOut grp_qrate(FP tmp, int ts, QP q, const E &e, const TT &T, LV lvSep);
 
 // Forward transform + quantization + distortion + rate of the residual res (W x H, row-major), by the 32 lanes of
 // the calling group, with tmp (th x (W + 1) floats) as scratch.  Levels into q (natural order, tw x th).  All lanes
 // return the same values.
-template <int W, int H, typename RP, typename FP, typename QP, typename E, typename TT>
-__device__ EvalOut grp_eval(RP res, FP tmp, QP q, const E &e, const TT &T) {
+template <int W, int H, typename RP, typename FP, typename QP, typename E, typename TT, typename LV = std::nullptr_t>
+__device__ EvalOut grp_eval(RP res, FP tmp, QP q, const E &e, const TT &T, LV lvSep = nullptr) {
     constexpr int TW = W, TH = H, TS = W + 1;
     constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : 4, LH = H == 4 ? 2 : H == 8 ? 3 : 4;
     const int lane = glane();
@@ -313,14 +347,17 @@ __device__ EvalOut grp_eval(RP res, FP tmp, QP q, const E &e, const TT &T) {
         }
     }
     gsync();
-    return grp_qrate<W, H>(tmp, TS, q, e, T);
+    return grp_qrate<W, H>(tmp, TS, q, e, T, lvSep);
 }
 
 // Quantization, distortion and rate of the coefficients of a W x H tx block held in tmp (row i of the kept tw x th
 // region at tmp + i * ts), levels into q (natural order, tw x th).  All lanes of the group return the same values.
-template <int W, int H, typename FP, typename QP, typename E, typename TT>
-__device__ __forceinline__ EvalOut grp_qrate(FP tmp, int ts, QP q, const E &e, const TT &T) {
+// lvSep: where the magnitudes go, or null: over the coefficients, which then all pass through registers (where a lane has
+// eight of them and 168 registers that costs 40 in spills: the analysis of 16x16 keeps the two apart, 1.48 -> 1.2 ms on 12 MP).
+template <int W, int H, typename FP, typename QP, typename E, typename TT, typename LV>
+__device__ __forceinline__ EvalOut grp_qrate(FP tmp, int ts, QP q, const E &e, const TT &T, LV lvSep) {
     static_assert(W <= 16 && H <= 16, "larger tx blocks: wave_qrate");
+    static_assert((H + 4) * lv_stride<W>() <= H * (W + 1) * 4, "the magnitudes fit in the coefficients' space");
     constexpr int TW = W, TH = H;
     constexpr int LTW = TW == 4 ? 2 : TW == 8 ? 3 : 4;
     constexpr int N = TW * TH;
@@ -335,17 +372,33 @@ __device__ __forceinline__ EvalOut grp_qrate(FP tmp, int ts, QP q, const E &e, c
     float dist = 0.f;
     int last = 0;
     constexpr int NE = (N + GW - 1) / GW;   // per lane; a 4x4 leaves the upper half of the lanes a zero
-#pragma unroll 4
+    constexpr bool SEP = !std::is_same_v<LV, std::nullptr_t>;
+    auto coef = [&](int idx) {
+        const float v = tmp[(idx >> LTW) * ts + (idx & (TW - 1))];
+        return N >= GW || lane < N ? v : 0.f;
+    };
+    float x[NE];
+    if constexpr (!SEP) {
+#pragma unroll
+        for (int t = 0; t < NE; t++) x[t] = coef(N < GW ? lane & (N - 1) : lane + GW * t);
+        gsync();
+    }
+    const auto lv = [&] { if constexpr (SEP) return lvSep; else return lv_of(tmp); }();
+    lv_margins<TW, TH, GW>(lv, lane);
+    constexpr int UNR = SEP ? 4 : NE;
+#pragma unroll UNR
     for (int t = 0; t < NE; t++) {
         const int idx = N < GW ? lane & (N - 1) : lane + GW * t;
-        float v = tmp[(idx >> LTW) * ts + (idx & (TW - 1))];
-        if constexpr (N < GW) v = lane < N ? v : 0.f;
+        const float v = SEP ? coef(idx) : x[t];
         const int step = idx == 0 ? e.dcQ : e.acQ;
         const float a = quot_step(fabsf(v) * (float)den, (float)step, idx == 0 ? e.dcRcp : e.acRcp);
         int l = a < e.zbin ? 0 : (int)(a + e.rnd);
         l = min(l, 16383);
         const int qv = v < 0 ? -l : l;
-        if (N >= GW || lane < N) q[idx] = (int16_t)qv;
+        if (N >= GW || lane < N) {
+            q[idx] = (int16_t)qv;
+            lv[(idx >> LTW) * lv_stride<TW>() + (idx & (TW - 1))] = (uint8_t)min(l, 15);
+        }
         const int c0 = (int)iscan[idx], c = sk == 0 ? c0 : sk == 1 ? (idx & (TW - 1)) * TH + (idx >> LTW) : idx;
         last = max(last, l ? c + 1 : 0);
         const float dq = (float)dequant(qv, step, dsh, e.bd);   // 0 for level 0
@@ -359,7 +412,7 @@ __device__ __forceinline__ EvalOut grp_qrate(FP tmp, int ts, QP q, const E &e, c
     const auto cbOff = cboff_ptr<TSZ>(T);
     int eob;
     EvalOut o;
-    grp_rate<TSZ>(q, dscan, cbOff, e, sk, last, eob, o.R);
+    grp_rate<TSZ>(lv, q, dscan, cbOff, e, sk, last, eob, o.R);
     const float g = T.txg[e.txSz][e.txType];
     o.D = g * distS;
     o.eob = eob;
@@ -392,16 +445,26 @@ __device__ EvalOut half_qrate(FP tmp, int ts, QP q, const E &e, const TT &T) {
     const int den = dq_denom(e.txSz), dsh = den == 4 ? 2 : den == 2 ? 1 : 0;
     float dist[2] = {0.f, 0.f};
     int last = 0;
+    float x[N / 16];
+#pragma unroll
+    for (int t = 0; t < N / 16; t++) {
+        const int idx = lane + 16 * t;
+        x[t] = tmp[(idx >> LTW) * ts + (idx & (TW - 1))];
+    }
+    gsync();
+    const auto lv = lv_of(tmp);
+    lv_margins<TW, TH, 16>(lv, lane);
 #pragma unroll
     for (int t = 0; t < N / 16; t++) {   // virtual lane lane + 16 (t & 1)
         const int idx = lane + 16 * t;
-        const float v = tmp[(idx >> LTW) * ts + (idx & (TW - 1))];
+        const float v = x[t];
         const int step = idx == 0 ? e.dcQ : e.acQ;
         const float a = quot_step(fabsf(v) * (float)den, (float)step, idx == 0 ? e.dcRcp : e.acRcp);
         int l = a < e.zbin ? 0 : (int)(a + e.rnd);
         l = min(l, 16383);
         const int qv = v < 0 ? -l : l;
         q[idx] = (int16_t)qv;
+        lv[(idx >> LTW) * lv_stride<TW>() + (idx & (TW - 1))] = (uint8_t)min(l, 15);
         const int c0 = (int)iscan[idx], c = sk == 0 ? c0 : sk == 1 ? (idx & (TW - 1)) * TH + (idx >> LTW) : idx;
         last = max(last, l ? c + 1 : 0);
         const float dq = (float)dequant(qv, step, dsh, e.bd);
@@ -416,11 +479,12 @@ __device__ EvalOut half_qrate(FP tmp, int ts, QP q, const E &e, const TT &T) {
     const int eob = hmaxi(last);
     const float base = base_bits<TSZ>(e, eob);
     float b0 = lane == 0 ? base : 0.f, b1 = 0.f;
+    const CoefIn in = coef_in<TSZ>(q, e, sk);
     // the lane's two virtual lanes side by side: their chains of reads overlap
     for (int c = lane; c < eob; c += GW) {
         const int d = c + 16 < N ? c + 16 : c;
-        const float v0 = coeff_bits<TSZ>(c, eob, sk, q, dscan, cbOff, e.plane > 0, e.dcCtx, *e.C);
-        const float v1 = coeff_bits<TSZ>(d, eob, sk, q, dscan, cbOff, e.plane > 0, e.dcCtx, *e.C);
+        const float v0 = coeff_bits<TSZ>(c, eob, in, lv, q, dscan, cbOff, e.plane > 0, *e.C);
+        const float v1 = coeff_bits<TSZ>(d, eob, in, lv, q, dscan, cbOff, e.plane > 0, *e.C);
         b0 += v0;
         if (c + 16 < eob) b1 += v1;
     }
@@ -648,7 +712,7 @@ __device__ __forceinline__ float wave_fwd_dct(FP tmp, const DevTables &T, float 
     return 0.f;
 }
 
-// Quantization, distortion and rate of those coefficients (row stride ts), levels into q (natural order; may overlay tmp: every
+// Quantization, distortion and rate of those coefficients (row stride ts), levels into q (natural order; the front of tmp: every
 // coefficient is read before the first level is written).  Each virtual lane v of the 32-lane form is two lanes here: the
 // lower half's takes the first half of its elements, the upper half's the rest, and the sequential sums are handed over
 // once; the rate's scan positions alternate between the two.  All lanes return the same values.
@@ -657,6 +721,7 @@ __device__ __forceinline__ EvalOut wave_qrate(FP tmp, int ts, QP q, const E &e, 
     constexpr int TW = W > 32 ? 32 : W, TH = H > 32 ? 32 : H;
     constexpr int LTW = TW == 8 ? 3 : TW == 16 ? 4 : 5;
     constexpr int N = TW * TH, NE = N / 64, TSZ = tx_of(W, H);
+    static_assert(N * 2 + (TH + 4) * lv_stride<TW>() <= TH * (TW + 1) * 4, "levels and magnitudes fit in the coefficients' space");
     constexpr bool E64 = W == 64 || H == 64;
     const int v = threadIdx.x & 31, h = (threadIdx.x >> 5) & 1;
     const auto iscan = iscan_ptr<TSZ>(T);
@@ -668,6 +733,9 @@ __device__ __forceinline__ EvalOut wave_qrate(FP tmp, int ts, QP q, const E &e, 
         x[u] = tmp[(idx >> LTW) * ts + (idx & (TW - 1))];
     }
     gsync();
+    // the levels take the front of the coefficients' space, their magnitudes what follows
+    const auto lv = lv_of(tmp) + N * 2;
+    lv_margins<TW, TH, 64>(lv, wlane());
     int last = 0;
 #pragma unroll
     for (int u = 0; u < NE; u++) {
@@ -678,6 +746,7 @@ __device__ __forceinline__ EvalOut wave_qrate(FP tmp, int ts, QP q, const E &e, 
         l = min(l, 16383);
         const int qv = x[u] < 0 ? -l : l;
         q[idx] = (int16_t)qv;
+        lv[(idx >> LTW) * lv_stride<TW>() + (idx & (TW - 1))] = (uint8_t)min(l, 15);
         last = max(last, l ? (int)iscan[idx] + 1 : 0);
         const float d = x[u] - (float)dequant(qv, step, dsh, e.bd);
         sq[u] = d * d;
@@ -702,10 +771,11 @@ __device__ __forceinline__ EvalOut wave_qrate(FP tmp, int ts, QP q, const E &e, 
     last = max(last, other_half(last));
     const int eob = __builtin_amdgcn_readfirstlane(gmaxi(last));
     const float base = base_bits<TSZ>(e, eob);
+    const CoefIn in = coef_in<TSZ>(q, e, 0);
     float bits = v == 0 ? base : 0.f;
     for (int c0 = 0; c0 < eob; c0 += 64) {
         const int c = c0 + 32 * h + v;
-        const float b = coeff_bits<TSZ>(min(c, N - 1), eob, 0, q, dscan, cbOff, e.plane > 0, e.dcCtx, *e.C);
+        const float b = coeff_bits<TSZ>(min(c, N - 1), eob, in, lv, q, dscan, cbOff, e.plane > 0, *e.C);
         const Halves p = halves(c < eob ? b : 0.f);
         bits += p.lo;
         bits += p.hi;

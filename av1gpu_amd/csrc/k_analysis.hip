@@ -29,9 +29,13 @@ struct EvalScrWave {
     float tmp[TH * TS];
     __device__ lev16 *lev() { return reinterpret_cast<lev16 *>(tmp); }
 };
+struct EvalScr16 : EvalScr<16, 16> {   // with its magnitudes apart (grp_qrate)
+    uint32_t mag[20 * 20 / 4];
+    __device__ uint8_t *lv() { return (uint8_t *)mag; }
+};
 template <int W, int H>
 struct AnScr {
-    std::conditional_t<an_wave<W, H>(), EvalScrWave<W, H>, EvalScr<W, H>> ev;
+    std::conditional_t<an_wave<W, H>(), EvalScrWave<W, H>, std::conditional_t<W == 16 && H == 16, EvalScr16, EvalScr<W, H>>> ev;
     uint16_t ea[EDGE_LEN], el[EDGE_LEN];   // source edges
     uint16_t pa[EDGE_LEN], pl[EDGE_LEN];   // edge-filtered copies of the candidate under evaluation
     int satdI[32];
@@ -394,7 +398,7 @@ __global__ void __launch_bounds__(AN_NT) __attribute__((amdgpu_waves_per_eu(an_w
             }
             e.txType = t;
             e.intraDir = m;
-            const EvalOut o = grp_eval<W, H>(S.ev.res, S.ev.tmp, S.ev.q, e, T);
+            const EvalOut o = grp_eval<W, H>(S.ev.res, S.ev.tmp, S.ev.q, e, T, S.ev.lv());
             const float J = fmaf(lambda, (o.R + mbits(c)) + overhead, o.D);
             if (J < bestJ) {
                 bestJ = J;
