@@ -12,7 +12,7 @@
 //       and 13 luma-mode logits (the mode is used by some block of the superblock).
 // Convolutions are implicit GEMMs on v_mfma_f32_16x16x16_bf16 (positions x input taps times taps x channels), weights
 // and activations BF16, accumulation and biases FP32.  Training runs the same forward kernels, then FP32 backward
-// kernels (convolution weight gradients accumulated with float atomics) and Adam on FP32 master weights.
+// kernels on v_mfma_f32_32x32x2 (FP32 operands and sums) and Adam on FP32 master weights.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <string.h>
@@ -214,31 +214,61 @@ __global__ void __launch_bounds__(256) k_ln_conv12(const bf16_t *in, const bf16_
 }
 
 // ---- fully connected head: logits[item][o] = b[o] + sum_f W[o][f] a4[item][f] (FP32, f ascending) ----
-// LN_FC_IT items per block share each weight read; their features sit in LDS (one fmaf chain per item and output)
-constexpr int LN_FC_IT = 16;
-__global__ void __launch_bounds__(128) k_ln_fc(const bf16_t *a4, const float *W, const float *b, float *logits, uint32_t n) {
-    __shared__ float f[LN_FC_IT][LN_FEAT];
-    const uint32_t i0 = blockIdx.x * LN_FC_IT;
-    if (i0 >= n) return;
-    const int ni = (int)min((uint32_t)LN_FC_IT, n - i0);
-    for (int e = threadIdx.x; e < LN_FC_IT * LN_FEAT; e += 128) {
-        const int i = e / LN_FEAT, k = e % LN_FEAT;
-        f[i][k] = i < ni ? from_bf16(a4[(size_t)(i0 + i) * LN_FEAT + k]) : 0.f;
+// A 16 x 16 tile of items and outputs per wave on v_mfma_f32_16x16x4: each step adds its four products one after the
+// other in ascending f, so a logit is the fmaf chain from b[o] that a scalar loop would make, bit for bit.  A scalar
+// chain per thread and 16 items held 3 waves on as many compute units as there are groups of 16 items, 512 dependent
+// steps of 16 LDS reads each: 149 us for 512 items, now 12;
+// 186 -> 52 us for the 6000 superblocks of a 24 MP image against one load per step.  Lane l holds row l % 16 of either operand at
+// f = 4 s + l / 16.
+// A lane loads 4 consecutive features (16 and 8 bytes) of its row, and two lane swaps bring 16 x 16 of them into step
+// order.
+constexpr int LN_FC_UNR = 8;
+// 4 x 4 transposition over a lane's four values and the four groups of 16 lanes
+__device__ __forceinline__ void swap_4x4(float (&v)[4]) {
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[j]), __float_as_uint(v[2 + j]), false, false);
+        v[j] = __uint_as_float(p[0]); v[2 + j] = __uint_as_float(p[1]);
     }
-    __syncthreads();
-    for (int o = threadIdx.x; o < LN_OUT; o += 128) {
-        const float *w = W + (size_t)o * LN_FEAT;
-        float s[LN_FC_IT];
 #pragma unroll
-        for (int i = 0; i < LN_FC_IT; i++) s[i] = b[o];
-        for (int k = 0; k < LN_FEAT; k++) {
-            const float wk = w[k];
+    for (int j = 0; j < 4; j += 2) {
+        const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[j]), __float_as_uint(v[j + 1]), false, false);
+        v[j] = __uint_as_float(p[0]); v[j + 1] = __uint_as_float(p[1]);
+    }
+}
+__global__ void __launch_bounds__(256) k_ln_fc(const bf16_t *a4, const float *W, const float *b, float *logits, uint32_t n) {
+    const int l = threadIdx.x & 63, c = l & 15, q = l >> 4;
+    const uint32_t i0 = blockIdx.x * 16;
+    const int o0 = ((int)blockIdx.y * 4 + (int)(threadIdx.x >> 6)) * 16, o = min(o0 + c, LN_OUT - 1);
+    if (i0 >= n || o0 >= LN_OUT) return;
+    const bf16_t *x = a4 + (size_t)min(i0 + c, n - 1) * LN_FEAT + 4 * q;
+    const float *w = W + (size_t)o * LN_FEAT + 4 * q;
+    const float bo = b[o];
+    float4_t acc = {bo, bo, bo, bo};
+#pragma unroll 1
+    for (int k = 0; k < LN_FEAT; k += 16 * LN_FC_UNR) {
+        float4_t wv[LN_FC_UNR];
+        short4_t xv[LN_FC_UNR];
 #pragma unroll
-            for (int i = 0; i < LN_FC_IT; i++) s[i] = fmaf(wk, f[i][k], s[i]);
+        for (int s = 0; s < LN_FC_UNR; s++) {
+            wv[s] = *(const float4_t *)(w + k + 16 * s);
+            xv[s] = *(const short4_t *)(x + k + 16 * s);
         }
 #pragma unroll
-        for (int i = 0; i < LN_FC_IT; i++)
-            if (i < ni) logits[(size_t)(i0 + i) * LN_OUT + o] = s[i];
+        for (int s = 0; s < LN_FC_UNR; s++) {
+            float av[4], bv[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) { av[j] = from_bf16((bf16_t)xv[s][j]); bv[j] = wv[s][j]; }
+            swap_4x4(av);
+            swap_4x4(bv);
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j], bv[j], acc, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const uint32_t it = i0 + 4 * q + r;
+        if (it < n && o0 + c < LN_OUT) logits[(size_t)it * LN_OUT + o0 + c] = acc[r];
     }
 }
 
@@ -291,10 +321,12 @@ __global__ void __launch_bounds__(64) k_ln_decide(const float *logits, const Img
 
 // ================================ training ================================
 
-// loss (binary cross-entropy with logits, masked) and its gradient / count
-__global__ void __launch_bounds__(128) k_ln_loss(const float *logits, const float *label, const float *lmask, uint32_t n, float scale,
-                                                 float *dlog, float *lossOut) {
-    const uint32_t i = blockIdx.x * 128 + threadIdx.x;
+// loss (binary cross-entropy with logits, masked) and its gradient / count.  One addition to the loss per 1024 outputs:
+// one per wave queued 2144 of them on the same address for 512 items.
+__global__ void __launch_bounds__(1024) k_ln_loss(const float *logits, const float *label, const float *lmask, uint32_t n, float scale,
+                                                  float *dlog, float *lossOut) {
+    __shared__ float part[16];
+    const uint32_t i = blockIdx.x * 1024 + threadIdx.x;
     float l = 0.f;
     if (i < n * LN_OUT) {
         const float z = logits[i], y = label[i], w = lmask[i];
@@ -303,86 +335,231 @@ __global__ void __launch_bounds__(128) k_ln_loss(const float *logits, const floa
         l = w * (fmaxf(z, 0.f) - z * y + log1pf(expf(-fabsf(z))));
     }
     for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o, 64);
-    if ((threadIdx.x & 63) == 0 && l != 0.f) atomicAdd(lossOut, l * scale);
-}
-
-// FC backward, inputs: da4[item][f] = sum_o dlog[item][o] W[o][f], masked by the ReLU of a4
-__global__ void __launch_bounds__(256) k_ln_fc_bwd_in(const bf16_t *a4, const float *W, const float *dlog, uint32_t n, float *da4) {
-    const uint32_t item = blockIdx.x;
-    if (item >= n) return;
-    const float *g = dlog + (size_t)item * LN_OUT;
-    for (int k = threadIdx.x; k < LN_FEAT; k += 256) {
-        float s = 0.f;
-        for (int o = 0; o < LN_OUT; o++) s = fmaf(g[o], W[(size_t)o * LN_FEAT + k], s);
-        da4[(size_t)item * LN_FEAT + k] = from_bf16(a4[(size_t)item * LN_FEAT + k]) > 0.f ? s : 0.f;
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = l;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        float t = 0.f;
+        for (int k = 0; k < 16; k++) t += part[k];
+        if (t != 0.f) atomicAdd(lossOut, t * scale);
     }
 }
-// FC backward, weights: one thread per (o, f) over the items (no atomics); the bias row uses f = LN_FEAT
+
+// The backward kernels are FP32 contractions on v_mfma_f32_32x32x2: A 32 rows x 2, lane l holds row l % 32 at step
+// 2 s + l / 32, B likewise with columns; D: lane l holds column l % 32 of rows 8 (r / 4) + 4 (l / 32) + r % 4.
+// The operands keep their types (FP32 gradients and weights; BF16 activations are exact in FP32) and so do the sums.
+// Scalar fmaf chains, a thread per output, read two operands per multiplication and made 5.13 of the 5.55 ms of a
+// 512-item gradient (now 0.22 of 0.39); per kernel the figures stand below.
+typedef float float16_t __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ int d_row(int r, int h) { return 8 * (r >> 2) + 4 * h + (r & 3); }
+__device__ __forceinline__ float16_t mfma32(float a, float b, float16_t c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
+
+// FC backward, inputs: da4[item][f] = sum_o dlog[item][o] W[o][f] (o ascending), masked by the ReLU of a4.  A wave per
+// tile of 32 items x 32 features.
+__global__ void __launch_bounds__(64) k_ln_fc_bwd_in(const bf16_t *a4, const float *W, const float *dlog, uint32_t n, float *da4) {
+    const int l = threadIdx.x, c = l & 31, h = l >> 5, f = (int)blockIdx.x * 32 + c;
+    const uint32_t i0 = blockIdx.y * 32;
+    if (i0 >= n) return;
+    const float *g = dlog + (size_t)min(i0 + c, n - 1) * LN_OUT + h;
+    const float *w = W + (size_t)h * LN_FEAT + f;
+    float16_t acc = {};
+    static_assert(LN_OUT % 4 == 0, "whole steps of two outputs, two at a time");
+#pragma unroll 16
+    for (int s = 0; s < LN_OUT / 2; s++) acc = mfma32(g[2 * s], w[(size_t)2 * s * LN_FEAT], acc);
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        const uint32_t it = i0 + d_row(r, h);
+        if (it < n) da4[(size_t)it * LN_FEAT + f] = from_bf16(a4[(size_t)it * LN_FEAT + f]) > 0.f ? acc[r] : 0.f;
+    }
+}
+// FC backward, weights: dW[o][f] = sum over the items of dlog[item][o] a4[item][f].  A workgroup per tile of 32 outputs
+// x 32 features, its four waves taking every fourth pair of items and adding their sums in wave order; the workgroups
+// of the first features also sum the bias.
 __global__ void __launch_bounds__(256) k_ln_fc_bwd_w(const bf16_t *a4, const float *dlog, uint32_t n, float *dW, float *db) {
-    const uint32_t e = blockIdx.x * 256 + threadIdx.x;
-    if (e >= (uint32_t)LN_OUT * (LN_FEAT + 1)) return;
-    const int o = (int)(e / (LN_FEAT + 1)), k = (int)(e % (LN_FEAT + 1));
-    float s = 0.f;
-    for (uint32_t it = 0; it < n; it++) {
-        const float g = dlog[(size_t)it * LN_OUT + o];
-        s = fmaf(g, k < LN_FEAT ? from_bf16(a4[(size_t)it * LN_FEAT + k]) : 1.f, s);
+    __shared__ float red[4][32 * 32];
+    __shared__ float redb[4][64];
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, c = l & 31, h = l >> 5;
+    const int o0 = (int)blockIdx.y * 32, f0 = (int)blockIdx.x * 32, o = min(o0 + c, LN_OUT - 1);
+    float16_t acc = {};
+    float sb = 0.f;
+    for (uint32_t i0 = 2 * w; i0 < n; i0 += 8 * 8) {
+        float av[8], bv[8];
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            const uint32_t it = i0 + 8 * s + h, ic = min(it, n - 1);
+            const float g = dlog[(size_t)ic * LN_OUT + o];
+            av[s] = it < n ? g : 0.f;
+            bv[s] = from_bf16(a4[(size_t)ic * LN_FEAT + f0 + c]);
+        }
+#pragma unroll
+        for (int s = 0; s < 8; s++) { acc = mfma32(av[s], bv[s], acc); sb += av[s]; }
     }
-    if (k < LN_FEAT) dW[(size_t)o * LN_FEAT + k] += s;
-    else db[o] += s;
+#pragma unroll
+    for (int r = 0; r < 16; r++) red[w][d_row(r, h) * 32 + c] = acc[r];
+    redb[w][l] = sb;
+    __syncthreads();
+    for (int e = threadIdx.x; e < 32 * 32; e += 256)
+        if (o0 + (e >> 5) < LN_OUT) dW[(size_t)(o0 + (e >> 5)) * LN_FEAT + f0 + (e & 31)] = ((red[0][e] + red[1][e]) + red[2][e]) + red[3][e];
+    if (blockIdx.x == 0 && threadIdx.x < 32 && o0 + (int)threadIdx.x < LN_OUT) {
+        float s = 0.f;
+        for (int k = 0; k < 4; k++) s += redb[k][threadIdx.x] + redb[k][32 + threadIdx.x];
+        db[o0 + threadIdx.x] = s;
+    }
 }
 
-// convolution backward.  dz: gradient at the convolution's output before the ReLU (already masked), FP32 NHWC.
-// Weights: dW[co][k] += sum over items and output positions of dz[pos][co] * im2col(in)[pos][k]; db[co] += sum dz.
+// Convolution backward.  dz: gradient at the convolution's output before the ReLU (already masked), FP32 NHWC.
+// Weights: dW[co][k] = sum over items and output positions of dz[pos][co] * im2col(in)[pos][k]; db[co] = sum dz.
+// A wave takes output rows, two positions a step, and keeps the sums of every tap (a 32 x 32 tile of co x ci each, or
+// all 18 taps x channels of the first layer in one) in registers over all its rows; one dz load serves the nine
+// products.  Two waves per SIMD (more would not hold the 144 sums).  The workgroup's eight waves add their sums
+// pairwise through LDS into one partial row, and k_ln_conv_bwd_sum adds the rows: no atomics, so the gradient of a batch is
+// the same each time.  Layers of 32 / 16 / 8 / 64 inputs a side, 512 items: 2870 / 393 / 93 / 902 us as scalar chains
+// with float atomics, now 46 / 17 / 11 / 36.
+constexpr int LN_BW_WAVES = 8;
 template <int CIN, int HIN>
-__global__ void __launch_bounds__(256) k_ln_conv_bwd_w(const bf16_t *in, const float *dz, uint32_t n, float *dW, float *db) {
-    constexpr int HOUT = HIN / 2, NPOS = HOUT * HOUT, K = 9 * CIN, KP = (K + 15) / 16 * 16;
-    const uint32_t item = blockIdx.x;
-    if (item >= n) return;
-    const bf16_t *x = in + (size_t)item * HIN * HIN * CIN;
-    const float *g = dz + (size_t)item * NPOS * LN_C;
-    for (int e = threadIdx.x; e < LN_C * K; e += 256) {
-        const int co = e / K, k = e % K, t = k / CIN, ci = k % CIN, ky = t / 3, kx = t % 3;
-        float s = 0.f;
-        for (int pos = 0; pos < NPOS; pos++) {
-            const int oy = pos / HOUT, ox = pos % HOUT, iy = 2 * oy - 1 + ky, ix = 2 * ox - 1 + kx;
-            if (iy < 0 || iy >= HIN || ix < 0 || ix >= HIN) continue;
-            s = fmaf(g[(size_t)pos * LN_C + co], from_bf16(x[((size_t)iy * HIN + ix) * CIN + ci]), s);
+__global__ void __launch_bounds__(64 * LN_BW_WAVES) k_ln_conv_bwd_w(const bf16_t *in, const float *dz, uint32_t n, float *part, uint32_t stride) {
+    constexpr int HOUT = HIN / 2, K = 9 * CIN, KP = (K + 15) / 16 * 16, NT = CIN == 32 ? 9 : 1, UNR = CIN == 32 ? 4 : 8;
+    static_assert(CIN == 32 || (K <= 32 && KP == 32), "a tile of 32 channels per tap, or every tap and channel in one");
+    static_assert(HOUT / 2 % UNR == 0 || HOUT / 2 < UNR, "whole groups of steps");
+    __shared__ float4_t red[LN_BW_WAVES / 2][NT * 4][64];
+    __shared__ float redb[LN_BW_WAVES][LN_C];
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, c = l & 31, h = l >> 5;
+    float16_t acc[NT] = {};
+    float sb = 0.f;
+    const int ty = (c >> 1) / 3, tx = (c >> 1) % 3;   // the lane's column of the first layer: tap c / 2, channel c % 2
+    const bool col = c < K;
+    for (uint32_t row = blockIdx.x * LN_BW_WAVES + w; row < n * HOUT; row += gridDim.x * LN_BW_WAVES) {
+        const int oy = (int)(row % HOUT);
+        const float *g = dz + (size_t)row * HOUT * LN_C + l;
+        const bf16_t *x = in + (size_t)(row / HOUT) * HIN * HIN * CIN;
+#pragma unroll 1
+        for (int s0 = 0; s0 < HOUT / 2; s0 += UNR) {
+            constexpr int NS = UNR < HOUT / 2 ? UNR : HOUT / 2;
+            float a[NS], b[NS][NT];
+#pragma unroll
+            for (int s = 0; s < NS; s++) {
+                const int ox = 2 * (s0 + s) + h;
+                a[s] = g[(size_t)64 * (s0 + s)];
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    const int ky = NT == 9 ? t / 3 : ty, kx = NT == 9 ? t % 3 : tx;
+                    const int iy = 2 * oy - 1 + ky, ix = 2 * ox - 1 + kx;   // only the first row and column reach outside
+                    const int at = NT == 9 ? (max(iy, 0) * HIN + max(ix, 0)) * CIN + c
+                                           : (col ? (max(iy, 0) * HIN + max(ix, 0)) * CIN + (c & 1) : 0);
+                    const float v = from_bf16(x[at]);
+                    b[s][t] = iy >= 0 && ix >= 0 && (NT == 9 || col) ? v : 0.f;
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < NS; s++) {
+                sb += a[s];
+#pragma unroll
+                for (int t = 0; t < NT; t++) acc[t] = mfma32(a[s], b[s][t], acc[t]);
+            }
         }
-        if (s != 0.f) atomicAdd(&dW[(size_t)co * KP + k], s);
     }
-    for (int co = threadIdx.x; co < LN_C; co += 256) {
-        float s = 0.f;
-        for (int pos = 0; pos < NPOS; pos++) s += g[(size_t)pos * LN_C + co];
-        if (s != 0.f) atomicAdd(&db[co], s);
+    sb += __shfl_xor(sb, 32, 64);
+    if (h == 0) redb[w][c] = sb;
+#pragma unroll
+    for (int half = LN_BW_WAVES / 2; half > 0; half >>= 1) {   // waves half .. 2 half - 1 hand their sums to 0 .. half - 1
+        if (w >= half && w < 2 * half)
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    red[w - half][t * 4 + v][l] = float4_t{acc[t][4 * v], acc[t][4 * v + 1], acc[t][4 * v + 2], acc[t][4 * v + 3]};
+        __syncthreads();
+        if (w < half)
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const float4_t o = red[w][t * 4 + v][l];
+#pragma unroll
+                    for (int j = 0; j < 4; j++) acc[t][4 * v + j] += o[j];
+                }
+        __syncthreads();
     }
+    float *p = part + (size_t)blockIdx.x * stride;
+    if (w == 0) {
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) p[d_row(r, h) * KP + t * 32 + c] = acc[t][r];
+    } else if (w == 1 && h == 0) {
+        float t = 0.f;
+        for (int k = 0; k < LN_BW_WAVES; k++) t += redb[k][c];
+        p[LN_C * KP + c] = t;
+    }
+}
+// g[e] = the sum of the rows' e-th partials: 64 elements per workgroup, a quarter of the rows per wave
+__global__ void __launch_bounds__(256) k_ln_conv_bwd_sum(const float *part, uint32_t rows, uint32_t stride, float *g) {
+    __shared__ float red[4][64];
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint32_t e = blockIdx.x * 64 + l, r1 = rows * (w + 1) / 4;
+    float s = 0.f;
+    if (e < stride)
+#pragma unroll 16
+        for (uint32_t r = rows * w / 4; r < r1; r++) s += part[(size_t)r * stride + e];
+    red[w][l] = s;
+    __syncthreads();
+    if (w == 0 && e < stride) g[e] = ((red[0][l] + red[1][l]) + red[2][l]) + red[3][l];
 }
 // Input: dIn[iy][ix][ci] = sum over taps (ky, kx) and channels co of dz[oy][ox][co] W[co][tap][ci] with
 // iy = 2 oy - 1 + ky, then masked by the ReLU of that input (the previous layer's output > 0): the previous dz.
-template <int CIN, int HIN>
-__global__ void __launch_bounds__(256) k_ln_conv_bwd_in(const bf16_t *in, const float *W, const float *dz, uint32_t n, float *dzPrev) {
-    constexpr int HOUT = HIN / 2, K = 9 * CIN, KP = (K + 15) / 16 * 16;
-    const uint32_t item = blockIdx.x;
-    if (item >= n) return;
-    const bf16_t *x = in + (size_t)item * HIN * HIN * CIN;
-    const float *g = dz + (size_t)item * HOUT * HOUT * LN_C;
-    float *d = dzPrev + (size_t)item * HIN * HIN * CIN;
-    for (int e = threadIdx.x; e < HIN * HIN * CIN; e += 256) {
-        const int ci = e % CIN, p = e / CIN, iy = p / HIN, ix = p % HIN;
-        float s = 0.f;
-        if (from_bf16(x[e]) > 0.f) {
-            for (int ky = 0; ky < 3; ky++) {
-                const int ty = iy + 1 - ky;
-                if (ty < 0 || (ty & 1) || (ty >> 1) >= HOUT) continue;
-                for (int kx = 0; kx < 3; kx++) {
-                    const int tx = ix + 1 - kx;
-                    if (tx < 0 || (tx & 1) || (tx >> 1) >= HOUT) continue;
-                    const float *gz = g + ((size_t)(ty >> 1) * HOUT + (tx >> 1)) * LN_C;
-                    const int k = (ky * 3 + kx) * CIN + ci;
-                    for (int co = 0; co < LN_C; co++) s = fmaf(gz[co], W[(size_t)co * KP + k], s);
-                }
+// A wave takes 32 output positions at a time and makes the 2 x 2 input samples of each, four 32 x 32 tiles of
+// positions x ci: sample (a, b) = (0, 0) has one tap, (0, 1) and (1, 0) two, (1, 1) four, over dz of the position, its
+// right, lower and lower right neighbour (zero past the border).  The co of a step are 16 h + s, so that a lane's
+// dz are 16 consecutive floats; the weights lie in LDS in that order.  Layers of 32 / 16 / 8 inputs a side, 512 items:
+// 544 / 130 / 33 us as scalar chains, now 42 / 17 / 15.
+template <int HIN>
+__global__ void __launch_bounds__(256, 2) k_ln_conv_bwd_in(const bf16_t *in, const float *W, const float *dz, uint32_t n, float *dzPrev) {
+    constexpr int HOUT = HIN / 2, NPOS = HOUT * HOUT, KP = 9 * LN_C;
+    __shared__ float lw[9 * 16 * 64];
+#pragma unroll
+    for (int k = 0; k < 9 * 4; k++) {   // [tap][s][lane], every load in flight before the first is stored
+        const int e = 256 * k + (int)threadIdx.x, t = e >> 10, s = (e >> 6) & 15, co = 16 * ((e >> 5) & 1) + s;
+        lw[e] = W[(size_t)co * KP + t * LN_C + (e & 31)];
+    }
+    __syncthreads();
+    const int l = threadIdx.x & 63, c = l & 31, h = l >> 5;
+    const uint32_t total = n * NPOS, tiles = (total + 31) / 32, waves = gridDim.x * 4;
+    for (uint32_t tile = blockIdx.x * 4 + (threadIdx.x >> 6); tile < tiles; tile += waves) {
+        const uint32_t P = min(tile * 32 + c, total - 1);
+        const int oy = (int)(P % NPOS) / HOUT, ox = (int)(P % HOUT);
+        float16_t acc[4] = {};   // (a, b) = (0, 0), (0, 1), (1, 0), (1, 1)
+#pragma unroll
+        for (int sh = 0; sh < 4; sh++) {
+            const int sy = sh >> 1, sx = sh & 1;
+            const bool ok = oy + sy < HOUT && ox + sx < HOUT;
+            const float4 *g = (const float4 *)(dz + (size_t)(ok ? P + sy * HOUT + sx : P) * LN_C + 16 * h);
+            float a[16];
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const float4 q = g[v];
+                a[4 * v] = ok ? q.x : 0.f; a[4 * v + 1] = ok ? q.y : 0.f; a[4 * v + 2] = ok ? q.z : 0.f; a[4 * v + 3] = ok ? q.w : 0.f;
+            }
+#pragma unroll
+            for (int k = 3; k >= 0; k--) {
+                // sample (ay, ax) reads dz (sy, sx) through tap ky = ay ? 2 - 2 sy : 1 (sy = 0 only), kx likewise
+                const int ay = k >> 1, ax = k & 1;
+                if (sy > ay || sx > ax) continue;
+                const int t = (ay ? 2 - 2 * sy : 1) * 3 + (ax ? 2 - 2 * sx : 1);
+#pragma unroll
+                for (int s = 0; s < 16; s++) acc[k] = mfma32(a[s], lw[(t * 16 + s) * 64 + l], acc[k]);
             }
         }
-        d[e] = s;
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const uint32_t p = tile * 32 + d_row(r, h);
+            if (p >= total) continue;
+            const int py = (int)(p % NPOS) / HOUT, px = (int)(p % HOUT);
+            const size_t at = (((size_t)(p / NPOS) * HIN + 2 * py) * HIN + 2 * px) * LN_C + c;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const size_t e = at + ((size_t)(k >> 1) * HIN + (k & 1)) * LN_C;
+                dzPrev[e] = from_bf16(in[e]) > 0.f ? acc[k][r] : 0.f;
+            }
+        }
     }
 }
 
@@ -410,6 +587,7 @@ __global__ void __launch_bounds__(256) k_ln_to_bf16(const float *w, bf16_t *bf, 
 constexpr int LN_KP1 = 32, LN_KP = 288;
 constexpr size_t LN_W_OFF[4] = {0, 32 * LN_KP1 + 32, 32 * LN_KP1 + 32 + 32 * LN_KP + 32, 32 * LN_KP1 + 32 + 2 * (32 * LN_KP + 32)};
 constexpr size_t LN_FC_OFF = 32 * LN_KP1 + 32 + 3 * (32 * LN_KP + 32);
+constexpr uint32_t LN_PART_ROWS = 256;   // workgroups of a convolution's weight gradient: one per compute unit
 constexpr size_t LN_NPARAM = LN_FC_OFF + (size_t)LN_OUT * LN_FEAT + LN_OUT;
 constexpr size_t LN_NBF = 32 * LN_KP1 + 3 * 32 * LN_KP;   // the BF16 copies of the convolution weights
 inline size_t ln_kp(int l) { return l == 0 ? LN_KP1 : LN_KP; }
@@ -445,6 +623,7 @@ struct LnNet {
     LnActs act;
     // training state (allocated on first use)
     float *g = nullptr, *m = nullptr, *v = nullptr, *dlog = nullptr, *d4 = nullptr, *d3 = nullptr, *d2 = nullptr, *d1 = nullptr, *loss = nullptr;
+    float *part = nullptr;         // partial convolution weight gradients: LN_PART_ROWS rows of LN_FC_OFF
     float *label = nullptr, *lmask = nullptr;
     uint8_t *tiles = nullptr, *q = nullptr;
     uint32_t dcap = 0;             // items the gradient buffers hold
@@ -478,8 +657,8 @@ static void ln_forward(const LnNet &N, const LnActs &a, uint32_t n, hipStream_t 
     }
     hipLaunchKernelGGL((k_ln_conv<32, 16, 4>), dim3(n), dim3(64), 0, st, a.a2, N.wb + ln_bf_off(2), w + LN_W_OFF[2] + 32 * LN_KP, a.a3, n);
     hipLaunchKernelGGL((k_ln_conv<32, 8, 1>), dim3(n), dim3(64), 0, st, a.a3, N.wb + ln_bf_off(3), w + LN_W_OFF[3] + 32 * LN_KP, a.a4, n);
-    hipLaunchKernelGGL(k_ln_fc, dim3((n + LN_FC_IT - 1) / LN_FC_IT), dim3(128), 0, st, a.a4, w + LN_FC_OFF, w + LN_FC_OFF + (size_t)LN_OUT * LN_FEAT,
-                       a.logits, n);
+    hipLaunchKernelGGL(k_ln_fc, dim3((n + 15) / 16, (LN_OUT + 63) / 64), dim3(256), 0, st, a.a4, w + LN_FC_OFF,
+                       w + LN_FC_OFF + (size_t)LN_OUT * LN_FEAT, a.logits, n);
 }
 
 static void ln_refresh_bf16(LnNet &N, hipStream_t st) {
@@ -498,7 +677,7 @@ static hipError_t ln_upload(LnNet &N, const float *params) {
 }
 
 static void ln_free(LnNet &N) {
-    void *p[] = {N.w, N.wb, N.actMem, N.g, N.m, N.v, N.dlog, N.d4, N.d3, N.d2, N.d1, N.loss, N.label, N.lmask,
+    void *p[] = {N.w, N.wb, N.actMem, N.g, N.m, N.v, N.dlog, N.d4, N.d3, N.d2, N.d1, N.loss, N.part, N.label, N.lmask,
                  N.tiles, N.q};
     for (void *x : p) if (x) (void)hipFree(x);
     N = LnNet();
@@ -623,12 +802,14 @@ int av1mi_ln_set_data(av1mi_learner *L, const uint8_t *tiles, const uint8_t *q, 
 static int ln_grad(LnNet &N, uint32_t first, uint32_t n, float *loss, hipStream_t st) {
     if (n == 0 || first >= N.ndata || n > N.ndata - first) return -1;   // items past the data on the device
     if (ln_alloc_acts(N, n) != hipSuccess) return -1;
-    if (!N.g) {
+    if (!N.part) {   // the last of them: after a failure all are allocated again
+        for (float **p : {&N.g, &N.m, &N.v, &N.loss}) { (void)hipFree(*p); *p = nullptr; }
         if (hipMalloc(&N.g, LN_NPARAM * 4) != hipSuccess || hipMalloc(&N.m, LN_NPARAM * 4) != hipSuccess ||
             hipMalloc(&N.v, LN_NPARAM * 4) != hipSuccess || hipMalloc(&N.loss, 4) != hipSuccess)
             return -1;
         (void)hipMemset(N.m, 0, LN_NPARAM * 4);
         (void)hipMemset(N.v, 0, LN_NPARAM * 4);
+        if (hipMalloc(&N.part, LN_PART_ROWS * LN_FC_OFF * 4) != hipSuccess) return -1;
     }
     if (n > N.dcap || !N.dlog) {
         (void)hipFree(N.dlog); (void)hipFree(N.d4); (void)hipFree(N.d3); (void)hipFree(N.d2); (void)hipFree(N.d1);
@@ -638,26 +819,29 @@ static int ln_grad(LnNet &N, uint32_t first, uint32_t n, float *loss, hipStream_
             return -1;
         N.dcap = n;
     }
-    (void)hipMemsetAsync(N.g, 0, LN_NPARAM * 4, st);
     (void)hipMemsetAsync(N.loss, 0, 4, st);
     hipLaunchKernelGGL(k_ln_tiles, dim3(n), dim3(256), 0, st, N.tiles + (size_t)first * 4096, N.q + first, n, N.act.x0);
     ln_forward(N, N.act, n, st);
     const float scale = 1.0f / (float)n;
-    hipLaunchKernelGGL(k_ln_loss, dim3((n * LN_OUT + 127) / 128), dim3(128), 0, st, N.act.logits, N.label + (size_t)first * LN_OUT,
+    hipLaunchKernelGGL(k_ln_loss, dim3((n * LN_OUT + 1023) / 1024), dim3(1024), 0, st, N.act.logits, N.label + (size_t)first * LN_OUT,
                        N.lmask + (size_t)first * LN_OUT, n, scale, N.dlog, N.loss);
     float *g = N.g;
     const float *w = N.w;
-    hipLaunchKernelGGL(k_ln_fc_bwd_w, dim3((LN_OUT * (LN_FEAT + 1) + 255) / 256), dim3(256), 0, st, N.act.a4, N.dlog, n, g + LN_FC_OFF,
+    hipLaunchKernelGGL(k_ln_fc_bwd_w, dim3(LN_FEAT / 32, (LN_OUT + 31) / 32), dim3(256), 0, st, N.act.a4, N.dlog, n, g + LN_FC_OFF,
                        g + LN_FC_OFF + (size_t)LN_OUT * LN_FEAT);
-    hipLaunchKernelGGL(k_ln_fc_bwd_in, dim3(n), dim3(256), 0, st, N.act.a4, w + LN_FC_OFF, N.dlog, n, N.d4);
-    // layer 4 (input a3, 8x8): weights, then the gradient at a3 (masked by its ReLU)
-    hipLaunchKernelGGL((k_ln_conv_bwd_w<32, 8>), dim3(n), dim3(256), 0, st, N.act.a3, N.d4, n, g + LN_W_OFF[3], g + LN_W_OFF[3] + 32 * LN_KP);
-    hipLaunchKernelGGL((k_ln_conv_bwd_in<32, 8>), dim3(n), dim3(256), 0, st, N.act.a3, w + LN_W_OFF[3], N.d4, n, N.d3);
-    hipLaunchKernelGGL((k_ln_conv_bwd_w<32, 16>), dim3(n), dim3(256), 0, st, N.act.a2, N.d3, n, g + LN_W_OFF[2], g + LN_W_OFF[2] + 32 * LN_KP);
-    hipLaunchKernelGGL((k_ln_conv_bwd_in<32, 16>), dim3(n), dim3(256), 0, st, N.act.a2, w + LN_W_OFF[2], N.d3, n, N.d2);
-    hipLaunchKernelGGL((k_ln_conv_bwd_w<32, 32>), dim3(n), dim3(256), 0, st, N.act.a1, N.d2, n, g + LN_W_OFF[1], g + LN_W_OFF[1] + 32 * LN_KP);
-    hipLaunchKernelGGL((k_ln_conv_bwd_in<32, 32>), dim3(n), dim3(256), 0, st, N.act.a1, w + LN_W_OFF[1], N.d2, n, N.d1);
-    hipLaunchKernelGGL((k_ln_conv_bwd_w<2, 64>), dim3(n), dim3(256), 0, st, N.act.x0, N.d1, n, g + LN_W_OFF[0], g + LN_W_OFF[0] + 32 * LN_KP1);
+    hipLaunchKernelGGL(k_ln_fc_bwd_in, dim3(LN_FEAT / 32, (n + 31) / 32), dim3(64), 0, st, N.act.a4, w + LN_FC_OFF, N.dlog, n, N.d4);
+    // layer 4 (input a3, 8x8): weights, then the gradient at a3 (masked by its ReLU); and so on down to the first
+    const uint32_t rows = n < LN_PART_ROWS ? n : LN_PART_ROWS, stride = (uint32_t)LN_FC_OFF;
+    const dim3 bw(64 * LN_BW_WAVES);
+    auto in_grid = [&](uint32_t npos) { const uint32_t t = (n * npos + 127) / 128; return dim3(t < 512 ? t : 512); };
+    hipLaunchKernelGGL((k_ln_conv_bwd_w<32, 8>), dim3(rows), bw, 0, st, N.act.a3, N.d4, n, N.part + LN_W_OFF[3], stride);
+    hipLaunchKernelGGL((k_ln_conv_bwd_in<8>), in_grid(16), dim3(256), 0, st, N.act.a3, w + LN_W_OFF[3], N.d4, n, N.d3);
+    hipLaunchKernelGGL((k_ln_conv_bwd_w<32, 16>), dim3(rows), bw, 0, st, N.act.a2, N.d3, n, N.part + LN_W_OFF[2], stride);
+    hipLaunchKernelGGL((k_ln_conv_bwd_in<16>), in_grid(64), dim3(256), 0, st, N.act.a2, w + LN_W_OFF[2], N.d3, n, N.d2);
+    hipLaunchKernelGGL((k_ln_conv_bwd_w<32, 32>), dim3(rows), bw, 0, st, N.act.a1, N.d2, n, N.part + LN_W_OFF[1], stride);
+    hipLaunchKernelGGL((k_ln_conv_bwd_in<32>), in_grid(256), dim3(256), 0, st, N.act.a1, w + LN_W_OFF[1], N.d2, n, N.d1);
+    hipLaunchKernelGGL((k_ln_conv_bwd_w<2, 64>), dim3(rows), bw, 0, st, N.act.x0, N.d1, n, N.part + LN_W_OFF[0], stride);
+    hipLaunchKernelGGL(k_ln_conv_bwd_sum, dim3((stride + 63) / 64), dim3(256), 0, st, N.part, rows, stride, g);
     if (hipGetLastError() != hipSuccess) return -1;
     if (loss && hipMemcpyAsync(loss, N.loss, 4, hipMemcpyDeviceToHost, st) != hipSuccess) return -1;
     return hipStreamSynchronize(st) == hipSuccess ? 0 : -1;

@@ -69,6 +69,36 @@ def test_gradient_matches_reference():
     L.close()
 
 
+@pytest.mark.parametrize("n", [1, 2, 15, 33, 257])
+def test_gradient_at_batch_edges(n):
+    """Batches below, at and past the tiles' sides (16 items of the head, two items of 4 x 4 positions or 32 items of
+    the backward tiles, 64 items a round of the head's weights) and past the 256 workgroups of the weight gradients,
+    starting past the data's first item.  A gradient is a sum of at most n x 1024 products in FP32, each chain at most
+    2048 long: within 2048 x 2^-24 = 1.2e-4 of the sum of magnitudes; 1e-3 of the largest entry holds that with the
+    cancellation seen between items."""
+    rng = np.random.default_rng(n)
+    p = Ln.init_params(14)
+    tiles = rng.integers(0, 256, (n + 1, 64, 64)).astype(np.uint8)
+    q = rng.integers(1, 256, n + 1).astype(np.uint8)
+    lab = (rng.uniform(size=(n + 1, Ln.N_OUT)) < 0.4).astype(np.float32)
+    msk = (rng.uniform(size=(n + 1, Ln.N_OUT)) < 0.9).astype(np.float32)
+    L = Ln.Learner(p)
+    L.set_data(tiles, q, lab, msk)
+    loss, g = L.gradient(1, n)
+    again = L.gradient(1, n)[1]
+    assert np.array_equal(g.view(np.uint32), again.view(np.uint32))   # no sum depends on the order of workgroups
+    shapes = [(64, 64, 2), (32, 32, 32), (16, 16, 32), (8, 8, 32), (4, 4, 32)]
+    acts = [L.activations(k, n).reshape((n,) + s) for k, s in enumerate(shapes)]
+    assert np.array_equal(acts[0], R.input_tensor(tiles[1:], q[1:]))
+    lr, gr = R.ref_grads(p, acts, lab[1:], msk[1:])
+    assert abs(loss - lr) < 1e-4 * max(1.0, abs(lr))
+    (gc, gw5, gb5), (rc, rw5, rb5) = Ln.unpack(g.astype(np.float64)), Ln.unpack(gr)
+    for a, b, name in [(gw5, rw5, "fc W"), (gb5, rb5, "fc b")] + [(gc[l][k], rc[l][k], "conv%d %s" % (l, "Wb"[k]))
+                                                                  for l in range(4) for k in range(2)]:
+        assert np.max(np.abs(a - b)) <= 1e-3 * np.max(np.abs(b)) + 1e-7, name
+    L.close()
+
+
 def test_training_lowers_the_loss():
     tiles, q = _data(4)
     rng = np.random.default_rng(6)
