@@ -578,6 +578,7 @@ __device__ __forceinline__ int other_half(int v) {
     const auto p = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
     return (int)((threadIdx.x & 32) ? p[0] : p[1]);
 }
+__device__ __forceinline__ int wsumi(int v) { v = gsumi(v); return v + other_half(v); }   // over the wave
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 

@@ -133,7 +133,8 @@ struct RcShared {
     int errFlag[2], nzFlag[2];               // range violations, nonzero levels left (luma or U, V)
     int flopsOn;                             // count the forward-transform work (Batch::flops set)
     unsigned long long flops;                // of the superblock so far
-    int am, lm, mode, delta, uvMode, uvDelta, nuv, bsize;
+    int am, lm, mode, uvMode, uvDelta, nuv, bsize;
+    int nSkip, nCfl;                         // skipped blocks and CfL blocks of the item
     uint32_t qItem;                          // persistent schedule: the item taken
     uint16_t leaf[MAX_LEAVES];               // the superblock's blocks: size | x4 << 5 | y4 << 9
     uint32_t cand[MAX_LEAVES][2];            // luma: their analysis candidates (6 bytes), count and tx type (BlockRes)
@@ -470,11 +471,11 @@ __device__ void wg_luma_residuals(lds<RcShared> &S, const lds<Img> &I) {
 // task t0 + 1 behind U's t0): the winner's levels and prepared edges (a larger block evaluates the task again if its team
 // ran another after it), exact dequantization and inverse transform with the conformance repair (spec 7.13.3, 7.12.3
 // step 3: halve the levels until no range is violated), prediction + residual written once, then the record: levels, txb
-// entry (index txb, + txbStep for V), context maps, BlockDecoded.  One wave of each half keeps the record, so the only
-// barriers are those of the inverse and one at the end.  (px, py): the tx block's first sample in its planes.
-template <int W, int H, int NP, typename Px>
+// entry (index txb, + txbStep for V), context maps, BlockDecoded, and what done(eob, lane) adds.  One wave of each half
+// keeps the record, so the only barriers are those of the inverse and one at the end.  (px, py): the tx block's first sample in its planes.
+template <int W, int H, int NP, typename Px, typename Done>
 __device__ __forceinline__ void wg_finish(lds<RcShared> &S, const Batch &B, const lds<SearchParams> &P, const DevTables &T, uint32_t sb, const lds<Img> &I,
-                                          int t0, int slot0, int txType, int px, int py, uint32_t txb, uint32_t txbStep, uint32_t coef) {
+                                          int t0, int slot0, int txType, int px, int py, uint32_t txb, uint32_t txbStep, uint32_t coef, Done done) {
     constexpr bool big = W > 16 || H > 16;
     constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 4 ? 2 : H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
     constexpr int TW = W > 32 ? 32 : W, TH = H > 32 ? 32 : H, N = TW * TH, txSz = tx_of(W, H), NT = RC_NT / NP;
@@ -596,13 +597,14 @@ __device__ __forceinline__ void wg_finish(lds<RcShared> &S, const Batch &B, cons
             B.oTxb[(size_t)sb * B.txbCap + txb + half * txbStep] = r;
             S.winEob[p] = eob;
         }
+        done(eob, tl);
     }
     __syncthreads();
 }
 
 template <int W, int H, typename Px>
 __device__ __noinline__ void rc_luma(lds<RcShared> &S, const Batch &B, const lds<SearchParams> &P, uint32_t sb, const lds<Img> &I, int bsize, int x, int y, int availU,
-                        int availL, int tx0, int ty0, float lambda, int li, uint32_t txb, uint32_t coef) {
+                        int availL, int tx0, int ty0, float lambda, int li, int hasC, uint32_t txb, uint32_t coef) {
     constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : W == 16 ? 4 : W == 32 ? 5 : 6, LH = H == 4 ? 2 : H == 8 ? 3 : H == 16 ? 4 : H == 32 ? 5 : 6;
     const DevTables &T = *B.T;
     const int tid = threadIdx.x, txSz = tx_of(W, H);
@@ -661,9 +663,32 @@ __device__ __noinline__ void rc_luma(lds<RcShared> &S, const Batch &B, const lds
         __syncthreads();
         wg_run_tasks<W, H>(S, I, T, P, lambda, true, true);
     }
-    const int win = S.win;
-    if (tid == 0) { S.mode = cand_mode(S.taskC[win]); S.delta = cand_delta(S.taskC[win]); }
-    wg_finish<W, H, 1, Px>(S, B, P, T, sb, I, win, S.taskK[win], S.taskT[win], x, y, txb, 0, coef);
+    const int win = S.win, yMode = cand_mode(S.taskC[win]), yDelta = cand_delta(S.taskC[win]);
+    // the 4x4 maps and the block's record (the chroma item completes that of a block that carries chroma), with the tx
+    // block's own record, so that the block ends at one barrier
+    constexpr int W4 = W / 4, H4 = H / 4;
+    auto each4x4 = [&](int l0, int dl, auto f) {
+        for (int k = l0; k < W4 * H4; k += dl) {
+            const int r = mi_row + (k >> (LW - 2)), c = mi_col + (k & (W4 - 1));
+            if (r < I.MiRows && c < I.MiCols) f((size_t)r * I.MiCols + c);
+        }
+    };
+    each4x4(tid, RC_NT, [&](size_t o) { map8(I.mY)[o] = (uint8_t)yMode; map8(I.mMiSize)[o] = (uint8_t)bsize; map8(I.mTx)[o] = (uint8_t)txSz; });
+    wg_finish<W, H, 1, Px>(S, B, P, T, sb, I, win, S.taskK[win], S.taskT[win], x, y, txb, 0, coef, [&](int eob, int l) {
+        const int skip = eob == 0;
+        if (!hasC) each4x4(l, 64, [&](size_t o) { map8(I.mSkip)[o] = (uint8_t)skip; });
+        if (l == 0) {
+            RecBlock b;
+            b.mi_row = (uint16_t)mi_row; b.mi_col = (uint16_t)mi_col; b.bsize = (uint8_t)bsize; b.skip = (uint8_t)skip; b.tx_depth = 0;
+            b.y_mode = (uint8_t)yMode;
+            b.angle_delta_y = (int8_t)(bsize >= BLOCK_8X8 && is_dir(yMode) ? yDelta : 0);
+            b.uv_mode = 0; b.angle_delta_uv = 0; b.cfl_alpha_u = 0; b.cfl_alpha_v = 0;
+            b.filter_intra = 0; b.cdef_idx = 0; b.sb_qindex = 0;
+            B.oBlocks[(size_t)sb * MAX_LEAVES + li] = b;
+            B.oBlockTxb[(size_t)sb * MAX_LEAVES + li] = (uint16_t)txb;
+            if (skip && !hasC) S.nSkip++;
+        }
+    });
 }
 
 template <int W, int H, typename Px>
@@ -691,10 +716,48 @@ __device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const l
     }
     if (tid < 32) S.satdI[tid] = 0;
     if (tid < 8) S.acc64[tid] = 0;
+    if (tid < 13) S.uvc[tid] = cand_pack(tid, 0);
+    // CfL of up to 256 samples: the last wave alone, up to 4 samples a lane.  Here their luma and its average; the alphas
+    // while wave 0 chooses the deltas to screen (they are read from the ranking on).  Every sum fits in 32 bits: at 10 bits
+    // |l| <= 8184 gives |l x residual| x 256 < 2^31; the squared deviations of values in 0 .. 8184 from their rounded mean
+    // are at most 4092^2 + 1/4 on average, 256 of them < 2^32.  In steps of its own with 64-bit shuffles this took 20% of
+    // a chroma block, and a 4:4:4 image waits for its chroma: closed loop of one of 1021 x 767, 10 bits, 20.2 -> 17.6 ms,
+    // of nine 36.4 -> 31.8 ms.
+    constexpr bool CFLW = W * H <= 256;
+    constexpr int NPL = W * H <= 64 ? 1 : CFLW ? W * H / 64 : 1;
+    const bool cflOk = P.cfl && cfl_allowed(bsize), cflWave = tid >= RC_NT - 64;
+    const int cl = tid & 63;
+    int cv[NPL], cavg = 0;
+    if constexpr (CFLW) if (cflOk && cflWave) {
+        const int lt = av1t::Max_Tx_Size_Rect[bsize], tw = tx_w(lt), th = tx_h(lt);
+        int maxLumaW = 0, maxLumaH = 0;
+        for (int ly = mi_row * 4; ly < mi_row * 4 + 4 * bh4(bsize); ly += th)
+            for (int lx = mi_col * 4; lx < mi_col * 4 + 4 * bw4(bsize); lx += tw)
+                if (lx < I.MiCols * 4 && ly < I.MiRows * 4) { maxLumaW = lx + tw; maxLumaH = ly + th; }
+        const glb<Px> *luma = rec_plane<Px>(I, 0);
+        const int lp = I.pitch[0];
+        int sum = 0;
+#pragma unroll
+        for (int k = 0; k < NPL; k++) {
+            const int q = cl + 64 * k, i = q >> LW, j = q & (W - 1);
+            cv[k] = 0;
+            if (W * H >= 64 || q < W * H) {
+                if (ss) {
+                    const int ly = min((cy + i) << 1, maxLumaH - 2), lx = min((cx + j) << 1, maxLumaW - 2);
+                    const glb<Px> *r = luma + (size_t)ly * lp + lx;
+                    cv[k] = ((int)r[0] + r[1] + r[lp] + r[lp + 1]) << 1;
+                } else {
+                    cv[k] = (int)luma[(size_t)min(cy + i, maxLumaH - 1) * lp + min(cx + j, maxLumaW - 1)] << 3;
+                }
+                S.cflL[q] = cv[k];
+            }
+            sum += cv[k];
+        }
+        cavg = round2(wsumi(sum), LW + LH);
+    }
     __syncthreads();
     const int sp = S.srcSp;
     const lds<uint16_t> *srcU = stage_src(S, 1), *srcV = stage_src(S, 2);
-    const bool cflOk = P.cfl && cfl_allowed(bsize);
     const float lamS = P.satdLambda * T.lamS[bd == 10][I.qindex];   // the luma lambda's screening weight
     const int yMode = S.mode;
     auto uvbits = [&](int m) -> float { return cfl_allowed(bsize) ? C.uv_cfl_yes[yMode][m] : C.uv_cfl_no[yMode][m < 13 ? m : 0]; };
@@ -704,79 +767,52 @@ __device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const l
         if (bsize >= BLOCK_8X8 && is_dir(m)) b += C.angle_delta[m - V_PRED][cand_delta(c) + 3];
         return b;
     };
-    // ---- CfL: luma values, average, least-squares alpha, +-1 refinement by exact SSE ----
-    if constexpr (W * H <= 64) if (cflOk) {
-        // up to 64 samples: wave 0 alone, one sample per lane, with 64-lane integer sums (the same integers as the
-        // workgroup form below) and no barrier until the result
-        if (tid < 64) {
-            const int lt = av1t::Max_Tx_Size_Rect[bsize], tw = tx_w(lt), th = tx_h(lt);
-            int maxLumaW = 0, maxLumaH = 0;
-            for (int ly = mi_row * 4; ly < mi_row * 4 + 4 * bh4(bsize); ly += th)
-                for (int lx = mi_col * 4; lx < mi_col * 4 + 4 * bw4(bsize); lx += tw)
-                    if (lx < I.MiCols * 4 && ly < I.MiRows * 4) { maxLumaW = lx + tw; maxLumaH = ly + th; }
-            const glb<Px> *luma = rec_plane<Px>(I, 0);
-            const int lp = I.pitch[0], i = tid >> LW, j = tid & (W - 1);
-            const bool in = tid < W * H;
-            int v = 0;
-            if (in) {
-                if (ss) {
-                    const int ly = min((cy + i) << 1, maxLumaH - 2), lx = min((cx + j) << 1, maxLumaW - 2);
-                    v = ((int)luma[(size_t)ly * lp + lx] + luma[(size_t)ly * lp + lx + 1] + luma[(size_t)(ly + 1) * lp + lx] + luma[(size_t)(ly + 1) * lp + lx + 1]) << 1;
-                } else {
-                    v = (int)luma[(size_t)min(cy + i, maxLumaH - 1) * lp + min(cx + j, maxLumaW - 1)] << 3;
-                }
-                S.cflL[tid] = v;
-            }
-            int sum = v;
+    // ---- CfL: least-squares alpha, +-1 refinement by exact SSE ----
+    auto wave_cfl = [&] {   // CFLW: by the last wave, from the samples it holds
+        int nU = 0, nV = 0;
+        uint32_t dd = 0;
 #pragma unroll
-            for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
-            const int avg = round2(sum, LW + LH);
-            const long long l = in ? (long long)(v - avg) : 0;
-            long long nU = in ? l * ((int)srcU[i * sp + j] - S.dcv[1]) : 0, nV = in ? l * ((int)srcV[i * sp + j] - S.dcv[2]) : 0, dd = l * l;
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-                nU += __shfl_xor(nU, o, 64);
-                nV += __shfl_xor(nV, o, 64);
-                dd += __shfl_xor(dd, o, 64);
-            }
-            int alpha[2];
-            for (int k = 0; k < 2; k++) {
-                const long long n = k == 0 ? nU : nV;
-                const int a = dd > 0 ? (int)rintf(64.f * (float)n / (float)dd) : 0;
-                alpha[k] = max(-16, min(16, a));
-            }
-            long long sse[6] = {0, 0, 0, 0, 0, 0};
-            if (in) {
-#pragma unroll
-                for (int pl = 0; pl < 2; pl++) {
-                    const int s = pl == 0 ? srcU[i * sp + j] : srcV[i * sp + j];
-#pragma unroll
-                    for (int k = 0; k < 3; k++) {
-                        const int a = max(-16, min(16, alpha[pl] + k - 1));
-                        const int d = s - clip3(0, (1 << bd) - 1, S.dcv[pl + 1] + round2signed(a * (int)l, 6));
-                        sse[pl * 3 + k] = (long long)d * d;
-                    }
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < 6; k++)
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) sse[k] += __shfl_xor(sse[k], o, 64);
-            if (tid == 0) {
-                S.cflAvg = avg;
-                for (int pl = 0; pl < 2; pl++) {
-                    int bk = 1;
-                    for (int k = 0; k < 3; k++) if (sse[pl * 3 + k] < sse[pl * 3 + bk]) bk = k;
-                    S.cflAlpha[pl] = max(-16, min(16, alpha[pl] + bk - 1));
-                }
+        for (int k = 0; k < NPL; k++) {
+            const int q = cl + 64 * k, i = q >> LW, j = q & (W - 1), l = cv[k] - cavg;
+            if (W * H >= 64 || q < W * H) {
+                nU += l * ((int)srcU[i * sp + j] - S.dcv[1]);
+                nV += l * ((int)srcV[i * sp + j] - S.dcv[2]);
+                dd += (uint32_t)(l * l);
             }
         }
-        if (tid < 32) S.satdI[tid] = 0;
-        __syncthreads();
-    } else if (tid == 0) {
-        S.cflAlpha[0] = S.cflAlpha[1] = 0;
-    }
-    if constexpr (W * H > 64) if (cflOk) {
+        nU = wsumi(nU); nV = wsumi(nV); dd = (uint32_t)wsumi((int)dd);
+        int alpha[2], sse[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int pl = 0; pl < 2; pl++) {
+            const int a = dd > 0 ? (int)rintf(64.f * (float)(pl ? nV : nU) / (float)dd) : 0;
+            alpha[pl] = max(-16, min(16, a));
+        }
+#pragma unroll
+        for (int k = 0; k < NPL; k++) {
+            const int q = cl + 64 * k, i = q >> LW, j = q & (W - 1), l = cv[k] - cavg;
+            if (W * H >= 64 || q < W * H)
+#pragma unroll
+                for (int c = 0; c < 6; c++) {
+                    const int pl = c / 3, a = max(-16, min(16, alpha[pl] + c % 3 - 1));
+                    const int d = (int)(pl ? srcV : srcU)[i * sp + j] - clip3(0, (1 << bd) - 1, S.dcv[pl + 1] + round2signed(a * l, 6));
+                    sse[c] += d * d;
+                }
+        }
+#pragma unroll
+        for (int c = 0; c < 6; c++) sse[c] = wsumi(sse[c]);
+        if (cl == 0) {
+            S.cflAvg = cavg;
+#pragma unroll
+            for (int pl = 0; pl < 2; pl++) {
+                int bk = 1;
+#pragma unroll
+                for (int k = 0; k < 3; k++) if (sse[pl * 3 + k] < (bk == 0 ? sse[pl * 3] : sse[pl * 3 + 1])) bk = k;
+                S.cflAlpha[pl] = max(-16, min(16, alpha[pl] + bk - 1));
+            }
+        }
+    };
+    if (tid == 0 && (!CFLW || !cflOk)) S.cflAlpha[0] = S.cflAlpha[1] = 0;
+    if constexpr (!CFLW) if (cflOk) {
         const int lt = av1t::Max_Tx_Size_Rect[bsize], tw = tx_w(lt), th = tx_h(lt);
         int maxLumaW = 0, maxLumaH = 0;
         for (int ly = mi_row * 4; ly < mi_row * 4 + 4 * bh4(bsize); ly += th)
@@ -855,12 +891,8 @@ __device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const l
             }
         if (tid < 32) S.satdI[tid] = 0;
         __syncthreads();
-    } else if (tid == 0) {
-        S.cflAlpha[0] = S.cflAlpha[1] = 0;
     }
     // ---- SATD screening of the UV candidates over U and V (unfiltered edges) ----
-    if (tid < 13) S.uvc[tid] = cand_pack(tid, 0);
-    __syncthreads();
     constexpr int NSUB = (W / 4) * (H / 4), NSX = W / 4;
     // screening of blocks of up to 16 4x4s: item = (candidate, plane, pixel), 16 lanes per 4x4 and the Hadamard
     // across them, so a wave holds at most two candidates (modes); larger blocks: item = (candidate, plane, 4x4).  A
@@ -957,6 +989,7 @@ __device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const l
         }
         if (tid == 0) S.nuv = dl ? 19 : 13;
     }
+    if constexpr (CFLW) if (cflOk && cflWave) wave_cfl();
     __syncthreads();
     if (S.nuv > 13) screen(13, 19);
     if (tid < GW) {   // the uvK candidates of smallest screening cost (first minimum each round), U and V tasks each
@@ -1018,7 +1051,7 @@ __device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const l
     // a closed-loop final quantization with the chosen mode, and is not coded outside the coded area
     const int win = S.win, uvTxType = S.taskT[win], winC = S.taskC[win];
     const uint32_t perPlane = (uint32_t)nTxb / 2;
-    wg_finish<W, H, 2, Px>(S, B, P, T, sb, I, win, win, uvTxType, cx, cy, txb, perPlane, coef);
+    wg_finish<W, H, 2, Px>(S, B, P, T, sb, I, win, win, uvTxType, cx, cy, txb, perPlane, coef, [](int, int) {});
     // only a chroma tx block with a 32-sample side belongs to a 64-sided 4:4:4 block
     if constexpr (W == 32 || H == 32) if (perPlane > 1) {
         const int nTxX = (4 * bw4(bsize)) / W, nTxY = (4 * bh4(bsize)) / H;
@@ -1047,7 +1080,7 @@ __device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const l
             if (tid == 0) S.nTask = 2;
             __syncthreads();
             wg_run_tasks<W, H>(S, I, T, P, lambda, false, false);
-            wg_finish<W, H, 2, Px>(S, B, P, T, sb, I, 0, 0, uvTxType, cx + ox, cy + oy, txb + n, perPlane, coef + n * tx_ncoef(txSz));
+            wg_finish<W, H, 2, Px>(S, B, P, T, sb, I, 0, 0, uvTxType, cx + ox, cy + oy, txb + n, perPlane, coef + n * tx_ncoef(txSz), [](int, int) {});
             eobU |= S.winEob[1]; eobV |= S.winEob[2];
         }
         __syncthreads();
@@ -1181,6 +1214,7 @@ __device__ bool recon_part(lds<RcShared> &S, const Batch &B, uint32_t sb, const 
         S.dcRcp = 1.f / (float)S.dcQ; S.acRcp = 1.f / (float)S.acQ;
         for (int k = 0; k < 4; k++) S.known[k] = 0;
         S.errFlag[0] = S.errFlag[1] = 0;
+        S.nSkip = S.nCfl = 0;
     }
     __syncthreads();
     const float lambda = T.lambda[I.bd == 10][I.qindex] * P.lambdaMul;
@@ -1231,43 +1265,16 @@ __device__ bool recon_part(lds<RcShared> &S, const Batch &B, uint32_t sb, const 
             S.srcAt = PL == 0 ? ly4 * 256 + lx4 * 4 : I.ss ? (ay >> 1) * 128 + (ax >> 1) * 4 : 0;
             S.srcSp = PL == 0 ? 64 : I.ss ? 32 : tx_w(uv_tx_size(bsize, 0));
         }
-        RecBlock *const rb = B.oBlocks + (size_t)sb * MAX_LEAVES + li;
-        int skip = 0;
         if constexpr (PL == 0) {
             const int availU = inside(mi_row - 1, mi_col), availL = inside(mi_row, mi_col - 1);
-#define RC_LUMA(w, h) rc_luma<w, h, Px>(S, B, P, sb, I, bsize, x, y, availU, availL, tx0, ty0, lambda, li, firstTxb, firstCoef)
+#define RC_LUMA(w, h) rc_luma<w, h, Px>(S, B, P, sb, I, bsize, x, y, availU, availL, tx0, ty0, lambda, li, hasC, firstTxb, firstCoef)
             AV1M_TX_SWITCH(txSz, RC_LUMA)
 #undef RC_LUMA
-            __syncthreads();
-            skip = S.winEob[0] == 0;   // of the luma; the chroma item completes the record of a block that carries chroma
-            const int yMode = S.mode;
-            for (int k = tid; k < bw * bh; k += RC_NT) {
-                const int r = mi_row + (k >> lbw), c = mi_col + (k & (bw - 1));
-                if (r < I.MiRows && c < I.MiCols) {
-                    const size_t o = (size_t)r * I.MiCols + c;
-                    map8(I.mY)[o] = (uint8_t)yMode;
-                    if (!hasC) map8(I.mSkip)[o] = (uint8_t)skip;
-                    map8(I.mMiSize)[o] = (uint8_t)bsize;
-                    map8(I.mTx)[o] = (uint8_t)txSz;
-                }
-            }
-            if (tid == 0) {
-                RecBlock b;
-                b.mi_row = (uint16_t)mi_row; b.mi_col = (uint16_t)mi_col; b.bsize = (uint8_t)bsize; b.skip = (uint8_t)skip; b.tx_depth = 0;
-                b.y_mode = (uint8_t)yMode;
-                b.angle_delta_y = (int8_t)(bsize >= BLOCK_8X8 && is_dir(yMode) ? S.delta : 0);
-                b.uv_mode = 0; b.angle_delta_uv = 0; b.cfl_alpha_u = 0; b.cfl_alpha_v = 0;
-                b.filter_intra = 0; b.cdef_idx = 0; b.sb_qindex = 0;
-                *rb = b;
-                B.oBlockTxb[(size_t)sb * MAX_LEAVES + li] = (uint16_t)firstTxb;
-                atomicAdd(&B.stats[0], 1u);
-                if (skip && !hasC) atomicAdd(&B.stats[1], 1u);
-            }
         } else {
+            RecBlock *const rb = B.oBlocks + (size_t)sb * MAX_LEAVES + li;
             const int availUC = (I.ss && bh == 1) ? inside(mi_row - 2, mi_col) : inside(mi_row - 1, mi_col);
             const int availLC = (I.ss && bw == 1) ? inside(mi_row, mi_col - 2) : inside(mi_row, mi_col - 1);
-            if (tid == 0) { S.mode = rb->y_mode; S.winEob[0] = !rb->skip; }
-            __syncthreads();
+            if (tid == 128) { S.mode = rb->y_mode; S.winEob[0] = !rb->skip; }   // read from the first barrier on
             const int uvTx = uv_tx_size(bsize, I.ss);
 #define RC_CHROMA(w, h) rc_chroma<w, h, Px>(S, B, P, sb, I, bsize, mi_row, mi_col, availUC, availLC, tx0, ty0, lambda * P.lambdaCMul, \
                                                    firstTxb + 1, firstCoef + tx_ncoef(txSz), cTxb)
@@ -1280,7 +1287,7 @@ __device__ bool recon_part(lds<RcShared> &S, const Batch &B, uint32_t sb, const 
             }
 #undef RC_CHROMA
             __syncthreads();
-            skip = S.winEob[0] == 0 && S.winEob[1] == 0 && S.winEob[2] == 0;
+            const int skip = S.winEob[0] == 0 && S.winEob[1] == 0 && S.winEob[2] == 0;
             const int uv = S.uvMode;
             for (int k = tid; k < bw * bh; k += RC_NT) {
                 const int r = mi_row + (k >> lbw), c = mi_col + (k & (bw - 1));
@@ -1297,13 +1304,13 @@ __device__ bool recon_part(lds<RcShared> &S, const Batch &B, uint32_t sb, const 
                 rb->angle_delta_uv = (int8_t)(bsize >= BLOCK_8X8 && is_dir(uv) ? S.uvDelta : 0);
                 rb->cfl_alpha_u = (int8_t)(cfl ? S.cflAlpha[0] : 0);
                 rb->cfl_alpha_v = (int8_t)(cfl ? S.cflAlpha[1] : 0);
-                if (skip) atomicAdd(&B.stats[1], 1u);
-                if (cfl) atomicAdd(&B.stats[2], 1u);
+                S.nSkip += skip;
+                S.nCfl += cfl;
             }
+            __syncthreads();
         }
         if (ax + aw == 16) ownR = ay + ah;
         if (ay + ah == 16) ownB = ax + aw;
-        __syncthreads();
         if (Q && tid == RC_NT - 64) {   // the last wave, which has the least to do while the next block is set up
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
             __hip_atomic_store(prog, ownR | ownB << 8 | (uint32_t)(li + 1) << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1314,7 +1321,11 @@ __device__ bool recon_part(lds<RcShared> &S, const Batch &B, uint32_t sb, const 
             SbOut o;
             o.nBlocks = (uint32_t)nLeaves; o.nTxb = (uint32_t)nTxb; o.nCoeffs = (uint32_t)nCoef; o.pad = 0;
             B.sbOut[sb] = o;
+            atomicAdd(&B.stats[0], (uint32_t)nLeaves);
+        } else if (S.nCfl) {
+            atomicAdd(&B.stats[2], (uint32_t)S.nCfl);
         }
+        if (S.nSkip) atomicAdd(&B.stats[1], (uint32_t)S.nSkip);
         if (S.flopsOn && S.flops) atomicAdd(&B.flops[32 + (sb & 31)], S.flops);
     }
     return true;
