@@ -239,24 +239,38 @@ struct Inv {
     static AV1M_HD int32_t mul(int32_t a, int32_t b) { return (int32_t)((uint32_t)a * (uint32_t)b); }
     static AV1M_HD int32_t add(int32_t a, int32_t b) { return (int32_t)((uint32_t)a + (uint32_t)b); }
     static AV1M_HD int32_t sub(int32_t a, int32_t b) { return (int32_t)((uint32_t)a - (uint32_t)b); }
+    // a * b for factors of at most 24 bits: the vector unit has that at the full rate, a 32-bit product at a quarter of it.
+    // A factor is a value inside its range (at most 18 bits) and a constant of at most 14; in a pass that is discarded
+    // anyway it may be cut.
+    static AV1M_HD int32_t mul24(int32_t a, int32_t b) {
+#ifdef __HIP_DEVICE_COMPILE__
+        return __mul24(a, b);
+#else
+        return mul((int32_t)((uint32_t)a << 8) >> 8, (int32_t)((uint32_t)b << 8) >> 8);
+#endif
+    }
+    // the lowest and the highest value of the range-checked ones: two instructions per rotation, and one test per transform
+    struct Span { int32_t lo = 0, hi = 0; };
+    static AV1M_HD int32_t imin(int32_t a, int32_t b) { return a < b ? a : b; }
+    static AV1M_HD int32_t imax(int32_t a, int32_t b) { return a > b ? a : b; }
+    static AV1M_HD uint32_t outside(const Span &v, int bits) { return v.lo < -(1 << (bits - 1)) || v.hi > (1 << (bits - 1)) - 1 ? 1u : 0u; }
     static AV1M_HD int32_t rnd12(int32_t v) { return add(v, 2048) >> 12; }
     static AV1M_HD void range(int32_t v, int bits, uint32_t &err, uint32_t f) {
         if (v < -(1 << (bits - 1)) || v > (1 << (bits - 1)) - 1) err |= f;
     }
-    static AV1M_HD void B(int32_t *T, int a, int b, int ang, int flip, int r, uint32_t &err) {
+    static AV1M_HD void B(int32_t *T, int a, int b, int ang, int flip, Span &sp) {
         const int32_t c = cos128(ang), s = cos128(ang - 64);
-        const int32_t x = rnd12(sub(mul(T[a], c), mul(T[b], s))), y = rnd12(add(mul(T[a], s), mul(T[b], c)));
-        range(x, r, err, 1u);
-        range(y, r, err, 1u);
+        const int32_t x = rnd12(sub(mul24(T[a], c), mul24(T[b], s))), y = rnd12(add(mul24(T[a], s), mul24(T[b], c)));
+        sp.lo = imin(sp.lo, imin(x, y));
+        sp.hi = imax(sp.hi, imax(x, y));
         T[a] = flip ? y : x;
         T[b] = flip ? x : y;
     }
     static AV1M_HD void H(int32_t *T, int a, int b, int flip, int r) {
         const int aa = flip ? b : a, bb = flip ? a : b;
         const int32_t x = T[aa], y = T[bb], lo = -(1 << (r - 1)), hi = (1 << (r - 1)) - 1;
-        const int32_t s = add(x, y), d = sub(x, y);
-        T[aa] = s < lo ? lo : s > hi ? hi : s;
-        T[bb] = d < lo ? lo : d > hi ? hi : d;
+        T[aa] = imin(imax(add(x, y), lo), hi);
+        T[bb] = imin(imax(sub(x, y), lo), hi);
     }
     static constexpr int brev(int bits, int x) {
         int t = 0;
@@ -264,6 +278,7 @@ struct Inv {
         return t;
     }
     template <int n> static AV1M_HD void dct(int32_t *T, int r, uint32_t &err) {
+        Span sp;
         constexpr int n0 = 1 << n;
         int32_t c[n0];
 #pragma unroll
@@ -272,11 +287,11 @@ struct Inv {
         for (int i = 0; i < n0; i++) T[i] = c[brev(n, i)];
         if (n == 6) {
 #pragma unroll
-            for (int i = 0; i < 16; i++) B(T, 32 + i, 63 - i, 63 - 4 * brev(4, i), 0, r, err);
+            for (int i = 0; i < 16; i++) B(T, 32 + i, 63 - i, 63 - 4 * brev(4, i), 0, sp);
         }
         if (n >= 5) {
 #pragma unroll
-            for (int i = 0; i < 8; i++) B(T, 16 + i, 31 - i, 6 + (brev(3, 7 - i) << 3), 0, r, err);
+            for (int i = 0; i < 8; i++) B(T, 16 + i, 31 - i, 6 + (brev(3, 7 - i) << 3), 0, sp);
         }
         if (n == 6) {
 #pragma unroll
@@ -284,7 +299,7 @@ struct Inv {
         }
         if (n >= 4) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) B(T, 8 + i, 15 - i, 12 + (brev(2, 3 - i) << 4), 0, r, err);
+            for (int i = 0; i < 4; i++) B(T, 8 + i, 15 - i, 12 + (brev(2, 3 - i) << 4), 0, sp);
         }
         if (n >= 5) {
 #pragma unroll
@@ -294,11 +309,11 @@ struct Inv {
 #pragma unroll
             for (int i = 0; i < 4; i++)
 #pragma unroll
-                for (int j = 0; j < 2; j++) B(T, 62 - i * 4 - j, 33 + i * 4 + j, 60 - 16 * brev(2, i) + 64 * j, 1, r, err);
+                for (int j = 0; j < 2; j++) B(T, 62 - i * 4 - j, 33 + i * 4 + j, 60 - 16 * brev(2, i) + 64 * j, 1, sp);
         }
         if (n >= 3) {
 #pragma unroll
-            for (int i = 0; i < 2; i++) B(T, 4 + i, 7 - i, 56 - 32 * i, 0, r, err);
+            for (int i = 0; i < 2; i++) B(T, 4 + i, 7 - i, 56 - 32 * i, 0, sp);
         }
         if (n >= 4) {
 #pragma unroll
@@ -308,7 +323,7 @@ struct Inv {
 #pragma unroll
             for (int i = 0; i < 2; i++)
 #pragma unroll
-                for (int j = 0; j < 2; j++) B(T, 30 - 4 * i - j, 17 + 4 * i + j, 24 + (j << 6) + ((1 - i) << 5), 1, r, err);
+                for (int j = 0; j < 2; j++) B(T, 30 - 4 * i - j, 17 + 4 * i + j, 24 + (j << 6) + ((1 - i) << 5), 1, sp);
         }
         if (n == 6) {
 #pragma unroll
@@ -317,14 +332,14 @@ struct Inv {
                 for (int j = 0; j < 2; j++) H(T, 32 + i * 4 + j, 35 + i * 4 - j, i & 1, r);
         }
 #pragma unroll
-        for (int i = 0; i < 2; i++) B(T, 2 * i, 2 * i + 1, 32 + 16 * i, 1 - i, r, err);
+        for (int i = 0; i < 2; i++) B(T, 2 * i, 2 * i + 1, 32 + 16 * i, 1 - i, sp);
         if (n >= 3) {
 #pragma unroll
             for (int i = 0; i < 2; i++) H(T, 4 + 2 * i, 5 + 2 * i, i, r);
         }
         if (n >= 4) {
 #pragma unroll
-            for (int i = 0; i < 2; i++) B(T, 14 - i, 9 + i, 48 + 64 * i, 1, r, err);
+            for (int i = 0; i < 2; i++) B(T, 14 - i, 9 + i, 48 + 64 * i, 1, sp);
         }
         if (n >= 5) {
 #pragma unroll
@@ -336,11 +351,11 @@ struct Inv {
 #pragma unroll
             for (int i = 0; i < 2; i++)
 #pragma unroll
-                for (int j = 0; j < 4; j++) B(T, 61 - i * 8 - j, 34 + i * 8 + j, 56 - i * 32 + (j >> 1) * 64, 1, r, err);
+                for (int j = 0; j < 4; j++) B(T, 61 - i * 8 - j, 34 + i * 8 + j, 56 - i * 32 + (j >> 1) * 64, 1, sp);
         }
 #pragma unroll
         for (int i = 0; i < 2; i++) H(T, i, 3 - i, 0, r);
-        if (n >= 3) B(T, 6, 5, 32, 1, r, err);
+        if (n >= 3) B(T, 6, 5, 32, 1, sp);
         if (n >= 4) {
 #pragma unroll
             for (int i = 0; i < 2; i++)
@@ -349,7 +364,7 @@ struct Inv {
         }
         if (n >= 5) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) B(T, 29 - i, 18 + i, 48 + (i >> 1) * 64, 1, r, err);
+            for (int i = 0; i < 4; i++) B(T, 29 - i, 18 + i, 48 + (i >> 1) * 64, 1, sp);
         }
         if (n == 6) {
 #pragma unroll
@@ -363,7 +378,7 @@ struct Inv {
         }
         if (n >= 4) {
 #pragma unroll
-            for (int i = 0; i < 2; i++) B(T, 13 - i, 10 + i, 32, 1, r, err);
+            for (int i = 0; i < 2; i++) B(T, 13 - i, 10 + i, 32, 1, sp);
         }
         if (n >= 5) {
 #pragma unroll
@@ -373,7 +388,7 @@ struct Inv {
         }
         if (n == 6) {
 #pragma unroll
-            for (int i = 0; i < 8; i++) B(T, 59 - i, 36 + i, i < 4 ? 48 : 112, 1, r, err);
+            for (int i = 0; i < 8; i++) B(T, 59 - i, 36 + i, i < 4 ? 48 : 112, 1, sp);
         }
         if (n >= 4) {
 #pragma unroll
@@ -381,7 +396,7 @@ struct Inv {
         }
         if (n >= 5) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) B(T, 27 - i, 20 + i, 32, 1, r, err);
+            for (int i = 0; i < 4; i++) B(T, 27 - i, 20 + i, 32, 1, sp);
         }
         if (n == 6) {
 #pragma unroll
@@ -393,10 +408,11 @@ struct Inv {
         }
         if (n == 6) {
 #pragma unroll
-            for (int i = 0; i < 8; i++) B(T, 55 - i, 40 + i, 32, 1, r, err);
+            for (int i = 0; i < 8; i++) B(T, 55 - i, 40 + i, 32, 1, sp);
 #pragma unroll
             for (int i = 0; i < 32; i++) H(T, i, 63 - i, 0, r);
         }
+        err |= outside(sp, r);
     }
     template <int n> static AV1M_HD void adst_in(int32_t *T) {
         constexpr int n0 = 1 << n;
@@ -437,29 +453,32 @@ struct Inv {
         T[0] = rnd12(x0); T[1] = rnd12(x1); T[2] = rnd12(x2); T[3] = rnd12(x3);
     }
     static AV1M_HD void adst8(int32_t *T, int r, uint32_t &err) {
+        Span sp;
         adst_in<3>(T);
 #pragma unroll
-        for (int i = 0; i < 4; i++) B(T, 2 * i, 2 * i + 1, 60 - 16 * i, 1, r, err);
+        for (int i = 0; i < 4; i++) B(T, 2 * i, 2 * i + 1, 60 - 16 * i, 1, sp);
 #pragma unroll
         for (int i = 0; i < 4; i++) H(T, i, 4 + i, 0, r);
 #pragma unroll
-        for (int i = 0; i < 2; i++) B(T, 4 + 3 * i, 5 + i, 48 - 32 * i, 1, r, err);
+        for (int i = 0; i < 2; i++) B(T, 4 + 3 * i, 5 + i, 48 - 32 * i, 1, sp);
 #pragma unroll
         for (int i = 0; i < 2; i++)
 #pragma unroll
             for (int j = 0; j < 2; j++) H(T, 4 * j + i, 2 + 4 * j + i, 0, r);
 #pragma unroll
-        for (int i = 0; i < 2; i++) B(T, 2 + 4 * i, 3 + 4 * i, 32, 1, r, err);
+        for (int i = 0; i < 2; i++) B(T, 2 + 4 * i, 3 + 4 * i, 32, 1, sp);
+        err |= outside(sp, r);
         adst_out<3>(T);
     }
     static AV1M_HD void adst16(int32_t *T, int r, uint32_t &err) {
+        Span sp;
         adst_in<4>(T);
 #pragma unroll
-        for (int i = 0; i < 8; i++) B(T, 2 * i, 2 * i + 1, 62 - 8 * i, 1, r, err);
+        for (int i = 0; i < 8; i++) B(T, 2 * i, 2 * i + 1, 62 - 8 * i, 1, sp);
 #pragma unroll
         for (int i = 0; i < 8; i++) H(T, i, 8 + i, 0, r);
 #pragma unroll
-        for (int i = 0; i < 2; i++) { B(T, 8 + 2 * i, 9 + 2 * i, 56 - 32 * i, 1, r, err); B(T, 13 + 2 * i, 12 + 2 * i, 8 + 32 * i, 1, r, err); }
+        for (int i = 0; i < 2; i++) { B(T, 8 + 2 * i, 9 + 2 * i, 56 - 32 * i, 1, sp); B(T, 13 + 2 * i, 12 + 2 * i, 8 + 32 * i, 1, sp); }
 #pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -467,21 +486,22 @@ struct Inv {
 #pragma unroll
         for (int i = 0; i < 2; i++)
 #pragma unroll
-            for (int j = 0; j < 2; j++) B(T, 4 + 8 * j + 3 * i, 5 + 8 * j + i, 48 - 32 * i, 1, r, err);
+            for (int j = 0; j < 2; j++) B(T, 4 + 8 * j + 3 * i, 5 + 8 * j + i, 48 - 32 * i, 1, sp);
 #pragma unroll
         for (int i = 0; i < 2; i++)
 #pragma unroll
             for (int j = 0; j < 4; j++) H(T, 4 * j + i, 2 + 4 * j + i, 0, r);
 #pragma unroll
-        for (int i = 0; i < 4; i++) B(T, 2 + 4 * i, 3 + 4 * i, 32, 1, r, err);
+        for (int i = 0; i < 4; i++) B(T, 2 + 4 * i, 3 + 4 * i, 32, 1, sp);
+        err |= outside(sp, r);
         adst_out<4>(T);
     }
     template <int n> static AV1M_HD void idt(int32_t *T) {
 #pragma unroll
         for (int i = 0; i < (1 << n); i++) {
-            if (n == 2) T[i] = rnd12(mul(T[i], 5793));
+            if (n == 2) T[i] = rnd12(mul24(T[i], 5793));
             else if (n == 3) T[i] = mul(T[i], 2);
-            else if (n == 4) T[i] = rnd12(mul(T[i], 11586));
+            else if (n == 4) T[i] = rnd12(mul24(T[i], 11586));
             else T[i] = mul(T[i], 4);
         }
     }
