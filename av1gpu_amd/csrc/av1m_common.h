@@ -63,7 +63,6 @@ inline constexpr uint8_t Part_Order[10] = {PARTITION_SPLIT, PARTITION_NONE, PART
 
 AV1M_HD int clip3(int lo, int hi, int x) { return x < lo ? lo : x > hi ? hi : x; }
 AV1M_HD int round2(int x, int n) { return n == 0 ? x : (x + (1 << (n - 1))) >> n; }
-AV1M_HD int64_t round2l(int64_t x, int n) { return n == 0 ? x : (x + ((int64_t)1 << (n - 1))) >> n; }
 AV1M_HD int round2signed(int x, int n) { return x >= 0 ? round2(x, n) : -round2(-x, n); }
 AV1M_HD int bw4(int bs) { return av1t::Num_4x4_Blocks_Wide[bs]; }
 AV1M_HD int square_bsize(int n) { return n == 8 ? BLOCK_8X8 : n == 16 ? BLOCK_16X16 : n == 32 ? BLOCK_32X32 : BLOCK_64X64; }

@@ -118,6 +118,16 @@ struct EvalOut { float D, R; int eob; };
 
 __device__ __forceinline__ int txsz_ctx(int t) { return (av1t::Tx_Size_Sqr[t] + av1t::Tx_Size_Sqr_Up[t] + 1) >> 1; }
 
+// Indexes of the cost tables' entries of a transform-size context, tx size or plane kind: a table that holds one of them
+// only (the analysis's LDS copy) has its own overloads that return 0.
+template <typename CT> __device__ __forceinline__ int cost_i(const CT &, int i) { return i; }
+// the eob position bits of an area class ms (16 << ms coefficients)
+template <int MS, typename CT>
+__device__ __forceinline__ float eob_pt_bits(const CT &C, int pt, int ec, int i) {
+    return MS == 0 ? C.eob_pt16[pt][ec][i] : MS == 1 ? C.eob_pt32[pt][ec][i] : MS == 2 ? C.eob_pt64[pt][ec][i] : MS == 3 ? C.eob_pt128[pt][ec][i]
+         : MS == 4 ? C.eob_pt256[pt][ec][i] : MS == 5 ? C.eob_pt512[pt][i] : C.eob_pt1024[pt][i];
+}
+
 // txb_skip, luma tx type and eob position bits of a tx block of size TSZ (no branch per lane: the terms that do not apply
 // are read at clamped positions and dropped)
 template <int TSZ, typename E>
@@ -125,32 +135,30 @@ __device__ __forceinline__ float base_bits(const E &e, int eob) {
     const auto &C = *e.C;
     constexpr int t = TSZ, ctx = txsz_ctx_of(t);
     const int pt = e.plane > 0;
-    const float skip = C.txb_skip[ctx][e.skipCtx][eob == 0 ? 1 : 0];
+    const float skip = C.txb_skip[cost_i(C, ctx)][e.skipCtx][eob == 0 ? 1 : 0];
     float b = skip;
     constexpr int set = tx_set_intra(t), sqr = av1t::Tx_Size_Sqr[t];
     if constexpr (set == TX_SET_INTRA_1) {
         int idx = 0;
 #pragma unroll
         for (int i = 0; i < 7; i++) idx = av1t::Tx_Type_Intra_Inv_Set1[i] == e.txType ? i : idx;
-        const float x = C.tx_set1[sqr][e.intraDir][idx];
+        const float x = C.tx_set1[cost_i(C, sqr)][e.intraDir][idx];
         b += pt ? 0.f : x;
     } else if constexpr (set == TX_SET_INTRA_2) {
         int idx = 0;
 #pragma unroll
         for (int i = 0; i < 5; i++) idx = av1t::Tx_Type_Intra_Inv_Set2[i] == e.txType ? i : idx;
-        const float x = C.tx_set2[sqr][e.intraDir][idx];
+        const float x = C.tx_set2[cost_i(C, sqr)][e.intraDir][idx];
         b += pt ? 0.f : x;
     }
     constexpr int lw = av1t::Tx_Width_Log2[t], lh = av1t::Tx_Height_Log2[t];
     constexpr int ms = (lw < 5 ? lw : 5) + (lh < 5 ? lh : 5) - 4;
     const int eobPt = eob <= 2 ? max(eob, 1) : 2 + (31 - __clz(eob - 1));
     const int ec = tx_class(e.txType) == TX_CLASS_2D ? 0 : 1;
-    const float p = ms == 0 ? C.eob_pt16[pt][ec][eobPt - 1] : ms == 1 ? C.eob_pt32[pt][ec][eobPt - 1]
-                  : ms == 2 ? C.eob_pt64[pt][ec][eobPt - 1] : ms == 3 ? C.eob_pt128[pt][ec][eobPt - 1]
-                  : ms == 4 ? C.eob_pt256[pt][ec][eobPt - 1] : ms == 5 ? C.eob_pt512[pt][eobPt - 1] : C.eob_pt1024[pt][eobPt - 1];
+    const float p = eob_pt_bits<ms>(C, pt, ec, eobPt - 1);
     b += p;
     const int x = max(eobPt - 3, 0), rem = eob - ((1 << (x + 1)) + 1);
-    const float ex = C.eob_extra[ctx][pt][x][(rem >> x) & 1];
+    const float ex = C.eob_extra[cost_i(C, ctx)][cost_i(C, pt)][x][(rem >> x) & 1];
     b += eobPt >= 3 ? ex : 0.f;
     b += (float)x;
     return eob == 0 ? skip : b;
@@ -191,7 +199,7 @@ __device__ __forceinline__ CoefIn coef_in(QP q, const E &e, int sk) {
     static_assert(av1t::Sig_Ref_Diff_Offset[0][2][0] == 1 && av1t::Sig_Ref_Diff_Offset[1][2][1] == 2 && av1t::Sig_Ref_Diff_Offset[2][4][0] == 4,
                   "neighbour order: right, below, then the class's own three");
     return CoefIn{sk, sk == 0 ? S + 1 : sk == 1 ? 2 : 2 * S, sk == 0 ? 2 : sk == 1 ? 3 : 3 * S, sk == 1 ? 4 : sk == 0 ? 2 * S : 4 * S,
-                  (&(*e.C).dc_sign[e.plane > 0][e.dcCtx][0])[q[0] < 0]};
+                  (&(*e.C).dc_sign[cost_i(*e.C, e.plane > 0)][e.dcCtx][0])[q[0] < 0]};
 }
 
 // Bits of the coefficient at scan position c (< eob) of a tx block of size TSZ given its magnitudes lv and levels q (natural
@@ -225,13 +233,13 @@ __device__ __forceinline__ float coeff_bits(int c, int eob, const CoefIn &in, LV
         bctx = sk == 0 ? bctx : m + 26 + 5 * min(sk == 1 ? col : row, 2);
     }
     const int ectx = c == 0 ? 0 : c <= (height << bwl) / 8 ? 1 : c <= (height << bwl) / 4 ? 2 : 3;
-    const auto *pb = c == eob - 1 ? &C.coeff_base_eob[ctx][pt][ectx][min(max(level, 1), 3) - 1] : &C.coeff_base[ctx][pt][bctx][min(level, 3)];
+    const auto *pb = c == eob - 1 ? &C.coeff_base_eob[cost_i(C, ctx)][cost_i(C, pt)][ectx][min(max(level, 1), 3) - 1] : &C.coeff_base[cost_i(C, ctx)][cost_i(C, pt)][bctx][min(level, 3)];
     float b = *pb, golomb = 0.f;
     if (level > 2) {
         const int mb = min((a0 + a1 + a2 + 1) >> 1, 6);
         bool near0 = row < 2 && col < 2;
         if constexpr (!only2d) near0 = sk == 0 ? near0 : sk == 1 ? col == 0 : row == 0;
-        const auto *br = C.coeff_br[min(ctx, (int)TX_32X32)][pt][pos == 0 ? mb : near0 ? mb + 7 : mb + 14];
+        const auto *br = C.coeff_br[cost_i(C, min(ctx, (int)TX_32X32))][cost_i(C, pt)][pos == 0 ? mb : near0 ? mb + 7 : mb + 14];
         // up to four symbols of at most 3: n3 full ones, then the rest
         const int rem = level - 3, n3 = (rem * 11) >> 5;   // rem / 3 for 0 .. 12
         const float full = br[3], rest = br[rem - 3 * n3];
@@ -320,7 +328,7 @@ __device__ EvalOut grp_eval(RP res, FP tmp, QP q, const E &e, const TT &T, LV lv
         constexpr int ORF = TW * TH / GW, OR = ORF < 1 ? 1 : ORF > TW ? TW : ORF, NR = TH * (TW / OR);
         static_assert(NR <= GW, "one row item per lane");
         const auto *FrT = T.fwdT + T.fwdOff[rk][LW];
-        const float scale = T.txScale[e.txSz];
+        const float scale = T.txScale[cost_i(T, e.txSz)];
         const int i = lane % TH, o0 = (lane / TH) * OR;
         auto *row = tmp + i * TS;
         float acc[OR];
@@ -413,7 +421,7 @@ __device__ __forceinline__ EvalOut grp_qrate(FP tmp, int ts, QP q, const E &e, c
     int eob;
     EvalOut o;
     grp_rate<TSZ>(lv, q, dscan, cbOff, e, sk, last, eob, o.R);
-    const float g = T.txg[e.txSz][e.txType];
+    const float g = T.txg[cost_i(T, e.txSz)][e.txType];
     o.D = g * distS;
     o.eob = eob;
     return o;
@@ -490,7 +498,7 @@ __device__ EvalOut half_qrate(FP tmp, int ts, QP q, const E &e, const TT &T) {
     }
     EvalOut o;
     o.R = hsum2(b0, b1);
-    o.D = T.txg[e.txSz][e.txType] * distS;
+    o.D = T.txg[cost_i(T, e.txSz)][e.txType] * distS;
     o.eob = eob;
     return o;
 }
@@ -532,7 +540,7 @@ __device__ EvalOut half_eval(RP res, FP tmp, QP q, const E &e, const TT &T) {
         constexpr int ORF = TW * TH / 16, OR = ORF < 1 ? 1 : ORF > TW ? TW : ORF, NR = TH * (TW / OR);
         static_assert(NR <= 16, "one row item per lane");
         const auto *FrT = T.fwdT + T.fwdOff[rk][LW];
-        const float scale = T.txScale[e.txSz];
+        const float scale = T.txScale[cost_i(T, e.txSz)];
         const int i = lane % TH, o0 = (lane / TH) * OR;
         auto *row = tmp + i * TS;
         float acc[OR];
@@ -783,7 +791,7 @@ __device__ __forceinline__ EvalOut wave_qrate(FP tmp, int ts, QP q, const E &e, 
     }
     EvalOut o;
     o.R = gsum(bits);
-    const float g = T.txg[e.txSz][e.txType];
+    const float g = T.txg[cost_i(T, e.txSz)][e.txType];
     o.D = g * distS;
     if constexpr (E64) {
         const float keptS = gsum(halves(kept).hi);

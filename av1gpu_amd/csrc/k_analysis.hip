@@ -55,8 +55,94 @@ struct AnScr {
     int cand[32];
 };
 
-// threads of a workgroup and blocks it takes at a time: 8 groups of 32 lanes, or 4 waves for the shapes of a wave per block
+// threads of a workgroup: 8 groups of 32 lanes, or 4 waves for the shapes of a wave per block
 constexpr int AN_NT = 256;
+
+// What an evaluation of a luma tx block of up to 16x16 reads in chains (scan -> magnitudes -> context -> cost), in LDS: the
+// matrices and scans of its size and, for the four quantizer contexts a batch may mix, the costs of its size's contexts.
+// From the device tables each of these was a 64-lane gather through the vector cache at a 64-bit address, whose registers
+// spilled besides.  Analysis of a 12 MP image searched in full 23.7 -> 22.0 ms, of 16 of them, learned, 69.6 -> 64.5 ms.
+struct AnCost {   // members as in CostTab, with one entry per transform-size context, tx size and plane kind
+    float angle_delta[8][7];
+    float txb_skip[1][1][2];
+    float tx_set1[1][13][7], tx_set2[1][13][5];
+    float eob_pt[2][9];
+    float eob_extra[1][1][9][2];
+    float dc_sign[1][1][2];
+    float coeff_base_eob[1][1][4][3], coeff_base[1][1][42][4], coeff_br[1][1][21][4];
+};
+template <int W, int H>
+struct AnTabs {
+    static constexpr int TSZ = tx_of(W, H), NF = W == H ? W * W : W * W + H * H;
+    float fwdT[3 * NF];
+    int fwdOff[3][7];
+    float txScale[1], txg[1][16];
+    uint8_t scan8[W * H], iscan8[W * H], cbOff[25];
+    AnCost cost[4];
+};
+struct AnNoTabs {};
+__device__ __forceinline__ int cost_i(const lds<AnCost> &, int) { return 0; }
+template <int W, int H> __device__ __forceinline__ int cost_i(const lds<AnTabs<W, H>> &, int) { return 0; }
+template <int MS> __device__ __forceinline__ float eob_pt_bits(const lds<AnCost> &C, int, int ec, int i) { return C.eob_pt[ec][i]; }
+template <int TSZ, int W, int H> __device__ __forceinline__ const lds<uint8_t> *dscan_ptr(const lds<AnTabs<W, H>> &T) { return T.scan8; }
+template <int TSZ, int W, int H> __device__ __forceinline__ const lds<uint8_t> *iscan_ptr(const lds<AnTabs<W, H>> &T) { return T.iscan8; }
+template <int TSZ, int W, int H> __device__ __forceinline__ const lds<uint8_t> *cboff_ptr(const lds<AnTabs<W, H>> &T) { return T.cbOff; }
+
+template <int W, int H>
+__device__ __forceinline__ void an_stage(lds<AnTabs<W, H>> &D, const DevTables &T, int tid) {
+    using A = AnTabs<W, H>;
+    constexpr int TSZ = A::TSZ, ctx = txsz_ctx_of(TSZ), sqr = av1t::Tx_Size_Sqr[TSZ], N = W * H, ms = (N == 16 ? 0 : N == 32 ? 1 : N == 64 ? 2 : N == 128 ? 3 : 4);
+    constexpr int LW = W == 4 ? 2 : W == 8 ? 3 : 4, LH = H == 4 ? 2 : H == 8 ? 3 : 4, NM = (3 * A::NF + AN_NT - 1) / AN_NT;
+    const glb<DevTables> &G = *(const glb<DevTables> *)&T;
+    // every load before the first store: a workgroup whose blocks are all pruned does nothing else
+    float m[NM], c[4][9];
+    int8_t sc = 0, isc = 0;
+#pragma unroll
+    for (int i = 0; i < NM; i++) {
+        const int k = min(tid + AN_NT * i, 3 * A::NF - 1), kind = k / A::NF, r = k % A::NF;
+        m[i] = G.fwdT[r < W * W ? G.fwdOff[kind][LW] + r : G.fwdOff[kind][LH] + r - W * W];
+    }
+    if (tid < N) { sc = (int8_t)G.scan8[scan8_off(TSZ) + tid]; isc = (int8_t)G.iscan8[scan8_off(TSZ) + tid]; }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const glb<CostTab> &S = G.cost[q];
+        auto at = [&](const glb<float> *p, int n) { return p[min(tid, n - 1)]; };
+        c[q][0] = at(&S.angle_delta[0][0], 56);
+        c[q][1] = at(&S.txb_skip[ctx][0][0], 2);
+        c[q][2] = tx_set_intra(TSZ) == TX_SET_INTRA_1 ? at(&S.tx_set1[sqr][0][0], 91) : at(&S.tx_set2[sqr][0][0], 65);
+        c[q][3] = at(ms == 0 ? &S.eob_pt16[0][0][0] : ms == 1 ? &S.eob_pt32[0][0][0] : ms == 2 ? &S.eob_pt64[0][0][0] : ms == 3 ? &S.eob_pt128[0][0][0] : &S.eob_pt256[0][0][0], 2 * (5 + ms));
+        c[q][4] = at(&S.eob_extra[ctx][0][0][0], 18);
+        c[q][5] = at(&S.dc_sign[0][0][0], 2);
+        c[q][6] = at(&S.coeff_base_eob[ctx][0][0][0], 12);
+        c[q][7] = at(&S.coeff_base[ctx][0][0][0], 168);
+        c[q][8] = at(&S.coeff_br[ctx < TX_32X32 ? ctx : TX_32X32][0][0][0], 84);
+    }
+    const float tg = G.txg[TSZ][tid & 15], ts = G.txScale[TSZ];
+    const uint8_t cb = (&av1t::Coeff_Base_Ctx_Offset[TSZ][0][0])[min(tid, 24)];
+#pragma unroll
+    for (int i = 0; i < NM; i++) if (tid + AN_NT * i < 3 * A::NF) D.fwdT[tid + AN_NT * i] = m[i];
+    if (tid < N) { D.scan8[tid] = (uint8_t)sc; D.iscan8[tid] = (uint8_t)isc; }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        lds<AnCost> &C = D.cost[q];
+        if (tid < 56) (&C.angle_delta[0][0])[tid] = c[q][0];
+        if (tid < 2) (&C.txb_skip[0][0][0])[tid] = c[q][1];
+        if (tx_set_intra(TSZ) == TX_SET_INTRA_1 ? tid < 91 : tid < 65)
+            (tx_set_intra(TSZ) == TX_SET_INTRA_1 ? &C.tx_set1[0][0][0] : &C.tx_set2[0][0][0])[tid] = c[q][2];
+        if (tid < 2 * (5 + ms)) C.eob_pt[tid / (5 + ms)][tid % (5 + ms)] = c[q][3];
+        if (tid < 18) (&C.eob_extra[0][0][0][0])[tid] = c[q][4];
+        if (tid < 2) (&C.dc_sign[0][0][0])[tid] = c[q][5];
+        if (tid < 12) (&C.coeff_base_eob[0][0][0][0])[tid] = c[q][6];
+        if (tid < 168) (&C.coeff_base[0][0][0][0])[tid] = c[q][7];
+        if (tid < 84) (&C.coeff_br[0][0][0][0])[tid] = c[q][8];
+    }
+    if (tid < 3) { D.fwdOff[tid][LW] = tid * A::NF; if (W != H) D.fwdOff[tid][LH] = tid * A::NF + W * W; }
+    if (tid == 0) D.txScale[0] = ts;
+    if (tid < 16) D.txg[0][tid] = tg;
+    if (tid < 25) D.cbOff[tid] = cb;
+}
+
+// blocks a workgroup takes at a time
 constexpr int an_groups(int W, int H) { return W >= 32 || H >= 32 ? AN_NT / 64 : AN_NT / 32; }
 
 struct TileBox { int x0, y0, x1, y1; };
@@ -106,6 +192,18 @@ __global__ void __launch_bounds__(AN_NT) __attribute__((amdgpu_waves_per_eu(an_w
     AnScr<W, H> &S = sm[blk];
     const DevTables &T = *B.T;
     const int lane = glane();
+    __shared__ std::conditional_t<WAVE, AnNoTabs, AnTabs<W, H>> tabMem;
+    using Tab = std::conditional_t<WAVE, const DevTables, const lds<std::conditional_t<WAVE, AnNoTabs, AnTabs<W, H>>>>;
+    using Cost = std::conditional_t<WAVE, const CostTab, const lds<AnCost>>;
+    Tab *tp;
+    if constexpr (WAVE) tp = &T;
+    else {
+        auto *d = (lds<AnTabs<W, H>> *)(lds<char> *)(char *)&tabMem;
+        an_stage<W, H>(*d, T, threadIdx.x);
+        __syncthreads();
+        tp = d;
+    }
+    Tab &TL = *tp;
     const uint32_t *starts = B.shStart + (size_t)BS * (B.nimg + 1);
     const int set = tx_set_intra(TXS);
     // a block list (k_an_blank has set every record of the shape to "not analysed"): the groups take its entries
@@ -163,7 +261,7 @@ __global__ void __launch_bounds__(AN_NT) __attribute__((amdgpu_waves_per_eu(an_w
         const Px *plane = (const Px *)I.src[0];
         const Px *src = plane + (size_t)y * sp + x;
         const float lambda = T.lambda[bd == 10][I.qindex] * P.lambdaMul, lamS = P.satdLambda * T.lamS[bd == 10][I.qindex];
-        const CostTab &C = T.cost[I.qctx];
+        Cost &C = TL.cost[I.qctx];
         uint16_t *A = S.ea + EDGE_OFF, *L = S.el + EDGE_OFF;
         grp_build_edges(plane, sp, x, y, LW, LH, haveL, haveA, haveAR, haveBL, maxX, maxY, A, L, bd);
         const int dcv = grp_dc_value(A, L, haveL, haveA, LW, LH, bd);
@@ -353,7 +451,7 @@ __global__ void __launch_bounds__(AN_NT) __attribute__((amdgpu_waves_per_eu(an_w
         // ---- RD of the top-K (DCT_DCT), then the tx types of the set for the winner ----
         const int hasC = has_chroma(BS, y >> 2, x >> 2, I.mono, I.ss);
         const float overhead = (hasC ? P.uvOverheadBits : 0.f) + T.avgSkip0;
-        EvalIn e;
+        EvalInT<Cost *> e;
         e.txSz = TXS; e.plane = 0; e.dcQ = dc_q(I.qindex, bd); e.acQ = ac_q(I.qindex, bd);
         e.dcRcp = 1.f / (float)e.dcQ; e.acRcp = 1.f / (float)e.acQ; e.skipCtx = 0; e.dcCtx = 0;
         e.bd = bd; e.rnd = P.rnd; e.zbin = P.zbin; e.resEnergy = 0.f; e.C = &C; e.intraDir = 0; e.txType = 0;
@@ -398,7 +496,7 @@ __global__ void __launch_bounds__(AN_NT) __attribute__((amdgpu_waves_per_eu(an_w
                 const int k = hf ? k1 : k0, c = S.cand[top[k]];
                 e.txType = hf ? t1 : t0;
                 e.intraDir = cand_mode(c);
-                const EvalOut o = half_eval<W, H>(S.ev.res[k > 2 * (nD - 1) || (r < nD && k > k0) ? 1 : 0], S.ev.tmp[hf], S.ev.q[hf], e, T);
+                const EvalOut o = half_eval<W, H>(S.ev.res[k > 2 * (nD - 1) || (r < nD && k > k0) ? 1 : 0], S.ev.tmp[hf], S.ev.q[hf], e, TL);
                 const float J = fmaf(lambda, (o.R + mbits(c)) + overhead, o.D), Jx = lane_xorf<16>(J);
                 const float J0 = hf ? Jx : J, J1 = hf ? J : Jx;
                 // the lowest J; of equal ones the first candidate and the lowest type
@@ -444,7 +542,7 @@ __global__ void __launch_bounds__(AN_NT) __attribute__((amdgpu_waves_per_eu(an_w
             }
             e.txType = t;
             e.intraDir = m;
-            const EvalOut o = grp_eval<W, H>(S.ev.res, S.ev.tmp, S.ev.q, e, T, S.ev.lv());
+            const EvalOut o = grp_eval<W, H>(S.ev.res, S.ev.tmp, S.ev.q, e, TL, S.ev.lv());
             const float J = fmaf(lambda, (o.R + mbits(c)) + overhead, o.D);
             if (J < bestJ) {
                 bestJ = J;
@@ -485,11 +583,11 @@ __global__ void k_an_blank(BlockRes *blk, uint32_t n) {
 // workgroups of a shape's launch: the kernels loop over the blocks (grid stride), so the grid is capped at
 // AN_WAVES_PER_SLOT times what the device holds at once -- most blocks of the small shapes are pruned by the learned
 // network and take a few instructions each, which one workgroup per 8 blocks spent on workgroup dispatch instead.
-// Measured on MI355X (analysis of the 256-image batch): 908 ms uncapped, 836 / 811 / 771 / 771 / 780 / 798 ms at 2 /
-// 4 / 16 / 32 / 64 / 128 (few workgroups balance the unevenly pruned blocks worse)
-constexpr int AN_WAVES_PER_SLOT = 16;
-// twice that for the shapes that measured faster at 32 (kernel trace of the same batch, every shape at 8 / 16 / 32:
-// 4x4 29.2 -> 27.8 ms, 64x32 55.7 -> 54.6, 64x64 49.4 -> 48.6, 4x8, 8x4, 16x32, 32x64 0.5-0.9 ms each)
+// Measured on MI355X (kernel traces, every shape together): 8 against 16 on 16 images of 12 MP, learned, 64.5 / 66.8 ms, on
+// 24 MP learned 10.03 / 10.30, 12 MP in full 21.99 / 22.26 (a workgroup stages its tables first, so fewer of them pay);
+// without a cap the 256-image batch's analysis took 908 ms against 771 when the cap was introduced.
+constexpr int AN_WAVES_PER_SLOT = 8;
+// twice that for the shapes that measured faster so on the 256-image batch (0.5-1.4 ms each)
 constexpr int an_slot_mult(int W, int H) {
     return (W == 4 && H <= 8) || (W == 8 && H == 4) || (W == 16 && H == 32) || (W == 32 && H == 64) || (W == 64 && H >= 32) ? 2 : 1;
 }
