@@ -361,7 +361,7 @@ __device__ EvalOut grp_eval(RP res, FP tmp, QP q, const E &e, const TT &T, LV lv
 // Quantization, distortion and rate of the coefficients of a W x H tx block held in tmp (row i of the kept tw x th
 // region at tmp + i * ts), levels into q (natural order, tw x th).  All lanes of the group return the same values.
 // lvSep: where the magnitudes go, or null: over the coefficients, which then all pass through registers (where a lane has
-// eight of them and 168 registers that costs 40 in spills: the analysis of 16x16 keeps the two apart, 1.48 -> 1.2 ms on 12 MP).
+// eight of them and 168 registers that costs 40 in spills: the analysis of 16x16 keeps the two apart, 1.48 -> 1.14 ms on 12 MP).
 template <int W, int H, typename FP, typename QP, typename E, typename TT, typename LV>
 __device__ __forceinline__ EvalOut grp_qrate(FP tmp, int ts, QP q, const E &e, const TT &T, LV lvSep) {
     static_assert(W <= 16 && H <= 16, "larger tx blocks: wave_qrate");
