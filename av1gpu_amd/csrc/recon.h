@@ -360,6 +360,18 @@ __device__ __forceinline__ uint32_t inv_col(int j, int W, int ck, int bd, lds<in
     return err;
 }
 
+// The barrier that closes a block, before one wave publishes it (recon_part).  A workgroup barrier by itself does not wait
+// for the waves' stores to global memory (its release is of workgroup scope, which the compute unit's order of
+// accesses provides), and the publisher's agent-scope release waits for its own wave's stores only: another wave's store could
+// reach the L2 after that write-back and a workgroup on another XCD, which sees the progress word, read the old sample.
+// So every wave first waits until its stores have arrived in the L2; the publisher's release then writes them all back.
+// The wait costs 0.7 % of the closed loop of a 512 x 512 image (one launch per step: 27.59 -> 27.75 ms); a release by every
+// wave in its place, a write-back of the L2 each, made the whole encode of 16 images of 12 MP 142 -> 211 ms.
+__device__ __forceinline__ void block_barrier() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+}
+
 // source of plane p in the staging buffer
 __device__ __forceinline__ const lds<uint16_t> *stage_src(const lds<RcShared> &S, int p) { return S.srcb + S.srcAt + (p == 2 ? 2048 : 0); }
 
@@ -602,7 +614,7 @@ __device__ __forceinline__ void wg_finish(lds<RcShared> &S, const Batch &B, cons
         }
         done(eob, tl);
     }
-    __syncthreads();
+    block_barrier();
 }
 
 template <int W, int H, typename Px>
@@ -1310,11 +1322,13 @@ __device__ bool recon_part(lds<RcShared> &S, const Batch &B, uint32_t sb, const 
                 S.nSkip += skip;
                 S.nCfl += cfl;
             }
-            __syncthreads();
+            block_barrier();
         }
         if (ax + aw == 16) ownR = ay + ah;
         if (ay + ah == 16) ownB = ax + aw;
-        if (Q && tid == RC_NT - 64) {   // the last wave, which has the least to do while the next block is set up
+        // the block's stores have all arrived (block_barrier): one lane writes them back and publishes, in the last wave,
+        // which has the least to do while the next block is set up
+        if (Q && tid == RC_NT - 64) {
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
             __hip_atomic_store(prog, ownR | ownB << 8 | (uint32_t)(li + 1) << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
