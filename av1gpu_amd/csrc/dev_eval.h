@@ -175,6 +175,8 @@ __device__ __forceinline__ lds<uint8_t> *lv_of(lds<float> *p) { return (lds<uint
 typedef uint32_t __attribute__((may_alias)) word_a;
 __device__ __forceinline__ void lv_zero(uint8_t *p) { *(word_a *)p = 0; }
 __device__ __forceinline__ void lv_zero(lds<uint8_t> *p) { *(lds<word_a> *)p = 0; }
+// a level's magnitude byte (a rounding offset below -1 makes levels of the other sign)
+__device__ __forceinline__ uint8_t lv_byte(int l) { return (uint8_t)min(max(l, -l), 15); }
 // the margins of a TW x TH block by NL lanes
 template <int TW, int TH, int NL, typename LV>
 __device__ __forceinline__ void lv_margins(LV lv, int lane) {
@@ -405,7 +407,7 @@ __device__ __forceinline__ EvalOut grp_qrate(FP tmp, int ts, QP q, const E &e, c
         const int qv = v < 0 ? -l : l;
         if (N >= GW || lane < N) {
             q[idx] = (int16_t)qv;
-            lv[(idx >> LTW) * lv_stride<TW>() + (idx & (TW - 1))] = (uint8_t)min(l, 15);
+            lv[(idx >> LTW) * lv_stride<TW>() + (idx & (TW - 1))] = lv_byte(l);
         }
         const int c0 = (int)iscan[idx], c = sk == 0 ? c0 : sk == 1 ? (idx & (TW - 1)) * TH + (idx >> LTW) : idx;
         last = max(last, l ? c + 1 : 0);
@@ -472,7 +474,7 @@ __device__ EvalOut half_qrate(FP tmp, int ts, QP q, const E &e, const TT &T) {
         l = min(l, 16383);
         const int qv = v < 0 ? -l : l;
         q[idx] = (int16_t)qv;
-        lv[(idx >> LTW) * lv_stride<TW>() + (idx & (TW - 1))] = (uint8_t)min(l, 15);
+        lv[(idx >> LTW) * lv_stride<TW>() + (idx & (TW - 1))] = lv_byte(l);
         const int c0 = (int)iscan[idx], c = sk == 0 ? c0 : sk == 1 ? (idx & (TW - 1)) * TH + (idx >> LTW) : idx;
         last = max(last, l ? c + 1 : 0);
         const float dq = (float)dequant(qv, step, dsh, e.bd);
@@ -755,7 +757,7 @@ __device__ __forceinline__ EvalOut wave_qrate(FP tmp, int ts, QP q, const E &e, 
         l = min(l, 16383);
         const int qv = x[u] < 0 ? -l : l;
         q[idx] = (int16_t)qv;
-        lv[(idx >> LTW) * lv_stride<TW>() + (idx & (TW - 1))] = (uint8_t)min(l, 15);
+        lv[(idx >> LTW) * lv_stride<TW>() + (idx & (TW - 1))] = lv_byte(l);
         last = max(last, l ? (int)iscan[idx] + 1 : 0);
         const float d = x[u] - (float)dequant(qv, step, dsh, e.bd);
         sq[u] = d * d;
