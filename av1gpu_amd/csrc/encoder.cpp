@@ -739,12 +739,26 @@ static int encode_impl(av1mi_encoder *enc, const av1mi_frame_in *in, int n, av1m
     for (auto &v : steps) { stepOff.push_back((uint32_t)stepFlat.size()); stepFlat.insert(stepFlat.end(), v.begin(), v.end()); }
     stepOff.push_back((uint32_t)stepFlat.size());
     if (stepFlat.size() != nSb) { snprintf(err, errlen, "internal: wavefront order covers %zu of %u superblocks", stepFlat.size(), nSb); return -1; }
+    // ---- schedule knobs: the config's, or the autotuner's for this batch shape ----
+    std::vector<uint64_t> sig = {(uint64_t)n, (uint64_t)bd, (uint64_t)(enc->ln != nullptr), enc->gen, enc->lnChunk};
+    for (int i = 0; i < n; i++)
+        sig.insert(sig.end(), {(uint64_t)imgs[i].W, (uint64_t)imgs[i].H, (uint64_t)imgs[i].aw, (uint64_t)imgs[i].ah, (uint64_t)imgs[i].ss,
+                               (uint64_t)imgs[i].mono});
+    int anS = std::max(1, enc->cfg.anStreams), sched = enc->cfg.schedule, cand = -1, occ = enc->cfg.queueOcc;
+    av1mi_encoder::Tune *tu = nullptr;
+    if (enc->cfg.tune) {
+        tu = &enc->tunes[sig];
+        const int k = tu->next < av1mi_encoder::NTUNE ? (cand = tu->next) : tu->best;
+        anS = (k & 1) ? 4 : 1;
+        sched = (k >> 1) == 2 ? 1 : 0;
+        occ = (k >> 1) == 2 ? 0 : (k >> 1) + 1;
+    }
     // the persistent schedule's items: each superblock's luma, and its chroma (none of monochrome frames)
     uint32_t nItems = nSb;
     for (int i = 0; i < n; i++) if (!imgs[i].mono) nItems += (uint32_t)(imgs[i].sbCols * imgs[i].sbRows);
-    uint32_t *dSteps, *dOrder, *dLnMask = nullptr;
+    uint32_t *dItems, *dLnMask = nullptr;   // the schedule's list: the items, or the superblocks step by step
     PackOff *dPO;
-    A.add(dSteps, stepFlat.size()); A.add(dOrder, nItems); A.add(dPO, nSb);
+    A.add(dItems, sched == 1 ? nSb : nItems); A.add(dPO, nSb);
     // deblocking work units per image (pass 0: each plane's rows x 4-sample columns; pass 1: 4-sample rows x columns)
     uint64_t *dDbStart = nullptr;
     std::vector<uint64_t> dbStart(2 * ((size_t)n + 1), 0);
@@ -770,20 +784,6 @@ static int encode_impl(av1mi_encoder *enc, const av1mi_frame_in *in, int n, av1m
     if (enc->ln) { A.add(dLnMask, (size_t)nSb * 12); A.add(dLnAct, ln_scratch_bytes(lnN)); }
     float *dDpRel = nullptr;
     if (enc->dpExport) A.add(dDpRel, (size_t)nSb * 255);
-    // ---- schedule knobs: the config's, or the autotuner's for this batch shape ----
-    std::vector<uint64_t> sig = {(uint64_t)n, (uint64_t)bd, (uint64_t)(enc->ln != nullptr), enc->gen, enc->lnChunk};
-    for (int i = 0; i < n; i++)
-        sig.insert(sig.end(), {(uint64_t)imgs[i].W, (uint64_t)imgs[i].H, (uint64_t)imgs[i].aw, (uint64_t)imgs[i].ah, (uint64_t)imgs[i].ss,
-                               (uint64_t)imgs[i].mono});
-    int anS = std::max(1, enc->cfg.anStreams), sched = enc->cfg.schedule, cand = -1, occ = enc->cfg.queueOcc;
-    av1mi_encoder::Tune *tu = nullptr;
-    if (enc->cfg.tune) {
-        tu = &enc->tunes[sig];
-        const int k = tu->next < av1mi_encoder::NTUNE ? (cand = tu->next) : tu->best;
-        anS = (k & 1) ? 4 : 1;
-        sched = (k >> 1) == 2 ? 1 : 0;
-        occ = (k >> 1) == 2 ? 0 : (k >> 1) + 1;
-    }
     // closed-loop instance: two workgroups per CU when the batch keeps more superblocks ready per wavefront step than the
     // device has CUs (throughput), else one with the larger register budget (the latency of a superblock chain)
     const int wpe = occ ? occ : (uint64_t)nSb >= (uint64_t)std::max(1, enc->cus) * std::max<size_t>(1, steps.size()) ? 2 : 1;
@@ -793,14 +793,19 @@ static int encode_impl(av1mi_encoder *enc, const av1mi_frame_in *in, int n, av1m
     // block, so an item runs beside its unfinished neighbours, and the lag keeps workgroups from being held by chroma
     // that waits for its luma (16 images of 12 MP, closed loop on MI355X: 94 ms; 105 ms with each superblock's chroma
     // right behind its luma, 116 ms with neighbours complete before an item starts).
-    std::vector<uint32_t> order;
-    order.reserve(nItems);
-    for (size_t k = 0; k <= steps.size(); k++) {
-        if (k < steps.size()) order.insert(order.end(), steps[k].begin(), steps[k].end());
-        if (k)
-            for (uint32_t sb : steps[k - 1])
-                if (!imgs[sbImg[sb]].mono) order.push_back(sb | RC_CHROMA);
-    }
+    // Made only where it is uploaded: not for one launch per step, nor for the replay of a captured plan, which keeps its own.
+    const auto item_list = [&] {
+        if (sched == 1) return stepFlat;
+        std::vector<uint32_t> order;
+        order.reserve(nItems);
+        for (size_t k = 0; k <= steps.size(); k++) {
+            if (k < steps.size()) order.insert(order.end(), steps[k].begin(), steps[k].end());
+            if (k)
+                for (uint32_t sb : steps[k - 1])
+                    if (!imgs[sbImg[sb]].mono) order.push_back(sb | RC_CHROMA);
+        }
+        return order;
+    };
     // ---- device memory: stream-ordered per call, or the captured plan's (graph mode) ----
     bool capture = false;
     const bool graph = enc->cfg.graph && !na;
@@ -879,21 +884,22 @@ static int encode_impl(av1mi_encoder *enc, const av1mi_frame_in *in, int n, av1m
         launch_dp(B, P, s);
         if (events) (void)hipEventRecord(enc->ev[3], s);
         if (sched == 1) {
-            for (size_t k = 0; k + 1 < stepOff.size(); k++) launch_recon(B, P, dSteps + stepOff[k], stepOff[k + 1] - stepOff[k], bd, s);
+            for (size_t k = 0; k + 1 < stepOff.size(); k++) launch_recon(B, P, dItems + stepOff[k], stepOff[k + 1] - stepOff[k], bd, s);
         } else {
             RcQueue Q;
-            Q.order = dOrder; Q.n = nItems; Q.nSb = nSb; Q.head = dQctl; Q.abort = dQctl + 1; Q.prog = dProg;
+            Q.order = dItems; Q.n = nItems; Q.nSb = nSb; Q.head = dQctl; Q.abort = dQctl + 1; Q.prog = dProg;
             Q.spinTicks = enc->clockHz * 30;   // no legitimate wait comes near 30 s
             launch_recon_queue(B, P, Q, std::min<uint32_t>(qBlocks, nItems), bd, wpe, s);
         }
         return hipGetLastError() == hipSuccess ? 0 : -1;
     };
+    std::vector<uint32_t> items;   // held until the call's end: the copy may read it until then
     if (graph) {
         if (capture) {   // shape data once, then the capture
             HCK(hipMemcpy(dShStart, shStart.data(), shStart.size() * 4, hipMemcpyHostToDevice));
             HCK(hipMemcpy(dSbImg, sbImg.data(), (size_t)nSb * 4, hipMemcpyHostToDevice));
-            HCK(hipMemcpy(dSteps, stepFlat.data(), stepFlat.size() * 4, hipMemcpyHostToDevice));
-            HCK(hipMemcpy(dOrder, order.data(), order.size() * 4, hipMemcpyHostToDevice));
+            items = item_list();
+            HCK(hipMemcpy(dItems, items.data(), items.size() * 4, hipMemcpyHostToDevice));
             HCK(hipStreamBeginCapture(enc->cap, hipStreamCaptureModeThreadLocal));
             const int r = device_part(enc->cap, false);
             hipGraph_t g = nullptr;
@@ -917,8 +923,8 @@ static int encode_impl(av1mi_encoder *enc, const av1mi_frame_in *in, int n, av1m
         HCK(hipMemcpyAsync(dImg, imgs.data(), n * sizeof(Img), hipMemcpyHostToDevice, st));
         HCK(hipMemcpyAsync(dShStart, shStart.data(), shStart.size() * 4, hipMemcpyHostToDevice, st));
         HCK(hipMemcpyAsync(dSbImg, sbImg.data(), (size_t)nSb * 4, hipMemcpyHostToDevice, st));
-        if (sched == 1) HCK(hipMemcpyAsync(dSteps, stepFlat.data(), stepFlat.size() * 4, hipMemcpyHostToDevice, st));
-        else HCK(hipMemcpyAsync(dOrder, order.data(), order.size() * 4, hipMemcpyHostToDevice, st));
+        items = item_list();
+        HCK(hipMemcpyAsync(dItems, items.data(), items.size() * 4, hipMemcpyHostToDevice, st));
         if (device_part(st, true)) { snprintf(err, errlen, "HIP: launch failed (%s)", hipGetErrorString(hipGetLastError())); A.release(st); return -1; }
     }
     tm.schedule = (uint32_t)sched;
