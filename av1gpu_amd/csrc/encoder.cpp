@@ -1315,7 +1315,7 @@ size_t av1mi_frame_bytes(int W, int H, int bitDepth, int yuv444) {
     const size_t planes = yuv444 ? aw * ah * bps * 3 : aw * ah * bps * 3 / 2;
     const size_t arena = planes + 5 * mi + 2 * (mi + 2 * c1) + blocks * sizeof(BlockRes) +
                          nSb * (4 + 2 + MAX_LEAVES * sizeof(Leaf) + 4 + sizeof(SbOut) + MAX_LEAVES * (sizeof(RecBlock) + 2) +
-                                txbCap * sizeof(RecTxb) + coefCap * 2 + 4 + sizeof(PackOff) + 4);
+                                txbCap * sizeof(RecTxb) + coefCap * 2 + sizeof(PackOff) + 2 * 4 + 2 * 4);   // progress words, items
     const size_t records = nSb * (MAX_LEAVES * (sizeof(RecBlock) + 4) + txbCap * sizeof(RecTxb) + coefCap * 2);
     const size_t network = nSb * 48 + ln_scratch_bytes((uint32_t)std::min<size_t>(nSb, 65536));   // masks, activations
     return planes + arena + records + network + 64 * 1024;
