@@ -366,7 +366,7 @@ __device__ EvalOut grp_eval(RP res, FP tmp, QP q, const E &e, const TT &T, LV lv
 // eight of them and 168 registers that costs 40 in spills: the analysis of 16x16 keeps the two apart, 1.48 -> 1.14 ms on 12 MP).
 template <int W, int H, typename FP, typename QP, typename E, typename TT, typename LV>
 __device__ __forceinline__ EvalOut grp_qrate(FP tmp, int ts, QP q, const E &e, const TT &T, LV lvSep) {
-    static_assert(W <= 16 && H <= 16, "larger tx blocks: wave_qrate");
+    static_assert(W <= 16 && H <= 16 && W * H >= GW, "larger tx blocks: wave_qrate; smaller ones: half_qrate");
     static_assert((H + 4) * lv_stride<W>() <= H * (W + 1) * 4, "the magnitudes fit in the coefficients' space");
     constexpr int TW = W, TH = H;
     constexpr int LTW = TW == 4 ? 2 : TW == 8 ? 3 : 4;
@@ -381,16 +381,13 @@ __device__ __forceinline__ EvalOut grp_qrate(FP tmp, int ts, QP q, const E &e, c
     const int den = dq_denom(e.txSz), dsh = den == 4 ? 2 : den == 2 ? 1 : 0;
     float dist = 0.f;
     int last = 0;
-    constexpr int NE = (N + GW - 1) / GW;   // per lane; a 4x4 leaves the upper half of the lanes a zero
+    constexpr int NE = N / GW;   // per lane
     constexpr bool SEP = !std::is_same_v<LV, std::nullptr_t>;
-    auto coef = [&](int idx) {
-        const float v = tmp[(idx >> LTW) * ts + (idx & (TW - 1))];
-        return N >= GW || lane < N ? v : 0.f;
-    };
+    auto coef = [&](int idx) -> float { return tmp[(idx >> LTW) * ts + (idx & (TW - 1))]; };
     float x[NE];
     if constexpr (!SEP) {
 #pragma unroll
-        for (int t = 0; t < NE; t++) x[t] = coef(N < GW ? lane & (N - 1) : lane + GW * t);
+        for (int t = 0; t < NE; t++) x[t] = coef(lane + GW * t);
         gsync();
     }
     const auto lv = [&] { if constexpr (SEP) return lvSep; else return lv_of(tmp); }();
@@ -398,17 +395,15 @@ __device__ __forceinline__ EvalOut grp_qrate(FP tmp, int ts, QP q, const E &e, c
     constexpr int UNR = SEP ? 4 : NE;
 #pragma unroll UNR
     for (int t = 0; t < NE; t++) {
-        const int idx = N < GW ? lane & (N - 1) : lane + GW * t;
+        const int idx = lane + GW * t;
         const float v = SEP ? coef(idx) : x[t];
         const int step = idx == 0 ? e.dcQ : e.acQ;
         const float a = quot_step(fabsf(v) * (float)den, (float)step, idx == 0 ? e.dcRcp : e.acRcp);
         int l = a < e.zbin ? 0 : (int)(a + e.rnd);
         l = min(l, 16383);
         const int qv = v < 0 ? -l : l;
-        if (N >= GW || lane < N) {
-            q[idx] = (int16_t)qv;
-            lv[(idx >> LTW) * lv_stride<TW>() + (idx & (TW - 1))] = lv_byte(l);
-        }
+        q[idx] = (int16_t)qv;
+        lv[(idx >> LTW) * lv_stride<TW>() + (idx & (TW - 1))] = lv_byte(l);
         const int c0 = (int)iscan[idx], c = sk == 0 ? c0 : sk == 1 ? (idx & (TW - 1)) * TH + (idx >> LTW) : idx;
         last = max(last, l ? c + 1 : 0);
         const float dq = (float)dequant(qv, step, dsh, e.bd);   // 0 for level 0

@@ -377,7 +377,7 @@ __device__ __forceinline__ const lds<uint16_t> *stage_src(const lds<RcShared> &S
 
 // Inlined into each per-shape leaf function (rc_luma / rc_chroma): as a call of its own it would run on the ~140
 // registers outside the callee-saved ones and spill; inlined, the leaf function's one frame covers it.
-// run S.taskC/T/P[0 .. nTask) on the 8 groups (the source block staged in S.srcb, row stride W); per task
+// run S.taskC/T/P[0 .. nTask) on the RC_NG groups (the source staged in S.srcb, row stride S.srcSp); per task
 // J = fmaf(lambda, R + extra, D) with extra = luma mode bits (plane 0) or 0; S.taskJ / taskE.  Then S.win = the first
 // minimum over the tasks.  Blocks up to 16x16: luma tasks read the residual of their candidate (S.taskK), made by
 // wg_luma_residuals; chroma tasks make their own in slot t; levels of task t go to S.u.s.lev[t].  Larger blocks:
@@ -394,11 +394,10 @@ __device__ __forceinline__ void wg_run_tasks(lds<RcShared> &S, const lds<Img> &I
     }
     const int g = gid(), lane = glane();
     const lds<CostTab> &C = S.tab.cost;
-    // blocks of up to 64 coefficients: 16 half groups, two tasks per group at once; luma residuals are ready, chroma
+    // blocks of up to 64 coefficients: 2 RC_NG half groups, two tasks per group at once; luma residuals are ready, chroma
     // tasks first make theirs (one task per group, as below), then the halves evaluate
-    bool done = false;
-    if constexpr (!big && W * H <= 64) {
-        done = true;
+    constexpr bool halves = !big && W * H <= 64;
+    if constexpr (halves) {
         if (!lumaBits) {
             for (int t = g; t < S.nTask; t += RC_NG)
                 grp_residual<W, H>(S, I.edgeFilter ? S.u.s.g[g].ea : nullptr, S.u.s.g[g].el, S.taskP[t], S.taskC[t], stage_src(S, S.taskP[t]), S.srcSp,
@@ -430,7 +429,7 @@ __device__ __forceinline__ void wg_run_tasks(lds<RcShared> &S, const lds<Img> &I
     constexpr int NGT = big ? RC_NTEAM : RC_NG;
     const int me = big ? (int)(threadIdx.x >> 6) : g;
     const int tFirst = big ? (me < S.nTask ? me + ((S.nTask - 1 - me) / NGT) * NGT : -1) : me, tStep = big ? -NGT : NGT;
-    if (!done) for (int t = tFirst; t >= 0 && t < S.nTask; t += tStep) {
+    if constexpr (!halves) for (int t = tFirst; t >= 0 && t < S.nTask; t += tStep) {
         int c = S.taskC[t], p = S.taskP[t];
         const int tt = S.taskT[t];
         if constexpr (big) { c = __builtin_amdgcn_readfirstlane(c); p = __builtin_amdgcn_readfirstlane(p); }   // the wave's task
