@@ -710,7 +710,7 @@ static int encode_impl(av1mi_encoder *enc, const av1mi_frame_in *in, int n, av1m
         anyCdef = true;
         A.add(cdefMem[i], ((size_t)I.aw * I.ah + 2 * (size_t)(I.aw >> I.ss) * (I.ah >> I.ss)) * bps);
     }
-    // everything so far starts each call at zero (reconstruction, maps, counters, done flags): one fill kernel; the
+    // everything so far starts each call at zero (reconstruction, maps, counters, progress words): one fill kernel; the
     // padding beyond the coded area is never reconstructed, so the returned planes are fully defined
     const size_t zeroBytes = A.total;
     Img *dImg; BlockRes *dBlk; uint32_t *dShStart, *dSbImg; uint16_t *dLeafCount; Leaf *dLeaves; float *dSbJ; SbOut *dSbOut;
@@ -785,7 +785,7 @@ static int encode_impl(av1mi_encoder *enc, const av1mi_frame_in *in, int n, av1m
     float *dDpRel = nullptr;
     if (enc->dpExport) A.add(dDpRel, (size_t)nSb * 255);
     // closed-loop instance: two workgroups per CU when the batch keeps more superblocks ready per wavefront step than the
-    // device has CUs (throughput), else one with the larger register budget (the latency of a superblock chain)
+    // device has CUs (throughput), else one of twice the threads (the latency of a superblock chain)
     const int wpe = occ ? occ : (uint64_t)nSb >= (uint64_t)std::max(1, enc->cus) * std::max<size_t>(1, steps.size()) ? 2 : 1;
     const int slots = enc->slots[bd == 10][wpe - 1] > 0 ? enc->slots[bd == 10][wpe - 1] : 1;
     const uint32_t qBlocks = enc->cfg.queueBlocks > 0 ? (uint32_t)enc->cfg.queueBlocks : (uint32_t)std::max(1, enc->cus * slots);

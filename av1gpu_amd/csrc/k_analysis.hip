@@ -170,11 +170,13 @@ __device__ __forceinline__ int ol_decoded(int px, int py, int x, int y, const Ti
 }
 
 // Occupancy target per shape, in waves per SIMD.  At 4 the compiler keeps a kernel under 128 VGPRs and the extra waves
-// hide the LDS and table latency, which outweighs the spills that costs most small shapes; 8x16, 16x8 and 16x16 spill
-// 150-340 bytes per lane at 4 and run faster with 168 VGPRs, as do the shapes of a wave per block (MI355X, 16 images of 12
-// MP, learned: 64x64 9.7 / 7.3 / 6.9 ms, 64x32 9.3 / 7.9 / 8.4, 32x64 9.7 / 7.6 / 7.6, 32x16 6.4 / 5.1 / 6.0, 16x32 5.6 / 5.0
-// / 6.3 at 2 / 3 / 4; all ten 50.9 / 41.0 / 43.8).  Where LDS allows fewer waves than the target the compiler notes that
-// it cannot reach it; the build silences that.
+// hide the LDS and table latency, which outweighs the spills that costs most small shapes.  The shapes of a wave per block
+// run faster with 168 VGPRs (MI355X, 16 images of 12 MP, learned, at 2 / 3 / 4: 64x64 9.7 / 7.3 / 6.9 ms, 64x32 9.3 / 7.9 /
+// 8.4, 32x64 9.7 / 7.6 / 7.6, 32x16 6.4 / 5.1 / 6.0, 16x32 5.6 / 5.0 / 6.3; all ten 50.9 / 41.0 / 43.8).  8x16, 16x8 and 16x16
+// were given 3 when they read device tables and spilled 150-340 bytes per lane at 4.  With the tables in LDS that holds for
+// 16x16 only: at 3 / 4 on the same images 16x16 6.0 / 6.1 ms, 8x16 6.4 / 5.2, 16x8 7.1 / 6.1; one 12 MP image searched in
+// full 1.22 / 1.33, 1.55 / 1.28, 1.61 / 1.37.  Where LDS allows fewer waves than the target the compiler notes that it cannot
+// reach it; the build silences that.
 constexpr int an_wpe(int W, int H) {
     return W >= 32 || H >= 32 || (W == 8 && H == 16) || (W == 16 && H == 8) || (W == 16 && H == 16) ? 3 : 4;
 }
@@ -299,9 +301,9 @@ __global__ void __launch_bounds__(AN_NT) __attribute__((amdgpu_waves_per_eu(an_w
         const int n13 = __popc(modeMask);
         if (lane < 13 && ((modeMask >> lane) & 1)) S.cand[__popc(modeMask & ((1u << lane) - 1))] = cand_pack(lane, 0);
         gsync();
-        // blocks of up to 8 4x4s: item = (candidate, pixel), 16 lanes per 4x4 and the Hadamard across them, so a
-        // round holds at most two candidates (modes); larger blocks: item = (candidate, 4x4).  A candidate's items are
-        // consecutive, so each segment of up to 32 lanes sums its Hadamard costs with shuffles before one LDS atomic.
+        // blocks of up to 8 4x4s: a lane predicts pixels, 16 lanes per 4x4 and the Hadamard across them, so a round holds
+        // at most two candidates (modes); larger blocks: a lane keeps its 4x4s of the block for every candidate and
+        // predicts each whole.  The lanes of a candidate sum their costs among them before one adds the sum in LDS.
         auto screen = [&](int c0, int c1) {
             constexpr int NSY = NSUB / NSX;
             if constexpr (NSUB >= 4 && NSUB <= 8 && NSY >= 2) {
@@ -583,11 +585,12 @@ __global__ void k_an_blank(BlockRes *blk, uint32_t n) {
 // workgroups of a shape's launch: the kernels loop over the blocks (grid stride), so the grid is capped at
 // AN_WAVES_PER_SLOT times what the device holds at once -- most blocks of the small shapes are pruned by the learned
 // network and take a few instructions each, which one workgroup per 8 blocks spent on workgroup dispatch instead.
-// Measured on MI355X (kernel traces, every shape together): 8 against 16 on 16 images of 12 MP, learned, 64.5 / 66.8 ms, on
-// 24 MP learned 10.03 / 10.30, 12 MP in full 21.99 / 22.26 (a workgroup stages its tables first, so fewer of them pay);
-// without a cap the 256-image batch's analysis took 908 ms against 771 when the cap was introduced.
+// Measured on MI355X (kernel traces) at 8 / 16: 16 images of 12 MP, learned, the shapes up to 16x16 (whose workgroups stage
+// their tables first) 35.2 / 36.6 ms, the shapes of a wave per block 29.8 / 30.6; one 12 MP image in full 15.3 / 15.5 and 6.68 /
+// 6.69.  Without a cap the 256-image batch's analysis took 908 ms against 771 when the cap was introduced.
 constexpr int AN_WAVES_PER_SLOT = 8;
-// twice that for the shapes that measured faster so on the 256-image batch (0.5-1.4 ms each)
+// twice that for these shapes: the 256-image batch's analysis 463.5 ms against 467.5 with 8 for every shape; 16 images of 12 MP
+// 65.0 / 65.0 and one 22.0 / 21.9, where it makes no difference
 constexpr int an_slot_mult(int W, int H) {
     return (W == 4 && H <= 8) || (W == 8 && H == 4) || (W == 16 && H == 32) || (W == 32 && H == 64) || (W == 64 && H >= 32) ? 2 : 1;
 }

@@ -583,7 +583,7 @@ __global__ void __launch_bounds__(256) k_ln_to_bf16(const float *w, bf16_t *bf, 
 // ================================ host side ================================
 
 // parameter layout (FP32 masters): per convolution l = 1..4 the weights [32][KP_l] (taps past 9 Cin are zero) and the
-// bias [32], then the FC weights [98][512] and bias [98]
+// bias [32], then the FC weights [LN_OUT][512] and bias [LN_OUT]
 constexpr int LN_KP1 = 32, LN_KP = 288;
 constexpr size_t LN_W_OFF[4] = {0, 32 * LN_KP1 + 32, 32 * LN_KP1 + 32 + 32 * LN_KP + 32, 32 * LN_KP1 + 32 + 2 * (32 * LN_KP + 32)};
 constexpr size_t LN_FC_OFF = 32 * LN_KP1 + 32 + 3 * (32 * LN_KP + 32);
@@ -755,7 +755,7 @@ int av1mi_ln_get_params(av1mi_learner *L, float *params) {
     return hipMemcpy(params, L->net.w, LN_NPARAM * 4, hipMemcpyDeviceToHost) == hipSuccess ? 0 : -1;
 }
 
-// forward of n 64x64 8-bit luma tiles (host arrays: tiles n x 4096, q n) -> logits (n x 98)
+// forward of n 64x64 8-bit luma tiles (host arrays: tiles n x 4096, q n) -> logits (n x LN_OUT)
 int av1mi_ln_forward(av1mi_learner *L, const uint8_t *tiles, const uint8_t *q, uint32_t n, float *logits) {
     LnNet &N = L->net;
     if (n == 0) return 0;
@@ -780,7 +780,7 @@ int av1mi_ln_activations(av1mi_learner *L, int layer, uint32_t n, uint16_t *out)
     return hipMemcpy(out, src[layer], n * per[layer] * 2, hipMemcpyDeviceToHost) == hipSuccess ? 0 : -1;
 }
 
-// Training data on the device: n tiles (n x 4096 8-bit luma), their qindex, labels and label masks (n x 98 each).
+// Training data on the device: n tiles (n x 4096 8-bit luma), their qindex, labels and label masks (n x LN_OUT each).
 int av1mi_ln_set_data(av1mi_learner *L, const uint8_t *tiles, const uint8_t *q, const float *label, const float *lmask, uint32_t n) {
     LnNet &N = L->net;
     (void)hipFree(N.tiles); (void)hipFree(N.q); (void)hipFree(N.label); (void)hipFree(N.lmask);

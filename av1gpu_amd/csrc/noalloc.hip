@@ -8,7 +8,8 @@
 
 namespace av1m {
 
-// (the last 64 KiB hold the closed loop's item order and progress words: 16 bytes for each of the at most 3.9 k superblocks)
+// the 64 KiB beyond the nominal size: the closed loop's list and progress words take 8 bytes per superblock more than its
+// superblock list and done flags did, and at least 30 KB of arrays per superblock let at most 5.6 k of them in
 constexpr size_t NOALLOC_SCRATCH_BYTES = ((size_t)AV1MI_NOALLOC_SCRATCH_MIB << 20) + (64 << 10);
 
 static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];

@@ -5,11 +5,11 @@
 // 1220-1686 (chroma), 139-197 (inverse + add), 203-238 (contexts), 685-730 (records).
 //
 // What bounds it: the latency of the chain of blocks.  A block's steps depend on each other and on the blocks before it,
-// so a superblock keeps one workgroup's four waves mostly waiting, and an image keeps about one superblock per wavefront
+// so a superblock keeps its workgroup's waves mostly waiting, and an image keeps about one superblock per wavefront
 // column ready.  Two splits shorten the chain: luma needs nothing of chroma, so the two run as separate items beside each
 // other; and progress published per block lets a superblock start beside its unfinished neighbours (recon_part).
-// Closed loop of one 512 x 512 image 48.7 -> 20.2 ms, 24 MP learned 115 -> 54 ms; 16 images of 12 MP 175 -> 119 ms (per
-// superblock there; the smaller items also spill less).
+// When the two came in, the closed loop of one 512 x 512 image went 48.7 -> 20.2 ms, 24 MP learned 115 -> 54 ms, 16 images
+// of 12 MP 175 -> 94 ms; with all that the comments below name they take 10.6, 29 and 66 ms.
 //
 // Per block:
 //   luma    every re-checked analysis candidate x every intra tx type of the set (tx blocks up to 16x16; DCT_DCT only
@@ -55,10 +55,10 @@ struct RcTeam {
 };
 template <typename X> __device__ __forceinline__ lds<int16_t> *team_lev(X &t) { return (lds<int16_t> *)(lds<char> *)t.tmp; }
 // The tables the evaluations and the decisions read, staged once per workgroup (the costs: per quantizer context of the
-// images it meets).  An evaluation reads them in chains (level -> context -> cost) that nothing else hides in one
-// workgroup's four waves.  From the device tables they were about 480 flat loads per wave and block; in LDS the closed loop
-// of a 512 x 512 image went 52.7 -> 48.7 ms, of 16 12 MP images 191 -> 175 ms (two workgroups per CU still fit: the
-// inverse's scratch and the levels share the evaluations' scratch).
+// images it meets).  An evaluation reads them in chains (level -> context -> cost) that nothing else hides in the few
+// waves of one workgroup.  From the device tables they were about 480 flat loads per wave and block; when they moved to LDS,
+// before the other steps named here, the closed loop of a 512 x 512 image went 52.7 -> 48.7 ms, of 16 12 MP images 191 ->
+// 175 ms (two workgroups per CU still fit: the inverse's scratch and the levels share the evaluations' scratch).
 struct RcTabs {
     float fwdT[3 * 336];     // DCT, ADST, identity for n = 4, 8, 16, transposed (offsets fwdOff)
     int fwdOff[3][7];
@@ -365,7 +365,7 @@ __device__ __forceinline__ uint32_t inv_col(int j, int W, int ck, int bd, lds<in
 // accesses provides), and the publisher's agent-scope release waits for its own wave's stores only: another wave's store could
 // reach the L2 after that write-back and a workgroup on another XCD, which sees the progress word, read the old sample.
 // So every wave first waits until its stores have arrived in the L2; the publisher's release then writes them all back.
-// The wait costs 0.7 % of the closed loop of a 512 x 512 image (one launch per step: 27.59 -> 27.75 ms); a release by every
+// The wait costs 0.6 % of the closed loop of a 512 x 512 image (one launch per step: 27.55 -> 27.72 ms); a release by every
 // wave in its place, a write-back of the L2 each, made the whole encode of 16 images of 12 MP 142 -> 211 ms.
 __device__ __forceinline__ void block_barrier() {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -908,9 +908,9 @@ __device__ __noinline__ void rc_chroma(lds<RcShared> &S, const Batch &B, const l
     }
     // ---- SATD screening of the UV candidates over U and V (unfiltered edges) ----
     constexpr int NSUB = (W / 4) * (H / 4), NSX = W / 4;
-    // screening of blocks of up to 16 4x4s: item = (candidate, plane, pixel), 16 lanes per 4x4 and the Hadamard
-    // across them, so a wave holds at most two candidates (modes); larger blocks: item = (candidate, plane, 4x4).  A
-    // candidate's items are consecutive, so each segment of up to 32 lanes sums its costs with shuffles before one LDS
+    // screening of blocks of up to 16 4x4s: item = (candidate, plane, pixel or run of pixels), 16 lanes per 4x4 and the
+    // Hadamard across them, so a wave holds at most two candidates (modes); larger blocks: item = (candidate, plane, 4x4).
+    // A candidate's items are consecutive, so each segment of up to 32 lanes sums its costs across lanes before one LDS
     // atomic.
     auto screen = [&](int c0, int c1) {
         constexpr int NSY = NSUB / NSX;

@@ -193,8 +193,8 @@ void av1mi_dev_records_free(av1mi_dev_records *dev, void *stream);
  * No counterpart in the reference.  For callers that cannot allocate device memory: code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc.  av1mi_encode_noalloc is av1mi_encode_dev with every internal buffer
  * (analysis records, leaves, superblock slots, maps, the pruning network's activations, the unpacked reconstruction) in
- * one file-scope device array of AV1MI_NOALLOC_SCRATCH_MIB MiB per device, reserved with the library's code and held
- * until the process ends; it calls no hipMalloc / hipFree / hipHostMalloc.  The caller passes the outputs: the packed
+ * one file-scope device array of AV1MI_NOALLOC_SCRATCH_MIB MiB and 64 KiB per device, reserved with the library's code and
+ * held until the process ends; it calls no hipMalloc / hipFree / hipHostMalloc.  The caller passes the outputs: the packed
  * records in device buffers (frames back to back in batch order; block_txb each block's first tx block relative to its
  * frame, txb.coeff_off relative to its frame, as av1mi_dev_records), and optionally the reconstruction per frame.
  * out[i] receives the frame's sizes and counts (its pointers stay NULL).  A batch needing more scratch than the array, or
